@@ -22,7 +22,7 @@ struct LevelCounters {
   unsigned long long alive[16];  // batched: OR of the level's frontier words, one
                                  // per 64 lanes (lanes that can still reach new vertices)
   unsigned int qlen;          // queue entries written for this level
-  unsigned int pad;
+  unsigned int hqlen;         // heavy-chunk entries (single-source engines)
 };
 
 constexpr int kRing = 4;          // ring of LevelCounters indexed by level % 4

@@ -8,13 +8,17 @@
 //
 // Layout in HBM (per graph, reused across calls):
 //   dist   int32[n]                      distances (INF = unreached)
-//   q      int32[3][n]                   frontier queue of level l in slot l%3
+//   q      int32[2][n]                   frontier queue of level l in slot l&1:
+//                                        vertices of out-degree <= hchunk
+//   hq     int2[2][hcap]                 (vertex, first edge) of every hchunk-edge
+//                                        chunk of the frontier's other vertices
 //   bm     uint32[3][words]              frontier bitmap of level l in slot l%3
 //   ring   LevelCounters[4]              per-level counters, level l in l%4
 //   state  SchedState                    step / done / mode / rule state
 // Every step writes BOTH the queue and the bitmap of the new level, so the
 // three modes are interchangeable from step to step with no conversion:
-//   PUSH    queue in: workgroup-balanced edge expansion (LDS degree scan)
+//   PUSH    queue in: wave-balanced edge expansion (chunks of the heavy
+//           vertices one wave each, the others 1 to 64 per wave by LDS scan)
 //   PULL    bitmap in: unvisited vertices scan in-edges (CSC) with early exit
 //   BITMAP  bitmap in: dense scan of the frontier bitmap, top-down expansion
 // The step loop is decide(1 wave) + expand(grid), captured K steps at a
@@ -44,8 +48,16 @@ struct SsArgs {
   const int32_t* in_col;
   const int32_t* in_w;
   int32_t* dist;
-  int32_t* q;        // 3 * n
+  int32_t* q;        // 2 * n
+  int2* hq;          // 2 * hcap
+  int64_t hcap;      // >= 2 m / hchunk: every heavy vertex's chunks fit
+  int32_t hchunk;    // edges per heavy chunk; longer lists are cut
+  int32_t heavy;     // degree from which the static chunk lists hold a vertex
   uint32_t* bm;      // 3 * words
+  const int32_t* oc_v;  // static out-edge chunks (BITMAP steps)
+  const int32_t* oc_beg;
+  const int32_t* oc_end;
+  int64_t num_oc;
   LevelCounters* ring;
   unsigned long long* part;  // kRing x kStripes counter stripes
   SchedState* st;
@@ -58,8 +70,16 @@ struct SsArgs {
 constexpr int kStripes = 64;
 constexpr int kStripeU64 = 16;  // 128 bytes per stripe
 constexpr int kPartU64 = kRing * kStripes * kStripeU64;
+// Threads per workgroup of the step kernels, and workgroups per launch (two
+// per CU).  Every workgroup that found something reserves its queue ranges
+// with atomics on one address each, about 12 ns apiece in turn: 4096
+// workgroups of 256 threads spent up to 50 us of a step on them, and an
+// idle launch of 4096 workgroups takes 4.4 us, of 512 less than half.
+constexpr int kSsBlock = 1024;
+constexpr unsigned kSsGrid = 512;
+constexpr int kSsWaves = kSsBlock / kWave;
 // Queue entries a workgroup stages in LDS before reserving global space.
-constexpr int kStageCap = 4096;
+constexpr int kStageCap = 8192;
 // Queue length of a level whose queue was not written (a pull step writes
 // the bitmap only): a top-down step that follows reads the bitmap instead.
 constexpr unsigned kNoQueue = 0xFFFFFFFFu;
@@ -69,6 +89,8 @@ struct SsWorkspace {
   int32_t n = 0;
   int64_t words = 0;
   DevBuf<int32_t> dist, q;
+  DevBuf<int2> hq;
+  int64_t hcap = 0;
   DevBuf<uint32_t> bm;
   DevBuf<LevelCounters> ring;
   DevBuf<unsigned long long> part;
@@ -100,33 +122,36 @@ void ss_workspace_free(SsWorkspace* ws) {
 
 namespace {
 
+// Four columns of an edge list, read by one load at any 4-byte offset.
+struct __attribute__((packed, aligned(4))) Cols4 {
+  int32_t c[4];
+};
+
 __device__ __forceinline__ bool test_bit(const uint32_t* bm, int32_t v) {
   return (bm[v >> 5] >> (v & 31)) & 1u;
 }
 
-// Largest j in [0, kBlock) with off[j] <= e (off non-decreasing).
+// Largest j in [0, kWave) with off[j] <= e (off non-decreasing, off[0] <= e).
 __device__ __forceinline__ int owner_of(const int* off, int e) {
-  int lo = 0, hi = kBlock - 1;
-  while (lo < hi) {
-    int mid = (lo + hi + 1) >> 1;
-    if (off[mid] <= e) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
+  int j = 0;
+#pragma unroll
+  for (int o = kWave / 2; o >= 1; o >>= 1)
+    if (off[j + o] <= e) j += o;
+  return j;
 }
 
 struct Acc {
   unsigned long long fv = 0, fe = 0, scout = 0;
-  __device__ void add(const int32_t* row_ptr, int32_t v) {
-    int d = row_ptr[v + 1] - row_ptr[v];
+  __device__ void add(int d) {
     fv += 1;
     fe += (unsigned)d;
     scout += (unsigned)(d > 0 ? d : 1);
   }
   // Wave sums into the workgroup's LDS totals (all 64 lanes).
   __device__ void reduce(unsigned long long* s_tot) {
+    if (!__ballot(fv != 0)) return;
     unsigned long long a = wave_sum_u64(fv), b = wave_sum_u64(fe), s = wave_sum_u64(scout);
-    if (lane_id() == 0 && a) {
+    if (lane_id() == 0) {
       atomicAdd(&s_tot[0], a);
       atomicAdd(&s_tot[1], b);
       atomicAdd(&s_tot[2], s);
@@ -134,22 +159,163 @@ struct Acc {
   }
 };
 
-// Workgroup-level staging of a step's outputs: the new level's queue
-// entries and its counters.
+// Edges per heavy chunk: two rounds of a wave.
+constexpr int kHeavyChunk = 128;
+
+// Chunks of a vertex of out-degree d.
+__device__ __forceinline__ int chunks_of(const SsArgs& a, int d) {
+  return (d + a.hchunk - 1) / a.hchunk;
+}
+
+// Writes the heavy-chunk entries of vertex u (degree d, first edge rb) from
+// slot `at` on: entries first, first + step, ...
+__device__ __forceinline__ void put_chunks(const SsArgs& a, int2* hq, unsigned at, int32_t u,
+                                           int rb, int d, int first, int step) {
+  const int k = chunks_of(a, d);
+  for (int i = first; i < k; i += step) hq[at + i] = make_int2(u, rb + i * a.hchunk);
+}
+
+// Heavy-chunk entries of the wave's lanes with d > hchunk: lists of up to
+// eight entries by their own lane, longer ones by the whole wave in turn (a
+// hub's hundreds of entries written by one lane took longer than the step's
+// edges).  *len is the counter to reserve from, in LDS or global memory.
+// Called by all 64 lanes.
+__device__ __forceinline__ void wave_put_chunks(const SsArgs& a, int2* hq, unsigned* len,
+                                                int32_t u, int rb, int d) {
+  const int k = d > a.hchunk ? chunks_of(a, d) : 0;
+  unsigned at = 0;
+  if (k) at = atomicAdd(len, (unsigned)k);
+  if (k && k <= 8) put_chunks(a, hq, at, u, rb, d, 0, 1);
+  uint64_t hm = __ballot(k > 8);
+  while (hm) {
+    const int l = __ffsll((unsigned long long)hm) - 1;
+    hm &= hm - 1;
+    put_chunks(a, hq, __shfl(at, l), __shfl(u, l), __shfl(rb, l), __shfl(d, l), lane_id(), kWave);
+  }
+}
+
+// Exclusive scan of one int per thread over a kSsBlock-thread workgroup.
+// scratch: kSsWaves ints of LDS; *total receives the sum.
+__device__ __forceinline__ int ss_scan(int x, int* scratch, int* total) {
+  const int l = lane_id(), w = threadIdx.x / kWave;
+  int inc = x;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int y = __shfl_up(inc, o);
+    if (l >= o) inc += y;
+  }
+  if (l == kWave - 1) scratch[w] = inc;
+  __syncthreads();
+  int before = 0, sum = 0;
+#pragma unroll
+  for (int i = 0; i < kSsWaves; i++) {
+    const int t = scratch[i];
+    if (i < w) before += t;
+    sum += t;
+  }
+  __syncthreads();
+  *total = sum;
+  return before + inc - x;
+}
+
+// Workgroup-level staging of a step's outputs: the vertices found in the
+// step and the level's counters.  Waves reserve LDS slots with LDS atomics;
+// flush() reads the staged vertices' degrees (independent loads, one after
+// the other hidden behind each other), splits them into the light queue and
+// heavy chunks, and reserves each global range once per workgroup: a global
+// counter that every wave bumps serialises at one address.  Vertices beyond
+// the LDS capacity go straight to the global queues, wave by wave.
 struct SsStage {
-  LdsQueue<kStageCap> q;
+  int32_t v[kStageCap];
+  unsigned n;        // slots reserved (may pass kStageCap)
+  unsigned base[2];  // global positions of the workgroup's ranges
+  int scan[kSsWaves];
   unsigned long long tot[3];
   __device__ void init() {
     if (threadIdx.x == 0) {
-      q.init();
+      n = 0u;
       tot[0] = tot[1] = tot[2] = 0ull;
     }
     __syncthreads();
   }
-  // Every thread, once, at the end of the step kernel.
-  __device__ void flush(const SsArgs& a, Acc& acc, int lv, unsigned* qlen, int32_t* q_out) {
+  // Records a vertex found in level lv (each vertex once per level).  Called
+  // by all 64 lanes of a wave.
+  __device__ void append(const SsArgs& a, bool pred, int32_t x, int lv, Acc& acc) {
+    const uint64_t m = __ballot(pred);
+    if (m == 0) return;
+    const int leader = __ffsll((unsigned long long)m) - 1;
+    const unsigned cnt = (unsigned)__popcll(m);
+    unsigned b = 0;
+    if (lane_id() == leader) b = atomicAdd(&n, cnt);
+    b = __shfl(b, leader);
+    const unsigned idx = b + (unsigned)__popcll(m & lanes_below_mask());
+    if (pred && idx < (unsigned)kStageCap) v[idx] = x;
+    if (b + cnt > (unsigned)kStageCap) spill(a, pred && idx >= (unsigned)kStageCap, x, lv, acc);
+  }
+  __device__ void spill(const SsArgs& a, bool pred, int32_t x, int lv, Acc& acc) {
+    LevelCounters* c = a.ring + (lv % kRing);
+    int32_t* q_out = a.q + (int64_t)(lv & 1) * a.n;
+    int2* hq_out = a.hq + (int64_t)(lv & 1) * a.hcap;
+    int rb = 0, d = 0;
+    if (pred) {
+      rb = a.row_ptr[x];
+      d = a.row_ptr[x + 1] - rb;
+      acc.add(d);
+    }
+    const bool light = d > 0 && d <= a.hchunk;
+    const int at = wave_append(&c->qlen, light);
+    if (light) q_out[at] = x;
+    wave_put_chunks(a, hq_out, &c->hqlen, x, rb, d);
+  }
+  // Every thread, once, at the end of the step kernel.  The staged order is
+  // kept: vertices found together are neighbours in the next queue, so the
+  // lanes that expand them read neighbouring rows and distances (queue
+  // entries interleaved by thread made push steps on a 2048^2 grid 2-3x
+  // slower).
+  __device__ void flush(const SsArgs& a, Acc& acc, int lv) {
+    __syncthreads();
+    const unsigned cnt = n < (unsigned)kStageCap ? n : (unsigned)kStageCap;
+    if (cnt) {  // block-uniform
+      int nl = 0, nh = 0, tl, th;
+      for (unsigned i = threadIdx.x; i < cnt; i += kSsBlock) {
+        const int d = a.row_ptr[v[i] + 1] - a.row_ptr[v[i]];
+        acc.add(d);
+        if (d > a.hchunk) nh += chunks_of(a, d);
+        else if (d > 0) nl += 1;
+      }
+      (void)ss_scan(nl, scan, &tl);
+      (void)ss_scan(nh, scan, &th);
+      if (threadIdx.x == 0) {
+        LevelCounters* c = a.ring + (lv % kRing);
+        base[0] = tl ? atomicAdd(&c->qlen, (unsigned)tl) : 0u;
+        base[1] = th ? atomicAdd(&c->hqlen, (unsigned)th) : 0u;
+      }
+      __syncthreads();
+      int32_t* q_out = a.q + (int64_t)(lv & 1) * a.n + base[0];
+      int2* hq_out = a.hq + (int64_t)(lv & 1) * a.hcap;
+      if ((unsigned)tl == cnt) {  // block-uniform: every vertex is light
+        for (unsigned i = threadIdx.x; i < cnt; i += kSsBlock) q_out[i] = v[i];
+      } else {
+        for (unsigned i0 = 0; i0 < cnt; i0 += kSsBlock) {
+          const unsigned i = i0 + threadIdx.x;
+          int rb = 0, d = 0;
+          int32_t x = 0;
+          if (i < cnt) {
+            x = v[i];
+            rb = a.row_ptr[x];
+            d = a.row_ptr[x + 1] - rb;
+          }
+          const bool light = d > 0 && d <= a.hchunk;
+          int tr;
+          const int ol = ss_scan(light ? 1 : 0, scan, &tr);
+          if (light) q_out[ol] = x;
+          q_out += tr;
+          wave_put_chunks(a, hq_out, &base[1], x, rb, d);
+        }
+      }
+    }
     acc.reduce(tot);
-    q.flush(qlen, q_out);  // synchronises the workgroup first
+    __syncthreads();
     if (threadIdx.x < 3 && tot[threadIdx.x]) {
       unsigned long long* stripe =
           a.part + ((size_t)(lv % kRing) * kStripes + blockIdx.x % kStripes) * kStripeU64;
@@ -158,12 +324,70 @@ struct SsStage {
   }
 };
 
-// Records a newly discovered vertex of the level: staged queue slot and
-// counters.  Called by every lane of the wave.
-__device__ __forceinline__ void emit(bool disc, int32_t v, SsStage& sg, unsigned* qlen,
-                                     int32_t* q_out, Acc& acc, const int32_t* row_ptr) {
-  sg.q.append(disc, v, qlen, q_out);
-  if (disc) acc.add(row_ptr, v);
+// Out-edges of level lv-1's queue, spread over the waves of the grid: a wave
+// takes the heavy chunks one by one, and of the light queue 1 to 64
+// vertices at a time (as few as the grid's waves need to cover the queue),
+// whose edge lists it walks as one (LDS degree scan, two edges per lane and
+// round).  edge(u_dist, k0, k1) handles edges k0 and k1 (-1: none) in one
+// wave-uniform call.  Bound by the latency of the dependent loads per edge
+// (column, then its distance): with whole workgroups taking 256 queue
+// entries each, a frontier of a few thousand vertices ran on a few CUs and
+// a hub's list on one (RMAT scale 22, 10.2 M edges of 3133 vertices: 29.7 ms,
+// now 0.25 ms; scale 20, 1.03 M edges of 434: 6.9 ms, now 0.18 ms, where the
+// atomics on the few bitmap words of the hubs bound it).
+template <bool DU, class F>
+__device__ __forceinline__ void push_edges(const SsArgs& a, int lv, F&& edge) {
+  __shared__ int s_off[kSsWaves][kWave];
+  __shared__ int s_beg[kSsWaves][kWave];
+  __shared__ int s_du[DU ? kSsWaves : 1][kWave];
+  const LevelCounters* c_in = a.ring + ((lv + kRing - 1) % kRing);
+  const unsigned qn = c_in->qlen, hn = c_in->hqlen;
+  const int32_t* q_in = a.q + (int64_t)((lv + 1) & 1) * a.n;
+  const int2* hq_in = a.hq + (int64_t)((lv + 1) & 1) * a.hcap;
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  const int64_t wid = (int64_t)blockIdx.x * (kSsWaves) + wv;
+  const int64_t nw = (int64_t)gridDim.x * (kSsWaves);
+  for (int64_t c = wid; c < hn; c += nw) {  // wave-uniform
+    const int2 h = hq_in[c];
+    const int end = min(h.y + a.hchunk, a.row_ptr[h.x + 1]);
+    const int du = DU ? a.dist[h.x] : 0;
+    for (int k = h.y; k < end; k += 2 * kWave) {
+      const int k0 = k + lane, k1 = k0 + kWave;
+      edge(du, du, k0 < end ? k0 : -1, k1 < end ? k1 : -1);
+    }
+  }
+  int64_t per = (qn + nw - 1) / nw;
+  per = per < 1 ? 1 : per > kWave ? kWave : per;
+  int* off = s_off[wv];
+  int* begs = s_beg[wv];
+  int* dus = s_du[DU ? wv : 0];
+  for (int64_t c = wid * per; c < qn; c += nw * per) {  // wave-uniform
+    int beg = 0, deg = 0, du = 0;
+    if (lane < per && c + lane < qn) {
+      const int32_t u = q_in[c + lane];
+      beg = a.row_ptr[u];
+      deg = a.row_ptr[u + 1] - beg;
+      if (DU) du = a.dist[u];
+    }
+    int inc = deg;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int y = __shfl_up(inc, o);
+      if (lane >= o) inc += y;
+    }
+    const int total = __shfl(inc, kWave - 1);
+    off[lane] = inc - deg;
+    begs[lane] = beg - (inc - deg);
+    if (DU) dus[lane] = du;
+    wave_lds_sync();
+    for (int e = lane; e - lane < total; e += 2 * kWave) {
+      const int e1 = e + kWave;
+      const int j0 = owner_of(off, e), j1 = owner_of(off, e1);
+      edge(DU ? dus[j0] : 0, DU ? dus[j1] : 0, e < total ? begs[j0] + e : -1,
+           e1 < total ? begs[j1] + e1 : -1);
+    }
+    wave_lds_sync();
+  }
 }
 
 // Clears the counter stripes of level lv (grid-stride).
@@ -195,11 +419,13 @@ __global__ void ss_fill_kernel(SsArgs a, int weighted) {
 }
 
 // Level 0 = {source}.  GAPBS starts scout_count at out_degree(source)
-// (test/gabps/bfs.cc:140).
+// (test/gabps/bfs.cc:140).  One wave.
 __global__ void bfs_seed_kernel(SsArgs a, int32_t policy) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  if (blockIdx.x != 0) return;
   const int32_t s = a.source;
-  const int d = a.row_ptr[s + 1] - a.row_ptr[s];
+  const int rb = a.row_ptr[s], d = a.row_ptr[s + 1] - rb;
+  if (d > a.hchunk) put_chunks(a, a.hq, 0, s, rb, d, threadIdx.x, blockDim.x);
+  if (threadIdx.x != 0) return;
   a.dist[s] = 0;
   a.bm[s >> 5] |= 1u << (s & 31);
   a.q[0] = s;
@@ -208,7 +434,8 @@ __global__ void bfs_seed_kernel(SsArgs a, int32_t policy) {
   c.fe = (unsigned)d;
   c.scout = (unsigned)d;
   c.flanes = 1;
-  c.qlen = 1;
+  if (d > a.hchunk) c.hqlen = (unsigned)((d + a.hchunk - 1) / a.hchunk);
+  else c.qlen = 1;
   seed_counters(a, 0, c);
   SchedState st{};
   st.step = 0;
@@ -225,29 +452,49 @@ __global__ void bfs_seed_kernel(SsArgs a, int32_t policy) {
 // (src/algorithm/cpu/sssp.cpp:40-46): every listed out-edge of the source
 // writes its weight in row order (a later duplicate overwrites an earlier
 // one), the distinct neighbours form the first frontier, distance[source]
-// = 0, and the source is never relaxed afterwards.
-__global__ void sssp_seed_kernel(SsArgs a) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// = 0, and the source is never relaxed afterwards.  One workgroup: each
+// neighbour's slot first takes -1 - (its last listed edge) by atomicMin,
+// then that edge alone replaces it by its weight (weights are >= 0, so no
+// other edge of the neighbour matches).  A hub source's list in one thread
+// took 100k dependent round trips.
+constexpr int kSeedBlock = 1024;
+__global__ void __launch_bounds__(kSeedBlock) sssp_seed_kernel(SsArgs a) {
+  __shared__ unsigned s_len[2];
+  __shared__ unsigned long long s_c[3];
   const int32_t s = a.source;
   const int32_t b = a.row_ptr[s], e = a.row_ptr[s + 1];
-  for (int32_t k = b; k < e; k++) a.dist[a.col[k]] = a.w[k];
-  a.dist[s] = 0;
+  if (threadIdx.x < 2) s_len[threadIdx.x] = 0u;
+  if (threadIdx.x < 3) s_c[threadIdx.x] = 0ull;
+  for (int32_t k = b + threadIdx.x; k < e; k += kSeedBlock) atomicMin(&a.dist[a.col[k]], -1 - k);
+  __syncthreads();
   uint32_t* bm1 = a.bm + a.words;  // level 1 slot
   int32_t* q1 = a.q + a.n;
-  LevelCounters c{};
-  for (int32_t k = b; k < e; k++) {
-    int32_t v = a.col[k];
+  int2* hq1 = a.hq + a.hcap;
+  for (int32_t k = b + threadIdx.x; k < e; k += kSeedBlock) {
+    const int32_t v = a.col[k];
+    if (__hip_atomic_load(&a.dist[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != -1 - k) continue;
+    __hip_atomic_store(&a.dist[v], a.w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (v == s) continue;
-    uint32_t bit = 1u << (v & 31);
-    if (bm1[v >> 5] & bit) continue;
-    bm1[v >> 5] |= bit;
-    q1[c.qlen++] = v;
-    int d = a.row_ptr[v + 1] - a.row_ptr[v];
-    c.fv += 1;
-    c.fe += (unsigned)d;
-    c.scout += (unsigned)(d > 0 ? d : 1);
+    atomicOr(&bm1[v >> 5], 1u << (v & 31));
+    const int rb = a.row_ptr[v], d = a.row_ptr[v + 1] - rb;
+    if (d > a.hchunk)
+      put_chunks(a, hq1, atomicAdd(&s_len[1], (unsigned)((d + a.hchunk - 1) / a.hchunk)), v, rb, d, 0, 1);
+    else if (d > 0)
+      q1[atomicAdd(&s_len[0], 1u)] = v;
+    atomicAdd(&s_c[0], 1ull);
+    atomicAdd(&s_c[1], (unsigned long long)d);
+    atomicAdd(&s_c[2], (unsigned long long)(d > 0 ? d : 1));
   }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  __hip_atomic_store(&a.dist[s], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  LevelCounters c{};
+  c.fv = s_c[0];
+  c.fe = s_c[1];
+  c.scout = s_c[2];
   c.flanes = c.fv;
+  c.qlen = s_len[0];
+  c.hqlen = s_len[1];
   seed_counters(a, 1, c);
   SchedState st{};
   st.step = 1;
@@ -292,91 +539,133 @@ __global__ void ss_decide_kernel(SsArgs a, SchedParams p, SchedTrace tr) {
   }
 }
 
-// One BOVM step: discovers level lv = st->step.
-__global__ void __launch_bounds__(kBlock) bfs_expand_kernel(SsArgs a) {
-  __shared__ int s_off[kBlock];
-  __shared__ int s_beg[kBlock];
-  __shared__ int s_scan[kBlock / kWave];
-  const SchedState st = *a.st;
-  if (st.done) return;
-  const int lv = st.step;
-  const int pi = (lv + 2) % 3, ci = lv % 3, ni = (lv + 1) % 3;
-  const uint32_t* bm_in = a.bm + pi * a.words;
-  uint32_t* bm_out = a.bm + ci * a.words;
-  uint32_t* bm_nx = a.bm + ni * a.words;
-  const int32_t* q_in = a.q + (int64_t)pi * a.n;
-  int32_t* q_out = a.q + (int64_t)ci * a.n;
-  LevelCounters* c_out = a.ring + (lv % kRing);
-  unsigned* qlen = &c_out->qlen;
-  const int lane = lane_id();
+// Per-step housekeeping shared by the step kernels: clears the next level's
+// bitmap, ring entry and counter stripes.
+__device__ __forceinline__ void clear_next(const SsArgs& a, int lv) {
   const int64_t gs = (int64_t)gridDim.x * blockDim.x;
   const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t* bm_nx = a.bm + (int64_t)((lv + 1) % 3) * a.words;
   for (int64_t i = gt; i < a.words; i += gs) bm_nx[i] = 0u;
   if (gt == 0) a.ring[(lv + 1) % kRing] = LevelCounters{};
   clear_stripes(a, lv + 1, gt, gs);
+}
+
+// Dense top-down over the frontier bitmap: vertices of out-degree < heavy
+// one lane each, the others by the graph's static out-edge chunks, a wave
+// each.  edge(v_dist, k) handles one edge per lane (k < 0: none) in
+// wave-uniform calls.
+template <bool DU, class F>
+__device__ __forceinline__ void bitmap_edges(const SsArgs& a, const uint32_t* bm_in, F&& edge) {
+  const int lane = lane_id();
+  const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
+  for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
+       base += wstride) {
+    const int32_t u = (int32_t)(base + lane);
+    const bool act = u < a.n && test_bit(bm_in, u);
+    if (__ballot(act) == 0) continue;
+    int beg = 0, deg = 0, du = 0;
+    if (act) {
+      beg = a.row_ptr[u];
+      deg = a.row_ptr[u + 1] - beg;
+      if (DU) du = a.dist[u];
+    }
+    const bool light = act && deg < a.heavy;
+    const int maxd = wave_max_i32(light ? deg : 0);
+    for (int j = 0; j < maxd; j++) edge(du, light && j < deg ? beg + j : -1);
+  }
+  const int64_t wid = ((int64_t)blockIdx.x * kSsBlock + threadIdx.x) / kWave;
+  const int64_t nw = (int64_t)gridDim.x * (kSsWaves);
+  // 64 chunks are probed at once, one per lane, as most are not in the
+  // frontier; a grid apart, as a hub's chunks are neighbours in the list.
+  for (int64_t c0 = wid; c0 < a.num_oc; c0 += nw * kWave) {  // wave-uniform
+    const int32_t mine = c0 + lane * nw < a.num_oc ? a.oc_v[c0 + lane * nw] : -1;
+    uint64_t m = __ballot(mine >= 0 && test_bit(bm_in, mine));
+    while (m) {
+      const int l = __ffsll((unsigned long long)m) - 1;
+      m &= m - 1;
+      const int du = DU ? a.dist[__shfl(mine, l)] : 0;
+      const int end = a.oc_end[c0 + l * nw];
+      for (int k = a.oc_beg[c0 + l * nw]; k < end; k += kWave) edge(du, k + lane < end ? k + lane : -1);
+    }
+  }
+}
+
+// One BOVM step: discovers level lv = st->step.
+__global__ void __launch_bounds__(kSsBlock, 8) bfs_expand_kernel(SsArgs a) {
+  const SchedState st = *a.st;
+  if (st.done) return;
+  const int lv = st.step;
+  const uint32_t* bm_in = a.bm + (int64_t)((lv + 2) % 3) * a.words;
+  uint32_t* bm_out = a.bm + (int64_t)(lv % 3) * a.words;
+  const int lane = lane_id();
+  clear_next(a, lv);
   __shared__ SsStage sg;
   sg.init();
   Acc acc;
+  // An unreached head joins the level once: the first to set its bitmap bit.
+  auto discover = [&](int32_t v) {
+    const uint32_t bit = 1u << (v & 31);
+    if (atomicOr(&bm_out[v >> 5], bit) & bit) return false;
+    a.dist[v] = lv;
+    return true;
+  };
 
   if (st.mode == DAWN_MODE_PUSH) {
-    const unsigned qn = a.ring[(lv + kRing - 1) % kRing].qlen;
-    for (int64_t c0 = (int64_t)blockIdx.x * kBlock; c0 < qn; c0 += (int64_t)gridDim.x * kBlock) {
-      const int64_t i = c0 + threadIdx.x;
-      int beg = 0, deg = 0;
-      if (i < qn) {
-        int u = q_in[i];
-        beg = a.row_ptr[u];
-        deg = a.row_ptr[u + 1] - beg;
-      }
-      int total;
-      int off = block_exclusive_scan(deg, s_scan, &total);
-      s_off[threadIdx.x] = off;
-      s_beg[threadIdx.x] = beg;
-      __syncthreads();
-      for (int e0 = 0; e0 < total; e0 += kBlock) {
-        const int e = e0 + threadIdx.x;
-        bool disc = false;
-        int32_t v = 0;
-        if (e < total) {
-          int j = owner_of(s_off, e);
-          v = a.col[s_beg[j] + (e - s_off[j])];
-          if (a.dist[v] == kInf && atomicCAS(&a.dist[v], kInf, lv) == kInf) {
-            disc = true;
-            atomicOr(&bm_out[v >> 5], 1u << (v & 31));
-          }
-        }
-        emit(disc, v, sg, qlen, q_out, acc, a.row_ptr);
-      }
-      __syncthreads();
-    }
+    push_edges<false>(a, lv, [&](int, int, int k0, int k1) {
+      const int32_t v0 = k0 >= 0 ? a.col[k0] : 0, v1 = k1 >= 0 ? a.col[k1] : 0;
+      const bool c0 = k0 >= 0 && a.dist[v0] == kInf, c1 = k1 >= 0 && a.dist[v1] == kInf;
+      const bool d0 = c0 && discover(v0), d1 = c1 && discover(v1);
+      sg.append(a, d0, v0, lv, acc);
+      sg.append(a, d1, v1, lv, acc);
+    });
   } else if (st.mode == DAWN_MODE_PULL) {
-    if (gt == 0) *qlen = kNoQueue;  // the level's bitmap only
-    const int64_t wstride = (int64_t)gridDim.x * kBlock;
-    for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.ring[lv % kRing].qlen = kNoQueue;  // bitmap only
+    const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
+    for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
          base += wstride) {
       const int32_t v = (int32_t)(base + lane);
-      bool cand = v < a.n && a.dist[v] == kInf;
       int beg = 0, deg = 0;
-      if (cand) {
+      if (v < a.n && a.dist[v] == kInf) {
         beg = a.in_row_ptr[v];
         deg = a.in_row_ptr[v + 1] - beg;
       }
-      const bool light = cand && deg < kHeavyDegree;
-      const int maxd = wave_max_i32(light ? deg : 0);
       bool found = false;
-      for (int j = 0; j < maxd; j++) {
-        if (light && !found && j < deg) found = test_bit(bm_in, a.in_col[beg + j]);
+      // Rounds of four in-edges per lane (columns by one 16-byte load, probed
+      // two by two), until every lane has found a frontier tail or run out;
+      // of a heavy vertex only the first two rounds, the rest by the whole
+      // wave.  Bound by requests (each lane reads its own list and probes a
+      // word per edge), so probes past the first hit cost: 128 edges of a
+      // heavy vertex probed at once made a sparse step on RMAT scale 22 60%
+      // slower than 64.
+      const int lim = deg < kHeavyDegree ? deg : 8;
+      for (int j = 0; __ballot(!found && j < lim); j += 4) {
+        if (!found && j < lim) {
+          const int32_t* p = a.in_col + beg + j;
+          Cols4 u;
+          if (j + 4 <= deg) {
+            u = *reinterpret_cast<const Cols4*>(p);
+          } else {
+            const int r = deg - 1 - j;  // 0..2: repeat the last column
+            u = {{p[0], p[min(1, r)], p[r], p[r]}};
+          }
+          const bool f0 = test_bit(bm_in, u.c[0]), f1 = test_bit(bm_in, u.c[1]);
+          found = f0 || f1;
+          if (!found) {
+            const bool f2 = test_bit(bm_in, u.c[2]), f3 = test_bit(bm_in, u.c[3]);
+            found = f2 || f3;
+          }
+        }
       }
-      uint64_t hm = __ballot(cand && deg >= kHeavyDegree);
+      uint64_t hm = __ballot(!found && deg >= kHeavyDegree);
       while (hm) {
         const int l = __ffsll((unsigned long long)hm) - 1;
         hm &= hm - 1;
         const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
         bool f = false;
-        for (int k0 = hb; k0 < he; k0 += kWave) {
+        for (int k0 = hb + 8; k0 < he; k0 += kWave) {
           const int k = k0 + lane;
-          const bool b = k < he && test_bit(bm_in, a.in_col[k]);
-          if (__ballot(b)) { f = true; break; }
+          const bool h = k < he && test_bit(bm_in, a.in_col[k]);
+          if (__ballot(h)) { f = true; break; }
         }
         if (lane == l) found = f;
       }
@@ -386,60 +675,20 @@ __global__ void __launch_bounds__(kBlock) bfs_expand_kernel(SsArgs a) {
         bm_out[base >> 5] = (uint32_t)fm;
         bm_out[(base >> 5) + 1] = (uint32_t)(fm >> 32);
       }
-      if (found) acc.add(a.row_ptr, v);  // bitmap only: no queue entries
+      if (found) acc.add(a.row_ptr[v + 1] - a.row_ptr[v]);  // bitmap only: no queue entries
     }
-  } else {  // DAWN_MODE_BITMAP: dense top-down over the frontier bitmap
-    const int64_t wstride = (int64_t)gridDim.x * kBlock;
-    for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
-         base += wstride) {
-      const int32_t u = (int32_t)(base + lane);
-      const bool act = u < a.n && test_bit(bm_in, u);
-      if (__ballot(act) == 0) continue;
-      int beg = 0, deg = 0;
-      if (act) {
-        beg = a.row_ptr[u];
-        deg = a.row_ptr[u + 1] - beg;
-      }
-      const bool light = act && deg < kHeavyDegree;
-      const int maxd = wave_max_i32(light ? deg : 0);
-      for (int j = 0; j < maxd; j++) {
-        bool disc = false;
-        int32_t v = 0;
-        if (light && j < deg) {
-          v = a.col[beg + j];
-          if (a.dist[v] == kInf && atomicCAS(&a.dist[v], kInf, lv) == kInf) {
-            disc = true;
-            atomicOr(&bm_out[v >> 5], 1u << (v & 31));
-          }
-        }
-        emit(disc, v, sg, qlen, q_out, acc, a.row_ptr);
-      }
-      uint64_t hm = __ballot(act && deg >= kHeavyDegree);
-      while (hm) {
-        const int l = __ffsll((unsigned long long)hm) - 1;
-        hm &= hm - 1;
-        const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
-        for (int k0 = hb; k0 < he; k0 += kWave) {
-          const int k = k0 + lane;
-          bool disc = false;
-          int32_t v = 0;
-          if (k < he) {
-            v = a.col[k];
-            if (a.dist[v] == kInf && atomicCAS(&a.dist[v], kInf, lv) == kInf) {
-              disc = true;
-              atomicOr(&bm_out[v >> 5], 1u << (v & 31));
-            }
-          }
-          emit(disc, v, sg, qlen, q_out, acc, a.row_ptr);
-        }
-      }
-    }
+  } else {  // DAWN_MODE_BITMAP
+    bitmap_edges<false>(a, bm_in, [&](int, int k) {
+      const int32_t v = k >= 0 ? a.col[k] : 0;
+      sg.append(a, k >= 0 && a.dist[v] == kInf && discover(v), v, lv, acc);
+    });
   }
-  sg.flush(a, acc, lv, qlen, q_out);
+  sg.flush(a, acc, lv);
 }
 
-// Relaxation of edge (u -> v, w) with du = current distance of u.  Returns
-// true when v joins the next frontier for the first time this level.
+// Relaxation of an edge to v of weight w with du = current distance of the
+// tail.  Returns true when v joins the next frontier for the first time this
+// level.
 __device__ __forceinline__ bool relax(const SsArgs& a, int32_t src, int32_t du, int32_t v,
                                       int32_t w, uint32_t* bm_out) {
   if (v == src) return false;
@@ -456,71 +705,35 @@ __device__ __forceinline__ bool relax(const SsArgs& a, int32_t src, int32_t du, 
 
 // One min-plus step (GOVM/GOVMP semantics): relaxes the out-edges of the
 // vertices whose distance dropped in the previous step.
-__global__ void __launch_bounds__(kBlock) sssp_expand_kernel(SsArgs a) {
-  __shared__ int s_off[kBlock];
-  __shared__ int s_beg[kBlock];
-  __shared__ int s_du[kBlock];
-  __shared__ int s_scan[kBlock / kWave];
+__global__ void __launch_bounds__(kSsBlock, 8) sssp_expand_kernel(SsArgs a) {
   const SchedState st = *a.st;
   if (st.done) return;
   const int32_t src = st.source;
   const int lv = st.step;
-  const int pi = (lv + 2) % 3, ci = lv % 3, ni = (lv + 1) % 3;
-  const uint32_t* bm_in = a.bm + pi * a.words;
-  uint32_t* bm_out = a.bm + ci * a.words;
-  uint32_t* bm_nx = a.bm + ni * a.words;
-  const int32_t* q_in = a.q + (int64_t)pi * a.n;
-  int32_t* q_out = a.q + (int64_t)ci * a.n;
-  LevelCounters* c_out = a.ring + (lv % kRing);
-  unsigned* qlen = &c_out->qlen;
+  const uint32_t* bm_in = a.bm + (int64_t)((lv + 2) % 3) * a.words;
+  uint32_t* bm_out = a.bm + (int64_t)(lv % 3) * a.words;
   const int lane = lane_id();
-  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
-  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int64_t i = gt; i < a.words; i += gs) bm_nx[i] = 0u;
-  if (gt == 0) a.ring[(lv + 1) % kRing] = LevelCounters{};
-  clear_stripes(a, lv + 1, gt, gs);
+  clear_next(a, lv);
   __shared__ SsStage sg;
   sg.init();
   Acc acc;
 
   if (st.mode == DAWN_MODE_PUSH) {
-    const unsigned qn = a.ring[(lv + kRing - 1) % kRing].qlen;
-    for (int64_t c0 = (int64_t)blockIdx.x * kBlock; c0 < qn; c0 += (int64_t)gridDim.x * kBlock) {
-      const int64_t i = c0 + threadIdx.x;
-      int beg = 0, deg = 0, du = 0;
-      if (i < qn) {
-        int u = q_in[i];
-        beg = a.row_ptr[u];
-        deg = a.row_ptr[u + 1] - beg;
-        du = a.dist[u];
-      }
-      int total;
-      int off = block_exclusive_scan(deg, s_scan, &total);
-      s_off[threadIdx.x] = off;
-      s_beg[threadIdx.x] = beg;
-      s_du[threadIdx.x] = du;
-      __syncthreads();
-      for (int e0 = 0; e0 < total; e0 += kBlock) {
-        const int e = e0 + threadIdx.x;
-        bool disc = false;
-        int32_t v = 0;
-        if (e < total) {
-          int j = owner_of(s_off, e);
-          int k = s_beg[j] + (e - s_off[j]);
-          v = a.col[k];
-          disc = relax(a, src, s_du[j], v, a.w[k], bm_out);
-        }
-        emit(disc, v, sg, qlen, q_out, acc, a.row_ptr);
-      }
-      __syncthreads();
-    }
+    push_edges<true>(a, lv, [&](int du0, int du1, int k0, int k1) {
+      const int32_t v0 = k0 >= 0 ? a.col[k0] : 0, v1 = k1 >= 0 ? a.col[k1] : 0;
+      const int32_t w0 = k0 >= 0 ? a.w[k0] : 0, w1 = k1 >= 0 ? a.w[k1] : 0;
+      const bool d0 = k0 >= 0 && relax(a, src, du0, v0, w0, bm_out);
+      const bool d1 = k1 >= 0 && relax(a, src, du1, v1, w1, bm_out);
+      sg.append(a, d0, v0, lv, acc);
+      sg.append(a, d1, v1, lv, acc);
+    });
   } else if (st.mode == DAWN_MODE_PULL) {
     // Every vertex takes the minimum over its in-edges from frontier
     // vertices; each vertex is written only by its own lane.  Bitmap only:
     // no queue entries.
-    if (gt == 0) *qlen = kNoQueue;
-    const int64_t wstride = (int64_t)gridDim.x * kBlock;
-    for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.ring[lv % kRing].qlen = kNoQueue;
+    const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
+    for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
          base += wstride) {
       const int32_t v = (int32_t)(base + lane);
       const bool cand = v < a.n && v != src;
@@ -566,53 +779,15 @@ __global__ void __launch_bounds__(kBlock) sssp_expand_kernel(SsArgs a) {
         bm_out[base >> 5] = (uint32_t)fm;
         bm_out[(base >> 5) + 1] = (uint32_t)(fm >> 32);
       }
-      if (found) acc.add(a.row_ptr, v);  // bitmap only: no queue entries
+      if (found) acc.add(a.row_ptr[v + 1] - a.row_ptr[v]);  // bitmap only: no queue entries
     }
   } else {  // DAWN_MODE_BITMAP (GOVMP shape: dense scan of the frontier)
-    const int64_t wstride = (int64_t)gridDim.x * kBlock;
-    for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
-         base += wstride) {
-      const int32_t u = (int32_t)(base + lane);
-      const bool act = u < a.n && test_bit(bm_in, u);
-      if (__ballot(act) == 0) continue;
-      int beg = 0, deg = 0;
-      int32_t du = 0;
-      if (act) {
-        beg = a.row_ptr[u];
-        deg = a.row_ptr[u + 1] - beg;
-        du = a.dist[u];
-      }
-      const bool light = act && deg < kHeavyDegree;
-      const int maxd = wave_max_i32(light ? deg : 0);
-      for (int j = 0; j < maxd; j++) {
-        bool disc = false;
-        int32_t v = 0;
-        if (light && j < deg) {
-          v = a.col[beg + j];
-          disc = relax(a, src, du, v, a.w[beg + j], bm_out);
-        }
-        emit(disc, v, sg, qlen, q_out, acc, a.row_ptr);
-      }
-      uint64_t hm = __ballot(act && deg >= kHeavyDegree);
-      while (hm) {
-        const int l = __ffsll((unsigned long long)hm) - 1;
-        hm &= hm - 1;
-        const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
-        const int32_t hdu = __shfl(du, l);
-        for (int k0 = hb; k0 < he; k0 += kWave) {
-          const int k = k0 + lane;
-          bool disc = false;
-          int32_t v = 0;
-          if (k < he) {
-            v = a.col[k];
-            disc = relax(a, src, hdu, v, a.w[k], bm_out);
-          }
-          emit(disc, v, sg, qlen, q_out, acc, a.row_ptr);
-        }
-      }
-    }
+    bitmap_edges<true>(a, bm_in, [&](int du, int k) {
+      const int32_t v = k >= 0 ? a.col[k] : 0;
+      sg.append(a, k >= 0 && relax(a, src, du, v, a.w[k], bm_out), v, lv, acc);
+    });
   }
-  sg.flush(a, acc, lv, qlen, q_out);
+  sg.flush(a, acc, lv);
 }
 
 // Sum of out-degree and count of reached vertices (GTEPS numerator):
@@ -642,6 +817,41 @@ __global__ void reach_kernel(const int32_t* dist, const int32_t* row_ptr, int32_
   if (threadIdx.x < 2 && s_t[threadIdx.x]) atomicAdd(&out[threadIdx.x], s_t[threadIdx.x]);
 }
 
+// Arguments that depend on the graph alone.
+SsArgs graph_args(const dawn_graph* g, int32_t source) {
+  SsArgs a{};
+  a.n = g->n;
+  a.source = source;
+  a.words = ((int64_t)g->n + 63) / 64 * 2;
+  a.row_ptr = g->row_ptr;
+  a.col = g->col;
+  a.w = g->weight;
+  a.in_row_ptr = g->in_row_ptr;
+  a.in_col = g->in_col;
+  a.in_w = g->in_weight;
+  a.oc_v = g->oc_v;
+  a.oc_beg = g->oc_beg;
+  a.oc_end = g->oc_end;
+  a.num_oc = g->num_oc;
+  a.heavy = g->knobs.heavy_degree;
+  return a;
+}
+
+// The same on the graph's workspace.
+SsArgs workspace_args(const dawn_graph* g, const SsWorkspace* ws, int32_t source) {
+  SsArgs a = graph_args(g, source);
+  a.dist = ws->dist.p;
+  a.q = ws->q.p;
+  a.hq = ws->hq.p;
+  a.hcap = ws->hcap;
+  a.hchunk = kHeavyChunk;
+  a.bm = ws->bm.p;
+  a.ring = ws->ring.p;
+  a.part = ws->part.p;
+  a.st = ws->st.p;
+  return a;
+}
+
 int ensure_ss(dawn_graph* g) {
   if (!g->ss) g->ss = new SsWorkspace();
   SsWorkspace* ws = g->ss;
@@ -649,7 +859,9 @@ int ensure_ss(dawn_graph* g) {
   ws->n = g->n;
   ws->words = ((int64_t)g->n + 63) / 64 * 2;
   DAWN_TRY(ws->dist.alloc(g->n));
-  DAWN_TRY(ws->q.alloc((size_t)3 * g->n));
+  DAWN_TRY(ws->q.alloc((size_t)2 * g->n));
+  ws->hcap = 2 * (g->m / kHeavyChunk) + 1;
+  DAWN_TRY(ws->hq.alloc((size_t)2 * ws->hcap));
   DAWN_TRY(ws->bm.alloc((size_t)3 * ws->words));
   DAWN_TRY(ws->ring.alloc(kRing));
   DAWN_TRY(ws->part.alloc(kPartU64));
@@ -680,22 +892,7 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   SsWorkspace* ws = g->ss;
   hipStream_t s = g->stream;
 
-  SsArgs a{};
-  a.n = g->n;
-  a.source = source;
-  a.words = ws->words;
-  a.row_ptr = g->row_ptr;
-  a.col = g->col;
-  a.w = g->weight;
-  a.in_row_ptr = g->in_row_ptr;
-  a.in_col = g->in_col;
-  a.in_w = g->in_weight;
-  a.dist = ws->dist.p;
-  a.q = ws->q.p;
-  a.bm = ws->bm.p;
-  a.ring = ws->ring.p;
-  a.part = ws->part.p;
-  a.st = ws->st.p;
+  const SsArgs a = workspace_args(g, ws, source);
 
   SchedParams p{};
   p.n = g->n;
@@ -713,7 +910,7 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   if (kind == 1 && policy == DAWN_POLICY_LEARNED) p.policy = DAWN_POLICY_FIXED;
   SchedTrace tr{ws->trace_feat.p, ws->trace_mode.p};
 
-  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kBlock, 4096);
+  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid);
   // A chunk = K decide+expand pairs, captured once per (kind, policy, mode,
   // K).  Without a knob K is what the last traversal on this graph took
   // (levels + 1, rounded up to even), so that one chunk and one read of the
@@ -738,9 +935,9 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
     for (int i = 0; i < K; i++) {
       ss_decide_kernel<<<1, 64, 0, s>>>(a, p, tr);
       if (kind == 0)
-        bfs_expand_kernel<<<grid, kBlock, 0, s>>>(a);
+        bfs_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
       else
-        sssp_expand_kernel<<<grid, kBlock, 0, s>>>(a);
+        sssp_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
     }
     DAWN_HIP(hipStreamEndCapture(s, &graph));
     hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
@@ -754,7 +951,7 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   if (kind == 0)
     bfs_seed_kernel<<<1, 64, 0, s>>>(a, policy);
   else
-    sssp_seed_kernel<<<1, 64, 0, s>>>(a);
+    sssp_seed_kernel<<<1, kSeedBlock, 0, s>>>(a);
   DAWN_HIP(hipGetLastError());
   if (force_mode >= 0) {
     // The seed kernel leaves force_mode = -1; set it before stepping.
@@ -870,7 +1067,7 @@ int ss_stepwise(dawn_graph* g, SsWorkspace* ws, const SsArgs& a, const SchedPara
       return DAWN_OK;
     }
     DAWN_HIP(hipEventRecord(ws->ev0, s));
-    bfs_expand_kernel<<<grid, kBlock, 0, s>>>(a);
+    bfs_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
     DAWN_HIP(hipGetLastError());
     DAWN_HIP(hipEventRecord(ws->ev1, s));
     DAWN_HIP(hipEventSynchronize(ws->ev1));
@@ -894,7 +1091,7 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
   DAWN_HIP(hipSetDevice(g->device));
   DAWN_TRY(ensure_ss(g));
   SsWorkspace* ws = g->ss;
-  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kBlock, 4096);
+  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid);
   int32_t rows = 0;
   std::vector<float> t, feat;
   std::vector<int32_t> modes;
@@ -902,22 +1099,7 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
     int64_t src = sources[i] % (int64_t)g->n;
     if (src < 0) src += g->n;
     if (g->h_row_ptr[src] == g->h_row_ptr[src + 1]) continue;  // isolated: no traversal
-    SsArgs a{};
-    a.n = g->n;
-    a.source = (int32_t)src;
-    a.words = ws->words;
-    a.row_ptr = g->row_ptr;
-    a.col = g->col;
-    a.w = g->weight;
-    a.in_row_ptr = g->in_row_ptr;
-    a.in_col = g->in_col;
-    a.in_w = g->in_weight;
-    a.dist = ws->dist.p;
-    a.q = ws->q.p;
-    a.bm = ws->bm.p;
-    a.ring = ws->ring.p;
-    a.part = ws->part.p;
-    a.st = ws->st.p;
+    const SsArgs a = workspace_args(g, ws, (int32_t)src);
     SchedParams p{};
     p.n = g->n;
     p.m = g->m;
@@ -965,7 +1147,7 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
 // that forbid hipMalloc): the single-source BOVM traversal on a fixed
 // scratch region instead of the graph's workspace.  The region is the
 // file-scope device array `scratch` below, sized for graphs of up to
-// kNoAllocMaxN vertices (66 MB); the code object carries it, so each GPU
+// kNoAllocMaxN vertices (57 MB); the code object carries it, so each GPU
 // the library runs on holds its own copy until the process ends.  Host code
 // never passes the array's name to a kernel (in host code it is a stand-in,
 // not a device address): once per device, with that device current, the
@@ -989,7 +1171,9 @@ constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 constexpr int64_t kNoAllocWords = ((int64_t)kNoAllocMaxN + 63) / 64 * 2;
 constexpr size_t kNaDist = 0;
 constexpr size_t kNaQ = align256(kNaDist + sizeof(int32_t) * (size_t)kNoAllocMaxN);
-constexpr size_t kNaBm = align256(kNaQ + sizeof(int32_t) * 3 * (size_t)kNoAllocMaxN);
+constexpr size_t kNaHq = align256(kNaQ + sizeof(int32_t) * 2 * (size_t)kNoAllocMaxN);
+constexpr int64_t kNoAllocHeavy = 1 << 18;  // heavy-chunk entries per level
+constexpr size_t kNaBm = align256(kNaHq + sizeof(int2) * 2 * (size_t)kNoAllocHeavy);
 constexpr size_t kNaRing = align256(kNaBm + sizeof(uint32_t) * 3 * (size_t)kNoAllocWords);
 constexpr size_t kNaPart = align256(kNaRing + sizeof(LevelCounters) * kRing);
 constexpr size_t kNaState = align256(kNaPart + sizeof(unsigned long long) * kPartU64);
@@ -1033,18 +1217,14 @@ int run_bfs_noalloc(dawn_graph* g, int32_t source, int32_t* dist_out, int32_t po
   }
   hipStream_t s = g->stream;
 
-  SsArgs a{};
-  a.n = g->n;
-  a.source = source;
-  a.words = ((int64_t)g->n + 63) / 64 * 2;
-  a.row_ptr = g->row_ptr;
-  a.col = g->col;
-  a.w = g->weight;
-  a.in_row_ptr = g->in_row_ptr;
-  a.in_col = g->in_col;
-  a.in_w = g->in_weight;
+  SsArgs a = graph_args(g, source);
   a.dist = (int32_t*)(base + kNaDist);
   a.q = (int32_t*)(base + kNaQ);
+  a.hq = (int2*)(base + kNaHq);
+  a.hcap = kNoAllocHeavy;
+  // Chunks long enough that the heavy lists of any graph fit the region.
+  a.hchunk = kHeavyChunk;
+  while (2 * (g->m / a.hchunk) + 1 > kNoAllocHeavy) a.hchunk *= 2;
   a.bm = (uint32_t*)(base + kNaBm);
   a.ring = (LevelCounters*)(base + kNaRing);
   a.part = (unsigned long long*)(base + kNaPart);
@@ -1064,7 +1244,7 @@ int run_bfs_noalloc(dawn_graph* g, int32_t source, int32_t* dist_out, int32_t po
   p.mlp = sched_single_mlp_if_present(g->device, &p.mlp_norm);
   SchedTrace tr{(float*)(base + kNaFeat), (int32_t*)(base + kNaMode)};
 
-  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kBlock, 4096);
+  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid);
   const int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : (g->n < (1 << 20) ? 8 : 16);
   const auto t0 = std::chrono::steady_clock::now();
   ss_fill_kernel<<<grid_for(std::max<int64_t>(3 * a.words, g->n)), kBlock, 0, s>>>(a, 0);
@@ -1076,7 +1256,7 @@ int run_bfs_noalloc(dawn_graph* g, int32_t source, int32_t* dist_out, int32_t po
   for (;;) {
     for (int i = 0; i < K; i++) {
       ss_decide_kernel<<<1, 64, 0, s>>>(a, p, tr);
-      bfs_expand_kernel<<<grid, kBlock, 0, s>>>(a);
+      bfs_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
     }
     DAWN_HIP(hipGetLastError());
     launched += K;

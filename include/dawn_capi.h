@@ -196,7 +196,7 @@ int dawn_sssp(const dawn_graph* g, int32_t source, int32_t* dist,
  * reference: for callers that cannot allocate device memory (serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, results and statuses as
  * dawn_bfs, but the traversal state lives in a fixed scratch region that
- * the library's code object carries (66 MB per GPU, held until the process
+ * the library's code object carries (57 MB per GPU, held until the process
  * ends) instead of the graph's workspace, so graphs of at most 4,194,304
  * vertices: larger ones return DAWN_ERR_SCRATCH_LIMIT.  The call allocates
  * nothing (no hipMalloc / hipFree, no captured graph), on the graph's
