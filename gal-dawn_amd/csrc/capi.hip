@@ -14,8 +14,7 @@
 namespace dawn {
 
 int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out, int32_t policy,
-                      dawn_stats* stats, int32_t force_mode, float* trace_feat,
-                      int32_t* trace_mode, int32_t trace_max, int32_t* trace_rows);
+                      dawn_stats* stats);
 // rows: with dist null, still compute every distance row (into a scratch
 // buffer) rather than only the per-source sums.
 int run_msbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64_t* sums,
@@ -144,14 +143,14 @@ int dawn_bfs(const dawn_graph* gc, int32_t source, int32_t* dist, int32_t policy
              dawn_stats* stats) {
   dawn_graph* g = const_cast<dawn_graph*>(gc);
   if (!g) return DAWN_ERR_INVALID_ARG;
-  return run_single_source(g, 0, source, dist, policy, stats, -1, nullptr, nullptr, 0, nullptr);
+  return run_single_source(g, 0, source, dist, policy, stats);
 }
 
 int dawn_sssp(const dawn_graph* gc, int32_t source, int32_t* dist, int32_t policy,
               dawn_stats* stats) {
   dawn_graph* g = const_cast<dawn_graph*>(gc);
   if (!g) return DAWN_ERR_INVALID_ARG;
-  return run_single_source(g, 1, source, dist, policy, stats, -1, nullptr, nullptr, 0, nullptr);
+  return run_single_source(g, 1, source, dist, policy, stats);
 }
 
 int dawn_mssp(const dawn_graph* gc, const int32_t* sources, int32_t count, int32_t* dist,

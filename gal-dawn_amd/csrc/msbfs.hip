@@ -174,7 +174,6 @@ struct MsWorkspace {
   hipEvent_t ev0 = nullptr, ev1 = nullptr, e_a = nullptr, e_b = nullptr;
 };
 
-void ss_invalidate_graphs(SsWorkspace* ws);
 void wms_invalidate_graphs(WmsWorkspace* ws);
 
 // Captured step graphs bake grid sizes, knobs and buffer addresses (the
@@ -186,7 +185,6 @@ void invalidate_graphs(dawn_graph* g) {
     for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
     ws->graphs.clear();
   }
-  ss_invalidate_graphs(g->ss);
   wms_invalidate_graphs(g->wms);
 }
 

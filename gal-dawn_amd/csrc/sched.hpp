@@ -22,7 +22,7 @@ struct LevelCounters {
   unsigned long long alive[16];  // batched: OR of the level's frontier words, one
                                  // per 64 lanes (lanes that can still reach new vertices)
   unsigned int qlen;          // queue entries written for this level
-  unsigned int hqlen;         // heavy-chunk entries (single-source engines)
+  unsigned int pad;
 };
 
 constexpr int kRing = 4;          // ring of LevelCounters indexed by level % 4
@@ -40,8 +40,7 @@ struct SchedState {
   int32_t last_mode;
   int32_t levels;    // number of non-empty levels (set when done)
   int32_t force_mode;// >= 0: every step uses this mode
-  int32_t source;    // single-source engines: the traversal's source (read by
-                     // captured step kernels; never a baked launch argument)
+  int32_t source;    // single-source engines: the traversal's source
   unsigned long long work_fv;  // frontier vertices expanded, summed over the steps
   unsigned long long work_fe;  // their out-edges (the relaxations of a push schedule)
 };

@@ -6,29 +6,35 @@
 // DAWN::BFS_CPU (src/algorithm/cpu/bfs.cpp:23-185) and DAWN::SSSP_CPU
 // (src/algorithm/cpu/sssp.cpp:23-199).
 //
-// Layout in HBM (per graph, reused across calls):
-//   dist   int32[n]                      distances (INF = unreached)
-//   q      int32[2][n]                   frontier queue of level l in slot l&1:
-//                                        vertices of out-degree <= hchunk
-//   hq     int2[2][hcap]                 (vertex, first edge) of every hchunk-edge
-//                                        chunk of the frontier's other vertices
-//   bm     uint32[3][words]              frontier bitmap of level l in slot l%3
-//   ring   LevelCounters[4]              per-level counters, level l in l%4
-//   state  SchedState                    step / done / mode / rule state
-// Every step writes BOTH the queue and the bitmap of the new level, so the
-// three modes are interchangeable from step to step with no conversion:
+// Layout in HBM (per graph, reused across calls; k: launch of the step kernel,
+// counted from 0 per traversal):
+//   dist   int32[n]         distances (INF = unreached): the caller's buffer when
+//                           it is device memory, else the workspace's
+//   q      int32[2][n]      frontier queue read by launch k in slot k&1: vertices
+//                           of out-degree 1 to hchunk
+//   hq     int2[2][hcap]    (vertex, first edge) of every hchunk-edge chunk of the
+//                           frontier's other vertices
+//   bm     uint32[3][words] frontier bitmap read by launch k in slot k%3
+//   slots  SsSlot[4]        queue lengths and counters of that frontier in slot k%4
+//   state  SsState[4]       step / done / mode / rule state in slot k%4
+// Launch k reads slot k, writes slot k+1 and clears slot k+2.  Every step but a
+// pull writes BOTH the queue and the bitmap of the new level, so the three modes
+// are interchangeable from step to step with no conversion:
 //   PUSH    queue in: wave-balanced edge expansion (chunks of the heavy
 //           vertices one wave each, the others 1 to 64 per wave by LDS scan)
 //   PULL    bitmap in: unvisited vertices scan in-edges (CSC) with early exit
 //   BITMAP  bitmap in: dense scan of the frontier bitmap, top-down expansion
-// The step loop is decide(1 wave) + expand(grid), captured K steps at a
-// time into a hipGraph; the host reads one flag per chunk.
+// The step loop is one kernel per step: every workgroup makes the same
+// decision from the last level's counters, then all expand the level; runs
+// of levels with few edges are walked by one workgroup within one launch.
+// The launch that finds the frontier empty writes the final state, with the
+// traversal's counts and device time, to pinned host memory, so a call is its
+// launches and one wait.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
 #include <cstdlib>
-#include <map>
 #include <mutex>
 #include <vector>
 
@@ -37,10 +43,33 @@
 
 namespace dawn {
 
+// Counters (frontier vertices, their out-edges, GAPBS scout) are added per
+// workgroup into one of kStripes stripes, each on its own 128-byte line, so
+// the atomics of the workgroups spread over 64 addresses; the next launch sums
+// them, one stripe per lane.
+constexpr int kStripes = 64;
+constexpr int kStripeU64 = 16;  // 128 bytes per stripe
+static_assert(kStripes == kWave, "one stripe per lane is summed");
+struct SsSlot {
+  unsigned long long part[kStripes][kStripeU64];
+  unsigned qlen, hqlen;  // queue entries, heavy-chunk entries
+  unsigned pad[30];
+};
+constexpr int kSsSlots = 4;
+
+struct SsState {
+  SchedState s;
+  int32_t launches;                   // step launches that did something
+  int32_t pad;
+  long long mode_steps[DAWN_NUM_MODES];
+  unsigned long long reached, edges;  // vertices reached, their out-edges (set when done)
+  long long t0, t1;                   // device clock at the first and the last launch
+};
+
 struct SsArgs {
   int32_t n;
-  int32_t source;    // read only by the (uncaptured) seed kernels
-  int64_t words;  // bitmap words per level slot
+  int32_t source;
+  int64_t words;  // bitmap words per slot
   const int32_t* row_ptr;
   const int32_t* col;
   const int32_t* w;
@@ -58,18 +87,21 @@ struct SsArgs {
   const int32_t* oc_beg;
   const int32_t* oc_end;
   int64_t num_oc;
-  LevelCounters* ring;
-  unsigned long long* part;  // kRing x kStripes counter stripes
-  SchedState* st;
+  SsSlot* slots;             // kSsSlots
+  unsigned long long* tot;   // kStripes stripes: vertices reached first, their out-edges
+  SsState* st;               // kSsSlots
+  SsState* host;             // pinned: the final state (null: not written)
 };
 
-// Level counters (fv, fe, scout) are added per workgroup into one of
-// kStripes stripes of the level, each on its own 128-byte line, so the
-// atomics of thousands of workgroups spread over 64 addresses; the decide
-// kernel sums the stripes of the level it reads.
-constexpr int kStripes = 64;
-constexpr int kStripeU64 = 16;  // 128 bytes per stripe
-constexpr int kPartU64 = kRing * kStripes * kStripeU64;
+// Everything a step launch needs but its number.
+struct SsRun {
+  SsArgs a;
+  SchedParams p;
+  SchedTrace tr;   // recording only (else null)
+  int32_t force;   // >= 0: every step in this mode
+  int32_t small;   // runs of small levels may be walked within a launch
+};
+
 // Threads per workgroup of the step kernels, and workgroups per launch (two
 // per CU).  Every workgroup that found something reserves its queue ranges
 // with atomics on one address each, about 12 ns apiece in turn: 4096
@@ -83,37 +115,25 @@ constexpr int kStageCap = 8192;
 // Queue length of a level whose queue was not written (a pull step writes
 // the bitmap only): a top-down step that follows reads the bitmap instead.
 constexpr unsigned kNoQueue = 0xFFFFFFFFu;
-static_assert(kStripes == kWave, "the decide kernel sums one stripe per lane");
 
 struct SsWorkspace {
   int32_t n = 0;
-  int64_t words = 0;
-  DevBuf<int32_t> dist, q;
+  DevBuf<int32_t> dist, q;  // dist: only for outputs that are not device memory
   DevBuf<int2> hq;
   int64_t hcap = 0;
   DevBuf<uint32_t> bm;
-  DevBuf<LevelCounters> ring;
-  DevBuf<unsigned long long> part;
-  DevBuf<SchedState> st;
-  DevBuf<float> trace_feat;
+  DevBuf<SsSlot> slots;
+  DevBuf<unsigned long long> tot;
+  DevBuf<SsState> st;
+  DevBuf<float> trace_feat;    // recording only
   DevBuf<int32_t> trace_mode;
-  DevBuf<unsigned long long> reach;  // [2]
-  SchedState* h_state = nullptr;     // pinned
-  int32_t last_pairs[2] = {0, 0};     // decide+expand pairs the last traversal (per kind) took
-  // Captured K-step chunks keyed by (kind, policy, K).
-  std::map<std::pair<long long, const void*>, hipGraphExec_t> graphs;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  SsState* h_state = nullptr;  // pinned
+  int32_t last_launches[2] = {0, 0};  // step launches the last traversal (per kind) took
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;  // recording only
 };
-
-void ss_invalidate_graphs(SsWorkspace* ws) {
-  if (!ws) return;
-  for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
-  ws->graphs.clear();
-}
 
 void ss_workspace_free(SsWorkspace* ws) {
   if (!ws) return;
-  for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
   if (ws->h_state) (void)hipHostFree(ws->h_state);
   if (ws->ev0) (void)hipEventDestroy(ws->ev0);
   if (ws->ev1) (void)hipEventDestroy(ws->ev1);
@@ -142,20 +162,16 @@ __device__ __forceinline__ int owner_of(const int* off, int e) {
 
 struct Acc {
   unsigned long long fv = 0, fe = 0, scout = 0;
+  unsigned rv = 0;            // vertices reached for the first time (min-plus)
+  unsigned long long re = 0;  // their out-edges
   __device__ void add(int d) {
     fv += 1;
     fe += (unsigned)d;
     scout += (unsigned)(d > 0 ? d : 1);
   }
-  // Wave sums into the workgroup's LDS totals (all 64 lanes).
-  __device__ void reduce(unsigned long long* s_tot) {
-    if (!__ballot(fv != 0)) return;
-    unsigned long long a = wave_sum_u64(fv), b = wave_sum_u64(fe), s = wave_sum_u64(scout);
-    if (lane_id() == 0) {
-      atomicAdd(&s_tot[0], a);
-      atomicAdd(&s_tot[1], b);
-      atomicAdd(&s_tot[2], s);
-    }
+  __device__ void reach(const SsArgs& a, int32_t v) {
+    rv += 1;
+    re += (unsigned)(a.row_ptr[v + 1] - a.row_ptr[v]);
   }
 };
 
@@ -218,6 +234,18 @@ __device__ __forceinline__ int ss_scan(int x, int* scratch, int* total) {
   return before + inc - x;
 }
 
+// Where a launch puts the new level.
+struct SsOut {
+  SsSlot* slot;
+  int32_t* q;
+  int2* hq;
+  unsigned long long* tot;
+};
+__device__ __forceinline__ SsOut out_of(const SsArgs& a, int k) {
+  return {a.slots + ((k + 1) % kSsSlots), a.q + (int64_t)((k + 1) & 1) * a.n,
+          a.hq + (int64_t)((k + 1) & 1) * a.hcap, a.tot + (blockIdx.x % kStripes) * kStripeU64};
+}
+
 // Workgroup-level staging of a step's outputs: the vertices found in the
 // step and the level's counters.  Waves reserve LDS slots with LDS atomics;
 // flush() reads the staged vertices' degrees (independent loads, one after
@@ -230,17 +258,15 @@ struct SsStage {
   unsigned n;        // slots reserved (may pass kStageCap)
   unsigned base[2];  // global positions of the workgroup's ranges
   int scan[kSsWaves];
-  unsigned long long tot[3];
+  unsigned long long tot[5];
   __device__ void init() {
-    if (threadIdx.x == 0) {
-      n = 0u;
-      tot[0] = tot[1] = tot[2] = 0ull;
-    }
+    if (threadIdx.x < 5) tot[threadIdx.x] = 0ull;
+    if (threadIdx.x == 0) n = 0u;
     __syncthreads();
   }
-  // Records a vertex found in level lv (each vertex once per level).  Called
+  // Records a vertex found in the step (each vertex once per level).  Called
   // by all 64 lanes of a wave.
-  __device__ void append(const SsArgs& a, bool pred, int32_t x, int lv, Acc& acc) {
+  __device__ void append(const SsArgs& a, const SsOut& o, bool pred, int32_t x, Acc& acc) {
     const uint64_t m = __ballot(pred);
     if (m == 0) return;
     const int leader = __ffsll((unsigned long long)m) - 1;
@@ -250,12 +276,9 @@ struct SsStage {
     b = __shfl(b, leader);
     const unsigned idx = b + (unsigned)__popcll(m & lanes_below_mask());
     if (pred && idx < (unsigned)kStageCap) v[idx] = x;
-    if (b + cnt > (unsigned)kStageCap) spill(a, pred && idx >= (unsigned)kStageCap, x, lv, acc);
+    if (b + cnt > (unsigned)kStageCap) spill(a, o, pred && idx >= (unsigned)kStageCap, x, acc);
   }
-  __device__ void spill(const SsArgs& a, bool pred, int32_t x, int lv, Acc& acc) {
-    LevelCounters* c = a.ring + (lv % kRing);
-    int32_t* q_out = a.q + (int64_t)(lv & 1) * a.n;
-    int2* hq_out = a.hq + (int64_t)(lv & 1) * a.hcap;
+  __device__ void spill(const SsArgs& a, const SsOut& o, bool pred, int32_t x, Acc& acc) {
     int rb = 0, d = 0;
     if (pred) {
       rb = a.row_ptr[x];
@@ -263,16 +286,16 @@ struct SsStage {
       acc.add(d);
     }
     const bool light = d > 0 && d <= a.hchunk;
-    const int at = wave_append(&c->qlen, light);
-    if (light) q_out[at] = x;
-    wave_put_chunks(a, hq_out, &c->hqlen, x, rb, d);
+    const int at = wave_append(&o.slot->qlen, light);
+    if (light) o.q[at] = x;
+    wave_put_chunks(a, o.hq, &o.slot->hqlen, x, rb, d);
   }
   // Every thread, once, at the end of the step kernel.  The staged order is
   // kept: vertices found together are neighbours in the next queue, so the
   // lanes that expand them read neighbouring rows and distances (queue
   // entries interleaved by thread made push steps on a 2048^2 grid 2-3x
   // slower).
-  __device__ void flush(const SsArgs& a, Acc& acc, int lv) {
+  __device__ void flush(const SsArgs& a, const SsOut& o, Acc& acc) {
     __syncthreads();
     const unsigned cnt = n < (unsigned)kStageCap ? n : (unsigned)kStageCap;
     if (cnt) {  // block-uniform
@@ -286,13 +309,11 @@ struct SsStage {
       (void)ss_scan(nl, scan, &tl);
       (void)ss_scan(nh, scan, &th);
       if (threadIdx.x == 0) {
-        LevelCounters* c = a.ring + (lv % kRing);
-        base[0] = tl ? atomicAdd(&c->qlen, (unsigned)tl) : 0u;
-        base[1] = th ? atomicAdd(&c->hqlen, (unsigned)th) : 0u;
+        base[0] = tl ? atomicAdd(&o.slot->qlen, (unsigned)tl) : 0u;
+        base[1] = th ? atomicAdd(&o.slot->hqlen, (unsigned)th) : 0u;
       }
       __syncthreads();
-      int32_t* q_out = a.q + (int64_t)(lv & 1) * a.n + base[0];
-      int2* hq_out = a.hq + (int64_t)(lv & 1) * a.hcap;
+      int32_t* q_out = o.q + base[0];
       if ((unsigned)tl == cnt) {  // block-uniform: every vertex is light
         for (unsigned i = threadIdx.x; i < cnt; i += kSsBlock) q_out[i] = v[i];
       } else {
@@ -310,21 +331,27 @@ struct SsStage {
           const int ol = ss_scan(light ? 1 : 0, scan, &tr);
           if (light) q_out[ol] = x;
           q_out += tr;
-          wave_put_chunks(a, hq_out, &base[1], x, rb, d);
+          wave_put_chunks(a, o.hq, &base[1], x, rb, d);
         }
       }
     }
-    acc.reduce(tot);
+    if (__ballot(acc.fv != 0 || acc.rv != 0)) {
+      const unsigned long long r[5] = {wave_sum_u64(acc.fv), wave_sum_u64(acc.fe),
+                                       wave_sum_u64(acc.scout), wave_sum_u64(acc.rv),
+                                       wave_sum_u64(acc.re)};
+      if (lane_id() == 0)
+        for (int i = 0; i < 5; i++)
+          if (r[i]) atomicAdd(&tot[i], r[i]);
+    }
     __syncthreads();
-    if (threadIdx.x < 3 && tot[threadIdx.x]) {
-      unsigned long long* stripe =
-          a.part + ((size_t)(lv % kRing) * kStripes + blockIdx.x % kStripes) * kStripeU64;
-      atomicAdd(&stripe[threadIdx.x], tot[threadIdx.x]);
+    if (threadIdx.x < 5 && tot[threadIdx.x]) {
+      const int i = threadIdx.x;
+      atomicAdd(i < 3 ? &o.slot->part[blockIdx.x % kStripes][i] : &o.tot[i - 3], tot[i]);
     }
   }
 };
 
-// Out-edges of level lv-1's queue, spread over the waves of the grid: a wave
+// Out-edges of the frontier queue of launch k, spread over the waves of the grid: a wave
 // takes the heavy chunks one by one, and of the light queue 1 to 64
 // vertices at a time (as few as the grid's waves need to cover the queue),
 // whose edge lists it walks as one (LDS degree scan, two edges per lane and
@@ -335,15 +362,17 @@ struct SsStage {
 // a hub's list on one (RMAT scale 22, 10.2 M edges of 3133 vertices: 29.7 ms,
 // now 0.25 ms; scale 20, 1.03 M edges of 434: 6.9 ms, now 0.18 ms, where the
 // atomics on the few bitmap words of the hubs bound it).
+template <bool DU>
+struct PushLds {
+  int off[kSsWaves][kWave];
+  int beg[kSsWaves][kWave];
+  int du[DU ? kSsWaves : 1][kWave];
+};
 template <bool DU, class F>
-__device__ __forceinline__ void push_edges(const SsArgs& a, int lv, F&& edge) {
-  __shared__ int s_off[kSsWaves][kWave];
-  __shared__ int s_beg[kSsWaves][kWave];
-  __shared__ int s_du[DU ? kSsWaves : 1][kWave];
-  const LevelCounters* c_in = a.ring + ((lv + kRing - 1) % kRing);
-  const unsigned qn = c_in->qlen, hn = c_in->hqlen;
-  const int32_t* q_in = a.q + (int64_t)((lv + 1) & 1) * a.n;
-  const int2* hq_in = a.hq + (int64_t)((lv + 1) & 1) * a.hcap;
+__device__ __forceinline__ void push_edges(const SsArgs& a, PushLds<DU>& s, int k, unsigned qn,
+                                           unsigned hn, F&& edge) {
+  const int32_t* q_in = a.q + (int64_t)(k & 1) * a.n;
+  const int2* hq_in = a.hq + (int64_t)(k & 1) * a.hcap;
   const int lane = lane_id(), wv = threadIdx.x / kWave;
   const int64_t wid = (int64_t)blockIdx.x * (kSsWaves) + wv;
   const int64_t nw = (int64_t)gridDim.x * (kSsWaves);
@@ -351,16 +380,16 @@ __device__ __forceinline__ void push_edges(const SsArgs& a, int lv, F&& edge) {
     const int2 h = hq_in[c];
     const int end = min(h.y + a.hchunk, a.row_ptr[h.x + 1]);
     const int du = DU ? a.dist[h.x] : 0;
-    for (int k = h.y; k < end; k += 2 * kWave) {
-      const int k0 = k + lane, k1 = k0 + kWave;
+    for (int kb = h.y; kb < end; kb += 2 * kWave) {
+      const int k0 = kb + lane, k1 = k0 + kWave;
       edge(du, du, k0 < end ? k0 : -1, k1 < end ? k1 : -1);
     }
   }
   int64_t per = (qn + nw - 1) / nw;
   per = per < 1 ? 1 : per > kWave ? kWave : per;
-  int* off = s_off[wv];
-  int* begs = s_beg[wv];
-  int* dus = s_du[DU ? wv : 0];
+  int* off = s.off[wv];
+  int* begs = s.beg[wv];
+  int* dus = s.du[DU ? wv : 0];
   for (int64_t c = wid * per; c < qn; c += nw * per) {  // wave-uniform
     int beg = 0, deg = 0, du = 0;
     if (lane < per && c + lane < qn) {
@@ -388,166 +417,6 @@ __device__ __forceinline__ void push_edges(const SsArgs& a, int lv, F&& edge) {
     }
     wave_lds_sync();
   }
-}
-
-// Clears the counter stripes of level lv (grid-stride).
-__device__ __forceinline__ void clear_stripes(const SsArgs& a, int lv, int64_t gt, int64_t gs) {
-  unsigned long long* p = a.part + (size_t)(lv % kRing) * kStripes * kStripeU64;
-  for (int64_t i = gt; i < kStripes * kStripeU64; i += gs) p[i] = 0ull;
-}
-
-// Level counters of a seed kernel: stripe 0 of the level (the others are
-// zero after the fill kernel) and the queue length in the ring.
-__device__ __forceinline__ void seed_counters(const SsArgs& a, int lv, const LevelCounters& c) {
-  a.ring[lv % kRing] = c;
-  unsigned long long* p = a.part + (size_t)(lv % kRing) * kStripes * kStripeU64;
-  p[0] = c.fv;
-  p[1] = c.fe;
-  p[2] = c.scout;
-}
-
-// ---------------------------------------------------------------- kernels ---
-
-__global__ void ss_fill_kernel(SsArgs a, int weighted) {
-  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
-  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int64_t i = t0; i < a.n; i += gs) a.dist[i] = kInf;
-  for (int64_t i = t0; i < 3 * a.words; i += gs) a.bm[i] = 0u;
-  if (t0 < kRing) a.ring[t0] = LevelCounters{};
-  for (int64_t i = t0; i < kPartU64; i += gs) a.part[i] = 0ull;
-  (void)weighted;
-}
-
-// Level 0 = {source}.  GAPBS starts scout_count at out_degree(source)
-// (test/gabps/bfs.cc:140).  One wave.
-__global__ void bfs_seed_kernel(SsArgs a, int32_t policy) {
-  if (blockIdx.x != 0) return;
-  const int32_t s = a.source;
-  const int rb = a.row_ptr[s], d = a.row_ptr[s + 1] - rb;
-  if (d > a.hchunk) put_chunks(a, a.hq, 0, s, rb, d, threadIdx.x, blockDim.x);
-  if (threadIdx.x != 0) return;
-  a.dist[s] = 0;
-  a.bm[s >> 5] |= 1u << (s & 31);
-  a.q[0] = s;
-  LevelCounters c{};
-  c.fv = 1;
-  c.fe = (unsigned)d;
-  c.scout = (unsigned)d;
-  c.flanes = 1;
-  if (d > a.hchunk) c.hqlen = (unsigned)((d + a.hchunk - 1) / a.hchunk);
-  else c.qlen = 1;
-  seed_counters(a, 0, c);
-  SchedState st{};
-  st.step = 0;
-  st.e2c = a.row_ptr[a.n];
-  st.scout = d;
-  st.force_mode = -1;
-  st.source = s;
-  st.last_mode = DAWN_MODE_PUSH;
-  *a.st = st;
-  (void)policy;
-}
-
-// Level 1 for min-plus, as SSSP_CPU::SSSP initialises it
-// (src/algorithm/cpu/sssp.cpp:40-46): every listed out-edge of the source
-// writes its weight in row order (a later duplicate overwrites an earlier
-// one), the distinct neighbours form the first frontier, distance[source]
-// = 0, and the source is never relaxed afterwards.  One workgroup: each
-// neighbour's slot first takes -1 - (its last listed edge) by atomicMin,
-// then that edge alone replaces it by its weight (weights are >= 0, so no
-// other edge of the neighbour matches).  A hub source's list in one thread
-// took 100k dependent round trips.
-constexpr int kSeedBlock = 1024;
-__global__ void __launch_bounds__(kSeedBlock) sssp_seed_kernel(SsArgs a) {
-  __shared__ unsigned s_len[2];
-  __shared__ unsigned long long s_c[3];
-  const int32_t s = a.source;
-  const int32_t b = a.row_ptr[s], e = a.row_ptr[s + 1];
-  if (threadIdx.x < 2) s_len[threadIdx.x] = 0u;
-  if (threadIdx.x < 3) s_c[threadIdx.x] = 0ull;
-  for (int32_t k = b + threadIdx.x; k < e; k += kSeedBlock) atomicMin(&a.dist[a.col[k]], -1 - k);
-  __syncthreads();
-  uint32_t* bm1 = a.bm + a.words;  // level 1 slot
-  int32_t* q1 = a.q + a.n;
-  int2* hq1 = a.hq + a.hcap;
-  for (int32_t k = b + threadIdx.x; k < e; k += kSeedBlock) {
-    const int32_t v = a.col[k];
-    if (__hip_atomic_load(&a.dist[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != -1 - k) continue;
-    __hip_atomic_store(&a.dist[v], a.w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (v == s) continue;
-    atomicOr(&bm1[v >> 5], 1u << (v & 31));
-    const int rb = a.row_ptr[v], d = a.row_ptr[v + 1] - rb;
-    if (d > a.hchunk)
-      put_chunks(a, hq1, atomicAdd(&s_len[1], (unsigned)((d + a.hchunk - 1) / a.hchunk)), v, rb, d, 0, 1);
-    else if (d > 0)
-      q1[atomicAdd(&s_len[0], 1u)] = v;
-    atomicAdd(&s_c[0], 1ull);
-    atomicAdd(&s_c[1], (unsigned long long)d);
-    atomicAdd(&s_c[2], (unsigned long long)(d > 0 ? d : 1));
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  __hip_atomic_store(&a.dist[s], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  LevelCounters c{};
-  c.fv = s_c[0];
-  c.fe = s_c[1];
-  c.scout = s_c[2];
-  c.flanes = c.fv;
-  c.qlen = s_len[0];
-  c.hqlen = s_len[1];
-  seed_counters(a, 1, c);
-  SchedState st{};
-  st.step = 1;
-  st.e2c = a.row_ptr[a.n];
-  st.scout = (long long)c.scout;
-  st.force_mode = -1;
-  st.source = s;
-  st.last_mode = DAWN_MODE_PUSH;
-  *a.st = st;
-}
-
-// One wave: sums the counter stripes of the last completed level into its
-// ring entry (an assignment, so running it twice is harmless), then decides.
-__global__ void ss_decide_kernel(SsArgs a, SchedParams p, SchedTrace tr) {
-  const SchedState s = *a.st;
-  if (!s.done) {
-    const int slot = s.step % kRing;
-    const unsigned long long* stripe =
-        a.part + ((size_t)slot * kStripes + lane_id()) * kStripeU64;
-    const unsigned long long fv = wave_sum_u64(stripe[0]);
-    const unsigned long long fe = wave_sum_u64(stripe[1]);
-    const unsigned long long sc = wave_sum_u64(stripe[2]);
-    if (threadIdx.x == 0) {
-      LevelCounters* c = a.ring + slot;
-      c->fv = fv;
-      c->fe = fe;
-      c->scout = sc;
-      c->flanes = fv;
-    }
-  }
-  sched_decide(a.st, a.ring, p, tr);
-  if (threadIdx.x == 0) {
-    SchedState* sp = a.st;
-    if (!sp->done && sp->mode == DAWN_MODE_PUSH &&
-        a.ring[(sp->step + kRing - 1) % kRing].qlen == kNoQueue) {
-      // The previous level has no queue: the same top-down step from its
-      // bitmap.
-      sp->mode = DAWN_MODE_BITMAP;
-      sp->last_mode = DAWN_MODE_BITMAP;
-      if (sp->step < kTraceMax && tr.mode) tr.mode[sp->step] = DAWN_MODE_BITMAP;
-    }
-  }
-}
-
-// Per-step housekeeping shared by the step kernels: clears the next level's
-// bitmap, ring entry and counter stripes.
-__device__ __forceinline__ void clear_next(const SsArgs& a, int lv) {
-  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
-  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t* bm_nx = a.bm + (int64_t)((lv + 1) % 3) * a.words;
-  for (int64_t i = gt; i < a.words; i += gs) bm_nx[i] = 0u;
-  if (gt == 0) a.ring[(lv + 1) % kRing] = LevelCounters{};
-  clear_stripes(a, lv + 1, gt, gs);
 }
 
 // Dense top-down over the frontier bitmap: vertices of out-degree < heavy
@@ -590,236 +459,704 @@ __device__ __forceinline__ void bitmap_edges(const SsArgs& a, const uint32_t* bm
   }
 }
 
-// One BOVM step: discovers level lv = st->step.
-__global__ void __launch_bounds__(kSsBlock, 8) bfs_expand_kernel(SsArgs a) {
-  const SchedState st = *a.st;
-  if (st.done) return;
-  const int lv = st.step;
-  const uint32_t* bm_in = a.bm + (int64_t)((lv + 2) % 3) * a.words;
-  uint32_t* bm_out = a.bm + (int64_t)(lv % 3) * a.words;
-  const int lane = lane_id();
-  clear_next(a, lv);
-  __shared__ SsStage sg;
-  sg.init();
-  Acc acc;
-  // An unreached head joins the level once: the first to set its bitmap bit.
-  auto discover = [&](int32_t v) {
-    const uint32_t bit = 1u << (v & 31);
-    if (atomicOr(&bm_out[v >> 5], bit) & bit) return false;
-    a.dist[v] = lv;
-    return true;
-  };
+// Clears what the next launch writes: its bitmap slot and its counters.
+__device__ __forceinline__ void clear_next(const SsArgs& a, int k) {
+  const int64_t gs = (int64_t)gridDim.x * blockDim.x;
+  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t* bm_nx = a.bm + (int64_t)((k + 2) % 3) * a.words;
+  for (int64_t i = gt; i < a.words; i += gs) bm_nx[i] = 0u;
+  unsigned long long* p = reinterpret_cast<unsigned long long*>(a.slots + ((k + 2) % kSsSlots));
+  for (int64_t i = gt; i < (int64_t)(sizeof(SsSlot) / 8); i += gs) p[i] = 0ull;
+}
 
-  if (st.mode == DAWN_MODE_PUSH) {
-    push_edges<false>(a, lv, [&](int, int, int k0, int k1) {
-      const int32_t v0 = k0 >= 0 ? a.col[k0] : 0, v1 = k1 >= 0 ? a.col[k1] : 0;
-      const bool c0 = k0 >= 0 && a.dist[v0] == kInf, c1 = k1 >= 0 && a.dist[v1] == kInf;
-      const bool d0 = c0 && discover(v0), d1 = c1 && discover(v1);
-      sg.append(a, d0, v0, lv, acc);
-      sg.append(a, d1, v1, lv, acc);
-    });
-  } else if (st.mode == DAWN_MODE_PULL) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.ring[lv % kRing].qlen = kNoQueue;  // bitmap only
-    const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
-    for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
-         base += wstride) {
-      const int32_t v = (int32_t)(base + lane);
-      int beg = 0, deg = 0;
-      if (v < a.n && a.dist[v] == kInf) {
-        beg = a.in_row_ptr[v];
-        deg = a.in_row_ptr[v + 1] - beg;
-      }
-      bool found = false;
-      // Rounds of four in-edges per lane (columns by one 16-byte load, probed
-      // two by two), until every lane has found a frontier tail or run out;
-      // of a heavy vertex only the first two rounds, the rest by the whole
-      // wave.  Bound by requests (each lane reads its own list and probes a
-      // word per edge), so probes past the first hit cost: 128 edges of a
-      // heavy vertex probed at once made a sparse step on RMAT scale 22 60%
-      // slower than 64.
-      const int lim = deg < kHeavyDegree ? deg : 8;
-      for (int j = 0; __ballot(!found && j < lim); j += 4) {
-        if (!found && j < lim) {
-          const int32_t* p = a.in_col + beg + j;
-          Cols4 u;
-          if (j + 4 <= deg) {
-            u = *reinterpret_cast<const Cols4*>(p);
-          } else {
-            const int r = deg - 1 - j;  // 0..2: repeat the last column
-            u = {{p[0], p[min(1, r)], p[r], p[r]}};
-          }
-          const bool f0 = test_bit(bm_in, u.c[0]), f1 = test_bit(bm_in, u.c[1]);
-          found = f0 || f1;
-          if (!found) {
-            const bool f2 = test_bit(bm_in, u.c[2]), f3 = test_bit(bm_in, u.c[3]);
-            found = f2 || f3;
-          }
-        }
-      }
-      uint64_t hm = __ballot(!found && deg >= kHeavyDegree);
-      while (hm) {
-        const int l = __ffsll((unsigned long long)hm) - 1;
-        hm &= hm - 1;
-        const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
-        bool f = false;
-        for (int k0 = hb + 8; k0 < he; k0 += kWave) {
-          const int k = k0 + lane;
-          const bool h = k < he && test_bit(bm_in, a.in_col[k]);
-          if (__ballot(h)) { f = true; break; }
-        }
-        if (lane == l) found = f;
-      }
-      if (found) a.dist[v] = lv;
-      const uint64_t fm = __ballot(found);
-      if (lane == 0) {
-        bm_out[base >> 5] = (uint32_t)fm;
-        bm_out[(base >> 5) + 1] = (uint32_t)(fm >> 32);
-      }
-      if (found) acc.add(a.row_ptr[v + 1] - a.row_ptr[v]);  // bitmap only: no queue entries
-    }
-  } else {  // DAWN_MODE_BITMAP
-    bitmap_edges<false>(a, bm_in, [&](int, int k) {
-      const int32_t v = k >= 0 ? a.col[k] : 0;
-      sg.append(a, k >= 0 && a.dist[v] == kInf && discover(v), v, lv, acc);
-    });
+// ---------------------------------------------------------------- kernels ---
+
+// Initial distances, bitmaps, counters; for BOVM also level 0 = {source}
+// (GAPBS starts scout_count at out_degree(source), test/gabps/bfs.cc:140).
+__global__ void __launch_bounds__(kBlock) ss_fill_kernel(SsArgs a, int bovm) {
+  const int64_t gs = (int64_t)gridDim.x * kBlock;
+  const int64_t gt = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int32_t s = a.source;
+  auto value = [&](int64_t v) { return bovm && v == s ? 0 : kInf; };
+  if (((uintptr_t)a.dist & 15) == 0) {
+    const int64_t n4 = a.n / 4;
+    for (int64_t i = gt; i < n4; i += gs)
+      reinterpret_cast<int4*>(a.dist)[i] =
+          make_int4(value(4 * i), value(4 * i + 1), value(4 * i + 2), value(4 * i + 3));
+    for (int64_t v = 4 * n4 + gt; v < a.n; v += gs) a.dist[v] = value(v);
+  } else {
+    for (int64_t v = gt; v < a.n; v += gs) a.dist[v] = value(v);
   }
-  sg.flush(a, acc, lv);
+  for (int64_t i = gt; i < 3 * a.words; i += gs)
+    a.bm[i] = bovm && i == s >> 5 ? 1u << (s & 31) : 0u;
+  if (blockIdx.x != 0) return;
+  unsigned long long* p = reinterpret_cast<unsigned long long*>(a.slots);
+  for (int i = threadIdx.x; i < (int)(kSsSlots * sizeof(SsSlot) / 8); i += kBlock) p[i] = 0ull;
+  for (int i = threadIdx.x; i < kStripes * kStripeU64; i += kBlock) a.tot[i] = 0ull;
+  __syncthreads();
+  SsState st{};
+  st.t0 = wall_clock64();
+  if (bovm) {
+    const int rb = a.row_ptr[s], d = a.row_ptr[s + 1] - rb;
+    if (d > a.hchunk) put_chunks(a, a.hq, 0, s, rb, d, threadIdx.x, kBlock);
+    if (threadIdx.x == 0) {
+      a.q[0] = s;
+      SsSlot& c = a.slots[0];
+      c.part[0][0] = 1ull;
+      c.part[0][1] = c.part[0][2] = (unsigned)d;
+      if (d > a.hchunk) c.hqlen = (unsigned)chunks_of(a, d);
+      else c.qlen = 1;
+      st.s.scout = d;
+    }
+  }
+  if (threadIdx.x == 0) {
+    st.s.e2c = a.row_ptr[a.n];
+    st.s.force_mode = -1;
+    st.s.source = s;
+    st.s.last_mode = DAWN_MODE_PUSH;
+    a.st[0] = st;
+  }
+}
+
+// Level 1 for min-plus, as SSSP_CPU::SSSP initialises it
+// (src/algorithm/cpu/sssp.cpp:40-46): every listed out-edge of the source
+// writes its weight in row order (a later duplicate overwrites an earlier
+// one), the distinct neighbours form the first frontier, distance[source]
+// = 0, and the source is never relaxed afterwards.  One workgroup: each
+// neighbour's slot first takes -1 - (its last listed edge) by atomicMin,
+// then that edge alone replaces it by its weight (weights are >= 0, so no
+// other edge of the neighbour matches).  A hub source's list in one thread
+// took 100k dependent round trips.
+__global__ void __launch_bounds__(kSsBlock) sssp_seed_kernel(SsArgs a) {
+  __shared__ unsigned s_len[2];
+  __shared__ unsigned long long s_c[3];
+  const int32_t s = a.source;
+  const int32_t b = a.row_ptr[s], e = a.row_ptr[s + 1];
+  if (threadIdx.x < 2) s_len[threadIdx.x] = 0u;
+  if (threadIdx.x < 3) s_c[threadIdx.x] = 0ull;
+  for (int32_t k = b + threadIdx.x; k < e; k += kSsBlock) atomicMin(&a.dist[a.col[k]], -1 - k);
+  __syncthreads();
+  for (int32_t k = b + threadIdx.x; k < e; k += kSsBlock) {
+    const int32_t v = a.col[k];
+    if (__hip_atomic_load(&a.dist[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != -1 - k) continue;
+    __hip_atomic_store(&a.dist[v], a.w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (v == s) continue;
+    atomicOr(&a.bm[v >> 5], 1u << (v & 31));
+    const int rb = a.row_ptr[v], d = a.row_ptr[v + 1] - rb;
+    if (d > a.hchunk)
+      put_chunks(a, a.hq, atomicAdd(&s_len[1], (unsigned)chunks_of(a, d)), v, rb, d, 0, 1);
+    else if (d > 0)
+      a.q[atomicAdd(&s_len[0], 1u)] = v;
+    atomicAdd(&s_c[0], 1ull);
+    atomicAdd(&s_c[1], (unsigned long long)d);
+    atomicAdd(&s_c[2], (unsigned long long)(d > 0 ? d : 1));
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  __hip_atomic_store(&a.dist[s], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  SsSlot& c = a.slots[0];
+  for (int i = 0; i < 3; i++) c.part[0][i] = s_c[i];
+  c.qlen = s_len[0];
+  c.hqlen = s_len[1];
+  a.tot[0] = 1 + s_c[0];
+  a.tot[1] = (unsigned long long)(e - b) + s_c[1];
+  SsState& st = a.st[0];
+  st.s.step = 1;
+  st.s.scout = (long long)s_c[2];
+}
+
+// An unreached head v joins level lv once: the first to set its bitmap bit.
+__device__ __forceinline__ bool discover(const SsArgs& a, int lv, int32_t v, uint32_t* bm_out) {
+  if (a.dist[v] != kInf) return false;
+  const uint32_t bit = 1u << (v & 31);
+  if (atomicOr(&bm_out[v >> 5], bit) & bit) return false;
+  a.dist[v] = lv;
+  return true;
 }
 
 // Relaxation of an edge to v of weight w with du = current distance of the
 // tail.  Returns true when v joins the next frontier for the first time this
 // level.
 __device__ __forceinline__ bool relax(const SsArgs& a, int32_t src, int32_t du, int32_t v,
-                                      int32_t w, uint32_t* bm_out) {
+                                      int32_t w, uint32_t* bm_out, Acc& acc) {
   if (v == src) return false;
-  const long long nd = (long long)du + (long long)w;
-  if (nd >= kInf) return false;
-  const int32_t ndi = (int32_t)nd;
-  if (ndi >= a.dist[v]) return false;
-  const int32_t old = atomicMin(&a.dist[v], ndi);
-  if (ndi >= old) return false;
+  const int32_t nd = minplus(du, w);
+  if (nd >= a.dist[v]) return false;
+  const int32_t old = atomicMin(&a.dist[v], nd);
+  if (nd >= old) return false;
+  if (old == kInf) acc.reach(a, v);
   const uint32_t bit = 1u << (v & 31);
-  const uint32_t prev = atomicOr(&bm_out[v >> 5], bit);
-  return (prev & bit) == 0;
+  return (atomicOr(&bm_out[v >> 5], bit) & bit) == 0;
 }
 
-// One min-plus step (GOVM/GOVMP semantics): relaxes the out-edges of the
-// vertices whose distance dropped in the previous step.
-__global__ void __launch_bounds__(kSsBlock, 8) sssp_expand_kernel(SsArgs a) {
-  const SchedState st = *a.st;
-  if (st.done) return;
-  const int32_t src = st.source;
-  const int lv = st.step;
-  const uint32_t* bm_in = a.bm + (int64_t)((lv + 2) % 3) * a.words;
-  uint32_t* bm_out = a.bm + (int64_t)(lv % 3) * a.words;
+// Counters of a completed level.
+struct SsLevel {
+  unsigned long long fv, fe, scout;
+  unsigned qlen, hqlen;
+};
+
+// What a step launch decides, in LDS; the same in every workgroup.
+struct SsCtl {
+  SsState st;  // state of the step to run (s.step = the level to discover)
+  SsLevel c;   // level s.step - 1
+  int run;     // 0: nothing left, 1: all workgroups expand, 2: one walks small levels
+  int fresh;   // run 0: this launch found the frontier empty
+  float x[8];
+};
+
+// Levels of at most kSmallEdges out-edges (and so at most as many vertices
+// found behind them) are walked by one workgroup, one after the other, within
+// a launch: a level costs about 4 us of dependent accesses there, and 9-12 us
+// as a step of its own (launch, decision, reservation of queue ranges, the
+// same accesses).  A level of 4000 edges takes one workgroup about 20 us, the
+// grid 12.  kSmallLevels bounds a launch on paths (about 20 ms).
+constexpr int kSmallEdges = 2048;
+constexpr int kSmallLevels = 4096;
+
+// Whether the level with counters c may be walked by one workgroup under
+// `mode`: its queue exists and holds every vertex with out-edges.
+__device__ __forceinline__ bool small_level(const SsLevel& c, int mode) {
+  return mode == DAWN_MODE_PUSH && c.qlen != kNoQueue && c.fe <= kSmallEdges && c.fv <= kSmallEdges;
+}
+
+// Mode of the step after the level with counters c, by the rule or the
+// forced policy; keeps the rule state current.  The learned network's choice
+// is made by the caller (it needs the workgroup).
+__device__ inline int ss_rule_mode(const SsRun& r, SchedState& s, const SsLevel& c) {
+  if (r.force >= 0) return r.force;
+  LevelCounters lc{};
+  lc.fv = c.fv;
+  lc.fe = c.fe;
+  lc.scout = c.scout;
+  const int mode = sched_fixed_mode(s, lc, r.p);
+  if (r.p.policy == DAWN_POLICY_PUSH) return DAWN_MODE_PUSH;
+  if (r.p.policy == DAWN_POLICY_PULL) return DAWN_MODE_PULL;
+  if (r.p.policy == DAWN_POLICY_BITMAP) return DAWN_MODE_BITMAP;
+  return mode;
+}
+
+__device__ __forceinline__ bool learned(const SsRun& r) {
+  return r.p.policy == DAWN_POLICY_LEARNED && r.p.mlp && r.force < 0;
+}
+
+// A frontier without a queue (after a pull step) is expanded top-down from
+// its bitmap.
+__device__ __forceinline__ int queue_mode(int mode, const SsLevel& c) {
+  return mode == DAWN_MODE_PUSH && c.qlen == kNoQueue ? DAWN_MODE_BITMAP : mode;
+}
+
+__device__ __forceinline__ void ss_advance(SchedState& s, const SsLevel& c, int mode) {
+  s.step += 1;
+  s.mode = mode;
+  s.last_mode = mode;
+  s.work_fv += c.fv;  // the level this step expands
+  s.work_fe += c.fe;
+}
+
+// Every workgroup decides from the same state and counters: a launch of its
+// own for the decision cost 4-5 us per step.  Called by all threads; the
+// result is in ctl after the last barrier.
+__device__ inline void ss_decide(const SsRun& r, int k, SsCtl& ctl) {
+  const SsArgs& a = r.a;
+  if (threadIdx.x < kWave) {
+    const SsSlot& slot = a.slots[k % kSsSlots];
+    SsState st = a.st[k % kSsSlots];
+    unsigned long long fv = slot.part[lane_id()][0], fe = slot.part[lane_id()][1],
+                       sc = slot.part[lane_id()][2];
+    const unsigned qlen = slot.qlen, hqlen = slot.hqlen;
+    fv = wave_sum_u64(fv);
+    fe = wave_sum_u64(fe);
+    sc = wave_sum_u64(sc);
+    if (threadIdx.x == 0) {
+      const SsLevel c{fv, fe, sc, qlen, hqlen};
+      ctl.c = c;
+      ctl.run = 0;
+      ctl.fresh = 0;
+      if (!st.s.done) {
+        if (c.fv == 0) {
+          st.s.done = 1;
+          st.s.levels = st.s.step;  // levels 0..step-1 are non-empty
+          ctl.fresh = 1;
+        } else {
+          const SchedState before = st.s;
+          const int mode = ss_rule_mode(r, st.s, c);
+          st.launches += 1;
+          // Small levels are pushed whatever the network would say.
+          ctl.run = r.small && small_level(c, learned(r) ? DAWN_MODE_PUSH : mode) ? 2 : 1;
+          if (ctl.run == 1 && (learned(r) || r.tr.feat)) {
+            LevelCounters lc{};
+            lc.fv = c.fv;
+            lc.fe = c.fe;
+            float x[8];
+            sched_features(lc, before.step + 1, r.p, before, x);
+            for (int i = 0; i < 8; i++) ctl.x[i] = x[i];
+          }
+          ss_advance(st.s, c, ctl.run == 2 ? DAWN_MODE_PUSH : queue_mode(mode, c));
+        }
+      }
+      ctl.st = st;
+    }
+  }
+  __syncthreads();
+  if (ctl.run == 1 && learned(r)) {
+    const int m = queue_mode(sched_mlp_mode(ctl.x, r.p), ctl.c);
+    if (threadIdx.x == 0) ctl.st.s.mode = ctl.st.s.last_mode = m;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && ctl.run) ctl.st.mode_steps[ctl.st.s.mode] += 1;
+}
+
+// LDS of the small-level walk: the level's vertices (min-plus: their slots in
+// a hash table that also holds their distances), then the scanned
+// out-degrees, first edges and distances of the level being expanded.
+template <bool MP>
+struct SmallLds {
+  static constexpr int kTab = MP ? 2 * kSmallEdges : 1;
+  int32_t q[kSmallEdges];
+  int off[kSmallEdges];
+  int beg[kSmallEdges];
+  int du[MP ? kSmallEdges : 1];
+  int32_t tab_v[kTab];
+  int32_t tab_d[kTab];
+  int scan[kSsWaves];
+  unsigned n, zero, hq, hn;
+  unsigned long long reach[2];
+};
+
+// Slot of v in the level's table (at most half full); *first: v was not there.
+template <bool MP>
+__device__ __forceinline__ unsigned tab_insert(SmallLds<MP>& s, int32_t v, bool* first) {
+  constexpr unsigned kTab = SmallLds<MP>::kTab;
+  unsigned h = ((unsigned)v * 2654435761u) % kTab;
+  for (;;) {
+    const int32_t old = atomicCAS(&s.tab_v[h], -1, v);
+    if (old == -1 || old == v) {
+      *first = old == -1;
+      return h;
+    }
+    h = (h + 1) % kTab;
+  }
+}
+
+// Walks levels in one workgroup, from level ctl.st.s.step on, until a level
+// is empty, too large, or the rule leaves PUSH; then writes the last level's
+// queue, bitmap bits and counters as a step of the whole grid would have left
+// them.  A level's edges are spread over the threads by one scan of its
+// vertices' out-degrees, so a level is one chain of three dependent accesses:
+// offsets, columns, and one atomicMin on the distance, whose old value tells
+// a first arrival (hop counts only grow) or an improvement.  The frontier
+// bitmap stays out of the loop: min-plus keeps the level's distinct vertices,
+// with their distances, in an LDS table.
+template <bool MP>
+__device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, SsCtl& ctl) {
+  constexpr int kPer = kSmallEdges / kSsBlock;
+  const SsArgs& a = run.a;
+  const int t = threadIdx.x;
+  const int32_t src = ctl.st.s.source;
+  const SsOut o = out_of(a, k);
+  auto clear_table = [&]() {
+    if (MP)
+      for (int i = t; i < SmallLds<MP>::kTab; i += kSsBlock) {
+        s.tab_v[i] = -1;
+        s.tab_d[i] = kInf;
+      }
+  };
+  {  // The level's vertices: the light queue and the first chunk of each heavy one.
+    const int32_t* q_in = a.q + (int64_t)(k & 1) * a.n;
+    const int2* hq_in = a.hq + (int64_t)(k & 1) * a.hcap;
+    const unsigned qn = ctl.c.qlen, hn = ctl.c.hqlen;
+    if (t == 0) s.n = 0u;
+    if (t < 2) s.reach[t] = 0ull;
+    clear_table();
+    __syncthreads();
+    for (unsigned i = t; i < qn + hn; i += kSsBlock) {
+      int32_t v;
+      if (i < qn) {
+        v = q_in[i];
+      } else {
+        const int2 h = hq_in[i - qn];
+        v = h.y == a.row_ptr[h.x] ? h.x : -1;
+      }
+      if (v < 0) continue;
+      if (MP) {
+        bool first;
+        const unsigned h = tab_insert(s, v, &first);
+        s.tab_d[h] = a.dist[v];
+        v = (int32_t)h;
+      }
+      s.q[atomicAdd(&s.n, 1u)] = v;
+    }
+    __syncthreads();
+  }
+  for (int it = 0;; it++) {
+    const unsigned cnt = s.n;
+    int32_t v[kPer];
+    int rb[kPer], d[kPer], du[MP ? kPer : 1], sum = 0;
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      const unsigned i = (unsigned)(t * kPer + r);
+      v[r] = -1;
+      rb[r] = d[r] = 0;
+      if (i < cnt) {
+        v[r] = MP ? s.tab_v[s.q[i]] : s.q[i];
+        if (MP) du[r] = s.tab_d[s.q[i]];
+        rb[r] = a.row_ptr[v[r]];
+        d[r] = a.row_ptr[v[r] + 1] - rb[r];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kPer; r++) sum += d[r];
+    if (t == 0) s.zero = 0u;
+    int total;
+    int off = ss_scan(sum, s.scan, &total);
+    if (t == 0) s.n = 0u;
+    clear_table();
+    if (it > 0) {  // the level just found: go on, or leave it to the grid?
+      int z = 0;
+#pragma unroll
+      for (int r = 0; r < kPer; r++) z += v[r] >= 0 && d[r] == 0;
+      if (z) atomicAdd(&s.zero, (unsigned)z);
+      __syncthreads();
+      if (t == 0) {
+        const SsLevel c{cnt, (unsigned long long)total, (unsigned long long)total + s.zero, cnt, 0u};
+        ctl.c = c;
+        if (cnt == 0) {
+          ctl.st.s.done = 1;
+          ctl.st.s.levels = ctl.st.s.step;
+          ctl.run = 0;
+          ctl.fresh = 1;
+        } else {
+          SchedState next = ctl.st.s;
+          const int mode = ss_rule_mode(run, next, c);
+          if (it < kSmallLevels && small_level(c, learned(run) ? DAWN_MODE_PUSH : mode)) {
+            ss_advance(next, c, DAWN_MODE_PUSH);
+            ctl.st.s = next;
+            ctl.st.mode_steps[DAWN_MODE_PUSH] += 1;
+          } else {
+            ctl.run = 1;
+          }
+        }
+      }
+      __syncthreads();
+      if (ctl.run != 2) {
+        if (MP && t < 2 && s.reach[t]) atomicAdd(&a.tot[t], s.reach[t]);
+        if (ctl.run == 1) {  // hand over
+          uint32_t* bm_out = a.bm + (int64_t)((k + 1) % 3) * a.words;
+          if (t == 0) s.hq = s.hn = 0u;
+          // Dealt out wave by wave, so that the chunk lists of neighbouring
+          // hubs are written by different waves.
+#pragma unroll
+          for (int r = 0; r < kPer; r++) s.off[t * kPer + r] = v[r];
+          __syncthreads();
+          for (int r = 0; r < kPer; r++) {
+            const int32_t x = s.off[r * kSsBlock + lane_id() * kSsWaves + t / kWave];
+            int xb = 0, xd = 0;
+            if (x >= 0) {
+              xb = a.row_ptr[x];
+              xd = a.row_ptr[x + 1] - xb;
+              atomicOr(&bm_out[x >> 5], 1u << (x & 31));
+            }
+            if (xd > 0 && xd <= a.hchunk) o.q[atomicAdd(&s.hq, 1u)] = x;
+            wave_put_chunks(a, o.hq, &s.hn, x, xb, xd);
+          }
+          __syncthreads();
+          if (t == 0) {
+            o.slot->part[0][0] = ctl.c.fv;
+            o.slot->part[0][1] = ctl.c.fe;
+            o.slot->part[0][2] = ctl.c.scout;
+            o.slot->qlen = s.hq;
+            o.slot->hqlen = s.hn;
+          }
+        }
+        return;
+      }
+    }
+    // Expand level step - 1 into level step.
+    const int lv = ctl.st.s.step;
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      const int i = t * kPer + r;
+      s.off[i] = off;
+      s.beg[i] = rb[r] - off;
+      if (MP) s.du[i] = du[r];
+      off += d[r];
+    }
+    __syncthreads();
+    int32_t hv[kPer], nd[kPer], old[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      const int e = t + r * kSsBlock;
+      hv[r] = -1;
+      nd[r] = lv;
+      if (e < total) {
+        int j = 0;  // the last entry that starts at or before e
+#pragma unroll
+        for (int w = kSmallEdges / 2; w >= 1; w >>= 1)
+          if (s.off[j + w] <= e) j += w;
+        const int ke = s.beg[j] + e;
+        hv[r] = a.col[ke];
+        if (MP) {
+          nd[r] = minplus(s.du[j], a.w[ke]);
+          if (hv[r] == src || nd[r] == kInf) hv[r] = -1;
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      old[r] = -1;
+      if (hv[r] >= 0) old[r] = atomicMin(&a.dist[hv[r]], nd[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      bool f = old[r] > nd[r];
+      if (MP && f) {
+        if (old[r] == kInf) {
+          atomicAdd(&s.reach[0], 1ull);
+          atomicAdd(&s.reach[1], (unsigned long long)(a.row_ptr[hv[r] + 1] - a.row_ptr[hv[r]]));
+        }
+        const unsigned h = tab_insert(s, hv[r], &f);
+        atomicMin(&s.tab_d[h], nd[r]);
+        hv[r] = (int32_t)h;
+      }
+      const int at = wave_append(&s.n, f);
+      if (f) s.q[at] = hv[r];
+    }
+    __syncthreads();
+  }
+}
+
+// The final state, once, to the host: the counts and the device time of the
+// traversal.  BOVM's levels are disjoint, so its expanded levels are the
+// vertices reached; min-plus counts first arrivals.
+template <bool MP>
+__device__ inline void ss_finish(const SsArgs& a, SsCtl& ctl) {
+  if (threadIdx.x >= kWave) return;
+  unsigned long long v = 0, e = 0;
+  if (MP) {
+    const unsigned long long* p = a.tot + lane_id() * kStripeU64;
+    v = wave_sum_u64(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    e = wave_sum_u64(__hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+  if (threadIdx.x != 0) return;
+  ctl.st.reached = MP ? v : ctl.st.s.work_fv;
+  ctl.st.edges = MP ? e : ctl.st.s.work_fe;
+  ctl.st.t1 = wall_clock64();
+  if (a.host) {
+    *a.host = ctl.st;
+    __threadfence_system();
+  }
+}
+
+// Unreached vertices look for a tail in the frontier bitmap; each vertex is
+// written only by its own lane.
+__device__ __forceinline__ void pull_bfs(const SsArgs& a, int lv, const uint32_t* bm_in,
+                                         uint32_t* bm_out, Acc& acc) {
   const int lane = lane_id();
-  clear_next(a, lv);
-  __shared__ SsStage sg;
+  const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
+  for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
+       base += wstride) {
+    const int32_t v = (int32_t)(base + lane);
+    int beg = 0, deg = 0;
+    if (v < a.n && a.dist[v] == kInf) {
+      beg = a.in_row_ptr[v];
+      deg = a.in_row_ptr[v + 1] - beg;
+    }
+    bool found = false;
+    // Rounds of four in-edges per lane (columns by one 16-byte load, probed
+    // two by two), until every lane has found a frontier tail or run out;
+    // of a heavy vertex only the first two rounds, the rest by the whole
+    // wave.  Bound by requests (each lane reads its own list and probes a
+    // word per edge), so probes past the first hit cost: 128 edges of a
+    // heavy vertex probed at once made a sparse step on RMAT scale 22 60%
+    // slower than 64.
+    const int lim = deg < kHeavyDegree ? deg : 8;
+    for (int j = 0; __ballot(!found && j < lim); j += 4) {
+      if (!found && j < lim) {
+        const int32_t* p = a.in_col + beg + j;
+        Cols4 u;
+        if (j + 4 <= deg) {
+          u = *reinterpret_cast<const Cols4*>(p);
+        } else {
+          const int r = deg - 1 - j;  // 0..2: repeat the last column
+          u = {{p[0], p[min(1, r)], p[r], p[r]}};
+        }
+        const bool f0 = test_bit(bm_in, u.c[0]), f1 = test_bit(bm_in, u.c[1]);
+        found = f0 || f1;
+        if (!found) {
+          const bool f2 = test_bit(bm_in, u.c[2]), f3 = test_bit(bm_in, u.c[3]);
+          found = f2 || f3;
+        }
+      }
+    }
+    uint64_t hm = __ballot(!found && deg >= kHeavyDegree);
+    while (hm) {
+      const int l = __ffsll((unsigned long long)hm) - 1;
+      hm &= hm - 1;
+      const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
+      bool f = false;
+      for (int k0 = hb + 8; k0 < he; k0 += kWave) {
+        const int k = k0 + lane;
+        const bool h = k < he && test_bit(bm_in, a.in_col[k]);
+        if (__ballot(h)) { f = true; break; }
+      }
+      if (lane == l) found = f;
+    }
+    if (found) a.dist[v] = lv;
+    const uint64_t fm = __ballot(found);
+    if (lane == 0) {
+      bm_out[base >> 5] = (uint32_t)fm;
+      bm_out[(base >> 5) + 1] = (uint32_t)(fm >> 32);
+    }
+    if (found) acc.add(a.row_ptr[v + 1] - a.row_ptr[v]);  // bitmap only: no queue entries
+  }
+}
+
+__device__ __forceinline__ void pull_minplus(const SsArgs& a, int32_t src, const uint32_t* bm_in,
+                                             uint32_t* bm_out, Acc& acc) {
+  const int lane = lane_id();
+  // Every vertex takes the minimum over its in-edges from frontier
+  // vertices; each vertex is written only by its own lane.
+  const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
+  for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
+       base += wstride) {
+    const int32_t v = (int32_t)(base + lane);
+    const bool cand = v < a.n && v != src;
+    int beg = 0, deg = 0;
+    int32_t cur = kInf;
+    if (cand) {
+      beg = a.in_row_ptr[v];
+      deg = a.in_row_ptr[v + 1] - beg;
+      cur = a.dist[v];
+    }
+    int32_t best = cur;
+    const bool light = cand && deg < kHeavyDegree;
+    const int maxd = wave_max_i32(light ? deg : 0);
+    for (int j = 0; j < maxd; j++) {
+      if (light && j < deg) {
+        const int32_t u = a.in_col[beg + j];
+        if (test_bit(bm_in, u)) {
+          long long nd = (long long)a.dist[u] + a.in_w[beg + j];
+          if (nd < best) best = (int32_t)nd;
+        }
+      }
+    }
+    uint64_t hm = __ballot(cand && deg >= kHeavyDegree);
+    while (hm) {
+      const int l = __ffsll((unsigned long long)hm) - 1;
+      hm &= hm - 1;
+      const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
+      int32_t hbest = kInf;
+      for (int k = hb + lane; k < he; k += kWave) {
+        const int32_t u = a.in_col[k];
+        if (test_bit(bm_in, u)) {
+          long long nd = (long long)a.dist[u] + a.in_w[k];
+          if (nd < hbest) hbest = (int32_t)nd;
+        }
+      }
+      for (int o = 32; o >= 1; o >>= 1) hbest = min(hbest, __shfl_xor(hbest, o));
+      if (lane == l && hbest < best) best = hbest;
+    }
+    const bool found = cand && best < cur;
+    if (found) {
+      a.dist[v] = best;
+      if (cur == kInf) acc.reach(a, v);
+    }
+    const uint64_t fm = __ballot(found);
+    if (lane == 0) {
+      bm_out[base >> 5] = (uint32_t)fm;
+      bm_out[(base >> 5) + 1] = (uint32_t)(fm >> 32);
+    }
+    if (found) acc.add(a.row_ptr[v + 1] - a.row_ptr[v]);  // bitmap only: no queue entries
+  }
+}
+
+// One step of the traversal: BOVM (discovers level lv) or min-plus
+// (GOVM/GOVMP semantics: relaxes the out-edges of the vertices whose distance
+// dropped in the previous step).  k: the launch's number modulo 12.
+template <bool MP>
+__global__ void __launch_bounds__(kSsBlock, 8) ss_step_kernel(SsRun run, int k) {
+  __shared__ SsCtl ctl;
+  __shared__ union {
+    struct {
+      SsStage sg;
+      PushLds<MP> push;
+    } wide;
+    SmallLds<MP> small;
+  } lds;
+  const SsArgs& a = run.a;
+  ss_decide(run, k, ctl);
+  if (ctl.run != 0) clear_next(a, k);
+  if (ctl.run != 1) {  // uniform over the grid: nothing left, or small levels
+    if (blockIdx.x != 0) return;
+    if (ctl.run == 2) {
+      small_levels<MP>(run, k, lds.small, ctl);
+      __syncthreads();
+    }
+    if (ctl.fresh) ss_finish<MP>(a, ctl);
+    if (threadIdx.x == 0) a.st[(k + 1) % kSsSlots] = ctl.st;
+    return;
+  }
+  const int lv = ctl.st.s.step, mode = ctl.st.s.mode;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    a.st[(k + 1) % kSsSlots] = ctl.st;
+    if (run.tr.mode && lv < kTraceMax) {
+      run.tr.mode[lv] = mode;
+      for (int i = 0; i < 8; i++) run.tr.feat[lv * 8 + i] = ctl.x[i];
+    }
+  }
+  const int32_t src = a.source;
+  const uint32_t* bm_in = a.bm + (int64_t)(k % 3) * a.words;
+  uint32_t* bm_out = a.bm + (int64_t)((k + 1) % 3) * a.words;
+  const SsOut o = out_of(a, k);
+  SsStage& sg = lds.wide.sg;
   sg.init();
   Acc acc;
-
-  if (st.mode == DAWN_MODE_PUSH) {
-    push_edges<true>(a, lv, [&](int du0, int du1, int k0, int k1) {
-      const int32_t v0 = k0 >= 0 ? a.col[k0] : 0, v1 = k1 >= 0 ? a.col[k1] : 0;
-      const int32_t w0 = k0 >= 0 ? a.w[k0] : 0, w1 = k1 >= 0 ? a.w[k1] : 0;
-      const bool d0 = k0 >= 0 && relax(a, src, du0, v0, w0, bm_out);
-      const bool d1 = k1 >= 0 && relax(a, src, du1, v1, w1, bm_out);
-      sg.append(a, d0, v0, lv, acc);
-      sg.append(a, d1, v1, lv, acc);
+  // Edge e (< 0: none) to the head v, tail distance du.
+  auto visit = [&](int e, int32_t v, int du, int32_t w) {
+    if (e < 0) return false;
+    return MP ? relax(a, src, du, v, w, bm_out, acc) : discover(a, lv, v, bm_out);
+  };
+  if (mode == DAWN_MODE_PUSH) {
+    push_edges<MP>(a, lds.wide.push, k, ctl.c.qlen, ctl.c.hqlen, [&](int du0, int du1, int e0, int e1) {
+      const int32_t v0 = e0 >= 0 ? a.col[e0] : 0, v1 = e1 >= 0 ? a.col[e1] : 0;
+      const int32_t w0 = MP && e0 >= 0 ? a.w[e0] : 0, w1 = MP && e1 >= 0 ? a.w[e1] : 0;
+      const bool f0 = visit(e0, v0, du0, w0), f1 = visit(e1, v1, du1, w1);
+      sg.append(a, o, f0, v0, acc);
+      sg.append(a, o, f1, v1, acc);
     });
-  } else if (st.mode == DAWN_MODE_PULL) {
-    // Every vertex takes the minimum over its in-edges from frontier
-    // vertices; each vertex is written only by its own lane.  Bitmap only:
-    // no queue entries.
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.ring[lv % kRing].qlen = kNoQueue;
-    const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
-    for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
-         base += wstride) {
-      const int32_t v = (int32_t)(base + lane);
-      const bool cand = v < a.n && v != src;
-      int beg = 0, deg = 0;
-      int32_t cur = kInf;
-      if (cand) {
-        beg = a.in_row_ptr[v];
-        deg = a.in_row_ptr[v + 1] - beg;
-        cur = a.dist[v];
-      }
-      int32_t best = cur;
-      const bool light = cand && deg < kHeavyDegree;
-      const int maxd = wave_max_i32(light ? deg : 0);
-      for (int j = 0; j < maxd; j++) {
-        if (light && j < deg) {
-          const int32_t u = a.in_col[beg + j];
-          if (test_bit(bm_in, u)) {
-            long long nd = (long long)a.dist[u] + a.in_w[beg + j];
-            if (nd < best) best = (int32_t)nd;
-          }
-        }
-      }
-      uint64_t hm = __ballot(cand && deg >= kHeavyDegree);
-      while (hm) {
-        const int l = __ffsll((unsigned long long)hm) - 1;
-        hm &= hm - 1;
-        const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
-        int32_t hbest = kInf;
-        for (int k = hb + lane; k < he; k += kWave) {
-          const int32_t u = a.in_col[k];
-          if (test_bit(bm_in, u)) {
-            long long nd = (long long)a.dist[u] + a.in_w[k];
-            if (nd < hbest) hbest = (int32_t)nd;
-          }
-        }
-        for (int o = 32; o >= 1; o >>= 1) hbest = min(hbest, __shfl_xor(hbest, o));
-        if (lane == l && hbest < best) best = hbest;
-      }
-      const bool found = cand && best < cur;
-      if (found) a.dist[v] = best;
-      const uint64_t fm = __ballot(found);
-      if (lane == 0) {
-        bm_out[base >> 5] = (uint32_t)fm;
-        bm_out[(base >> 5) + 1] = (uint32_t)(fm >> 32);
-      }
-      if (found) acc.add(a.row_ptr[v + 1] - a.row_ptr[v]);  // bitmap only: no queue entries
-    }
-  } else {  // DAWN_MODE_BITMAP (GOVMP shape: dense scan of the frontier)
-    bitmap_edges<true>(a, bm_in, [&](int du, int k) {
-      const int32_t v = k >= 0 ? a.col[k] : 0;
-      sg.append(a, k >= 0 && relax(a, src, du, v, a.w[k], bm_out), v, lv, acc);
+  } else if (mode == DAWN_MODE_BITMAP) {  // (min-plus: GOVMP shape)
+    bitmap_edges<MP>(a, bm_in, [&](int du, int e) {
+      const int32_t v = e >= 0 ? a.col[e] : 0;
+      sg.append(a, o, visit(e, v, du, MP && e >= 0 ? a.w[e] : 0), v, acc);
     });
+  } else {
+    // PULL: the bitmap only, no queue entries.
+    if (blockIdx.x == 0 && threadIdx.x == 0) o.slot->qlen = kNoQueue;
+    if constexpr (MP) pull_minplus(a, src, bm_in, bm_out, acc);
+    else pull_bfs(a, lv, bm_in, bm_out, acc);
   }
-  sg.flush(a, acc, lv);
+  sg.flush(a, o, acc);
 }
 
-// Sum of out-degree and count of reached vertices (GTEPS numerator):
-// wave sums, then one pair of atomics per workgroup (launched with at most
-// kReachBlocks workgroups: the two counters are single addresses).
-constexpr unsigned kReachBlocks = 512;
-__global__ void reach_kernel(const int32_t* dist, const int32_t* row_ptr, int32_t n,
-                             unsigned long long* out) {
-  __shared__ unsigned long long s_t[2];
-  if (threadIdx.x == 0) s_t[0] = s_t[1] = 0ull;
-  __syncthreads();
-  unsigned long long cnt = 0, edges = 0;
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-       v += (int64_t)gridDim.x * blockDim.x) {
-    if (dist[v] != kInf) {
-      cnt++;
-      edges += (unsigned)(row_ptr[v + 1] - row_ptr[v]);
-    }
-  }
-  cnt = wave_sum_u64(cnt);
-  edges = wave_sum_u64(edges);
-  if (lane_id() == 0 && cnt) {
-    atomicAdd(&s_t[0], cnt);
-    atomicAdd(&s_t[1], edges);
-  }
-  __syncthreads();
-  if (threadIdx.x < 2 && s_t[threadIdx.x]) atomicAdd(&out[threadIdx.x], s_t[threadIdx.x]);
+int ensure_ss(dawn_graph* g) {
+  if (!g->ss) g->ss = new SsWorkspace();
+  SsWorkspace* ws = g->ss;
+  if (ws->n == g->n && ws->st.p) return DAWN_OK;
+  ws->n = g->n;
+  ws->hcap = 2 * (g->m / kHeavyChunk) + 1;
+  DAWN_TRY(ws->q.alloc((size_t)2 * g->n));
+  DAWN_TRY(ws->hq.alloc((size_t)2 * ws->hcap));
+  DAWN_TRY(ws->bm.alloc((size_t)3 * (((int64_t)g->n + 63) / 64 * 2)));
+  DAWN_TRY(ws->slots.alloc(kSsSlots));
+  DAWN_TRY(ws->tot.alloc(kStripes * kStripeU64));
+  if (!ws->h_state) DAWN_HIP(hipHostMalloc((void**)&ws->h_state, sizeof(SsState)));
+  return ws->st.alloc(kSsSlots);
 }
 
-// Arguments that depend on the graph alone.
-SsArgs graph_args(const dawn_graph* g, int32_t source) {
-  SsArgs a{};
+// Launch arguments that depend on the graph and the call alone.
+SsRun make_run(const dawn_graph* g, int32_t source, int32_t policy) {
+  SsRun r{};
+  SsArgs& a = r.a;
   a.n = g->n;
   a.source = source;
   a.words = ((int64_t)g->n + 63) / 64 * 2;
@@ -834,67 +1171,7 @@ SsArgs graph_args(const dawn_graph* g, int32_t source) {
   a.oc_end = g->oc_end;
   a.num_oc = g->num_oc;
   a.heavy = g->knobs.heavy_degree;
-  return a;
-}
-
-// The same on the graph's workspace.
-SsArgs workspace_args(const dawn_graph* g, const SsWorkspace* ws, int32_t source) {
-  SsArgs a = graph_args(g, source);
-  a.dist = ws->dist.p;
-  a.q = ws->q.p;
-  a.hq = ws->hq.p;
-  a.hcap = ws->hcap;
-  a.hchunk = kHeavyChunk;
-  a.bm = ws->bm.p;
-  a.ring = ws->ring.p;
-  a.part = ws->part.p;
-  a.st = ws->st.p;
-  return a;
-}
-
-int ensure_ss(dawn_graph* g) {
-  if (!g->ss) g->ss = new SsWorkspace();
-  SsWorkspace* ws = g->ss;
-  if (ws->n == g->n && ws->dist.p) return DAWN_OK;
-  ws->n = g->n;
-  ws->words = ((int64_t)g->n + 63) / 64 * 2;
-  DAWN_TRY(ws->dist.alloc(g->n));
-  DAWN_TRY(ws->q.alloc((size_t)2 * g->n));
-  ws->hcap = 2 * (g->m / kHeavyChunk) + 1;
-  DAWN_TRY(ws->hq.alloc((size_t)2 * ws->hcap));
-  DAWN_TRY(ws->bm.alloc((size_t)3 * ws->words));
-  DAWN_TRY(ws->ring.alloc(kRing));
-  DAWN_TRY(ws->part.alloc(kPartU64));
-  DAWN_TRY(ws->st.alloc(1));
-  DAWN_TRY(ws->trace_feat.alloc((size_t)kTraceMax * 8));
-  DAWN_TRY(ws->trace_mode.alloc(kTraceMax));
-  DAWN_TRY(ws->reach.alloc(2));
-  if (!ws->h_state) DAWN_HIP(hipHostMalloc((void**)&ws->h_state, sizeof(SchedState)));
-  if (!ws->ev0) DAWN_HIP(hipEventCreate(&ws->ev0));
-  if (!ws->ev1) DAWN_HIP(hipEventCreate(&ws->ev1));
-  return DAWN_OK;
-}
-
-}  // namespace
-
-// Runs one single-source traversal.  kind 0: BOVM, 1: min-plus.
-// steps_per_chunk: decide+expand pairs per captured graph.
-int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out,
-                      int32_t policy, dawn_stats* stats, int32_t force_mode,
-                      float* trace_feat, int32_t* trace_mode, int32_t trace_max,
-                      int32_t* trace_rows) {
-  if (!g || source < 0 || source >= g->n) return DAWN_ERR_INVALID_ARG;
-  if (kind == 1 && !g->weighted) return DAWN_ERR_NOT_WEIGHTED;
-  if (g->h_row_ptr[source] == g->h_row_ptr[source + 1]) return DAWN_ERR_ISOLATED_SOURCE;
-  std::lock_guard<std::mutex> guard(g->lock);
-  DAWN_HIP(hipSetDevice(g->device));
-  DAWN_TRY(ensure_ss(g));
-  SsWorkspace* ws = g->ss;
-  hipStream_t s = g->stream;
-
-  const SsArgs a = workspace_args(g, ws, source);
-
-  SchedParams p{};
+  SchedParams& p = r.p;
   p.n = g->n;
   p.m = g->m;
   p.policy = policy;
@@ -904,129 +1181,122 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   p.allow_pull = 1;
   p.avg_degree = g->n ? (float)((double)g->m / g->n) : 0.f;
   p.max_degree = (float)g->max_out_degree;
+  r.force = -1;
+  r.small = 1;
+  return r;
+}
+
+// The graph's workspace.
+void use_workspace(SsRun& r, const SsWorkspace* ws) {
+  SsArgs& a = r.a;
+  a.dist = ws->dist.p;
+  a.q = ws->q.p;
+  a.hq = ws->hq.p;
+  a.hcap = ws->hcap;
+  a.hchunk = kHeavyChunk;
+  a.bm = ws->bm.p;
+  a.slots = ws->slots.p;
+  a.tot = ws->tot.p;
+  a.st = ws->st.p;
+}
+
+unsigned ss_grid(const dawn_graph* g) { return grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid); }
+
+int ss_start(const SsRun& r, int kind, hipStream_t s) {
+  ss_fill_kernel<<<grid_for(std::max<int64_t>(3 * r.a.words, r.a.n / 4)), kBlock, 0, s>>>(r.a, kind == 0);
+  if (kind) sssp_seed_kernel<<<1, kSsBlock, 0, s>>>(r.a);
+  DAWN_HIP(hipGetLastError());
+  return DAWN_OK;
+}
+
+void ss_step(const SsRun& r, int kind, int64_t k, unsigned grid, hipStream_t s) {
+  if (kind == 0) ss_step_kernel<false><<<grid, kSsBlock, 0, s>>>(r, (int)(k % 12));
+  else ss_step_kernel<true><<<grid, kSsBlock, 0, s>>>(r, (int)(k % 12));
+}
+
+// A whole traversal: the first `first` step launches, then more (twice as
+// many each time) while the frontier is not empty, one wait after each set.
+// A launch past the end costs 2-4 us, a wait too many about 15 us.  h: the
+// final state; without a pinned r.a.host it is copied from the device.
+int ss_traverse(const dawn_graph* g, const SsRun& r, int kind, int first, hipStream_t s, SsState* h) {
+  const unsigned grid = ss_grid(g);
+  const bool pinned = r.a.host != nullptr;
+  h->s.done = 0;
+  DAWN_TRY(ss_start(r, kind, s));
+  const int64_t limit = (int64_t)g->n + 2;
+  int64_t k = 0;
+  for (int K = first;; K = std::min(64, k == first ? 4 : 2 * K)) {
+    for (int i = 0; i < K; i++, k++) ss_step(r, kind, k, grid, s);
+    DAWN_HIP(hipGetLastError());
+    if (!pinned)
+      DAWN_HIP(hipMemcpyAsync(h, r.a.st + k % kSsSlots, sizeof(SsState), hipMemcpyDeviceToHost, s));
+    DAWN_HIP(hipStreamSynchronize(s));
+    if (h->s.done) return DAWN_OK;
+    if (k > limit) return DAWN_ERR_HIP;  // step bound exceeded
+  }
+}
+
+// Statistics of a finished traversal.
+int ss_stats(const dawn_graph* g, const SsState& h, dawn_stats* stats) {
+  int khz = 0;
+  DAWN_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g->device));
+  stats->device_ms += khz > 0 ? (double)(h.t1 - h.t0) / khz : 0.0;
+  stats->vertices_reached += (int64_t)h.reached;
+  stats->edges_reached += (int64_t)h.edges;
+  stats->batches += 1;
+  stats->frontier_edges += (int64_t)h.s.work_fe;
+  for (int m = 0; m < DAWN_NUM_MODES; m++) {
+    stats->steps += h.mode_steps[m];
+    stats->mode_steps[m] += h.mode_steps[m];
+  }
+  return DAWN_OK;
+}
+
+// Whether the traversal may run in the caller's buffer itself: plain memory
+// of the graph's own device, at int32 alignment.
+bool in_place(const dawn_graph* g, const void* p) {
+  if (!p || ((uintptr_t)p & 3)) return false;
+  hipPointerAttribute_t attr;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return attr.type == hipMemoryTypeDevice && attr.device == g->device;
+}
+
+}  // namespace
+
+// Runs one single-source traversal.  kind 0: BOVM, 1: min-plus.
+int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out, int32_t policy,
+                      dawn_stats* stats) {
+  if (!g || source < 0 || source >= g->n) return DAWN_ERR_INVALID_ARG;
+  if (kind == 1 && !g->weighted) return DAWN_ERR_NOT_WEIGHTED;
+  if (g->h_row_ptr[source] == g->h_row_ptr[source + 1]) return DAWN_ERR_ISOLATED_SOURCE;
+  std::lock_guard<std::mutex> guard(g->lock);
+  DAWN_HIP(hipSetDevice(g->device));
+  DAWN_TRY(ensure_ss(g));
+  SsWorkspace* ws = g->ss;
+  const bool direct = in_place(g, dist_out);
+  if (!direct) DAWN_TRY(ws->dist.alloc(g->n));
+  SsRun r = make_run(g, source, policy);
+  use_workspace(r, ws);
+  if (direct) r.a.dist = dist_out;
+  r.a.host = ws->h_state;
   // The single-source network (trained on single-source steps); without
   // one the learned policy takes the fixed rule.  Min-plus: the fixed rule.
-  p.mlp = kind == 0 ? sched_single_mlp_device(g->device, &p.mlp_norm) : nullptr;
-  if (kind == 1 && policy == DAWN_POLICY_LEARNED) p.policy = DAWN_POLICY_FIXED;
-  SchedTrace tr{ws->trace_feat.p, ws->trace_mode.p};
-
-  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid);
-  // A chunk = K decide+expand pairs, captured once per (kind, policy, mode,
-  // K).  Without a knob K is what the last traversal on this graph took
-  // (levels + 1, rounded up to even), so that one chunk and one read of the
-  // done flag usually suffice (BFS on ER n=65,536, 9 levels: 0.20 ms with
-  // K = 8, 0.156 ms with K = 10).
-  int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : (g->n < (1 << 20) ? 8 : 16);
-  if (g->knobs.ss_chunk <= 0 && ws->last_pairs[kind] > 0)
-    K = std::min(128, (ws->last_pairs[kind] + 1) & ~1);
-  // Launch arguments are baked into the graph: key it by every one that
-  // varies between calls (the network pointer changes when one is installed).
-  const std::pair<long long, const void*> key{
-      ((long long)kind << 40) | ((long long)(policy & 0xff) << 32) |
-          ((long long)(force_mode + 1) << 16) | K,
-      (const void*)p.mlp};
-  hipGraphExec_t exec = nullptr;
-  auto it = ws->graphs.find(key);
-  if (it != ws->graphs.end()) {
-    exec = it->second;
-  } else {
-    hipGraph_t graph;
-    DAWN_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < K; i++) {
-      ss_decide_kernel<<<1, 64, 0, s>>>(a, p, tr);
-      if (kind == 0)
-        bfs_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
-      else
-        sssp_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
-    }
-    DAWN_HIP(hipStreamEndCapture(s, &graph));
-    hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    DAWN_HIP(e);
-    ws->graphs[key] = exec;
-  }
-
-  DAWN_HIP(hipEventRecord(ws->ev0, s));
-  ss_fill_kernel<<<grid_for(std::max<int64_t>(3 * ws->words, g->n)), kBlock, 0, s>>>(a, kind);
-  if (kind == 0)
-    bfs_seed_kernel<<<1, 64, 0, s>>>(a, policy);
-  else
-    sssp_seed_kernel<<<1, kSeedBlock, 0, s>>>(a);
-  DAWN_HIP(hipGetLastError());
-  if (force_mode >= 0) {
-    // The seed kernel leaves force_mode = -1; set it before stepping.
-    const int32_t fm = force_mode;
-    DAWN_HIP(hipMemcpyAsync(&ws->st.p->force_mode, &fm, sizeof(int32_t),
-                            hipMemcpyHostToDevice, s));
-    DAWN_HIP(hipStreamSynchronize(s));
-  }
-  int64_t launched = 0;
-  const int64_t limit = (int64_t)g->n + 2;
-  for (;;) {
-    DAWN_HIP(hipGraphLaunch(exec, s));
-    launched += K;
-    DAWN_HIP(hipMemcpyAsync(ws->h_state, ws->st.p, sizeof(SchedState),
-                            hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
-    if (ws->h_state->done || launched > limit) break;
-  }
-  DAWN_HIP(hipEventRecord(ws->ev1, s));
-  DAWN_HIP(hipEventSynchronize(ws->ev1));
-  float ms = 0.f;
-  DAWN_HIP(hipEventElapsedTime(&ms, ws->ev0, ws->ev1));
-  if (!ws->h_state->done) return DAWN_ERR_HIP;  // step bound exceeded
-
-  const int levels = ws->h_state->levels;
-  const int first_step = kind == 0 ? 1 : 2;
-  // Decides that ran: one per expanded level after the seeded ones, plus
-  // the one that found the frontier empty.
-  ws->last_pairs[kind] = std::max(1, levels - first_step + 2);
-  if (stats) {
-    DAWN_HIP(hipMemsetAsync(ws->reach.p, 0, 2 * sizeof(unsigned long long), s));
-    reach_kernel<<<grid_for(g->n, kBlock, kReachBlocks), kBlock, 0, s>>>(ws->dist.p, g->row_ptr, g->n, ws->reach.p);
-    unsigned long long rr[2];
-    DAWN_HIP(hipMemcpyAsync(rr, ws->reach.p, sizeof rr, hipMemcpyDeviceToHost, s));
-    // Trace entries 1..levels hold the modes of the expanding steps.
-    std::vector<int32_t> modes(levels + 1);
-    const int nrec = std::min(levels + 1, kTraceMax);
-    if (nrec > 0)
-      DAWN_HIP(hipMemcpyAsync(modes.data(), ws->trace_mode.p, sizeof(int32_t) * nrec,
-                              hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
-    stats->device_ms += ms;
-    stats->vertices_reached += (int64_t)rr[0];
-    stats->edges_reached += (int64_t)rr[1];
-    stats->batches += 1;
-    stats->frontier_edges += (int64_t)ws->h_state->work_fe;
-    // Steps first_step..levels expanded a level; the final step found none.
-    for (int st = first_step; st <= levels && st < kTraceMax; st++) {
-      stats->steps += 1;
-      int md = modes[st];
-      if (md >= 0 && md < DAWN_NUM_MODES) stats->mode_steps[md] += 1;
-    }
-  }
-  if (trace_rows) {
-    int rows = 0;
-    int nrec = std::min(levels + 1, kTraceMax);
-    std::vector<int32_t> modes(nrec);
-    std::vector<float> feat((size_t)nrec * 8);
-    DAWN_HIP(hipMemcpyAsync(modes.data(), ws->trace_mode.p, sizeof(int32_t) * nrec,
-                            hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipMemcpyAsync(feat.data(), ws->trace_feat.p, sizeof(float) * 8 * nrec,
-                            hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
-    for (int st = first_step; st <= levels && st < nrec && rows < trace_max; st++, rows++) {
-      if (trace_mode) trace_mode[rows] = modes[st];
-      if (trace_feat)
-        for (int i = 0; i < 8; i++) trace_feat[rows * 8 + i] = feat[(size_t)st * 8 + i];
-    }
-    *trace_rows = rows;
-  }
-  if (dist_out) {
-    const bool dev = is_device_pointer(dist_out);
-    DAWN_HIP(hipMemcpyAsync(dist_out, ws->dist.p, sizeof(int32_t) * g->n,
-                            dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
+  r.p.mlp = kind == 0 ? sched_single_mlp_device(g->device, &r.p.mlp_norm) : nullptr;
+  if (kind == 1 && policy == DAWN_POLICY_LEARNED) r.p.policy = DAWN_POLICY_FIXED;
+  // Launches before the first look at the done flag: the knob, else what the
+  // last traversal of this kind on the graph took (and the one that finds
+  // the frontier empty).
+  int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : 8;
+  if (g->knobs.ss_chunk <= 0 && ws->last_launches[kind] > 0) K = std::min(256, ws->last_launches[kind]);
+  DAWN_TRY(ss_traverse(g, r, kind, K, g->stream, ws->h_state));
+  ws->last_launches[kind] = ws->h_state->launches + 1;
+  if (stats) DAWN_TRY(ss_stats(g, *ws->h_state, stats));
+  if (dist_out && !direct) {
+    DAWN_HIP(hipMemcpyAsync(dist_out, ws->dist.p, sizeof(int32_t) * g->n, hipMemcpyDefault, g->stream));
+    DAWN_HIP(hipStreamSynchronize(g->stream));
   }
   return DAWN_OK;
 }
@@ -1037,40 +1307,31 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
 // of vertices at hop distance l, whatever the modes of the steps before), so
 // a step starts from the same state in every run: one BOVM traversal per
 // mode with that mode forced, each step launched on its own with HIP events
-// around the expand kernel, gives the time of every mode at every step
+// around the step kernel, gives the time of every mode at every step
 // (minimum over `repeats` traversals); one traversal under `policy` gives
 // the step features and the policy's choices.
 
 namespace {
 
-// One traversal from a.source, step by step.  force < 0: the policy's
-// choices, else that mode at every step.  times: expand-kernel time of each
+// One traversal from r.a.source, step by step.  times: kernel time of each
 // step (steps 1..levels).
-int ss_stepwise(dawn_graph* g, SsWorkspace* ws, const SsArgs& a, const SchedParams& p,
-                SchedTrace tr, int force, unsigned grid, std::vector<float>* times,
-                int* levels) {
+int ss_stepwise(dawn_graph* g, SsWorkspace* ws, const SsRun& r, std::vector<float>* times, int* levels) {
   hipStream_t s = g->stream;
-  ss_fill_kernel<<<grid_for(std::max<int64_t>(3 * ws->words, g->n)), kBlock, 0, s>>>(a, 0);
-  bfs_seed_kernel<<<1, 64, 0, s>>>(a, p.policy);
-  DAWN_HIP(hipGetLastError());
-  if (force >= 0) {
-    const int32_t fm = force;
-    DAWN_HIP(hipMemcpyAsync(&ws->st.p->force_mode, &fm, sizeof(int32_t), hipMemcpyHostToDevice, s));
-  }
+  const unsigned grid = ss_grid(g);
+  DAWN_TRY(ss_start(r, 0, s));
   times->clear();
   for (int64_t k = 0; k <= (int64_t)g->n + 1; k++) {
-    ss_decide_kernel<<<1, 64, 0, s>>>(a, p, tr);
-    DAWN_HIP(hipMemcpyAsync(ws->h_state, ws->st.p, sizeof(SchedState), hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
-    if (ws->h_state->done) {
-      *levels = ws->h_state->levels;
-      return DAWN_OK;
-    }
     DAWN_HIP(hipEventRecord(ws->ev0, s));
-    bfs_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
+    ss_step(r, 0, k, grid, s);
     DAWN_HIP(hipGetLastError());
     DAWN_HIP(hipEventRecord(ws->ev1, s));
-    DAWN_HIP(hipEventSynchronize(ws->ev1));
+    DAWN_HIP(hipMemcpyAsync(ws->h_state, ws->st.p + (k + 1) % kSsSlots, sizeof(SsState),
+                            hipMemcpyDeviceToHost, s));
+    DAWN_HIP(hipStreamSynchronize(s));
+    if (ws->h_state->s.done) {
+      *levels = ws->h_state->s.levels;
+      return DAWN_OK;
+    }
     float ms = 0.f;
     DAWN_HIP(hipEventElapsedTime(&ms, ws->ev0, ws->ev1));
     times->push_back(ms);
@@ -1091,7 +1352,11 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
   DAWN_HIP(hipSetDevice(g->device));
   DAWN_TRY(ensure_ss(g));
   SsWorkspace* ws = g->ss;
-  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid);
+  DAWN_TRY(ws->dist.alloc(g->n));
+  DAWN_TRY(ws->trace_feat.alloc((size_t)kTraceMax * 8));
+  DAWN_TRY(ws->trace_mode.alloc(kTraceMax));
+  if (!ws->ev0) DAWN_HIP(hipEventCreate(&ws->ev0));
+  if (!ws->ev1) DAWN_HIP(hipEventCreate(&ws->ev1));
   int32_t rows = 0;
   std::vector<float> t, feat;
   std::vector<int32_t> modes;
@@ -1099,22 +1364,14 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
     int64_t src = sources[i] % (int64_t)g->n;
     if (src < 0) src += g->n;
     if (g->h_row_ptr[src] == g->h_row_ptr[src + 1]) continue;  // isolated: no traversal
-    const SsArgs a = workspace_args(g, ws, (int32_t)src);
-    SchedParams p{};
-    p.n = g->n;
-    p.m = g->m;
-    p.policy = policy;
-    p.alpha = 15;
-    p.beta = 18;
-    p.batched = 0;
-    p.allow_pull = 1;
-    p.avg_degree = g->n ? (float)((double)g->m / g->n) : 0.f;
-    p.max_degree = (float)g->max_out_degree;
-    p.mlp = sched_single_mlp_device(g->device, &p.mlp_norm);
-    SchedTrace tr{ws->trace_feat.p, ws->trace_mode.p};
+    SsRun r = make_run(g, (int32_t)src, policy);
+    use_workspace(r, ws);
+    r.p.mlp = sched_single_mlp_device(g->device, &r.p.mlp_norm);
+    r.tr = SchedTrace{ws->trace_feat.p, ws->trace_mode.p};
+    r.small = 0;  // every level a step of its own
     // The policy's run: features and choices of steps 1..levels.
     int levels = 0;
-    DAWN_TRY(ss_stepwise(g, ws, a, p, tr, -1, grid, &t, &levels));
+    DAWN_TRY(ss_stepwise(g, ws, r, &t, &levels));
     const int nrec = std::min(levels + 1, kTraceMax);
     modes.assign(nrec, 0);
     feat.assign((size_t)nrec * 8, 0.f);
@@ -1123,9 +1380,10 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
     // Every mode forced, minimum over the repeats.
     std::vector<float> best((size_t)levels * DAWN_NUM_MODES, 1e30f);
     for (int m = 0; m < DAWN_NUM_MODES; m++)
-      for (int r = 0; r < repeats; r++) {
+      for (int rep = 0; rep < repeats; rep++) {
         int lv = 0;
-        DAWN_TRY(ss_stepwise(g, ws, a, p, tr, m, grid, &t, &lv));
+        r.force = m;
+        DAWN_TRY(ss_stepwise(g, ws, r, &t, &lv));
         if (lv != levels || (int)t.size() != levels) return DAWN_ERR_HIP;  // modes must agree
         for (int k = 0; k < levels; k++)
           best[(size_t)k * DAWN_NUM_MODES + m] = std::min(best[(size_t)k * DAWN_NUM_MODES + m], t[k]);
@@ -1154,15 +1412,13 @@ int run_ss_record(dawn_graph* g, const int32_t* sources, int32_t S, int32_t repe
 // first call takes its device address from hipGetSymbolAddress and keeps it
 // per device; every kernel argument and copy uses that address.
 //
-// Every call re-initialises what it reads (fill and seed kernels, a zeroing
-// kernel for the reach counters).  Calls on one GPU share the array, so the
-// calls of a process are serialised per device by a lock (two calls that
-// overlapped on one GPU would race).  The step loop is launched directly,
-// K decide+expand pairs between reads of the done flag: instantiating a
-// captured graph would allocate.  The single-source scheduler network is
-// used only if it is already on the device (installing it allocates);
-// otherwise the learned policy falls back to the fixed rule, as when no
-// network is set.
+// Every call re-initialises what it reads.  Calls on one GPU share the array,
+// so the calls of a process are serialised per device by a lock (two calls
+// that overlapped on one GPU would race).  The final state is copied from the
+// device (pinned memory would have to be allocated), after sets of step
+// launches.  The single-source scheduler network is used only if it is
+// already on the device (installing it allocates); otherwise the learned
+// policy falls back to the fixed rule, as when no network is set.
 
 constexpr int32_t kNoAllocMaxN = 1 << 22;
 constexpr int kNoAllocMaxDevices = 64;
@@ -1174,13 +1430,10 @@ constexpr size_t kNaQ = align256(kNaDist + sizeof(int32_t) * (size_t)kNoAllocMax
 constexpr size_t kNaHq = align256(kNaQ + sizeof(int32_t) * 2 * (size_t)kNoAllocMaxN);
 constexpr int64_t kNoAllocHeavy = 1 << 18;  // heavy-chunk entries per level
 constexpr size_t kNaBm = align256(kNaHq + sizeof(int2) * 2 * (size_t)kNoAllocHeavy);
-constexpr size_t kNaRing = align256(kNaBm + sizeof(uint32_t) * 3 * (size_t)kNoAllocWords);
-constexpr size_t kNaPart = align256(kNaRing + sizeof(LevelCounters) * kRing);
-constexpr size_t kNaState = align256(kNaPart + sizeof(unsigned long long) * kPartU64);
-constexpr size_t kNaFeat = align256(kNaState + sizeof(SchedState));
-constexpr size_t kNaMode = align256(kNaFeat + sizeof(float) * 8 * (size_t)kTraceMax);
-constexpr size_t kNaReach = align256(kNaMode + sizeof(int32_t) * (size_t)kTraceMax);
-constexpr size_t kNoAllocBytes = align256(kNaReach + 2 * sizeof(unsigned long long));
+constexpr size_t kNaSlots = align256(kNaBm + sizeof(uint32_t) * 3 * (size_t)kNoAllocWords);
+constexpr size_t kNaTot = align256(kNaSlots + sizeof(SsSlot) * kSsSlots);
+constexpr size_t kNaState = align256(kNaTot + sizeof(unsigned long long) * kStripes * kStripeU64);
+constexpr size_t kNoAllocBytes = align256(kNaState + sizeof(SsState) * kSsSlots);
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -1188,11 +1441,6 @@ namespace {
 
 std::mutex g_noalloc_lock[kNoAllocMaxDevices];
 unsigned char* g_noalloc_base[kNoAllocMaxDevices] = {};  // device address of `scratch`
-
-__global__ void zero_u64_kernel(unsigned long long* p, int count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) p[i] = 0ull;
-}
 
 }  // namespace
 
@@ -1215,9 +1463,8 @@ int run_bfs_noalloc(dawn_graph* g, int32_t source, int32_t* dist_out, int32_t po
     if (!base) return DAWN_ERR_HIP;
     g_noalloc_base[g->device] = base;
   }
-  hipStream_t s = g->stream;
-
-  SsArgs a = graph_args(g, source);
+  SsRun r = make_run(g, source, policy);
+  SsArgs& a = r.a;
   a.dist = (int32_t*)(base + kNaDist);
   a.q = (int32_t*)(base + kNaQ);
   a.hq = (int2*)(base + kNaHq);
@@ -1226,75 +1473,29 @@ int run_bfs_noalloc(dawn_graph* g, int32_t source, int32_t* dist_out, int32_t po
   a.hchunk = kHeavyChunk;
   while (2 * (g->m / a.hchunk) + 1 > kNoAllocHeavy) a.hchunk *= 2;
   a.bm = (uint32_t*)(base + kNaBm);
-  a.ring = (LevelCounters*)(base + kNaRing);
-  a.part = (unsigned long long*)(base + kNaPart);
-  a.st = (SchedState*)(base + kNaState);
-  unsigned long long* reach = (unsigned long long*)(base + kNaReach);
-
-  SchedParams p{};
-  p.n = g->n;
-  p.m = g->m;
-  p.policy = policy;
-  p.alpha = 15;
-  p.beta = 18;
-  p.batched = 0;
-  p.allow_pull = 1;
-  p.avg_degree = g->n ? (float)((double)g->m / g->n) : 0.f;
-  p.max_degree = (float)g->max_out_degree;
-  p.mlp = sched_single_mlp_if_present(g->device, &p.mlp_norm);
-  SchedTrace tr{(float*)(base + kNaFeat), (int32_t*)(base + kNaMode)};
-
-  const unsigned grid = grid_for(std::max<int64_t>(g->n, 1), kSsBlock, kSsGrid);
-  const int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : (g->n < (1 << 20) ? 8 : 16);
+  a.slots = (SsSlot*)(base + kNaSlots);
+  a.tot = (unsigned long long*)(base + kNaTot);
+  a.st = (SsState*)(base + kNaState);
+  r.p.mlp = sched_single_mlp_if_present(g->device, &r.p.mlp_norm);
+  const int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : 8;
   const auto t0 = std::chrono::steady_clock::now();
-  ss_fill_kernel<<<grid_for(std::max<int64_t>(3 * a.words, g->n)), kBlock, 0, s>>>(a, 0);
-  bfs_seed_kernel<<<1, 64, 0, s>>>(a, policy);
-  DAWN_HIP(hipGetLastError());
-  SchedState h_state{};
-  int64_t launched = 0;
-  const int64_t limit = (int64_t)g->n + 2;
-  for (;;) {
-    for (int i = 0; i < K; i++) {
-      ss_decide_kernel<<<1, 64, 0, s>>>(a, p, tr);
-      bfs_expand_kernel<<<grid, kSsBlock, 0, s>>>(a);
-    }
-    DAWN_HIP(hipGetLastError());
-    launched += K;
-    DAWN_HIP(hipMemcpyAsync(&h_state, a.st, sizeof(SchedState), hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
-    if (h_state.done || launched > limit) break;
-  }
+  SsState h{};
+  DAWN_TRY(ss_traverse(g, r, 0, K, g->stream, &h));
   const double ms =
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  if (!h_state.done) return DAWN_ERR_HIP;  // step bound exceeded
-
   if (stats) {
-    const int levels = h_state.levels;
-    zero_u64_kernel<<<1, 64, 0, s>>>(reach, 2);
-    reach_kernel<<<grid_for(g->n, kBlock, kReachBlocks), kBlock, 0, s>>>(a.dist, g->row_ptr, g->n, reach);
-    DAWN_HIP(hipGetLastError());
-    unsigned long long rr[2];
-    DAWN_HIP(hipMemcpyAsync(rr, reach, sizeof rr, hipMemcpyDeviceToHost, s));
-    // Trace entries 1..levels hold the modes of the expanding steps.
-    std::vector<int32_t> modes(levels + 1);
-    const int nrec = std::min(levels + 1, kTraceMax);
-    if (nrec > 0)
-      DAWN_HIP(hipMemcpyAsync(modes.data(), tr.mode, sizeof(int32_t) * nrec,
-                              hipMemcpyDeviceToHost, s));
-    DAWN_HIP(hipStreamSynchronize(s));
+    dawn_stats st{};
+    DAWN_TRY(ss_stats(g, h, &st));
     stats->device_ms += ms;
-    stats->vertices_reached += (int64_t)rr[0];
-    stats->edges_reached += (int64_t)rr[1];
+    stats->vertices_reached += st.vertices_reached;
+    stats->edges_reached += st.edges_reached;
     stats->batches += 1;
-    for (int st = 1; st <= levels && st < kTraceMax; st++) {
-      stats->steps += 1;
-      const int md = modes[st];
-      if (md >= 0 && md < DAWN_NUM_MODES) stats->mode_steps[md] += 1;
-    }
+    stats->steps += st.steps;
+    for (int m = 0; m < DAWN_NUM_MODES; m++) stats->mode_steps[m] += st.mode_steps[m];
   }
   if (dist_out) {
-    DAWN_HIP(hipMemcpyAsync(dist_out, a.dist, sizeof(int32_t) * g->n, hipMemcpyDefault, s));
-    DAWN_HIP(hipStreamSynchronize(s));
+    DAWN_HIP(hipMemcpyAsync(dist_out, a.dist, sizeof(int32_t) * g->n, hipMemcpyDefault, g->stream));
+    DAWN_HIP(hipStreamSynchronize(g->stream));
   }
   return DAWN_OK;
 }

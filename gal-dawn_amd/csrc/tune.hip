@@ -4,7 +4,7 @@
 //
 // Knobs (dawn::TuneKnobs): grid cap of the batched dense kernels, the degree
 // from which edge lists are cut into wave chunks, the chunk length, the
-// single-source steps per captured hipGraph, the light-pull variant, the
+// single-source step launches per wait, the light-pull variant, the
 // batch width and the hub-first order.  dawn_tune sweeps them on a graph
 // (coordinate descent from the graph's current knobs), applies the winner
 // to the graph and caches it for the graph's class (log2 n, log2 average
@@ -35,8 +35,7 @@ namespace dawn {
 int run_msbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64_t* sums,
               int64_t* reached, int64_t* edges, int32_t policy, dawn_stats* stats, bool rows);
 int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out, int32_t policy,
-                      dawn_stats* stats, int32_t force_mode, float* trace_feat,
-                      int32_t* trace_mode, int32_t trace_max, int32_t* trace_rows);
+                      dawn_stats* stats);
 
 namespace {
 std::mutex g_tune_lock;
@@ -59,8 +58,7 @@ int sample_ms(dawn_graph* g, const std::vector<int32_t>& src, double* ms) {
     dawn_stats st{};
     if (g->weighted) {
       for (int32_t s : src)
-        DAWN_TRY(run_single_source(g, 1, s, nullptr, DAWN_POLICY_FIXED, &st, -1, nullptr, nullptr,
-                                   0, nullptr));
+        DAWN_TRY(run_single_source(g, 1, s, nullptr, DAWN_POLICY_FIXED, &st));
     } else {
       // The learned schedule where a network is installed (the fixed rule
       // otherwise), as traversals run by default.

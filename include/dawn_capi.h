@@ -73,7 +73,7 @@ typedef struct dawn_csr {
 
 /* Per-call statistics. */
 typedef struct dawn_stats {
-  double device_ms;          /* HIP-event time of the traversal            */
+  double device_ms;          /* device time of the traversal               */
   int64_t steps;             /* frontier steps executed (summed over batches) */
   int64_t mode_steps[DAWN_NUM_MODES];
   int64_t edges_reached;     /* sum over sources of out-degree of reached vertices */
@@ -403,7 +403,7 @@ int dawn_tune_save(const char* path);
 
 /* The knobs of one graph, in the order of DAWN_KNOB_*: grid cap of the
  * dense batched kernels, degree from which edge lists are cut into wave
- * chunks, chunk length, single-source steps per captured graph (0 = auto),
+ * chunks, chunk length, single-source step launches per wait (0 = auto),
  * light-pull variant (0..3), 64-lane words per vertex of the batched engine
  * (1, 2, 4, 8 or 16: 64 to 1024 sources per batch), hub-first vertex
  * order of the batched engine (0 or 1; graphs of 65,536 vertices or more).

@@ -82,3 +82,52 @@ def test_source_lists_its_edges_repeatedly(orc, policy):
     w = rng.integers(0, 500, len(col)).astype(np.int32)
     g = dawn.Graph(dawn.HostGraph.from_csr(rp, col, w, directed=True))
     assert np.array_equal(g.sssp(0, policy=policy), orc.sssp(rp, col, w, 0))
+
+
+def chain_and_fans():
+    """Chain, a fan of 3000 (a level of more edges than one workgroup walks),
+    all joined again, a hub of 300 and a fan of 1500 behind another chain:
+    levels change between small and large several times."""
+    u, v, at = [], [], 0
+
+    def link(a, b):
+        u.append(a)
+        v.append(b)
+    for fan_of, chain in ((3000, 12), (300, 3), (1500, 40), (2048, 5), (2047, 1)):
+        for _ in range(chain):
+            link(at, at + 1)
+            at += 1
+        root, join = at, at + fan_of + 1
+        for i in range(fan_of):
+            link(root, root + 1 + i)
+            link(root + 1 + i, join)
+        at = join
+    return at + 1, np.array(u, np.int32), np.array(v, np.int32)
+
+
+@pytest.mark.parametrize("kind", ["path", "fans"])
+def test_walks_of_small_levels_exact(orc, kind):
+    """Runs of small levels are walked in one launch (at most 4096 levels of
+    at most 2048 edges); every policy, both engines, and into a device buffer."""
+    n, u, v = chain_and_fans() if kind == "fans" else (9001, np.arange(9000), np.arange(1, 9001))
+    log(f"case: {kind}, n={n}")
+    w = np.random.default_rng(5).integers(0, 50, len(u)).astype(np.int32)
+    h, hw = dawn.HostGraph.from_edges(n, u, v), dawn.HostGraph.from_edges(n, u, v, w)
+    g, gw = dawn.Graph(h), dawn.Graph(hw)
+    for s in (0, 13, n // 2, n - 1):
+        ref, refw = orc.bfs(h.row_ptr, h.col, s), orc.sssp(hw.row_ptr, hw.col, hw.weight, s)
+        for p in ("fixed", "push") + (("pull", "bitmap") if kind == "fans" else ()):
+            d, st = g.bfs(s, policy=p, stats=True)
+            assert np.array_equal(d, ref), (s, p)
+            assert st["vertices_reached"] == n and st["edges_reached"] == h.m, (s, p)
+            assert st["steps"] == ref.max() + 1, (s, p)  # the last one finds nothing
+            dw, st = gw.sssp(s, policy=p, stats=True)
+            assert np.array_equal(dw, refw), (s, p)
+            assert st["vertices_reached"] == n and st["edges_reached"] == hw.m, (s, p)
+        out = dawn.DeviceArray(n + 1, np.int32)  # rows at any int32 offset
+        for off in (0, 4):
+            p = out.data_ptr() + off
+            assert dawn.lib().dawn_bfs(g.handle, s, p, 0, None) == 0
+            got = out.download()[off // 4:][:n]
+            assert np.array_equal(got, ref), (s, off)
+        assert np.array_equal(g.bfs_noalloc(s), ref), s
