@@ -43,10 +43,11 @@
 
 namespace dawn {
 
-// Counters (frontier vertices, their out-edges, GAPBS scout) are added per
-// workgroup into one of kStripes stripes, each on its own 128-byte line, so
-// the atomics of the workgroups spread over 64 addresses; the next launch sums
-// them, one stripe per lane.
+// Counters (frontier vertices, their out-edges, GAPBS scout; min-plus also the
+// smallest frontier distance, as the largest INF - distance, and the out-edges
+// of deferred vertices) are added per workgroup into one of kStripes stripes,
+// each on its own 128-byte line, so the atomics of the workgroups spread over
+// 64 addresses; the next launch sums them, one stripe per lane.
 constexpr int kStripes = 64;
 constexpr int kStripeU64 = 16;  // 128 bytes per stripe
 static_assert(kStripes == kWave, "one stripe per lane is summed");
@@ -64,6 +65,7 @@ struct SsState {
   long long mode_steps[DAWN_NUM_MODES];
   unsigned long long reached, edges;  // vertices reached, their out-edges (set when done)
   long long t0, t1;                   // device clock at the first and the last launch
+  long long delta, thr;               // min-plus: advance per step (0: none), threshold
 };
 
 struct SsArgs {
@@ -88,9 +90,11 @@ struct SsArgs {
   const int32_t* oc_end;
   int64_t num_oc;
   SsSlot* slots;             // kSsSlots
-  unsigned long long* tot;   // kStripes stripes: vertices reached first, their out-edges
+  unsigned long long* tot;   // reach counts: workgroups done, then a pair of parts each
   SsState* st;               // kSsSlots
   SsState* host;             // pinned: the final state (null: not written)
+  const unsigned long long* wsum;  // kWsumBlocks parts of the sum of the weights
+  double delta_scale;        // threshold advance per unit of that sum
 };
 
 // Everything a step launch needs but its number.
@@ -125,6 +129,7 @@ struct SsWorkspace {
   DevBuf<SsSlot> slots;
   DevBuf<unsigned long long> tot;
   DevBuf<SsState> st;
+  DevBuf<unsigned long long> wsum;  // min-plus: parts of the sum of the weights
   DevBuf<float> trace_feat;    // recording only
   DevBuf<int32_t> trace_mode;
   SsState* h_state = nullptr;  // pinned
@@ -160,19 +165,18 @@ __device__ __forceinline__ int owner_of(const int* off, int e) {
   return j;
 }
 
+// A thread's counts of the level it finds.
 struct Acc {
-  unsigned long long fv = 0, fe = 0, scout = 0;
-  unsigned rv = 0;            // vertices reached for the first time (min-plus)
-  unsigned long long re = 0;  // their out-edges
+  unsigned fv = 0, zero = 0;  // vertices, those without out-edges
+  unsigned long long fe = 0;  // their out-edges
+  unsigned long long de = 0;  // min-plus: out-edges of deferred vertices
+  unsigned near = 0;          // min-plus: largest INF - distance of a frontier vertex
   __device__ void add(int d) {
     fv += 1;
+    zero += d == 0;
     fe += (unsigned)d;
-    scout += (unsigned)(d > 0 ? d : 1);
   }
-  __device__ void reach(const SsArgs& a, int32_t v) {
-    rv += 1;
-    re += (unsigned)(a.row_ptr[v + 1] - a.row_ptr[v]);
-  }
+  __device__ void dist(int32_t d) { near = max(near, (unsigned)(kInf - d)); }
 };
 
 // Edges per heavy chunk: two rounds of a wave.
@@ -239,34 +243,35 @@ struct SsOut {
   SsSlot* slot;
   int32_t* q;
   int2* hq;
-  unsigned long long* tot;
 };
 __device__ __forceinline__ SsOut out_of(const SsArgs& a, int k) {
   return {a.slots + ((k + 1) % kSsSlots), a.q + (int64_t)((k + 1) & 1) * a.n,
-          a.hq + (int64_t)((k + 1) & 1) * a.hcap, a.tot + (blockIdx.x % kStripes) * kStripeU64};
+          a.hq + (int64_t)((k + 1) & 1) * a.hcap};
 }
 
 // Workgroup-level staging of a step's outputs: the vertices found in the
-// step and the level's counters.  Waves reserve LDS slots with LDS atomics;
-// flush() reads the staged vertices' degrees (independent loads, one after
-// the other hidden behind each other), splits them into the light queue and
-// heavy chunks, and reserves each global range once per workgroup: a global
-// counter that every wave bumps serialises at one address.  Vertices beyond
-// the LDS capacity go straight to the global queues, wave by wave.
+// step, with their out-degrees (read beside the atomic that found them), and
+// the level's counters.  Waves reserve LDS slots with LDS atomics; flush()
+// splits the staged vertices into the light queue and heavy chunks, and
+// reserves each global range once per workgroup: a global counter that every
+// wave bumps serialises at one address.  Vertices beyond the LDS capacity go
+// straight to the global queues, wave by wave.
 struct SsStage {
   int32_t v[kStageCap];
-  unsigned n;        // slots reserved (may pass kStageCap)
-  unsigned base[2];  // global positions of the workgroup's ranges
+  uint16_t d[kStageCap];  // out-degree, 65535 for any larger one
+  unsigned n;             // slots reserved (may pass kStageCap)
+  unsigned odd;           // staged vertices that are not light: no edges, or heavy
+  unsigned base[2];       // global positions of the workgroup's ranges
   int scan[kSsWaves];
   unsigned long long tot[5];
   __device__ void init() {
     if (threadIdx.x < 5) tot[threadIdx.x] = 0ull;
-    if (threadIdx.x == 0) n = 0u;
+    if (threadIdx.x == 0) n = odd = 0u;
     __syncthreads();
   }
-  // Records a vertex found in the step (each vertex once per level).  Called
-  // by all 64 lanes of a wave.
-  __device__ void append(const SsArgs& a, const SsOut& o, bool pred, int32_t x, Acc& acc) {
+  // Records a vertex of out-degree deg found in the step (each vertex once
+  // per level).  Called by all 64 lanes of a wave.
+  __device__ void append(const SsArgs& a, const SsOut& o, bool pred, int32_t x, int deg, Acc& acc) {
     const uint64_t m = __ballot(pred);
     if (m == 0) return;
     const int leader = __ffsll((unsigned long long)m) - 1;
@@ -275,36 +280,42 @@ struct SsStage {
     if (lane_id() == leader) b = atomicAdd(&n, cnt);
     b = __shfl(b, leader);
     const unsigned idx = b + (unsigned)__popcll(m & lanes_below_mask());
-    if (pred && idx < (unsigned)kStageCap) v[idx] = x;
-    if (b + cnt > (unsigned)kStageCap) spill(a, o, pred && idx >= (unsigned)kStageCap, x, acc);
-  }
-  __device__ void spill(const SsArgs& a, const SsOut& o, bool pred, int32_t x, Acc& acc) {
-    int rb = 0, d = 0;
-    if (pred) {
-      rb = a.row_ptr[x];
-      d = a.row_ptr[x + 1] - rb;
-      acc.add(d);
+    const bool in = pred && idx < (unsigned)kStageCap;
+    if (in) {
+      v[idx] = x;
+      d[idx] = (uint16_t)min(deg, 65535);
     }
-    const bool light = d > 0 && d <= a.hchunk;
+    if (pred) acc.add(deg);
+    const uint64_t om = __ballot(in && (deg == 0 || deg > a.hchunk));
+    if (om && lane_id() == leader) atomicAdd(&odd, (unsigned)__popcll(om));
+    if (b + cnt > (unsigned)kStageCap) spill(a, o, pred && !in, x, deg);
+  }
+  __device__ void spill(const SsArgs& a, const SsOut& o, bool pred, int32_t x, int deg) {
+    const bool light = pred && deg > 0 && deg <= a.hchunk;
     const int at = wave_append(&o.slot->qlen, light);
     if (light) o.q[at] = x;
-    wave_put_chunks(a, o.hq, &o.slot->hqlen, x, rb, d);
+    const bool heavy = pred && deg > a.hchunk;
+    wave_put_chunks(a, o.hq, &o.slot->hqlen, x, heavy ? a.row_ptr[x] : 0, heavy ? deg : 0);
   }
   // Every thread, once, at the end of the step kernel.  The staged order is
   // kept: vertices found together are neighbours in the next queue, so the
   // lanes that expand them read neighbouring rows and distances (queue
   // entries interleaved by thread made push steps on a 2048^2 grid 2-3x
   // slower).
+  template <bool MP>
   __device__ void flush(const SsArgs& a, const SsOut& o, Acc& acc) {
     __syncthreads();
     const unsigned cnt = n < (unsigned)kStageCap ? n : (unsigned)kStageCap;
-    if (cnt) {  // block-uniform
+    const bool all_light = odd == 0;
+    if (cnt && all_light) {  // block-uniform
+      if (threadIdx.x == 0) base[0] = atomicAdd(&o.slot->qlen, cnt);
+    } else if (cnt) {
       int nl = 0, nh = 0, tl, th;
       for (unsigned i = threadIdx.x; i < cnt; i += kSsBlock) {
-        const int d = a.row_ptr[v[i] + 1] - a.row_ptr[v[i]];
-        acc.add(d);
-        if (d > a.hchunk) nh += chunks_of(a, d);
-        else if (d > 0) nl += 1;
+        int g = d[i];
+        if (g == 65535) g = a.row_ptr[v[i] + 1] - a.row_ptr[v[i]];
+        if (g > a.hchunk) nh += chunks_of(a, g);
+        else if (g > 0) nl += 1;
       }
       (void)ss_scan(nl, scan, &tl);
       (void)ss_scan(nh, scan, &th);
@@ -312,74 +323,129 @@ struct SsStage {
         base[0] = tl ? atomicAdd(&o.slot->qlen, (unsigned)tl) : 0u;
         base[1] = th ? atomicAdd(&o.slot->hqlen, (unsigned)th) : 0u;
       }
-      __syncthreads();
-      int32_t* q_out = o.q + base[0];
-      if ((unsigned)tl == cnt) {  // block-uniform: every vertex is light
-        for (unsigned i = threadIdx.x; i < cnt; i += kSsBlock) q_out[i] = v[i];
-      } else {
-        for (unsigned i0 = 0; i0 < cnt; i0 += kSsBlock) {
-          const unsigned i = i0 + threadIdx.x;
-          int rb = 0, d = 0;
-          int32_t x = 0;
-          if (i < cnt) {
-            x = v[i];
-            rb = a.row_ptr[x];
-            d = a.row_ptr[x + 1] - rb;
-          }
-          const bool light = d > 0 && d <= a.hchunk;
-          int tr;
-          const int ol = ss_scan(light ? 1 : 0, scan, &tr);
-          if (light) q_out[ol] = x;
-          q_out += tr;
-          wave_put_chunks(a, o.hq, &base[1], x, rb, d);
-        }
-      }
     }
-    if (__ballot(acc.fv != 0 || acc.rv != 0)) {
-      const unsigned long long r[5] = {wave_sum_u64(acc.fv), wave_sum_u64(acc.fe),
-                                       wave_sum_u64(acc.scout), wave_sum_u64(acc.rv),
-                                       wave_sum_u64(acc.re)};
-      if (lane_id() == 0)
-        for (int i = 0; i < 5; i++)
-          if (r[i]) atomicAdd(&tot[i], r[i]);
+    if (__ballot(acc.fv != 0 || acc.near != 0)) {  // beside the reservation
+      const unsigned long long c =
+          wave_sum_u64((unsigned long long)acc.fv | ((unsigned long long)acc.zero << 32));
+      const unsigned long long fe = wave_sum_u64(acc.fe);
+      const unsigned long long de = MP ? wave_sum_u64(acc.de) : 0ull;
+      const int near = MP ? wave_max_i32((int)acc.near) : 0;
+      if (lane_id() == 0) {
+        atomicAdd(&tot[0], c & 0xFFFFFFFFull);
+        atomicAdd(&tot[1], fe);
+        atomicAdd(&tot[2], fe + (c >> 32));  // scout: max(degree, 1)
+        if (near) atomicMax(&tot[3], (unsigned long long)near);
+        if (de) atomicAdd(&tot[4], de);
+      }
     }
     __syncthreads();
     if (threadIdx.x < 5 && tot[threadIdx.x]) {
-      const int i = threadIdx.x;
-      atomicAdd(i < 3 ? &o.slot->part[blockIdx.x % kStripes][i] : &o.tot[i - 3], tot[i]);
+      unsigned long long* part = o.slot->part[blockIdx.x % kStripes];
+      if (threadIdx.x == 3) atomicMax(&part[3], tot[3]);
+      else atomicAdd(&part[threadIdx.x], tot[threadIdx.x]);
+    }
+    if (cnt && all_light) {
+      for (unsigned i = threadIdx.x; i < cnt; i += kSsBlock) o.q[base[0] + i] = v[i];
+    } else if (cnt) {
+      int32_t* q_out = o.q + base[0];
+      for (unsigned i0 = 0; i0 < cnt; i0 += kSsBlock) {
+        const unsigned i = i0 + threadIdx.x;
+        int rb = 0, g = 0;
+        int32_t x = 0;
+        if (i < cnt) {
+          x = v[i];
+          g = d[i];
+          if (g > a.hchunk) {
+            rb = a.row_ptr[x];
+            g = a.row_ptr[x + 1] - rb;
+          }
+        }
+        const bool light = g > 0 && g <= a.hchunk;
+        int tr;
+        const int ol = ss_scan(light ? 1 : 0, scan, &tr);
+        if (light) q_out[ol] = x;
+        q_out += tr;
+        wave_put_chunks(a, o.hq, &base[1], x, rb, g > a.hchunk ? g : 0);
+      }
     }
   }
 };
 
-// Out-edges of the frontier queue of launch k, spread over the waves of the grid: a wave
-// takes the heavy chunks one by one, and of the light queue 1 to 64
-// vertices at a time (as few as the grid's waves need to cover the queue),
-// whose edge lists it walks as one (LDS degree scan, two edges per lane and
-// round).  edge(u_dist, k0, k1) handles edges k0 and k1 (-1: none) in one
-// wave-uniform call.  Bound by the latency of the dependent loads per edge
-// (column, then its distance): with whole workgroups taking 256 queue
-// entries each, a frontier of a few thousand vertices ran on a few CUs and
-// a hub's list on one (RMAT scale 22, 10.2 M edges of 3133 vertices: 29.7 ms,
-// now 0.25 ms; scale 20, 1.03 M edges of 434: 6.9 ms, now 0.18 ms, where the
-// atomics on the few bitmap words of the hubs bound it).
+// LDS of one wave's batch of vertices: scanned out-degrees, first edges, tail
+// distances; for frontiers read from the bitmap also its words and their
+// scanned bit counts.
 template <bool DU>
 struct PushLds {
   int off[kSsWaves][kWave];
   int beg[kSsWaves][kWave];
   int du[DU ? kSsWaves : 1][kWave];
+  int woff[kSsWaves][kWave];
+  uint32_t word[kSsWaves][kWave];
 };
+
+__device__ __forceinline__ int wave_incl_scan(int x) {
+  const int l = lane_id();
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int y = __shfl_up(x, o);
+    if (l >= o) x += y;
+  }
+  return x;
+}
+
+// Edge lists of up to 64 vertices (one per lane: first edge, out-degree, tail
+// distance), walked as one by the wave: LDS degree scan, two edges per lane
+// and round.  edge(du0, du1, e0, e1) handles edges e0 and e1 (-1: none) in one
+// wave-uniform call.
 template <bool DU, class F>
+__device__ __forceinline__ void wave_edges(PushLds<DU>& s, int beg, int deg, int du, F&& edge) {
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  int* off = s.off[wv];
+  int* begs = s.beg[wv];
+  int* dus = s.du[DU ? wv : 0];
+  const int inc = wave_incl_scan(deg);
+  const int total = __shfl(inc, kWave - 1);
+  off[lane] = inc - deg;
+  begs[lane] = beg - (inc - deg);
+  if (DU) dus[lane] = du;
+  wave_lds_sync();
+  for (int e = lane; e - lane < total; e += 2 * kWave) {
+    const int e1 = e + kWave;
+    const int j0 = owner_of(off, e), j1 = owner_of(off, e1);
+    edge(DU ? dus[j0] : 0, DU ? dus[j1] : 0, e < total ? begs[j0] + e : -1,
+         e1 < total ? begs[j1] + e1 : -1);
+  }
+  wave_lds_sync();
+}
+
+// Out-edges of the frontier queue of launch k, spread over the waves of the
+// grid: a wave takes the heavy chunks one by one, and of the light queue 1 to
+// 64 vertices at a time (as few as the grid's waves need to cover the queue).
+// With DU, vertices at distance thr or more are not expanded: defer(yes, u,
+// its distance, its out-degree), wave-uniform too.  Bound by the latency of
+// the dependent loads per edge (column, then its distance): with whole
+// workgroups taking 256 queue entries each, a frontier of a few thousand
+// vertices ran on a few CUs and a hub's list on one (RMAT scale 22, 10.2 M
+// edges of 3133 vertices: 29.7 ms, now 0.25 ms; scale 20, 1.03 M edges of 434:
+// 6.9 ms, now 0.18 ms, where the atomics on the few bitmap words of the hubs
+// bound it).
+template <bool DU, class F, class D>
 __device__ __forceinline__ void push_edges(const SsArgs& a, PushLds<DU>& s, int k, unsigned qn,
-                                           unsigned hn, F&& edge) {
+                                           unsigned hn, int32_t thr, F&& edge, D&& defer) {
   const int32_t* q_in = a.q + (int64_t)(k & 1) * a.n;
   const int2* hq_in = a.hq + (int64_t)(k & 1) * a.hcap;
-  const int lane = lane_id(), wv = threadIdx.x / kWave;
-  const int64_t wid = (int64_t)blockIdx.x * (kSsWaves) + wv;
-  const int64_t nw = (int64_t)gridDim.x * (kSsWaves);
+  const int lane = lane_id();
+  const int64_t wid = (int64_t)blockIdx.x * kSsWaves + threadIdx.x / kWave;
+  const int64_t nw = (int64_t)gridDim.x * kSsWaves;
   for (int64_t c = wid; c < hn; c += nw) {  // wave-uniform
     const int2 h = hq_in[c];
     const int end = min(h.y + a.hchunk, a.row_ptr[h.x + 1]);
     const int du = DU ? a.dist[h.x] : 0;
+    if (DU && du >= thr) {  // once per vertex: by its first chunk
+      const int rb = a.row_ptr[h.x];
+      defer(lane == 0 && h.y == rb, h.x, du, a.row_ptr[h.x + 1] - rb);
+      continue;
+    }
     for (int kb = h.y; kb < end; kb += 2 * kWave) {
       const int k0 = kb + lane, k1 = k0 + kWave;
       edge(du, du, k0 < end ? k0 : -1, k1 < end ? k1 : -1);
@@ -387,63 +453,86 @@ __device__ __forceinline__ void push_edges(const SsArgs& a, PushLds<DU>& s, int 
   }
   int64_t per = (qn + nw - 1) / nw;
   per = per < 1 ? 1 : per > kWave ? kWave : per;
-  int* off = s.off[wv];
-  int* begs = s.beg[wv];
-  int* dus = s.du[DU ? wv : 0];
   for (int64_t c = wid * per; c < qn; c += nw * per) {  // wave-uniform
     int beg = 0, deg = 0, du = 0;
+    int32_t u = 0;
     if (lane < per && c + lane < qn) {
-      const int32_t u = q_in[c + lane];
+      u = q_in[c + lane];
       beg = a.row_ptr[u];
       deg = a.row_ptr[u + 1] - beg;
       if (DU) du = a.dist[u];
     }
-    int inc = deg;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int y = __shfl_up(inc, o);
-      if (lane >= o) inc += y;
+    if (DU) {
+      const bool later = deg > 0 && du >= thr;
+      defer(later, u, du, deg);
+      if (later) deg = 0;
     }
-    const int total = __shfl(inc, kWave - 1);
-    off[lane] = inc - deg;
-    begs[lane] = beg - (inc - deg);
-    if (DU) dus[lane] = du;
-    wave_lds_sync();
-    for (int e = lane; e - lane < total; e += 2 * kWave) {
-      const int e1 = e + kWave;
-      const int j0 = owner_of(off, e), j1 = owner_of(off, e1);
-      edge(DU ? dus[j0] : 0, DU ? dus[j1] : 0, e < total ? begs[j0] + e : -1,
-           e1 < total ? begs[j1] + e1 : -1);
-    }
-    wave_lds_sync();
+    wave_edges<DU>(s, beg, deg, du, edge);
   }
 }
 
-// Dense top-down over the frontier bitmap: vertices of out-degree < heavy
-// one lane each, the others by the graph's static out-edge chunks, a wave
-// each.  edge(v_dist, k) handles one edge per lane (k < 0: none) in
-// wave-uniform calls.
-template <bool DU, class F>
-__device__ __forceinline__ void bitmap_edges(const SsArgs& a, const uint32_t* bm_in, F&& edge) {
-  const int lane = lane_id();
-  const int64_t wstride = (int64_t)gridDim.x * kSsBlock;
-  for (int64_t base = (int64_t)blockIdx.x * kSsBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
-       base += wstride) {
-    const int32_t u = (int32_t)(base + lane);
-    const bool act = u < a.n && test_bit(bm_in, u);
-    if (__ballot(act) == 0) continue;
-    int beg = 0, deg = 0, du = 0;
-    if (act) {
-      beg = a.row_ptr[u];
-      deg = a.row_ptr[u + 1] - beg;
-      if (DU) du = a.dist[u];
+// Position of the r-th set bit of x (r < popcount).
+__device__ __forceinline__ int select_bit(uint32_t x, int r) {
+  int at = 0;
+#pragma unroll
+  for (int w = 16; w >= 1; w >>= 1) {
+    const int c = __popc((x >> at) & ((1u << w) - 1u));
+    if (r >= c) {
+      r -= c;
+      at += w;
     }
-    const bool light = act && deg < a.heavy;
-    const int maxd = wave_max_i32(light ? deg : 0);
-    for (int j = 0; j < maxd; j++) edge(du, light && j < deg ? beg + j : -1);
   }
-  const int64_t wid = ((int64_t)blockIdx.x * kSsBlock + threadIdx.x) / kWave;
-  const int64_t nw = (int64_t)gridDim.x * (kSsWaves);
+  return at;
+}
+
+// Out-edges of the frontier bitmap, in vertex order: a wave takes up to 64
+// consecutive words (fewer, so that the words are spread over the grid's
+// waves), 64 of their set bits at a time.  Neighbouring vertices are expanded
+// together, so their rows, columns and heads' distances share lines, where a
+// queue of some hundred thousand vertices, in the order they were found,
+// moves most of a line per access (2048^2 grid, min-plus: a traversal with its dense
+// steps in vertex order 1.61 ms, all by the queue 1.98).
+// Vertices of out-degree >= heavy go by the graph's static out-edge chunks, a
+// wave each.
+template <bool DU, class F, class D>
+__device__ __forceinline__ void bitmap_edges(const SsArgs& a, PushLds<DU>& s, const uint32_t* bm_in,
+                                             int32_t thr, F&& edge, D&& defer) {
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  const int64_t wid = (int64_t)blockIdx.x * kSsWaves + wv;
+  const int64_t nw = (int64_t)gridDim.x * kSsWaves;
+  int64_t per = (a.words + nw - 1) / nw;
+  per = per > kWave ? kWave : per;
+  int* woff = s.woff[wv];
+  uint32_t* word = s.word[wv];
+  for (int64_t w0 = wid * per; w0 < a.words; w0 += nw * per) {  // wave-uniform
+    const uint32_t x = lane < per && w0 + lane < a.words ? bm_in[w0 + lane] : 0u;
+    if (!__ballot(x != 0)) continue;
+    const int inc = wave_incl_scan(__popc(x));
+    const int total = __shfl(inc, kWave - 1);
+    woff[lane] = inc - __popc(x);
+    word[lane] = x;
+    wave_lds_sync();
+    for (int i0 = 0; i0 < total; i0 += kWave) {
+      const int i = i0 + lane;
+      int beg = 0, deg = 0, du = 0;
+      int32_t u = 0;
+      if (i < total) {
+        const int j = owner_of(woff, i);
+        u = (int32_t)((w0 + j) * 32 + select_bit(word[j], i - woff[j]));
+        beg = a.row_ptr[u];
+        deg = a.row_ptr[u + 1] - beg;
+        if (DU) du = a.dist[u];
+      }
+      if (DU) {
+        const bool later = deg > 0 && du >= thr;
+        defer(later, u, du, deg);
+        if (later) deg = 0;
+      }
+      if (deg >= a.heavy) deg = 0;
+      wave_edges<DU>(s, beg, deg, du, edge);
+    }
+    wave_lds_sync();
+  }
   // 64 chunks are probed at once, one per lane, as most are not in the
   // frontier; a grid apart, as a hub's chunks are neighbours in the list.
   for (int64_t c0 = wid; c0 < a.num_oc; c0 += nw * kWave) {  // wave-uniform
@@ -453,8 +542,10 @@ __device__ __forceinline__ void bitmap_edges(const SsArgs& a, const uint32_t* bm
       const int l = __ffsll((unsigned long long)m) - 1;
       m &= m - 1;
       const int du = DU ? a.dist[__shfl(mine, l)] : 0;
+      if (DU && du >= thr) continue;
       const int end = a.oc_end[c0 + l * nw];
-      for (int k = a.oc_beg[c0 + l * nw]; k < end; k += kWave) edge(du, k + lane < end ? k + lane : -1);
+      for (int e = a.oc_beg[c0 + l * nw] + lane; e - lane < end; e += 2 * kWave)
+        edge(du, du, e < end ? e : -1, e + kWave < end ? e + kWave : -1);
     }
   }
 }
@@ -492,7 +583,7 @@ __global__ void __launch_bounds__(kBlock) ss_fill_kernel(SsArgs a, int bovm) {
   if (blockIdx.x != 0) return;
   unsigned long long* p = reinterpret_cast<unsigned long long*>(a.slots);
   for (int i = threadIdx.x; i < (int)(kSsSlots * sizeof(SsSlot) / 8); i += kBlock) p[i] = 0ull;
-  for (int i = threadIdx.x; i < kStripes * kStripeU64; i += kBlock) a.tot[i] = 0ull;
+  if (threadIdx.x == 0) a.tot[0] = 0ull;
   __syncthreads();
   SsState st{};
   st.t0 = wall_clock64();
@@ -518,6 +609,23 @@ __global__ void __launch_bounds__(kBlock) ss_fill_kernel(SsArgs a, int bovm) {
   }
 }
 
+// Sum of the edge weights, in one part per workgroup (once per graph).
+constexpr int kWsumBlocks = 512;
+__global__ void __launch_bounds__(kBlock) ss_wsum_kernel(const int32_t* w, int64_t m,
+                                                         unsigned long long* out) {
+  __shared__ unsigned long long s_t[kBlock / kWave];
+  unsigned long long t = 0;
+  for (int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x; k < m; k += (int64_t)kWsumBlocks * kBlock)
+    t += (unsigned)w[k];
+  t = wave_sum_u64(t);
+  if (lane_id() == 0) s_t[threadIdx.x / kWave] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kBlock / kWave; i++) t += s_t[i];
+    out[blockIdx.x] = t;
+  }
+}
+
 // Level 1 for min-plus, as SSSP_CPU::SSSP initialises it
 // (src/algorithm/cpu/sssp.cpp:40-46): every listed out-edge of the source
 // writes its weight in row order (a later duplicate overwrites an earlier
@@ -528,12 +636,16 @@ __global__ void __launch_bounds__(kBlock) ss_fill_kernel(SsArgs a, int bovm) {
 // other edge of the neighbour matches).  A hub source's list in one thread
 // took 100k dependent round trips.
 __global__ void __launch_bounds__(kSsBlock) sssp_seed_kernel(SsArgs a) {
-  __shared__ unsigned s_len[2];
-  __shared__ unsigned long long s_c[3];
+  __shared__ unsigned s_len[2], s_near;
+  __shared__ unsigned long long s_c[3], s_wsum;
   const int32_t s = a.source;
   const int32_t b = a.row_ptr[s], e = a.row_ptr[s + 1];
   if (threadIdx.x < 2) s_len[threadIdx.x] = 0u;
   if (threadIdx.x < 3) s_c[threadIdx.x] = 0ull;
+  if (threadIdx.x == 3) {
+    s_near = 0u;
+    s_wsum = 0ull;
+  }
   for (int32_t k = b + threadIdx.x; k < e; k += kSsBlock) atomicMin(&a.dist[a.col[k]], -1 - k);
   __syncthreads();
   for (int32_t k = b + threadIdx.x; k < e; k += kSsBlock) {
@@ -541,6 +653,7 @@ __global__ void __launch_bounds__(kSsBlock) sssp_seed_kernel(SsArgs a) {
     if (__hip_atomic_load(&a.dist[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != -1 - k) continue;
     __hip_atomic_store(&a.dist[v], a.w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (v == s) continue;
+    atomicMax(&s_near, (unsigned)(kInf - a.w[k]));
     atomicOr(&a.bm[v >> 5], 1u << (v & 31));
     const int rb = a.row_ptr[v], d = a.row_ptr[v + 1] - rb;
     if (d > a.hchunk)
@@ -551,42 +664,61 @@ __global__ void __launch_bounds__(kSsBlock) sssp_seed_kernel(SsArgs a) {
     atomicAdd(&s_c[1], (unsigned long long)d);
     atomicAdd(&s_c[2], (unsigned long long)(d > 0 ? d : 1));
   }
+  if (threadIdx.x < kWsumBlocks) {
+    const unsigned long long x = wave_sum_u64(a.wsum[threadIdx.x]);
+    if (lane_id() == 0) atomicAdd(&s_wsum, x);
+  }
   __syncthreads();
   if (threadIdx.x != 0) return;
   __hip_atomic_store(&a.dist[s], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   SsSlot& c = a.slots[0];
   for (int i = 0; i < 3; i++) c.part[0][i] = s_c[i];
+  c.part[0][3] = s_near;
   c.qlen = s_len[0];
   c.hqlen = s_len[1];
-  a.tot[0] = 1 + s_c[0];
-  a.tot[1] = (unsigned long long)(e - b) + s_c[1];
   SsState& st = a.st[0];
   st.s.step = 1;
   st.s.scout = (long long)s_c[2];
+  if (a.delta_scale > 0) st.delta = max(1ll, (long long)ceil(a.delta_scale * (double)s_wsum));
 }
 
-// An unreached head v joins level lv once: the first to set its bitmap bit.
-__device__ __forceinline__ bool discover(const SsArgs& a, int lv, int32_t v, uint32_t* bm_out) {
-  if (a.dist[v] != kInf) return false;
-  const uint32_t bit = 1u << (v & 31);
-  if (atomicOr(&bm_out[v >> 5], bit) & bit) return false;
-  a.dist[v] = lv;
-  return true;
-}
+// A head that may join the new level: BOVM if unreached, min-plus if the path
+// over this edge is shorter than its distance.
+struct Head {
+  int32_t v, nd, deg;
+  bool cand, join;
+};
 
-// Relaxation of an edge to v of weight w with du = current distance of the
-// tail.  Returns true when v joins the next frontier for the first time this
-// level.
-__device__ __forceinline__ bool relax(const SsArgs& a, int32_t src, int32_t du, int32_t v,
-                                      int32_t w, uint32_t* bm_out, Acc& acc) {
-  if (v == src) return false;
-  const int32_t nd = minplus(du, w);
-  if (nd >= a.dist[v]) return false;
-  const int32_t old = atomicMin(&a.dist[v], nd);
-  if (nd >= old) return false;
-  if (old == kInf) acc.reach(a, v);
-  const uint32_t bit = 1u << (v & 31);
-  return (atomicOr(&bm_out[v >> 5], bit) & bit) == 0;
+// First half: the head's distance is compared; the second half's accesses
+// (which need no answer from each other) are the atomicMin (min-plus), the
+// atomicOr on the level's bitmap, whose first setter joins the vertex to the
+// level, and its out-degree.  A min-plus head whose distance another edge
+// has lowered below nd meanwhile may still be joined here: that edge's tail
+// was expanded in this step too, so the head belongs to the next frontier.
+template <bool MP>
+__device__ __forceinline__ Head head_of(const SsArgs& a, int lv, int32_t src, int e, int du) {
+  Head h{0, lv, 0, false, false};
+  if (e >= 0) {
+    h.v = a.col[e];
+    if (MP) h.nd = minplus(du, a.w[e]);
+    h.cand = MP ? h.v != src : true;
+  }
+  return h;
+}
+template <bool MP>
+__device__ __forceinline__ void test_head(const SsArgs& a, Head& h) {
+  if (h.cand) h.cand = MP ? h.nd < a.dist[h.v] : a.dist[h.v] == kInf;
+}
+template <bool MP>
+__device__ __forceinline__ void join_head(const SsArgs& a, Head& h, uint32_t* bm_out, Acc& acc) {
+  if (!h.cand) return;
+  const uint32_t bit = 1u << (h.v & 31);
+  if (MP) atomicMin(&a.dist[h.v], h.nd);
+  const uint32_t old = atomicOr(&bm_out[h.v >> 5], bit);
+  h.deg = a.row_ptr[h.v + 1] - a.row_ptr[h.v];
+  h.join = (old & bit) == 0;
+  if (MP) acc.dist(h.nd);
+  else if (h.join) a.dist[h.v] = h.nd;
 }
 
 // Counters of a completed level.
@@ -612,6 +744,8 @@ struct SsCtl {
 // grid 12.  kSmallLevels bounds a launch on paths (about 20 ms).
 constexpr int kSmallEdges = 2048;
 constexpr int kSmallLevels = 4096;
+// Min-plus: frontiers of at least n / kMpDense vertices are read from the bitmap.
+constexpr unsigned long long kMpDense = 32;
 
 // Whether the level with counters c may be walked by one workgroup under
 // `mode`: its queue exists and holds every vertex with out-edges.
@@ -621,18 +755,24 @@ __device__ __forceinline__ bool small_level(const SsLevel& c, int mode) {
 
 // Mode of the step after the level with counters c, by the rule or the
 // forced policy; keeps the rule state current.  The learned network's choice
-// is made by the caller (it needs the workgroup).
+// is made by the caller (it needs the workgroup).  Min-plus has no rule of
+// the reference: it pushes, in vertex order from the bitmap once the frontier
+// is dense enough for its vertices to share lines (from n / 32 on: 2048^2 grid
+// 1.61 ms, by the queue alone 1.98, by the bitmap alone 1.76; random graphs
+// within 3% of each other).  A pull relaxes every edge of the graph per step
+// and was never faster (2048^2 grid: 3.6 ms; RMAT scale 18: 14.5 against 0.7).
+template <bool MP>
 __device__ inline int ss_rule_mode(const SsRun& r, SchedState& s, const SsLevel& c) {
   if (r.force >= 0) return r.force;
+  if (r.p.policy == DAWN_POLICY_PUSH) return DAWN_MODE_PUSH;
+  if (r.p.policy == DAWN_POLICY_PULL) return DAWN_MODE_PULL;
+  if (r.p.policy == DAWN_POLICY_BITMAP) return DAWN_MODE_BITMAP;
+  if (MP) return c.fv * kMpDense >= (unsigned long long)r.p.n ? DAWN_MODE_BITMAP : DAWN_MODE_PUSH;
   LevelCounters lc{};
   lc.fv = c.fv;
   lc.fe = c.fe;
   lc.scout = c.scout;
-  const int mode = sched_fixed_mode(s, lc, r.p);
-  if (r.p.policy == DAWN_POLICY_PUSH) return DAWN_MODE_PUSH;
-  if (r.p.policy == DAWN_POLICY_PULL) return DAWN_MODE_PULL;
-  if (r.p.policy == DAWN_POLICY_BITMAP) return DAWN_MODE_BITMAP;
-  return mode;
+  return sched_fixed_mode(s, lc, r.p);
 }
 
 __device__ __forceinline__ bool learned(const SsRun& r) {
@@ -656,6 +796,7 @@ __device__ __forceinline__ void ss_advance(SchedState& s, const SsLevel& c, int 
 // Every workgroup decides from the same state and counters: a launch of its
 // own for the decision cost 4-5 us per step.  Called by all threads; the
 // result is in ctl after the last barrier.
+template <bool MP>
 __device__ inline void ss_decide(const SsRun& r, int k, SsCtl& ctl) {
   const SsArgs& a = r.a;
   if (threadIdx.x < kWave) {
@@ -664,6 +805,12 @@ __device__ inline void ss_decide(const SsRun& r, int k, SsCtl& ctl) {
     unsigned long long fv = slot.part[lane_id()][0], fe = slot.part[lane_id()][1],
                        sc = slot.part[lane_id()][2];
     const unsigned qlen = slot.qlen, hqlen = slot.hqlen;
+    unsigned near = 0;
+    unsigned long long de = 0;
+    if (MP) {
+      near = (unsigned)wave_max_i32((int)slot.part[lane_id()][3]);
+      de = wave_sum_u64(slot.part[lane_id()][4]);
+    }
     fv = wave_sum_u64(fv);
     fe = wave_sum_u64(fe);
     sc = wave_sum_u64(sc);
@@ -679,8 +826,12 @@ __device__ inline void ss_decide(const SsRun& r, int k, SsCtl& ctl) {
           ctl.fresh = 1;
         } else {
           const SchedState before = st.s;
-          const int mode = ss_rule_mode(r, st.s, c);
+          const int mode = ss_rule_mode<MP>(r, st.s, c);
           st.launches += 1;
+          if (MP) {
+            st.s.work_fe -= de;  // counted with the frontier, not expanded
+            if (st.delta > 0) st.thr = max(st.thr, (long long)(kInf - near)) + st.delta;
+          }
           // Small levels are pushed whatever the network would say.
           ctl.run = r.small && small_level(c, learned(r) ? DAWN_MODE_PUSH : mode) ? 2 : 1;
           if (ctl.run == 1 && (learned(r) || r.tr.feat)) {
@@ -719,8 +870,7 @@ struct SmallLds {
   int32_t tab_v[kTab];
   int32_t tab_d[kTab];
   int scan[kSsWaves];
-  unsigned n, zero, hq, hn;
-  unsigned long long reach[2];
+  unsigned n, zero, hq, hn, near;
 };
 
 // Slot of v in the level's table (at most half full); *first: v was not there.
@@ -766,7 +916,6 @@ __device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, Ss
     const int2* hq_in = a.hq + (int64_t)(k & 1) * a.hcap;
     const unsigned qn = ctl.c.qlen, hn = ctl.c.hqlen;
     if (t == 0) s.n = 0u;
-    if (t < 2) s.reach[t] = 0ull;
     clear_table();
     __syncthreads();
     for (unsigned i = t; i < qn + hn; i += kSsBlock) {
@@ -827,7 +976,7 @@ __device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, Ss
           ctl.fresh = 1;
         } else {
           SchedState next = ctl.st.s;
-          const int mode = ss_rule_mode(run, next, c);
+          const int mode = ss_rule_mode<MP>(run, next, c);
           if (it < kSmallLevels && small_level(c, learned(run) ? DAWN_MODE_PUSH : mode)) {
             ss_advance(next, c, DAWN_MODE_PUSH);
             ctl.st.s = next;
@@ -839,10 +988,9 @@ __device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, Ss
       }
       __syncthreads();
       if (ctl.run != 2) {
-        if (MP && t < 2 && s.reach[t]) atomicAdd(&a.tot[t], s.reach[t]);
         if (ctl.run == 1) {  // hand over
           uint32_t* bm_out = a.bm + (int64_t)((k + 1) % 3) * a.words;
-          if (t == 0) s.hq = s.hn = 0u;
+          if (t == 0) s.hq = s.hn = s.near = 0u;
           // Dealt out wave by wave, so that the chunk lists of neighbouring
           // hubs are written by different waves.
 #pragma unroll
@@ -859,8 +1007,16 @@ __device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, Ss
             if (xd > 0 && xd <= a.hchunk) o.q[atomicAdd(&s.hq, 1u)] = x;
             wave_put_chunks(a, o.hq, &s.hn, x, xb, xd);
           }
+          if (MP) {
+            unsigned near = 0;
+#pragma unroll
+            for (int r = 0; r < kPer; r++)
+              if (v[r] >= 0) near = max(near, (unsigned)(kInf - du[r]));
+            if (near) atomicMax(&s.near, near);
+          }
           __syncthreads();
           if (t == 0) {
+            if (MP) o.slot->part[0][3] = s.near;
             o.slot->part[0][0] = ctl.c.fv;
             o.slot->part[0][1] = ctl.c.fe;
             o.slot->part[0][2] = ctl.c.scout;
@@ -910,10 +1066,6 @@ __device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, Ss
     for (int r = 0; r < kPer; r++) {
       bool f = old[r] > nd[r];
       if (MP && f) {
-        if (old[r] == kInf) {
-          atomicAdd(&s.reach[0], 1ull);
-          atomicAdd(&s.reach[1], (unsigned long long)(a.row_ptr[hv[r] + 1] - a.row_ptr[hv[r]]));
-        }
         const unsigned h = tab_insert(s, hv[r], &f);
         atomicMin(&s.tab_d[h], nd[r]);
         hv[r] = (int32_t)h;
@@ -925,26 +1077,76 @@ __device__ inline void small_levels(const SsRun& run, int k, SmallLds<MP>& s, Ss
   }
 }
 
-// The final state, once, to the host: the counts and the device time of the
-// traversal.  BOVM's levels are disjoint, so its expanded levels are the
-// vertices reached; min-plus counts first arrivals.
+// The final state, once, to the host (one thread): BOVM's levels are
+// disjoint, so its expanded levels are the vertices reached.
 template <bool MP>
 __device__ inline void ss_finish(const SsArgs& a, SsCtl& ctl) {
-  if (threadIdx.x >= kWave) return;
-  unsigned long long v = 0, e = 0;
-  if (MP) {
-    const unsigned long long* p = a.tot + lane_id() * kStripeU64;
-    v = wave_sum_u64(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    e = wave_sum_u64(__hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  if (!MP) {
+    ctl.st.reached = ctl.st.s.work_fv;
+    ctl.st.edges = ctl.st.s.work_fe;
   }
-  if (threadIdx.x != 0) return;
-  ctl.st.reached = MP ? v : ctl.st.s.work_fv;
-  ctl.st.edges = MP ? e : ctl.st.s.work_fe;
   ctl.st.t1 = wall_clock64();
   if (a.host) {
     *a.host = ctl.st;
     __threadfence_system();
   }
+}
+
+// Min-plus, after the step launches up to launch k: vertices reached and
+// their out-edges, if the traversal is done.  Each workgroup writes its part;
+// the last one to count itself in (one atomic each: several same-address
+// atomics per workgroup took longer than the pass) sums them for the host.
+constexpr unsigned kReachBlocks = 256;
+__global__ void __launch_bounds__(kSsBlock) ss_reach_kernel(SsArgs a, int k) {
+  __shared__ unsigned long long s_t[2];
+  __shared__ unsigned s_last;
+  if (!a.st[k % kSsSlots].s.done) return;
+  if (threadIdx.x < 2) s_t[threadIdx.x] = 0ull;
+  __syncthreads();
+  unsigned long long cnt = 0, edges = 0;
+  const int64_t gs = (int64_t)gridDim.x * kSsBlock;
+  for (int64_t v0 = (int64_t)blockIdx.x * kSsBlock + threadIdx.x; v0 < a.n; v0 += 4 * gs) {
+    int d[4], g[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int64_t v = min(v0 + j * gs, (int64_t)a.n - 1);
+      d[j] = a.dist[v];
+      g[j] = a.row_ptr[v + 1] - a.row_ptr[v];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (v0 + j * gs < a.n && d[j] != kInf) {
+        cnt += 1;
+        edges += (unsigned)g[j];
+      }
+  }
+  cnt = wave_sum_u64(cnt);
+  edges = wave_sum_u64(edges);
+  if (lane_id() == 0 && cnt) {
+    atomicAdd(&s_t[0], cnt);
+    atomicAdd(&s_t[1], edges);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a.tot[1 + 2 * blockIdx.x] = s_t[0];
+    a.tot[2 + 2 * blockIdx.x] = s_t[1];
+    __threadfence();
+    s_last = atomicAdd(&a.tot[0], 1ull) + 1 == gridDim.x;
+  }
+  __syncthreads();
+  if (!s_last || threadIdx.x >= kWave) return;
+  __threadfence();
+  cnt = edges = 0;
+  for (unsigned b = threadIdx.x; b < gridDim.x; b += kWave) {
+    cnt += __hip_atomic_load(&a.tot[1 + 2 * b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    edges += __hip_atomic_load(&a.tot[2 + 2 * b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  cnt = wave_sum_u64(cnt);
+  edges = wave_sum_u64(edges);
+  if (threadIdx.x != 0) return;
+  a.host->reached = cnt;
+  a.host->edges = edges;
+  __threadfence_system();
 }
 
 // Unreached vertices look for a tail in the frontier bitmap; each vertex is
@@ -1059,7 +1261,7 @@ __device__ __forceinline__ void pull_minplus(const SsArgs& a, int32_t src, const
     const bool found = cand && best < cur;
     if (found) {
       a.dist[v] = best;
-      if (cur == kInf) acc.reach(a, v);
+      acc.dist(best);
     }
     const uint64_t fm = __ballot(found);
     if (lane == 0) {
@@ -1073,6 +1275,19 @@ __device__ __forceinline__ void pull_minplus(const SsArgs& a, int32_t src, const
 // One step of the traversal: BOVM (discovers level lv) or min-plus
 // (GOVM/GOVMP semantics: relaxes the out-edges of the vertices whose distance
 // dropped in the previous step).  k: the launch's number modulo 12.
+//
+// Min-plus relaxes in rough distance order: a step expands the frontier
+// vertices below a threshold that moves on by delta every step (and past the
+// smallest frontier distance), and leaves the others in the frontier.  The
+// fixed point is the same; vertices whose distance would still drop are
+// mostly not expanded too early.  delta = 2 x mean weight / mean degree, about
+// the distance the shortest paths' front covers per hop: in a CPU count the
+// steps stay as many as without (2048^2 grid with weights in [1, 1000]: 79 ->
+// 80; random graphs of degree 4-32: 27-35, the same) and the relaxations per
+// edge fall from 2.7-5.5 to 1.3-1.8; half of it takes 1.5-2x the steps, twice
+// of it saves almost no relaxations.  On skewed graphs (RMAT: 16 steps, 4.5
+// relaxations per edge) it takes 59 steps for 3.7, so graphs with a vertex of
+// more than 16 times the mean degree use no threshold.
 template <bool MP>
 __global__ void __launch_bounds__(kSsBlock, 8) ss_step_kernel(SsRun run, int k) {
   __shared__ SsCtl ctl;
@@ -1084,7 +1299,7 @@ __global__ void __launch_bounds__(kSsBlock, 8) ss_step_kernel(SsRun run, int k) 
     SmallLds<MP> small;
   } lds;
   const SsArgs& a = run.a;
-  ss_decide(run, k, ctl);
+  ss_decide<MP>(run, k, ctl);
   if (ctl.run != 0) clear_next(a, k);
   if (ctl.run != 1) {  // uniform over the grid: nothing left, or small levels
     if (blockIdx.x != 0) return;
@@ -1092,8 +1307,10 @@ __global__ void __launch_bounds__(kSsBlock, 8) ss_step_kernel(SsRun run, int k) 
       small_levels<MP>(run, k, lds.small, ctl);
       __syncthreads();
     }
-    if (ctl.fresh) ss_finish<MP>(a, ctl);
-    if (threadIdx.x == 0) a.st[(k + 1) % kSsSlots] = ctl.st;
+    if (threadIdx.x == 0) {
+      if (ctl.fresh) ss_finish<MP>(a, ctl);
+      a.st[(k + 1) % kSsSlots] = ctl.st;
+    }
     return;
   }
   const int lv = ctl.st.s.step, mode = ctl.st.s.mode;
@@ -1111,31 +1328,35 @@ __global__ void __launch_bounds__(kSsBlock, 8) ss_step_kernel(SsRun run, int k) 
   SsStage& sg = lds.wide.sg;
   sg.init();
   Acc acc;
-  // Edge e (< 0: none) to the head v, tail distance du.
-  auto visit = [&](int e, int32_t v, int du, int32_t w) {
-    if (e < 0) return false;
-    return MP ? relax(a, src, du, v, w, bm_out, acc) : discover(a, lv, v, bm_out);
+  // A frontier vertex at or beyond the threshold stays in the frontier.
+  const int32_t thr = MP && ctl.st.delta > 0 ? (int32_t)min(ctl.st.thr, (long long)kInf) : kInf;
+  auto defer = [&](bool yes, int32_t u, int du, int deg) {
+    const uint32_t bit = 1u << (u & 31);
+    const bool first = yes && (atomicOr(&bm_out[u >> 5], bit) & bit) == 0;
+    if (yes) acc.dist(du);
+    if (first) acc.de += (unsigned)deg;
+    sg.append(a, o, first, u, deg, acc);
+  };
+  auto edge = [&](int du0, int du1, int e0, int e1) {
+    Head h0 = head_of<MP>(a, lv, src, e0, du0), h1 = head_of<MP>(a, lv, src, e1, du1);
+    test_head<MP>(a, h0);
+    test_head<MP>(a, h1);
+    join_head<MP>(a, h0, bm_out, acc);
+    join_head<MP>(a, h1, bm_out, acc);
+    sg.append(a, o, h0.join, h0.v, h0.deg, acc);
+    sg.append(a, o, h1.join, h1.v, h1.deg, acc);
   };
   if (mode == DAWN_MODE_PUSH) {
-    push_edges<MP>(a, lds.wide.push, k, ctl.c.qlen, ctl.c.hqlen, [&](int du0, int du1, int e0, int e1) {
-      const int32_t v0 = e0 >= 0 ? a.col[e0] : 0, v1 = e1 >= 0 ? a.col[e1] : 0;
-      const int32_t w0 = MP && e0 >= 0 ? a.w[e0] : 0, w1 = MP && e1 >= 0 ? a.w[e1] : 0;
-      const bool f0 = visit(e0, v0, du0, w0), f1 = visit(e1, v1, du1, w1);
-      sg.append(a, o, f0, v0, acc);
-      sg.append(a, o, f1, v1, acc);
-    });
+    push_edges<MP>(a, lds.wide.push, k, ctl.c.qlen, ctl.c.hqlen, thr, edge, defer);
   } else if (mode == DAWN_MODE_BITMAP) {  // (min-plus: GOVMP shape)
-    bitmap_edges<MP>(a, bm_in, [&](int du, int e) {
-      const int32_t v = e >= 0 ? a.col[e] : 0;
-      sg.append(a, o, visit(e, v, du, MP && e >= 0 ? a.w[e] : 0), v, acc);
-    });
+    bitmap_edges<MP>(a, lds.wide.push, bm_in, thr, edge, defer);
   } else {
     // PULL: the bitmap only, no queue entries.
     if (blockIdx.x == 0 && threadIdx.x == 0) o.slot->qlen = kNoQueue;
     if constexpr (MP) pull_minplus(a, src, bm_in, bm_out, acc);
     else pull_bfs(a, lv, bm_in, bm_out, acc);
   }
-  sg.flush(a, o, acc);
+  sg.flush<MP>(a, o, acc);
 }
 
 int ensure_ss(dawn_graph* g) {
@@ -1148,7 +1369,7 @@ int ensure_ss(dawn_graph* g) {
   DAWN_TRY(ws->hq.alloc((size_t)2 * ws->hcap));
   DAWN_TRY(ws->bm.alloc((size_t)3 * (((int64_t)g->n + 63) / 64 * 2)));
   DAWN_TRY(ws->slots.alloc(kSsSlots));
-  DAWN_TRY(ws->tot.alloc(kStripes * kStripeU64));
+  DAWN_TRY(ws->tot.alloc(1 + 2 * kReachBlocks));
   if (!ws->h_state) DAWN_HIP(hipHostMalloc((void**)&ws->h_state, sizeof(SsState)));
   return ws->st.alloc(kSsSlots);
 }
@@ -1181,6 +1402,8 @@ SsRun make_run(const dawn_graph* g, int32_t source, int32_t policy) {
   p.allow_pull = 1;
   p.avg_degree = g->n ? (float)((double)g->m / g->n) : 0.f;
   p.max_degree = (float)g->max_out_degree;
+  const double avg = p.avg_degree;
+  a.delta_scale = g->m > 0 && g->max_out_degree <= 16 * avg ? 2.0 / (avg * (double)g->m) : 0.0;
   r.force = -1;
   r.small = 1;
   return r;
@@ -1217,8 +1440,10 @@ void ss_step(const SsRun& r, int kind, int64_t k, unsigned grid, hipStream_t s) 
 // A whole traversal: the first `first` step launches, then more (twice as
 // many each time) while the frontier is not empty, one wait after each set.
 // A launch past the end costs 2-4 us, a wait too many about 15 us.  h: the
-// final state; without a pinned r.a.host it is copied from the device.
-int ss_traverse(const dawn_graph* g, const SsRun& r, int kind, int first, hipStream_t s, SsState* h) {
+// final state; without a pinned r.a.host it is copied from the device.  reach:
+// count the vertices reached (min-plus).
+int ss_traverse(const dawn_graph* g, const SsRun& r, int kind, int first, bool reach, hipStream_t s,
+                SsState* h) {
   const unsigned grid = ss_grid(g);
   const bool pinned = r.a.host != nullptr;
   h->s.done = 0;
@@ -1227,6 +1452,7 @@ int ss_traverse(const dawn_graph* g, const SsRun& r, int kind, int first, hipStr
   int64_t k = 0;
   for (int K = first;; K = std::min(64, k == first ? 4 : 2 * K)) {
     for (int i = 0; i < K; i++, k++) ss_step(r, kind, k, grid, s);
+    if (reach) ss_reach_kernel<<<grid_for(g->n, kSsBlock, kReachBlocks), kSsBlock, 0, s>>>(r.a, (int)(k % 12));
     DAWN_HIP(hipGetLastError());
     if (!pinned)
       DAWN_HIP(hipMemcpyAsync(h, r.a.st + k % kSsSlots, sizeof(SsState), hipMemcpyDeviceToHost, s));
@@ -1282,6 +1508,12 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   use_workspace(r, ws);
   if (direct) r.a.dist = dist_out;
   r.a.host = ws->h_state;
+  if (kind == 1 && !ws->wsum.p) {
+    DAWN_TRY(ws->wsum.alloc(kWsumBlocks));
+    ss_wsum_kernel<<<kWsumBlocks, kBlock, 0, g->stream>>>(g->weight, g->m, ws->wsum.p);
+    DAWN_HIP(hipGetLastError());
+  }
+  r.a.wsum = ws->wsum.p;
   // The single-source network (trained on single-source steps); without
   // one the learned policy takes the fixed rule.  Min-plus: the fixed rule.
   r.p.mlp = kind == 0 ? sched_single_mlp_device(g->device, &r.p.mlp_norm) : nullptr;
@@ -1291,7 +1523,7 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   // the frontier empty).
   int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : 8;
   if (g->knobs.ss_chunk <= 0 && ws->last_launches[kind] > 0) K = std::min(256, ws->last_launches[kind]);
-  DAWN_TRY(ss_traverse(g, r, kind, K, g->stream, ws->h_state));
+  DAWN_TRY(ss_traverse(g, r, kind, K, kind == 1 && stats, g->stream, ws->h_state));
   ws->last_launches[kind] = ws->h_state->launches + 1;
   if (stats) DAWN_TRY(ss_stats(g, *ws->h_state, stats));
   if (dist_out && !direct) {
@@ -1432,7 +1664,7 @@ constexpr int64_t kNoAllocHeavy = 1 << 18;  // heavy-chunk entries per level
 constexpr size_t kNaBm = align256(kNaHq + sizeof(int2) * 2 * (size_t)kNoAllocHeavy);
 constexpr size_t kNaSlots = align256(kNaBm + sizeof(uint32_t) * 3 * (size_t)kNoAllocWords);
 constexpr size_t kNaTot = align256(kNaSlots + sizeof(SsSlot) * kSsSlots);
-constexpr size_t kNaState = align256(kNaTot + sizeof(unsigned long long) * kStripes * kStripeU64);
+constexpr size_t kNaState = align256(kNaTot + sizeof(unsigned long long));
 constexpr size_t kNoAllocBytes = align256(kNaState + sizeof(SsState) * kSsSlots);
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
@@ -1480,7 +1712,7 @@ int run_bfs_noalloc(dawn_graph* g, int32_t source, int32_t* dist_out, int32_t po
   const int K = g->knobs.ss_chunk > 0 ? g->knobs.ss_chunk : 8;
   const auto t0 = std::chrono::steady_clock::now();
   SsState h{};
-  DAWN_TRY(ss_traverse(g, r, 0, K, g->stream, &h));
+  DAWN_TRY(ss_traverse(g, r, 0, K, false, g->stream, &h));
   const double ms =
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (stats) {

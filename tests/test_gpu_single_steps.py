@@ -131,3 +131,26 @@ def test_walks_of_small_levels_exact(orc, kind):
             got = out.download()[off // 4:][:n]
             assert np.array_equal(got, ref), (s, off)
         assert np.array_equal(g.bfs_noalloc(s), ref), s
+
+
+@pytest.mark.parametrize("n,deg,wmax", [(1500, 3, 1), (5000, 4, 2), (30000, 12, 100000), (200000, 4, 1000)])
+def test_minplus_thresholds_exact(orc, n, deg, wmax):
+    """Distance thresholds (graphs without hubs): unit and tiny weights (an
+    advance of one), large ones, weights of zero, a few far heavier than the
+    mean, and vertices held back over many steps; all policies."""
+    log(f"case: random directed graph n={n} degree {deg}, weights up to {wmax}, every 50th 200 times that")
+    rng = np.random.default_rng(n)
+    m = n * deg
+    u, v = rng.integers(0, n, m).astype(np.int32), rng.integers(0, n, m).astype(np.int32)
+    w = rng.integers(0, wmax + 1, m).astype(np.int32)
+    w[::50] *= 200
+    h = dawn.HostGraph.from_edges(n, u, v, w, symmetrize=False)
+    g = dawn.Graph(h)
+    for s in np.flatnonzero(h.degrees() > 0)[[0, n // 3]]:
+        ref = orc.sssp(h.row_ptr, h.col, h.weight, int(s))
+        for p in POLICIES:
+            d, st = g.sssp(int(s), policy=p, stats=True)
+            assert np.array_equal(d, ref), (s, p)
+            reached = ref != dawn.INF
+            assert st["vertices_reached"] == reached.sum(), (s, p)
+            assert st["edges_reached"] == h.degrees()[reached].sum(), (s, p)
