@@ -8,9 +8,10 @@
 // no grid-wide synchronisation exists and every workgroup exits once the
 // task counter passes the last task).
 //
-// Unweighted task: all sources of one graph (or a share of them on the
-// largest graphs) as lanes of one word per vertex, as narrow as the lanes
-// allow (<= 64 lanes; 8 sources: a byte), sparse level-synchronous BOVM:
+// Unweighted task: all sources of one graph (or a share of them) as lanes of
+// one field per vertex, level-synchronous BOVM with the fields in LDS, pushed
+// and pulled (run_lds).  Graphs too large for a workgroup's LDS (more than 1.2
+// million vertices) keep words of up to 64 lanes in memory, sparse BOVM:
 //   Q_l = [(v, lanes that reached v at level l)]
 //   expand: for (u, f) in Q_l, w in N(u): nv = f & ~seen[w]; if nv,
 //           atomicOr(next[w], nv); the first writer appends w to `touched`
@@ -41,14 +42,18 @@ struct BatchGraph {
   const int32_t* row_ptr;
   const int32_t* col;
   const int32_t* w;
+  const int32_t* in_row_ptr;  // in-edges (the CSR for undirected graphs)
+  const int32_t* in_col;
   int64_t dist_off;  // first output row of this graph
+  int32_t max_deg;   // largest out-degree
+  int32_t pad;
 };
 
 struct BatchTask {
   int32_t graph;
   int32_t lane0;   // first source index within the graph's block
   int32_t lanes;   // sources in this task (1 for weighted)
-  int32_t pad;
+  int32_t bits;    // unweighted: log2 of the bits per vertex in LDS, -1: state in memory
 };
 
 struct BatchArgs {
@@ -68,7 +73,11 @@ struct BatchArgs {
   int32_t* qv;         // [grid][2][max_n]
   uint64_t* qw;        // [grid][2][max_n]
   int32_t* touched;    // [grid][max_n]
-  uint16_t* stage;     // [grid][max_n][8]: arrival levels of tasks of <= 8 lanes
+  uint8_t* stage;      // [grid][stage_cap]: arrival levels that are not in LDS
+  int64_t stage_cap;
+  int32_t* lds_q;      // [grid][max_lds_n]: vertex queue of the LDS tasks
+  int2* entries;       // [grid][max_lds_n]: expanded queue entries of the LDS tasks
+  int64_t max_lds_n;
 };
 
 namespace {
@@ -83,6 +92,9 @@ namespace {
 // spilled) made the batches slower (18.7 -> 24-27 ms unweighted, 46 -> 51 ms
 // weighted): twice the concurrent tasks' state no longer fits the caches.
 constexpr int kBatchBlock = 1024;
+constexpr int64_t kSpanFlat = 116000, kSpan = 262144;
+constexpr int32_t kHubDeg = 1024;
+constexpr int64_t kSplit2 = 500000, kSplit1 = 2000000;
 
 template <int BS>
 __device__ __forceinline__ int owner(const int* off, int e) {
@@ -172,7 +184,7 @@ __device__ void run_unweighted(const BatchArgs& a, const BatchGraph& G, const Ba
   // once) and write the rows in one coalesced pass at the end, instead of
   // 4-byte stores scattered over the rows as vertices are reached.
   constexpr bool kStage = sizeof(LT) == 1;
-  uint16_t* stage = a.stage + (int64_t)blockIdx.x * mn * 8;
+  uint16_t* stage = reinterpret_cast<uint16_t*>(a.stage + (int64_t)blockIdx.x * a.stage_cap);
   for (int32_t v = threadIdx.x; v < n; v += blockDim.x) {
     seen[v] = (LT)~lanemask;
     next[v] = 0;
@@ -305,6 +317,320 @@ __device__ void run_unweighted(const BatchArgs& a, const BatchGraph& G, const Ba
     }
   }
   if (threadIdx.x == 0) atomicAdd(a.levels_total, (unsigned long long)level);
+}
+
+// ---- unweighted tasks with their state in LDS -----------------------------
+//
+// A graph's traversal probes and updates its per-vertex lane words at random
+// per scanned edge; in memory each probe moved a line (512 graphs, 8 sources:
+// 41 GB, 18.7 ms).  Here a vertex has a field in a workgroup's LDS: for L > 1
+// lanes (1 << bits) 2L bits, A (lanes that have reached it) in the low half
+// and B (lanes that arrive at the level being found) in the high half, so that
+// one LDS atomic marks an arrival in both; for one lane A alone, as its queue
+// entries need no B.  Per level:
+//   gather  the queue's vertices give their B bits, offsets and degrees to
+//           the entry list; B is cleared
+//   pull    of the lanes whose frontier holds more than 1 / kPullShare of the
+//           graph's edges: every vertex that misses one of them ORs its in-
+//           neighbours' A bits until it has found them all (a lane that an
+//           in-neighbour has and the vertex lacks arrived there one level
+//           ago, or the vertex would have it); they enter A afterwards
+//   push    of the other lanes: short lists by a thread per entry, else the
+//           entries' edges spread over the threads (LDS degree scan), four
+//           edges in flight per thread: bits new in A arrive; the first
+//           arrival at a vertex in the level appends it to the queue
+// Arrival levels are staged in a byte per vertex and lane, in LDS where they
+// fit beside the fields (in memory, the scattered bytes of 256 workgroups are
+// most of the batch's traffic), and written as rows at the end.
+constexpr int kLdsWords = 37800;  // 151,200 bytes
+constexpr int kMaxBits = 4;       // up to 16 lanes per task
+constexpr int kPullShare = 8;
+constexpr int kSerialDeg = 12;    // largest out-degree of graphs whose lists threads walk alone
+constexpr uint32_t kStaged8 = 0xFFu;  // stage entry of a level that does not fit (in its row)
+
+// Lanes per vertex (log2) of a task of `lanes` sources on n vertices whose
+// fields fit the LDS, or -1.  A task's entries hold degree and lanes in 32
+// bits, so graphs with a larger degree than 65535 take one lane.
+inline int64_t lds_field_words(int64_t n, int bits) { return (n * (bits ? 2 << bits : 1) + 31) / 32; }
+inline int lds_bits(int64_t n, int lanes, int32_t max_deg) {
+  int b = 0;
+  while ((1 << b) < lanes) b++;
+  return b <= kMaxBits && (b == 0 || max_deg < 65536) && lds_field_words(n, b) <= kLdsWords ? b : -1;
+}
+
+struct LdsTask {
+  uint32_t W[kLdsWords];
+  unsigned lane_edges[1 << kMaxBits];
+};
+
+// Four columns of an edge list, read by one load at any 4-byte offset.
+struct __attribute__((packed, aligned(4))) Cols4 {
+  int32_t c[4];
+};
+// The columns at p, of which r + 1 >= 1 are there (the last one repeated).
+__device__ __forceinline__ Cols4 cols_at(const int32_t* p, int r) {
+  if (r >= 3) return *reinterpret_cast<const Cols4*>(p);
+  return Cols4{{p[0], p[min(1, r)], p[r], p[r]}};
+}
+
+template <int BS>
+__device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask& T, LdsTask& s,
+                        int32_t* qv, int2* ent, int* s_off, int* s_beg, uint32_t* s_f, int* s_scan,
+                        unsigned* s_cnt, uint32_t* s_red) {
+  const int32_t n = G.n;
+  const int t = threadIdx.x;
+  const bool one = T.bits == 0;
+  const int L = 1 << T.bits, fw = one ? 0 : T.bits + 1, fpw = 5 - fw;  // log2 field width, fields per word
+  const uint32_t fmask = (1u << L) - 1u;
+  uint32_t bmask = 0;  // the B halves of a word
+  if (!one)
+    for (int k = 0; k < 32; k += 2 * L) bmask |= fmask << (k + L);
+  const int words = (int)((((int64_t)n << fw) + 31) >> 5);
+  int32_t* drow = a.dist + G.dist_off + (int64_t)T.lane0 * n;
+  uint8_t* lstage = reinterpret_cast<uint8_t*>(s.W + words);
+  uint8_t* gstage = a.stage + (int64_t)blockIdx.x * a.stage_cap;
+  const bool in_lds = (int64_t)words * 4 + (int64_t)n * L <= (int64_t)kLdsWords * 4;
+  auto word_of = [&](int32_t v) { return v >> fpw; };
+  auto shift_of = [&](int32_t v) { return (v & ((1 << fpw) - 1)) << fw; };
+  auto mark = [&](uint32_t nv) { return one ? nv : nv | nv << L; };
+  auto put_level = [&](int32_t v, uint32_t bits, int32_t lv) {
+    for (; bits; bits &= bits - 1) {
+      const int b = __ffs(bits) - 1;
+      const uint8_t x = (uint8_t)min((uint32_t)lv, kStaged8);
+      const int64_t at = (int64_t)v * L + b;
+      if (in_lds) lstage[at] = x;
+      else gstage[at] = x;
+      if (x == kStaged8) drow[(int64_t)b * n + v] = lv;
+    }
+  };
+  for (int i = t; i < words; i += BS) s.W[i] = 0u;
+  if (t == 0) s_cnt[0] = 0u;
+  __syncthreads();
+  if (t < T.lanes) {
+    const int32_t v = a.sources[(int64_t)T.graph * a.spg + T.lane0 + t];
+    const uint32_t bit = 1u << t;
+    const uint32_t old = atomicOr(&s.W[word_of(v)], mark(bit) << shift_of(v)) >> shift_of(v);
+    put_level(v, bit, 0);
+    if (!(old & fmask)) qv[atomicAdd(&s_cnt[0], 1u)] = v;
+  }
+  __syncthreads();
+  int level = 0;
+  for (;; level++) {
+    const unsigned qn = s_cnt[0];
+    if (qn == 0) break;
+    const int32_t lv = level + 1;
+    // Gather: entries of the frontier, its edges, its live lanes.
+    if (t == 0) {
+      s_red[0] = 0u;
+      s_cnt[1] = 0u;
+    }
+    __syncthreads();
+    unsigned fe = 0;  // at most m < 2^31
+    uint32_t live = 0;
+    for (unsigned i = t; i < qn; i += BS) {
+      const int32_t v = qv[i];
+      const uint32_t f = one ? 1u : (s.W[word_of(v)] >> (shift_of(v) + L)) & fmask;
+      const int rb = G.row_ptr[v], d = G.row_ptr[v + 1] - rb;
+      ent[i] = make_int2(rb, one ? d : d | (int)(f << 16));
+      fe += (unsigned)d;
+      live |= f;
+    }
+    for (int o = 32; o >= 1; o >>= 1) {
+      fe += (unsigned)__shfl_xor((int)fe, o);
+      live |= (uint32_t)__shfl_xor((int)live, o);
+    }
+    if (lane_id() == 0) {
+      if (fe) atomicAdd(&s_cnt[1], fe);
+      if (live) atomicOr(&s_red[0], live);
+    }
+    __syncthreads();
+    live = s_red[0];
+    uint32_t pull = 0;  // lanes to pull
+    if ((unsigned long long)s_cnt[1] * kPullShare > (unsigned long long)G.m) {
+      // The frontier's edges lane by lane: the lanes with many are pulled
+      // (a lane with few would make every vertex scan its whole list).
+      if (one) {
+        pull = 1u;
+      } else {
+        if (t < 1 << kMaxBits) s.lane_edges[t] = 0u;
+        __syncthreads();
+        for (int b0 = 0; b0 < T.lanes; b0 += 4) {
+          unsigned c[4] = {0, 0, 0, 0};
+          for (unsigned i = t; i < qn; i += BS) {
+            const unsigned df = (unsigned)ent[i].y;
+#pragma unroll
+            for (int b = 0; b < 4; b++) c[b] += (df >> (16 + b0 + b)) & 1u ? df & 0xFFFFu : 0u;
+          }
+#pragma unroll
+          for (int b = 0; b < 4; b++) {
+            for (int o = 32; o >= 1; o >>= 1) c[b] += (unsigned)__shfl_xor((int)c[b], o);
+            if (lane_id() == 0 && c[b] && b0 + b < T.lanes) atomicAdd(&s.lane_edges[b0 + b], c[b]);
+          }
+        }
+        __syncthreads();
+        for (int b = 0; b < T.lanes; b++)
+          if ((unsigned long long)s.lane_edges[b] * kPullShare > (unsigned long long)G.m) pull |= 1u << b;
+      }
+    }
+    if (!one)
+      for (int i = t; i < words; i += BS) s.W[i] &= ~bmask;
+    if (t == 0) s_cnt[0] = 0u;
+    __syncthreads();
+    if (pull) {
+      for (int32_t v0 = 0; v0 < n; v0 += BS) {
+        const int32_t v = v0 + t;
+        uint32_t miss = 0, got = 0;
+        int beg = 0, deg = 0;
+        if (v < n) {
+          miss = pull & ~(s.W[word_of(v)] >> shift_of(v));
+          if (miss) {
+            beg = G.in_row_ptr[v];
+            deg = G.in_row_ptr[v + 1] - beg;
+          }
+        }
+        auto field = [&](int32_t u) { return s.W[word_of(u)] >> shift_of(u); };
+        const int lim = deg < 64 ? deg : 16;
+        for (int j = 0; j < lim && (got & miss) != miss; j += 4) {
+          const Cols4 u = cols_at(G.in_col + beg + j, deg - 1 - j);
+          got |= field(u.c[0]) | field(u.c[1]) | field(u.c[2]) | field(u.c[3]);
+        }
+        // The rest of long lists by the whole wave, four edges per lane.
+        uint64_t hm = __ballot(deg >= 64 && (got & miss) != miss);
+        while (hm) {
+          const int l = __ffsll((unsigned long long)hm) - 1;
+          hm &= hm - 1;
+          const int hb = __shfl(beg, l), he = hb + __shfl(deg, l);
+          const uint32_t want = (uint32_t)__shfl((int)miss, l);
+          uint32_t g = (uint32_t)__shfl((int)got, l);
+          for (int k0 = hb + 16; k0 < he && (g & want) != want; k0 += 4 * kWave) {
+            const int k = k0 + 4 * lane_id();
+            uint32_t x = 0;
+            if (k < he) {
+              const Cols4 u = cols_at(G.in_col + k, he - 1 - k);
+              x = field(u.c[0]) | field(u.c[1]) | field(u.c[2]) | field(u.c[3]);
+            }
+            for (int o = 32; o >= 1; o >>= 1) x |= (uint32_t)__shfl_xor((int)x, o);
+            g |= x;
+          }
+          if (lane_id() == l) got = g;
+        }
+        got &= miss;
+        if (got) {
+          if (!one) atomicOr(&s.W[word_of(v)], got << (shift_of(v) + L));
+          put_level(v, got, lv);
+        }
+        const int slot = lds_append(&s_cnt[0], got != 0);
+        if (got) qv[slot] = v;
+      }
+      __syncthreads();
+      if (one) {
+        const unsigned found = s_cnt[0];
+        for (unsigned i = t; i < found; i += BS) atomicOr(&s.W[word_of(qv[i])], 1u << shift_of(qv[i]));
+      } else {
+        for (int i = t; i < words; i += BS) s.W[i] |= (s.W[i] & bmask) >> L;
+      }
+      __syncthreads();
+      if (!(live & ~pull)) continue;
+    }
+    // Push the lanes that were not pulled (their bits are disjoint from the
+    // pulled lanes').  Four heads at a time: their words, the atomics on those
+    // that lack a lane, then one reservation of queue slots for the wave.
+    auto visit = [&](const int32_t (&w)[4], const uint32_t (&f)[4]) {
+      uint32_t nv[4], old[4];
+      bool first[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        nv[r] = f[r] ? f[r] & ~(*(volatile uint32_t*)&s.W[word_of(w[r])] >> shift_of(w[r])) : 0u;
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        old[r] = nv[r] ? atomicOr(&s.W[word_of(w[r])], mark(nv[r]) << shift_of(w[r])) >> shift_of(w[r])
+                       : 0u;
+      uint64_t m[4];
+      unsigned cnt = 0;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        nv[r] &= ~old[r];
+        first[r] = nv[r] != 0 && (one || ((old[r] >> L) & fmask) == 0);
+        m[r] = __ballot(first[r]);
+        cnt += (unsigned)__popcll(m[r]);
+      }
+      if (!__ballot((nv[0] | nv[1] | nv[2] | nv[3]) != 0)) return;
+      unsigned at = 0;
+      if (cnt && lane_id() == 0) at = atomicAdd(&s_cnt[0], cnt);
+#pragma unroll
+      for (int r = 0; r < 4; r++) put_level(w[r], nv[r], lv);
+      at = __shfl(at, 0);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        if (first[r]) qv[at + (unsigned)__popcll(m[r] & lanes_below_mask())] = w[r];
+        at += (unsigned)__popcll(m[r]);
+      }
+    };
+    if (G.max_deg <= kSerialDeg) {
+      // Short lists: a thread walks its own entry's, four columns per load.
+      for (unsigned c0 = t & ~(kWave - 1); c0 < qn; c0 += BS) {  // wave-uniform
+        const unsigned i = c0 + lane_id();
+        int2 e2 = make_int2(0, 0);
+        if (i < qn) e2 = ent[i];
+        const uint32_t f = (one ? 1u : (uint32_t)e2.y >> 16) & ~pull;
+        const int d = !f ? 0 : one ? e2.y : e2.y & 0xFFFF;
+        const int most = wave_max_i32(d);
+        for (int j = 0; j < most; j += 4) {
+          Cols4 u{{0, 0, 0, 0}};
+          if (j < d) u = cols_at(G.col + e2.x + j, d - 1 - j);
+          const uint32_t fr[4] = {j < d ? f : 0u, j + 1 < d ? f : 0u, j + 2 < d ? f : 0u,
+                                  j + 3 < d ? f : 0u};
+          visit(u.c, fr);
+        }
+      }
+      __syncthreads();
+      continue;
+    }
+    for (unsigned c0 = 0; c0 < qn; c0 += BS) {
+      const unsigned i = c0 + t;
+      int2 e2 = make_int2(0, 0);
+      if (i < qn) e2 = ent[i];
+      const uint32_t f0 = (one ? 1u : (uint32_t)e2.y >> 16) & ~pull;
+      int total;
+      const int off = scan_bs<BS>(!f0 ? 0 : one ? e2.y : e2.y & 0xFFFF, s_scan, &total);
+      s_off[t] = off;
+      s_beg[t] = e2.x - off;
+      s_f[t] = f0;
+      __syncthreads();
+      constexpr int U = 4;
+      for (int e0 = 0; e0 < total; e0 += U * BS) {
+        int32_t w[U];
+        uint32_t f[U];
+#pragma unroll
+        for (int r = 0; r < U; r++) {
+          const int e = e0 + r * BS + t;
+          f[r] = 0u;
+          w[r] = 0;
+          if (e < total) {
+            const int j = owner<BS>(s_off, e);
+            f[r] = s_f[j];
+            w[r] = G.col[s_beg[j] + e];
+          }
+        }
+        visit(w, f);
+      }
+      __syncthreads();
+    }
+  }
+  // Rows: a row store of a wave covers 64 consecutive vertices.
+  for (int32_t v = t; v < n; v += BS) {
+    const uint32_t got = s.W[word_of(v)] >> shift_of(v);
+    for (int b = 0; b < T.lanes; b++) {
+      const int64_t at = (int64_t)v * L + b;
+      if (!((got >> b) & 1u)) {
+        drow[(int64_t)b * n + v] = kInf;
+      } else {
+        const uint32_t l = in_lds ? lstage[at] : gstage[at];
+        if (l != kStaged8) drow[(int64_t)b * n + v] = (int32_t)l;
+      }
+    }
+  }
+  if (t == 0) atomicAdd(a.levels_total, (unsigned long long)level);
 }
 
 // One weighted source.  The reference's initialisation
@@ -514,11 +840,15 @@ template <int BS>
 __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
   __shared__ int s_off[BS];
   __shared__ int s_beg[BS];
-  __shared__ uint64_t s_f[BS];
+  __shared__ uint32_t s_lf[BS];
   __shared__ int s_scan[BS / kWave];
   __shared__ unsigned s_cnt[5];
   __shared__ int s_red[2];
   __shared__ int s_task;
+  __shared__ uint32_t s_or[1];
+  __shared__ LdsTask s_lds;
+  // The tasks with their state in memory use the LDS for what is left of theirs.
+  uint64_t* s_f = reinterpret_cast<uint64_t*>(s_lds.W);
   const int64_t mn = a.max_n;
   uint64_t* seen = a.seen + (int64_t)blockIdx.x * mn;
   uint64_t* next = a.next + (int64_t)blockIdx.x * mn;
@@ -536,6 +866,9 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
     if (G.weighted)
       run_weighted<BS>(a, G, T, (uint8_t*)next, qv, (int32_t*)qw, s_off, s_beg,
                        (int*)s_f, s_scan, s_cnt, s_red);
+    else if (T.bits >= 0)
+      run_lds<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
+                  a.entries + (int64_t)blockIdx.x * a.max_lds_n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or);
     else if (T.lanes <= 8)
       run_unweighted<BS, uint8_t>(a, G, T, (uint8_t*)seen, (uint8_t*)next, qv, (uint8_t*)qw,
                                   touched, s_off, s_beg, s_f, s_scan, s_cnt);
@@ -563,15 +896,17 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   if (!graphs || num_graphs <= 0 || !sources || spg <= 0 || spg > 64 || !dist_offsets)
     return DAWN_ERR_INVALID_ARG;
   const int device = graphs[0]->device;
-  int64_t max_n = 1, total = 0;
+  int64_t total = 0;
+  // Largest graphs of the tasks that keep state in memory, and in LDS.
+  int64_t max_n = 0, max_lds_n = 0, stage_cap = 0;
   std::vector<BatchGraph> hg(num_graphs);
   std::vector<BatchTask> ht;
   std::vector<int32_t> hs((size_t)num_graphs * spg);
   for (int32_t i = 0; i < num_graphs; i++) {
     dawn_graph* g = graphs[i];
     if (!g || g->device != device || g->n <= 0) return DAWN_ERR_INVALID_ARG;
-    max_n = std::max<int64_t>(max_n, g->n);
-    hg[i] = BatchGraph{g->n, g->weighted, g->m, g->row_ptr, g->col, g->weight, dist_offsets[i]};
+    hg[i] = BatchGraph{g->n, g->weighted, g->m, g->row_ptr, g->col, g->weight, g->in_row_ptr,
+                       g->in_col, dist_offsets[i], g->max_out_degree, 0};
     total = std::max<int64_t>(total, dist_offsets[i] + (int64_t)spg * g->n);
     for (int32_t j = 0; j < spg; j++) {
       int64_t s = sources[(int64_t)i * spg + j] % (int64_t)g->n;
@@ -580,46 +915,74 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
       if (stats && g->h_row_ptr[s] == g->h_row_ptr[s + 1]) stats->skipped_sources += 1;
     }
     if (g->weighted) {
-      for (int32_t j = 0; j < spg; j++) ht.push_back(BatchTask{i, j, 1, 0});
+      for (int32_t j = 0; j < spg; j++) ht.push_back(BatchTask{i, j, 1, -1});
+      max_n = std::max<int64_t>(max_n, g->n);
     } else {
-      // The sources of a graph share one task as lanes of a word, except
+      // The sources of a graph share one task as lanes of a field, except
       // on the largest graphs, whose tasks would be the batch's critical
-      // path: from 500k edges two tasks of half the lanes, from 2M edges a
-      // task per source (512 graphs of 1k-130k vertices, 8 sources each:
-      // 31.5 -> 25.5 ms).
-      const int32_t per = g->m >= 2000000 ? 1 : g->m >= 500000 ? std::max(1, spg / 2) : spg;
-      for (int32_t j = 0; j < spg; j += per) ht.push_back(BatchTask{i, j, std::min(per, spg - j), 0});
+      // path, and where fewer lanes keep the fields and staged levels in LDS
+      // (kSpan*: lanes x vertices; graphs with hubs pull most of their edges
+      // once for all lanes and take more).  512 graphs of 1k-130k vertices, 8
+      // sources: one task per graph 4.6 ms, at most 65,536 lanes x vertices
+      // 3.6, at most 116,000 with the levels in LDS 2.6.
+      int32_t per = std::min(spg, 1 << kMaxBits);
+      if (g->m >= kSplit1) per = 1;
+      else if (g->m >= kSplit2) per = std::max(1, spg / 2);
+      const int64_t span = g->max_out_degree <= kHubDeg ? kSpanFlat : kSpan;
+      while (per > 1 && (lds_bits(g->n, per, g->max_out_degree) < 0 || g->n * (int64_t)per > span))
+        per = (per + 1) / 2;
+      if (lds_bits(g->n, per, g->max_out_degree) < 0) {
+        // Graphs beyond the LDS: state in memory, lanes as wide as 64.
+        per = g->m >= 2000000 ? 1 : g->m >= 500000 ? std::max(1, spg / 2) : spg;
+        max_n = std::max<int64_t>(max_n, g->n);
+        if (per <= 8) stage_cap = std::max<int64_t>(stage_cap, (int64_t)g->n * 16);
+      } else {
+        max_lds_n = std::max<int64_t>(max_lds_n, g->n);
+      }
+      for (int32_t j = 0; j < spg; j += per) {
+        const int32_t lanes = std::min(per, spg - j);
+        const int bits =
+            lds_bits(g->n, per, g->max_out_degree) < 0 ? -1 : lds_bits(g->n, lanes, g->max_out_degree);
+        if (bits >= 0 && lds_field_words(g->n, bits) * 4 + ((int64_t)g->n << bits) > (int64_t)kLdsWords * 4)
+          stage_cap = std::max<int64_t>(stage_cap, (int64_t)g->n << bits);
+        ht.push_back(BatchTask{i, j, lanes, bits});
+      }
     }
   }
-  // Largest graphs first: the long tasks start early.
-  std::stable_sort(ht.begin(), ht.end(), [&](const BatchTask& x, const BatchTask& y) {
-    return hg[x.graph].n > hg[y.graph].n;
-  });
+  // The long tasks start early: graphs of short lists take many levels (a
+  // grid of 131,000 vertices 2.8 ms), the others go by their edges.
+  auto cost = [&](const BatchTask& x) {
+    const BatchGraph& g = hg[x.graph];
+    return (g.weighted ? 0 : (g.max_deg <= kSerialDeg ? 5 : 1) * x.lanes) * (int64_t)g.n + g.m;
+  };
+  std::stable_sort(ht.begin(), ht.end(),
+                   [&](const BatchTask& x, const BatchTask& y) { return cost(x) > cost(y); });
   DAWN_HIP(hipSetDevice(device));
   int cus = 0;
   DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   // One workgroup per CU: as many as are resident at once.
   const int grid = std::max(1, std::min<int>((int)ht.size(), cus));
 
-  DevBuf<BatchGraph> dg;
-  DevBuf<BatchTask> dt;
-  DevBuf<int32_t> ds, dq, dtouch, dout;
-  DevBuf<uint64_t> dseen, dnext, dqw;
-  DevBuf<uint16_t> dstage;
-  DevBuf<unsigned> dcnt;
-  DevBuf<unsigned long long> dlev, dwsum;
-  DAWN_TRY(dg.alloc(num_graphs));
-  DAWN_TRY(dt.alloc(ht.size()));
-  DAWN_TRY(ds.alloc(hs.size()));
-  DAWN_TRY(dseen.alloc((size_t)grid * max_n));
-  DAWN_TRY(dnext.alloc((size_t)grid * max_n));
-  DAWN_TRY(dq.alloc((size_t)grid * 2 * max_n));
-  DAWN_TRY(dqw.alloc((size_t)grid * 2 * max_n));
-  DAWN_TRY(dtouch.alloc((size_t)grid * max_n));
-  DAWN_TRY(dstage.alloc((size_t)grid * max_n * 8));
-  DAWN_TRY(dcnt.alloc(1));
-  DAWN_TRY(dlev.alloc(1));
-  DAWN_TRY(dwsum.alloc(num_graphs));
+  // One allocation for everything, cut at 256-byte offsets.
+  stage_cap = (stage_cap + 255) / 256 * 256;
+  DevBuf<unsigned char> mem;
+  DevBuf<int32_t> dout;
+  size_t bytes = 0;
+  auto cut = [&](size_t count, size_t size) {
+    const size_t at = bytes;
+    bytes += (count * size + 255) / 256 * 256;
+    return at;
+  };
+  const size_t g1 = (size_t)grid, mx = (size_t)max_n, lx = (size_t)max_lds_n;
+  const size_t o_graphs = cut(hg.size(), sizeof(BatchGraph)), o_tasks = cut(ht.size(), sizeof(BatchTask));
+  const size_t o_src = cut(hs.size(), sizeof(int32_t));
+  const size_t o_cnt = cut(1, sizeof(unsigned)), o_lev = cut(1, sizeof(unsigned long long));
+  const size_t o_wsum = cut(hg.size(), sizeof(unsigned long long)), o_zero_end = bytes;
+  const size_t o_seen = cut(g1 * mx, sizeof(uint64_t)), o_next = cut(g1 * mx, sizeof(uint64_t));
+  const size_t o_q = cut(g1 * 2 * mx, sizeof(int32_t)), o_qw = cut(g1 * 2 * mx, sizeof(uint64_t));
+  const size_t o_touch = cut(g1 * mx, sizeof(int32_t)), o_stage = cut(g1 * (size_t)stage_cap, 1);
+  const size_t o_ldsq = cut(g1 * lx, sizeof(int32_t)), o_ent = cut(g1 * lx, sizeof(int2));
+  DAWN_TRY(mem.alloc(bytes));
   const bool dev_out = is_device_pointer(dist);
   int32_t* out = dist;
   if (!dev_out) {
@@ -627,36 +990,39 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
     out = dout.p;
   }
   hipStream_t s = graphs[0]->stream;
-  DAWN_HIP(hipMemcpyAsync(dg.p, hg.data(), sizeof(BatchGraph) * hg.size(), hipMemcpyHostToDevice, s));
-  DAWN_HIP(hipMemcpyAsync(dt.p, ht.data(), sizeof(BatchTask) * ht.size(), hipMemcpyHostToDevice, s));
-  DAWN_HIP(hipMemcpyAsync(ds.p, hs.data(), sizeof(int32_t) * hs.size(), hipMemcpyHostToDevice, s));
-  DAWN_HIP(hipMemsetAsync(dcnt.p, 0, sizeof(unsigned), s));
-  DAWN_HIP(hipMemsetAsync(dlev.p, 0, sizeof(unsigned long long), s));
-  DAWN_HIP(hipMemsetAsync(dwsum.p, 0, sizeof(unsigned long long) * num_graphs, s));
+  unsigned char* const M = mem.p;
+  DAWN_HIP(hipMemcpyAsync(M + o_graphs, hg.data(), sizeof(BatchGraph) * hg.size(), hipMemcpyHostToDevice, s));
+  DAWN_HIP(hipMemcpyAsync(M + o_tasks, ht.data(), sizeof(BatchTask) * ht.size(), hipMemcpyHostToDevice, s));
+  DAWN_HIP(hipMemcpyAsync(M + o_src, hs.data(), sizeof(int32_t) * hs.size(), hipMemcpyHostToDevice, s));
+  DAWN_HIP(hipMemsetAsync(M + o_cnt, 0, o_zero_end - o_cnt, s));
   BatchArgs a{};
-  a.graphs = dg.p;
-  a.tasks = dt.p;
+  a.graphs = (const BatchGraph*)(M + o_graphs);
+  a.tasks = (const BatchTask*)(M + o_tasks);
   a.num_tasks = (int32_t)ht.size();
   a.spg = spg;
-  a.sources = ds.p;
+  a.sources = (const int32_t*)(M + o_src);
   a.dist = out;
-  a.task_counter = dcnt.p;
-  a.levels_total = dlev.p;
-  a.wsum = dwsum.p;
+  a.task_counter = (unsigned*)(M + o_cnt);
+  a.levels_total = (unsigned long long*)(M + o_lev);
+  a.wsum = (const unsigned long long*)(M + o_wsum);
   a.max_n = max_n;
-  a.seen = dseen.p;
-  a.next = dnext.p;
-  a.qv = dq.p;
-  a.qw = dqw.p;
-  a.touched = dtouch.p;
-  a.stage = dstage.p;
+  a.seen = (uint64_t*)(M + o_seen);
+  a.next = (uint64_t*)(M + o_next);
+  a.qv = (int32_t*)(M + o_q);
+  a.qw = (uint64_t*)(M + o_qw);
+  a.touched = (int32_t*)(M + o_touch);
+  a.stage = M + o_stage;
+  a.stage_cap = stage_cap;
+  a.lds_q = (int32_t*)(M + o_ldsq);
+  a.entries = (int2*)(M + o_ent);
+  a.max_lds_n = max_lds_n;
   hipEvent_t e0, e1;
   DAWN_HIP(hipEventCreate(&e0));
   DAWN_HIP(hipEventCreate(&e1));
   bool any_weighted = false;
   for (const BatchGraph& x : hg) any_weighted = any_weighted || x.weighted;
   DAWN_HIP(hipEventRecord(e0, s));
-  if (any_weighted) wsum_kernel<<<num_graphs * kWsumParts, kBlock, 0, s>>>(dg.p, dwsum.p);
+  if (any_weighted) wsum_kernel<<<num_graphs * kWsumParts, kBlock, 0, s>>>(a.graphs, (unsigned long long*)(M + o_wsum));
   batch_kernel<kBatchBlock><<<grid, kBatchBlock, 0, s>>>(a);
   DAWN_HIP(hipGetLastError());
   DAWN_HIP(hipEventRecord(e1, s));
@@ -666,7 +1032,7 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   unsigned long long levels = 0;
-  DAWN_HIP(hipMemcpy(&levels, dlev.p, sizeof levels, hipMemcpyDeviceToHost));
+  DAWN_HIP(hipMemcpy(&levels, a.levels_total, sizeof levels, hipMemcpyDeviceToHost));
   if (dist && !dev_out)
     DAWN_HIP(hipMemcpy(dist, out, sizeof(int32_t) * (size_t)total, hipMemcpyDeviceToHost));
   if (stats) {
