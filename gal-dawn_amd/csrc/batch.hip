@@ -18,8 +18,9 @@
 //   commit: for w in touched: nw = next[w] & ~seen[w]; next[w] = 0;
 //           seen[w] |= nw; dist[b][w] = l+1 for b in nw; Q_{l+1} += (w, nw)
 // Weighted task: one source, int32 min-plus (the fixed point of GOVM,
-// src/algorithm/cpu/sssp.cpp:141-199, from the reference's seeding), by
-// near-far relaxation: vertices whose distance dropped are relaxed next if
+// src/algorithm/cpu/sssp.cpp:141-199, from the reference's seeding), with its
+// state in LDS up to 134,000 vertices (run_weighted_lds).  Larger graphs by
+// near-far relaxation in memory: vertices whose distance dropped are relaxed next if
 // it is below a threshold (near), else set aside (far); when no near vertex
 // is left the threshold moves past the smallest far distance by delta and
 // the far pile is split.  Relaxing in distance order re-relaxes far fewer
@@ -35,15 +36,19 @@
 
 namespace dawn {
 
+// Device memory by type: through a plain pointer that was itself read from
+// memory the compiler emits flat loads, which also wait for the LDS.
+typedef const int32_t __attribute__((address_space(1)))* GlobalInts;
+
 struct BatchGraph {
   int32_t n;
   int32_t weighted;
   int64_t m;
-  const int32_t* row_ptr;
-  const int32_t* col;
-  const int32_t* w;
-  const int32_t* in_row_ptr;  // in-edges (the CSR for undirected graphs)
-  const int32_t* in_col;
+  GlobalInts row_ptr;
+  GlobalInts col;
+  GlobalInts w;
+  GlobalInts in_row_ptr;  // in-edges (the CSR for undirected graphs)
+  GlobalInts in_col;
   int64_t dist_off;  // first output row of this graph
   int32_t max_deg;   // largest out-degree
   int32_t pad;
@@ -105,6 +110,40 @@ __device__ __forceinline__ int owner(const int* off, int e) {
     else hi = mid - 1;
   }
   return lo;
+}
+
+// The owners of 4 x 64 consecutive edges from e0 on (wave-uniform), edge
+// e0 + 64 r + lane in o[r]; past the end the last edge, e[r].  First the
+// owners of the range's two ends, a ballot over BS/64 segments and one inside,
+// then each lane searches between those: 4 probes at a mean degree of 16
+// instead of 10, and without branches, so that the four searches interleave
+// and the loads that follow are all in flight (one weighted source of RMAT-17:
+// relaxations 5.1 ms -> 3.2 ms).
+template <int BS>
+__device__ __forceinline__ int wave_owner(const int* off, int e) {
+  constexpr int S = BS / kWave;
+  const int seg = __popcll(__ballot(off[lane_id() * S] <= e)) - 1;
+  const uint64_t in = __ballot(off[seg * S + lane_id() % S] <= e);
+  return seg * S + __popcll(in & ((1ull << S) - 1)) - 1;
+}
+template <int BS>
+__device__ __forceinline__ void owners4(const int* off, int e0, int edges, int (&e)[4], int (&o)[4]) {
+  const int lo = __builtin_amdgcn_readfirstlane(wave_owner<BS>(off, e0));
+  const int hi = __builtin_amdgcn_readfirstlane(wave_owner<BS>(off, min(e0 + 4 * kWave, edges) - 1));
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    e[r] = min(e0 + r * kWave + lane_id(), edges - 1);
+    o[r] = lo;
+  }
+  for (int step = hi > lo ? 1 << (31 - __clz(hi - lo)) : 0; step; step >>= 1) {
+    int to[4], at[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) to[r] = min(o[r] + step, hi);
+#pragma unroll
+    for (int r = 0; r < 4; r++) at[r] = off[to[r]];
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[r] = at[r] <= e[r] ? to[r] : o[r];
+  }
 }
 
 // Exclusive scan of one int per thread over a BS-thread workgroup.
@@ -359,7 +398,7 @@ inline int lds_bits(int64_t n, int lanes, int32_t max_deg) {
 }
 
 struct LdsTask {
-  uint32_t W[kLdsWords];
+  alignas(16) uint32_t W[kLdsWords];
   unsigned lane_edges[1 << kMaxBits];
 };
 
@@ -368,8 +407,8 @@ struct __attribute__((packed, aligned(4))) Cols4 {
   int32_t c[4];
 };
 // The columns at p, of which r + 1 >= 1 are there (the last one repeated).
-__device__ __forceinline__ Cols4 cols_at(const int32_t* p, int r) {
-  if (r >= 3) return *reinterpret_cast<const Cols4*>(p);
+__device__ __forceinline__ Cols4 cols_at(GlobalInts p, int r) {
+  if (r >= 3) return *(const Cols4*)(const int32_t*)p;
   return Cols4{{p[0], p[min(1, r)], p[r], p[r]}};
 }
 
@@ -540,7 +579,9 @@ __device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask
       bool first[4];
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        nv[r] = f[r] ? f[r] & ~(*(volatile uint32_t*)&s.W[word_of(w[r])] >> shift_of(w[r])) : 0u;
+        nv[r] = __hip_atomic_load(&s.W[word_of(w[r])], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+      for (int r = 0; r < 4; r++) nv[r] = f[r] & ~(nv[r] >> shift_of(w[r]));
 #pragma unroll
       for (int r = 0; r < 4; r++)
         old[r] = nv[r] ? atomicOr(&s.W[word_of(w[r])], mark(nv[r]) << shift_of(w[r])) >> shift_of(w[r])
@@ -597,21 +638,17 @@ __device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask
       s_beg[t] = e2.x - off;
       s_f[t] = f0;
       __syncthreads();
-      constexpr int U = 4;
-      for (int e0 = 0; e0 < total; e0 += U * BS) {
-        int32_t w[U];
-        uint32_t f[U];
+      for (int e0 = __builtin_amdgcn_readfirstlane(t / kWave) * 4 * kWave; e0 < total; e0 += 4 * BS) {
+        int e[4], o[4];
+        int32_t w[4];
+        uint32_t f[4];
+        owners4<BS>(s_off, e0, total, e, o);
 #pragma unroll
-        for (int r = 0; r < U; r++) {
-          const int e = e0 + r * BS + t;
-          f[r] = 0u;
-          w[r] = 0;
-          if (e < total) {
-            const int j = owner<BS>(s_off, e);
-            f[r] = s_f[j];
-            w[r] = G.col[s_beg[j] + e];
-          }
-        }
+        for (int r = 0; r < 4; r++) w[r] = G.col[s_beg[o[r]] + e[r]];
+#pragma unroll
+        for (int r = 0; r < 4; r++) f[r] = s_f[o[r]];
+#pragma unroll
+        for (int r = 0; r < 4; r++) f[r] = e0 + r * kWave + lane_id() < total ? f[r] : 0u;
         visit(w, f);
       }
       __syncthreads();
@@ -816,6 +853,318 @@ __device__ void run_weighted(const BatchArgs& a, const BatchGraph& G, const Batc
   if (threadIdx.x == 0) atomicAdd(a.levels_total, (unsigned long long)steps);
 }
 
+// ---- weighted tasks with LDS state ----------------------------------------
+//
+// Label-correcting relaxation to the same fixed point, with everything that
+// is probed at random per edge in LDS and no queues: what is to be expanded is
+// marked at the vertex, and every step scans the marks.
+//
+// Graphs of up to kDistN vertices keep the distances there (DL): a word
+// 2 d + mark, all ones for a vertex not reached.  An improvement is one
+// unsigned minimum with 2 nd + 1: it sets the mark, and an equal distance
+// changes nothing.  Larger graphs keep the distances in the output row and in
+// LDS a mark bit and a byte, d <= base + byte * 2^qs, 255 for none known: an
+// edge whose path is no shorter than that bound cannot improve the vertex and
+// touches no memory.  Bytes are stored without an atomic: of two improvements
+// the larger may stay, which only makes the bound looser and the vertex later.
+// When the bytes to come leave the lower half of the range, base moves up to
+// the smallest and all are rewritten (rebase).
+//
+// Graphs without hubs move the threshold by delta after every step (rolling:
+// few steps, 1.0-1.8 relaxations per edge); graphs with hubs exhaust what is
+// below it first (1.3 to 1.7 per edge where rolling takes 3.4).  delta, in mean
+// weights over the mean degree: 2 where the distances are in LDS and a step
+// costs about what its relaxations do (1: grids of up to 37,000 vertices 26%
+// slower, RMAT 13%); 1 (hubs: 1/2) where a relaxation may go to memory (2:
+// random graphs 33% slower, grids 7%, RMAT-17 13%).
+//
+// Measured, 512 graphs of 1,000 to 130,000 vertices, 8 sources each (1.7 G
+// edges to relax once): 45.0 ms with queues, marks and distances in memory and
+// one edge per thread in flight.  What bounds it now is the instructions of a
+// relaxation (RMAT-17, one CU: 2 G relaxations/s of 60 VALU and 15 LDS
+// operations per wave and edge) and, for small graphs, the step's scan (3 us).
+constexpr int64_t kDistN = kLdsWords - 3;  // words, rounded up to four
+constexpr int64_t kBoundN = 134000;        // a byte and a bit per vertex
+constexpr int64_t kSerialM = 4;            // edges of one load
+constexpr int64_t kLdsM = 1 << 30;         // edges reached by 32-bit byte offsets
+static_assert((kBoundN + 3) / 4 + (kBoundN + 31) / 32 <= kLdsWords, "bounds and marks");
+enum { kWeightedMemory = -1, kWeightedDist = 0, kWeightedBound = 1 };  // BatchTask::bits
+
+// p[i] by a 32-bit offset from a base in scalar registers.
+__device__ __forceinline__ int32_t at32(GlobalInts p, uint32_t i) {
+  return *(GlobalInts)((const char __attribute__((address_space(1)))*)p + i * 4u);
+}
+
+// Of two distances, kInf for none, in 32 bits (both are >= 0).
+__device__ __forceinline__ int32_t plus_sat(int32_t a, int32_t b) {
+  return (int32_t)min((uint32_t)a + (uint32_t)b, (uint32_t)kInf);
+}
+
+__device__ __forceinline__ Cols4 four_at(GlobalInts p, uint32_t i) {
+  return *(const Cols4*)((const char*)(const int32_t*)p + i * 4u);
+}
+
+template <int BS, bool DL>
+__device__ void run_weighted_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask& T, LdsTask& s,
+                                 int* s_off, int* s_beg, int* s_du, int* s_scan, int* s_red) {
+  // Vertices per thread: quads at a stride of BS quads, or words of 32 in order.
+  constexpr int kQuads = (int)((kDistN + 4 * BS - 1) / (4 * BS));
+  constexpr int kWords = (int)(((kBoundN + 31) / 32 + BS - 1) / BS);
+  static_assert(kQuads * 4 <= 64, "a bit each");
+  const int32_t n = G.n;
+  const int t = threadIdx.x;
+  const int32_t src = a.sources[(int64_t)T.graph * a.spg + T.lane0];
+  int32_t* dist = a.dist + G.dist_off + (int64_t)T.lane0 * n;
+  uint32_t* word = s.W;                               // DL
+  uint8_t* key = reinterpret_cast<uint8_t*>(s.W);     // otherwise
+  const int nb = (n + 31) / 32, n4 = (n + 3) / 4;
+  uint32_t* pend = s.W + n4;
+  const double avg_w = G.m > 0 ? (double)a.wsum[T.graph] / (double)G.m : 1.0;
+  const double avg_deg = n > 0 ? (double)G.m / (double)n : 1.0;
+  const bool roll = G.max_deg <= 16 * avg_deg;
+  const double delta = fmax(1.0, ceil((DL ? 2.0 : roll ? 1.0 : 0.5) * avg_w / fmax(avg_deg, 1.0)));
+  int qs = 0;  // two or three units to a delta
+  while (!DL && qs < 22 && (double)(2ll << qs) < delta * (2.0 / 3)) qs++;
+  const long long step_k = DL ? (long long)delta : (long long)ceil(delta / (double)(1 << qs));
+  uint32_t base = 0;
+  auto get = [&](int32_t v) {
+    return __hip_atomic_load((int32_t*)((char*)dist + (uint32_t)v * 4u), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto put = [&](int32_t v, int32_t d) {
+    __hip_atomic_store(dist + v, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto key_of = [&](int32_t v) {
+    return (uint32_t)__hip_atomic_load(key + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto units = [&](int32_t d) {  // smallest k >= 0 with d <= base + k * 2^qs, at most 255
+    return (uint32_t)d <= base ? 0u : min(((uint32_t)d - base + (1u << qs) - 1u) >> qs, 255u);
+  };
+  auto improved = [&](int32_t v, int32_t d) {
+    __hip_atomic_store(key + v, (uint8_t)units(d), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    atomicOr(&pend[v >> 5], 1u << (v & 31));
+  };
+  for (int32_t v = t; v < (DL ? n4 * 4 : n); v += BS) {
+    if (DL) word[v] = ~0u;
+    else dist[v] = kInf, key[v] = 255;
+  }
+  if (!DL)
+    for (int i = t; i < nb; i += BS) pend[i] = 0u;
+  __syncthreads();
+  // Reference initialisation (sssp.cpp:40-46), all edges at once: a
+  // neighbour's slot first takes a tag of its last listed edge, then that edge
+  // alone replaces it by its weight.  Tags are even (DL: the words of marked
+  // vertices are odd) or negative (weights are >= 0).
+  const int32_t sb = G.row_ptr[src], se = G.row_ptr[src + 1];
+  for (int32_t k = sb + t; k < se; k += BS) {
+    if (DL) atomicMin(&word[G.col[k]], (uint32_t)(kInf - k) * 2u);
+    else atomicMin(&dist[G.col[k]], -1 - k);
+  }
+  __syncthreads();
+  for (int32_t k = sb + t; k < se; k += BS) {
+    const int32_t v = G.col[k], w = G.w[k];
+    if (DL) {
+      if (word[v] == (uint32_t)(kInf - k) * 2u) word[v] = (uint32_t)w * 2u + 1u;
+    } else if (get(v) == -1 - k) {
+      put(v, w);
+      if (v != src && w != kInf) improved(v, w);
+    }
+  }
+  __syncthreads();
+  if (t == 0) {
+    if (DL) word[src] = 0u;
+    else put(src, 0), key[src] = 0;
+  }
+  // Four relaxations in flight: the keys, atomics on those that may improve.
+  auto relax = [&](const int32_t (&v)[4], const int32_t (&nd)[4]) {
+    if (DL) {
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        atomicMin(&word[v[r]], (uint32_t)nd[r] * 2u + 1u);
+      return;
+    }
+    bool may[4];
+    uint32_t k[4];
+    int32_t old[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) k[r] = key_of(v[r]);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      may[r] = (uint32_t)nd[r] < (k[r] == 255u ? (uint32_t)kInf : base + (k[r] << qs));
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      old[r] = may[r] ? atomicMin((int32_t*)((char*)dist + (uint32_t)v[r] * 4u), nd[r]) : -1;
+    // Opaque to the compiler, which else moves each comparison, and with it
+    // the wait for its atomic, up before the next atomic.
+#pragma unroll
+    for (int r = 0; r < 4; r++) asm volatile("" : "+v"(old[r]));
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (nd[r] < old[r]) improved(v[r], nd[r]);
+  };
+  long long thr = -1;  // set by the first pass, which selects nothing
+  uint32_t steps = 0;
+  for (;;) {
+    if (t == 0) s_red[0] = kInf;
+    __syncthreads();
+    // What is to be expanded with a key of at most thr, and the smallest key
+    // of the rest.
+    uint64_t quads = 0;
+    uint32_t sel[kWords];
+    int count = 0;
+    int32_t least = kInf;
+    if (DL) {
+      const uint32_t lim = thr < 0 ? 0u : (uint32_t)min(thr, (long long)kInf - 1) * 2u + 1u;
+      uint32_t lm = ~0u;
+#pragma unroll
+      for (int r = 0; r < kQuads; r++) {
+        const int q = r * BS + t;
+        if (q < n4) {
+          const uint4 x = reinterpret_cast<const uint4*>(word)[q];
+          const uint32_t y[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const bool marked = y[c] & 1u, in = marked && y[c] <= lim;
+            quads |= (uint64_t)in << (r * 4 + c);
+            if (marked && !in) lm = min(lm, y[c]);
+          }
+        }
+      }
+      count = __popcll(quads);
+      least = (int32_t)(lm >> 1);  // all ones (not reached): kInf
+    } else {
+#pragma unroll
+      for (int r = 0; r < kWords; r++) {
+        const int i = t * kWords + r;
+        uint32_t x = i < nb ? pend[i] : 0u;
+        sel[r] = 0u;
+        while (x) {
+          const int b = __ffs(x) - 1;
+          x &= x - 1;
+          const int32_t k = (int32_t)key_of(i * 32 + b);
+          if ((long long)k <= thr) sel[r] |= 1u << b;
+          else least = min(least, k);
+        }
+        count += __popc(sel[r]);
+      }
+    }
+    least = wave_min_i32(least);
+    if (lane_id() == 0 && least != kInf) atomicMin(&s_red[0], least);
+    int total;
+    int pos = scan_bs<BS>(count, s_scan, &total);
+    if (total == 0) {
+      const int32_t fm = s_red[0];  // scan_bs has synchronised
+      __syncthreads();
+      if (fm == kInf) break;
+      if (!DL && fm > 127) {
+        // Rebase.  Unknown bytes are set from the distances; where only such
+        // are to come, base moves to the smallest of their distances.
+        uint32_t shift = (uint32_t)(fm - 1);
+        if (fm == 255) {
+          int32_t dm = kInf;
+          for (int i = t; i < nb; i += BS)
+            for (uint32_t x = pend[i]; x; x &= x - 1) dm = min(dm, get(i * 32 + __ffs(x) - 1));
+          dm = wave_min_i32(dm);
+          if (t == 0) s_red[0] = kInf;
+          __syncthreads();
+          if (lane_id() == 0) atomicMin(&s_red[0], dm);
+          __syncthreads();
+          dm = s_red[0];
+          shift = (uint32_t)dm <= base ? 0u : ((uint32_t)dm - base) >> qs;
+        }
+        base += shift << qs;
+        for (int32_t v = t; v < n; v += BS) {
+          const uint32_t k = key[v];
+          if (k != 255u) {
+            key[v] = (uint8_t)(k > shift ? k - shift : 0u);
+          } else {
+            const int32_t d = get(v);
+            if (d != kInf) key[v] = (uint8_t)units(d);
+          }
+        }
+        thr = -1;
+        __syncthreads();
+      } else {
+        thr = (long long)fm + step_k;
+      }
+      continue;
+    }
+    steps++;
+    for (int w0 = 0; w0 < total; w0 += BS) {
+      // The next BS of them, off the marks before their distances are read:
+      // a later improvement marks them again.  No other thread is at this
+      // thread's marks here.
+      if (DL) {
+        for (; quads && pos < w0 + BS; quads &= quads - 1, pos++) {
+          const int b = __ffsll((unsigned long long)quads) - 1;
+          const int32_t v = ((b >> 2) * BS + t) * 4 + (b & 3);
+          s_beg[pos - w0] = v;
+          s_du[pos - w0] = (int32_t)(word[v] >> 1);
+          word[v] &= ~1u;
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < kWords; r++) {
+          const uint32_t before = sel[r];
+          for (; sel[r] && pos < w0 + BS; sel[r] &= sel[r] - 1, pos++)
+            s_beg[pos - w0] = (t * kWords + r) * 32 + __ffs(sel[r]) - 1;
+          if (before != sel[r]) pend[t * kWords + r] &= ~(before ^ sel[r]);
+        }
+      }
+      __syncthreads();
+      int beg = 0, deg = 0, du = 0;
+      if (w0 + t < total) {
+        const int32_t u = s_beg[t];
+        beg = at32(G.row_ptr, (uint32_t)u);
+        deg = at32(G.row_ptr, (uint32_t)u + 1u) - beg;
+        du = DL ? s_du[t] : get(u);
+      }
+      if (G.max_deg <= kSerialDeg && G.m >= kSerialM) {
+        // A thread per vertex, four edges by one load; what the load holds of
+        // other rows is relaxed at no distance.
+        const int most = wave_max_i32(deg), end = beg + deg;
+        for (int j = 0; j < most; j += 4) {
+          const int k0 = min(j < deg ? beg + j : 0, (int)G.m - 4);  // kSerialM <= m < kLdsM
+          const Cols4 u = four_at(G.col, k0), w = four_at(G.w, k0);
+          int32_t v[4], nd[4];
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            v[r] = u.c[r];
+            nd[r] = plus_sat(k0 + r >= beg + j && k0 + r < end ? du : kInf, w.c[r]);
+          }
+          relax(v, nd);
+        }
+      } else {
+        int edges;
+        const int off = scan_bs<BS>(deg, s_scan, &edges);
+        s_off[t] = off;
+        s_beg[t] = beg - off;
+        if (!DL) s_du[t] = du;
+        __syncthreads();
+        for (int e0 = __builtin_amdgcn_readfirstlane(t / kWave) * 4 * kWave; e0 < edges; e0 += 4 * BS) {
+          int e[4], o[4], k[4], du[4];
+          int32_t v[4], nd[4];
+          owners4<BS>(s_off, e0, edges, e, o);
+#pragma unroll
+          for (int r = 0; r < 4; r++) k[r] = s_beg[o[r]] + e[r], du[r] = s_du[o[r]];
+#pragma unroll
+          for (int r = 0; r < 4; r++) du[r] = e0 + r * kWave + lane_id() < edges ? du[r] : kInf;
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] = at32(G.col, k[r]), nd[r] = at32(G.w, k[r]);
+#pragma unroll
+          for (int r = 0; r < 4; r++) nd[r] = plus_sat(du[r], nd[r]);
+          relax(v, nd);
+        }
+      }
+      __syncthreads();
+    }
+    if (roll) thr = DL || thr <= 191 ? thr + step_k : -1;  // -1: towards a rebase
+  }
+  if (DL)
+    for (int32_t v = t; v < n; v += BS) dist[v] = (int32_t)(word[v] >> 1);
+  if (t == 0) atomicAdd(a.levels_total, (unsigned long long)steps);
+}
+
 // Sum of the edge weights of each weighted graph (the near-far delta):
 // kWsumParts workgroups per graph, one atomic each.
 constexpr int kWsumParts = 4;
@@ -836,7 +1185,10 @@ __global__ void __launch_bounds__(kBlock) wsum_kernel(const BatchGraph* graphs,
   if (threadIdx.x == 0 && s_t) atomicAdd(&out[blockIdx.x / kWsumParts], s_t);
 }
 
-template <int BS>
+// KIND: the tasks of the batch are all unweighted (0), all weighted (1) or
+// mixed (2); with one kind alone the compiler keeps the registers the other
+// would take (mixed: 145 scalar and 12 vector spills).
+template <int BS, int KIND>
 __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
   __shared__ int s_off[BS];
   __shared__ int s_beg[BS];
@@ -858,29 +1210,36 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
   for (;;) {
     if (threadIdx.x == 0) s_task = (int)atomicAdd(a.task_counter, 1u);
     __syncthreads();
-    const int t = s_task;
+    const int t = __builtin_amdgcn_readfirstlane(s_task);  // uniform: T and G in scalar registers
     __syncthreads();
     if (t >= a.num_tasks) break;  // every workgroup leaves once the queue is empty
     const BatchTask T = a.tasks[t];
     const BatchGraph G = a.graphs[T.graph];
-    if (G.weighted)
-      run_weighted<BS>(a, G, T, (uint8_t*)next, qv, (int32_t*)qw, s_off, s_beg,
-                       (int*)s_f, s_scan, s_cnt, s_red);
-    else if (T.bits >= 0)
-      run_lds<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
-                  a.entries + (int64_t)blockIdx.x * a.max_lds_n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or);
-    else if (T.lanes <= 8)
-      run_unweighted<BS, uint8_t>(a, G, T, (uint8_t*)seen, (uint8_t*)next, qv, (uint8_t*)qw,
-                                  touched, s_off, s_beg, s_f, s_scan, s_cnt);
-    else if (T.lanes <= 16)
-      run_unweighted<BS, uint16_t>(a, G, T, (uint16_t*)seen, (uint16_t*)next, qv, (uint16_t*)qw,
-                                   touched, s_off, s_beg, s_f, s_scan, s_cnt);
-    else if (T.lanes <= 32)
-      run_unweighted<BS, uint32_t>(a, G, T, (uint32_t*)seen, (uint32_t*)next, qv, (uint32_t*)qw,
-                                   touched, s_off, s_beg, s_f, s_scan, s_cnt);
-    else
-      run_unweighted<BS, uint64_t>(a, G, T, seen, next, qv, qw, touched, s_off, s_beg, s_f,
-                                   s_scan, s_cnt);
+    if (KIND == 1 || (KIND == 2 && G.weighted)) {
+      if (T.bits == kWeightedDist)
+        run_weighted_lds<BS, true>(a, G, T, s_lds, s_off, s_beg, (int*)s_lf, s_scan, s_red);
+      else if (T.bits == kWeightedBound)
+        run_weighted_lds<BS, false>(a, G, T, s_lds, s_off, s_beg, (int*)s_lf, s_scan, s_red);
+      else
+        run_weighted<BS>(a, G, T, (uint8_t*)next, qv, (int32_t*)qw, s_off, s_beg,
+                         (int*)s_f, s_scan, s_cnt, s_red);
+    } else {
+      if (T.bits >= 0)
+        run_lds<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
+                    a.entries + (int64_t)blockIdx.x * a.max_lds_n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or);
+      else if (T.lanes <= 8)
+        run_unweighted<BS, uint8_t>(a, G, T, (uint8_t*)seen, (uint8_t*)next, qv, (uint8_t*)qw,
+                                    touched, s_off, s_beg, s_f, s_scan, s_cnt);
+      else if (T.lanes <= 16)
+        run_unweighted<BS, uint16_t>(a, G, T, (uint16_t*)seen, (uint16_t*)next, qv, (uint16_t*)qw,
+                                     touched, s_off, s_beg, s_f, s_scan, s_cnt);
+      else if (T.lanes <= 32)
+        run_unweighted<BS, uint32_t>(a, G, T, (uint32_t*)seen, (uint32_t*)next, qv, (uint32_t*)qw,
+                                     touched, s_off, s_beg, s_f, s_scan, s_cnt);
+      else
+        run_unweighted<BS, uint64_t>(a, G, T, seen, next, qv, qw, touched, s_off, s_beg, s_f,
+                                     s_scan, s_cnt);
+    }
     __syncthreads();
   }
 }
@@ -905,8 +1264,9 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   for (int32_t i = 0; i < num_graphs; i++) {
     dawn_graph* g = graphs[i];
     if (!g || g->device != device || g->n <= 0) return DAWN_ERR_INVALID_ARG;
-    hg[i] = BatchGraph{g->n, g->weighted, g->m, g->row_ptr, g->col, g->weight, g->in_row_ptr,
-                       g->in_col, dist_offsets[i], g->max_out_degree, 0};
+    hg[i] = BatchGraph{g->n, g->weighted, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col,
+                       (GlobalInts)g->weight, (GlobalInts)g->in_row_ptr, (GlobalInts)g->in_col,
+                       dist_offsets[i], g->max_out_degree, 0};
     total = std::max<int64_t>(total, dist_offsets[i] + (int64_t)spg * g->n);
     for (int32_t j = 0; j < spg; j++) {
       int64_t s = sources[(int64_t)i * spg + j] % (int64_t)g->n;
@@ -915,8 +1275,11 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
       if (stats && g->h_row_ptr[s] == g->h_row_ptr[s + 1]) stats->skipped_sources += 1;
     }
     if (g->weighted) {
-      for (int32_t j = 0; j < spg; j++) ht.push_back(BatchTask{i, j, 1, -1});
-      max_n = std::max<int64_t>(max_n, g->n);
+      const int state = g->m >= kLdsM || g->n > kBoundN ? kWeightedMemory
+                        : g->n <= kDistN                ? kWeightedDist
+                                                        : kWeightedBound;
+      for (int32_t j = 0; j < spg; j++) ht.push_back(BatchTask{i, j, 1, state});
+      if (state == kWeightedMemory) max_n = std::max<int64_t>(max_n, g->n);
     } else {
       // The sources of a graph share one task as lanes of a field, except
       // on the largest graphs, whose tasks would be the batch's critical
@@ -1020,10 +1383,16 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   DAWN_HIP(hipEventCreate(&e0));
   DAWN_HIP(hipEventCreate(&e1));
   bool any_weighted = false;
-  for (const BatchGraph& x : hg) any_weighted = any_weighted || x.weighted;
+  bool all_weighted = true;
+  for (const BatchGraph& x : hg) {
+    any_weighted = any_weighted || x.weighted;
+    all_weighted = all_weighted && x.weighted;
+  }
   DAWN_HIP(hipEventRecord(e0, s));
   if (any_weighted) wsum_kernel<<<num_graphs * kWsumParts, kBlock, 0, s>>>(a.graphs, (unsigned long long*)(M + o_wsum));
-  batch_kernel<kBatchBlock><<<grid, kBatchBlock, 0, s>>>(a);
+  if (!any_weighted) batch_kernel<kBatchBlock, 0><<<grid, kBatchBlock, 0, s>>>(a);
+  else if (all_weighted) batch_kernel<kBatchBlock, 1><<<grid, kBatchBlock, 0, s>>>(a);
+  else batch_kernel<kBatchBlock, 2><<<grid, kBatchBlock, 0, s>>>(a);
   DAWN_HIP(hipGetLastError());
   DAWN_HIP(hipEventRecord(e1, s));
   DAWN_HIP(hipEventSynchronize(e1));
