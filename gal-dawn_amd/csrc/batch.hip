@@ -884,9 +884,9 @@ __device__ void run_weighted(const BatchArgs& a, const BatchGraph& G, const Batc
 // relaxation (RMAT-17, one CU: 2 G relaxations/s of 60 VALU and 15 LDS
 // operations per wave and edge) and, for small graphs, the step's scan (3 us).
 constexpr int64_t kDistN = kLdsWords - 3;  // words, rounded up to four
-constexpr int64_t kBoundN = 134000;        // a byte and a bit per vertex
+constexpr int64_t kBoundN = kSourcesN;     // a byte and a bit per vertex
 constexpr int64_t kSerialM = 4;            // edges of one load
-constexpr int64_t kLdsM = 1 << 30;         // edges reached by 32-bit byte offsets
+constexpr int64_t kLdsM = kSourcesMaxM;    // edges reached by 32-bit byte offsets
 static_assert((kBoundN + 3) / 4 + (kBoundN + 31) / 32 <= kLdsWords, "bounds and marks");
 enum { kWeightedMemory = -1, kWeightedDist = 0, kWeightedBound = 1 };  // BatchTask::bits
 
@@ -904,22 +904,23 @@ __device__ __forceinline__ Cols4 four_at(GlobalInts p, uint32_t i) {
   return *(const Cols4*)((const char*)(const int32_t*)p + i * 4u);
 }
 
+// One source.  dist: its row (DL: not touched, the words are left in s.W).
+// Returns the steps taken.
 template <int BS, bool DL>
-__device__ void run_weighted_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask& T, LdsTask& s,
-                                 int* s_off, int* s_beg, int* s_du, int* s_scan, int* s_red) {
+__device__ uint32_t run_weighted_lds(const BatchGraph& G, int32_t src, unsigned long long wsum,
+                                     int32_t* dist, LdsTask& s, int* s_off, int* s_beg, int* s_du,
+                                     int* s_scan, int* s_red) {
   // Vertices per thread: quads at a stride of BS quads, or words of 32 in order.
   constexpr int kQuads = (int)((kDistN + 4 * BS - 1) / (4 * BS));
   constexpr int kWords = (int)(((kBoundN + 31) / 32 + BS - 1) / BS);
   static_assert(kQuads * 4 <= 64, "a bit each");
   const int32_t n = G.n;
   const int t = threadIdx.x;
-  const int32_t src = a.sources[(int64_t)T.graph * a.spg + T.lane0];
-  int32_t* dist = a.dist + G.dist_off + (int64_t)T.lane0 * n;
   uint32_t* word = s.W;                               // DL
   uint8_t* key = reinterpret_cast<uint8_t*>(s.W);     // otherwise
   const int nb = (n + 31) / 32, n4 = (n + 3) / 4;
   uint32_t* pend = s.W + n4;
-  const double avg_w = G.m > 0 ? (double)a.wsum[T.graph] / (double)G.m : 1.0;
+  const double avg_w = G.m > 0 ? (double)wsum / (double)G.m : 1.0;
   const double avg_deg = n > 0 ? (double)G.m / (double)n : 1.0;
   const bool roll = G.max_deg <= 16 * avg_deg;
   const double delta = fmax(1.0, ceil((DL ? 2.0 : roll ? 1.0 : 0.5) * avg_w / fmax(avg_deg, 1.0)));
@@ -1160,9 +1161,19 @@ __device__ void run_weighted_lds(const BatchArgs& a, const BatchGraph& G, const 
     }
     if (roll) thr = DL || thr <= 191 ? thr + step_k : -1;  // -1: towards a rebase
   }
+  return steps;
+}
+
+template <int BS, bool DL>
+__device__ void weighted_task(const BatchArgs& a, const BatchGraph& G, const BatchTask& T, LdsTask& s,
+                              int* s_off, int* s_beg, int* s_du, int* s_scan, int* s_red) {
+  int32_t* dist = a.dist + G.dist_off + (int64_t)T.lane0 * G.n;
+  const uint32_t steps =
+      run_weighted_lds<BS, DL>(G, a.sources[(int64_t)T.graph * a.spg + T.lane0], a.wsum[T.graph], dist, s,
+                               s_off, s_beg, s_du, s_scan, s_red);
   if (DL)
-    for (int32_t v = t; v < n; v += BS) dist[v] = (int32_t)(word[v] >> 1);
-  if (t == 0) atomicAdd(a.levels_total, (unsigned long long)steps);
+    for (int32_t v = threadIdx.x; v < G.n; v += BS) dist[v] = (int32_t)(s.W[v] >> 1);
+  if (threadIdx.x == 0) atomicAdd(a.levels_total, (unsigned long long)steps);
 }
 
 // Sum of the edge weights of each weighted graph (the near-far delta):
@@ -1217,9 +1228,9 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
     const BatchGraph G = a.graphs[T.graph];
     if (KIND == 1 || (KIND == 2 && G.weighted)) {
       if (T.bits == kWeightedDist)
-        run_weighted_lds<BS, true>(a, G, T, s_lds, s_off, s_beg, (int*)s_lf, s_scan, s_red);
+        weighted_task<BS, true>(a, G, T, s_lds, s_off, s_beg, (int*)s_lf, s_scan, s_red);
       else if (T.bits == kWeightedBound)
-        run_weighted_lds<BS, false>(a, G, T, s_lds, s_off, s_beg, (int*)s_lf, s_scan, s_red);
+        weighted_task<BS, false>(a, G, T, s_lds, s_off, s_beg, (int*)s_lf, s_scan, s_red);
       else
         run_weighted<BS>(a, G, T, (uint8_t*)next, qv, (int32_t*)qw, s_off, s_beg,
                          (int*)s_f, s_scan, s_cnt, s_red);
@@ -1244,7 +1255,151 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
   }
 }
 
+// Many sources of one weighted graph, a workgroup each at a time.
+struct SourcesArgs {
+  BatchGraph G;
+  const int32_t* sources;
+  int32_t count;
+  int32_t* rows;            // [count][n], or null
+  int32_t* scratch;         // without rows and with more than kDistN vertices: [grid][n]
+  unsigned* counter;
+  unsigned long long* acc;  // per source: distance sum, vertices reached, their out-degrees, steps
+  const unsigned long long* wsum;
+};
+
+template <int BS, bool DL>
+__global__ void __launch_bounds__(BS) sources_kernel(SourcesArgs a) {
+  __shared__ int s_off[BS];
+  __shared__ int s_beg[BS];
+  __shared__ int s_du[BS];
+  __shared__ int s_scan[BS / kWave];
+  __shared__ int s_red[1];
+  __shared__ int s_next;
+  __shared__ unsigned long long s_acc[3];
+  __shared__ LdsTask s_lds;
+  const int t = threadIdx.x;
+  const int32_t n = a.G.n;
+  for (;;) {
+    if (t == 0) s_next = (int)atomicAdd(a.counter, 1u);
+    if (t < 3) s_acc[t] = 0ull;
+    __syncthreads();
+    const int i = __builtin_amdgcn_readfirstlane(s_next);
+    __syncthreads();
+    if (i >= a.count) break;  // every workgroup leaves once the sources are taken
+    int32_t* row = a.rows ? a.rows + (int64_t)i * n : DL ? nullptr : a.scratch + (int64_t)blockIdx.x * n;
+    const uint32_t steps = run_weighted_lds<BS, DL>(a.G, a.sources[i], *a.wsum, row, s_lds, s_off, s_beg,
+                                                    s_du, s_scan, s_red);
+    unsigned long long sum = 0, edges = 0;
+    unsigned reached = 0;
+    for (int32_t v = t; v < n; v += BS) {
+      const int32_t d = DL ? (int32_t)(s_lds.W[v] >> 1)
+                           : __hip_atomic_load(row + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (DL && row) row[v] = d;
+      if (d != kInf) {
+        sum += (unsigned)d;
+        reached++;
+        edges += (unsigned)(a.G.row_ptr[v + 1] - a.G.row_ptr[v]);
+      }
+    }
+    sum = wave_sum_u64(sum);
+    edges = wave_sum_u64(edges);
+    const unsigned long long many = wave_sum_u64(reached);
+    if (lane_id() == 0) {
+      atomicAdd(&s_acc[0], sum);
+      atomicAdd(&s_acc[1], many);
+      atomicAdd(&s_acc[2], edges);
+    }
+    __syncthreads();
+    if (t < 4) a.acc[(int64_t)i * 4 + t] = t < 3 ? s_acc[t] : steps;
+    __syncthreads();
+  }
+}
+
 }  // namespace
+
+// The batched min-plus engine's route for graphs whose state fits a
+// workgroup's LDS (wmsbfs.hip says when): sources already reduced mod n.
+int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources, int32_t S, int32_t* dist,
+                    int64_t* sums, dawn_stats* stats) {
+  if (g->n > kBoundN || g->m >= kLdsM) return DAWN_ERR_UNSUPPORTED;
+  const bool dl = g->n <= kDistN;
+  const bool dev_out = dist && is_device_pointer(dist);
+  int cus = 0;
+  DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
+  hipStream_t s = g->stream;
+  // Rows go to the caller's device memory; host rows in blocks of a full launch.
+  const int32_t per = dist && !dev_out ? std::min<int32_t>(S, std::max(cus / 64, 1) * 64) : S;
+  const int grid = std::max(1, std::min<int>(per, cus));
+  SourcesArgs a{};
+  a.G = BatchGraph{g->n, 1, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col, (GlobalInts)g->weight,
+                   (GlobalInts)g->in_row_ptr, (GlobalInts)g->in_col, 0, g->max_out_degree, 0};
+  if (!ws->graph.p) {
+    DAWN_TRY(ws->graph.alloc(sizeof(BatchGraph)));
+    DAWN_TRY(ws->wsum.alloc(1));
+    DAWN_HIP(hipMemcpyAsync(ws->graph.p, &a.G, sizeof(BatchGraph), hipMemcpyHostToDevice, s));
+    DAWN_HIP(hipMemsetAsync(ws->wsum.p, 0, sizeof(unsigned long long), s));
+    wsum_kernel<<<kWsumParts, kBlock, 0, s>>>((const BatchGraph*)ws->graph.p, ws->wsum.p);
+    DAWN_HIP(hipGetLastError());
+  }
+  for (hipEvent_t* e : {&ws->ev0, &ws->ev1})
+    if (!*e) DAWN_HIP(hipEventCreate(e));
+  DAWN_TRY(ws->counter.alloc(1));
+  DAWN_TRY(ws->sources.alloc((size_t)per));
+  DAWN_TRY(ws->acc.alloc((size_t)per * 4));
+  if (dist && !dev_out) DAWN_TRY(ws->rows.alloc((size_t)per * g->n));
+  else if (!dist && !dl) DAWN_TRY(ws->rows.alloc((size_t)grid * g->n));
+  a.sources = ws->sources.p;
+  a.scratch = ws->rows.p;
+  a.counter = ws->counter.p;
+  a.acc = ws->acc.p;
+  a.wsum = ws->wsum.p;
+  std::vector<unsigned long long> h((size_t)per * 4);
+  for (int32_t b0 = 0; b0 < S; b0 += per) {
+    const int32_t count = std::min(per, S - b0);
+    a.count = count;
+    a.rows = !dist ? nullptr : dev_out ? dist + (int64_t)b0 * g->n : ws->rows.p;
+    DAWN_HIP(hipMemcpyAsync(ws->sources.p, sources + b0, sizeof(int32_t) * (size_t)count,
+                            hipMemcpyHostToDevice, s));
+    DAWN_HIP(hipEventRecord(ws->ev0, s));
+    DAWN_HIP(hipMemsetAsync(ws->counter.p, 0, sizeof(unsigned), s));
+    if (dl) sources_kernel<kBatchBlock, true><<<grid, kBatchBlock, 0, s>>>(a);
+    else sources_kernel<kBatchBlock, false><<<grid, kBatchBlock, 0, s>>>(a);
+    DAWN_HIP(hipGetLastError());
+    DAWN_HIP(hipEventRecord(ws->ev1, s));
+    DAWN_HIP(hipMemcpyAsync(h.data(), ws->acc.p, sizeof(unsigned long long) * 4 * (size_t)count,
+                            hipMemcpyDeviceToHost, s));
+    DAWN_HIP(hipStreamSynchronize(s));
+    if (dist && !dev_out)
+      DAWN_HIP(hipMemcpy(dist + (int64_t)b0 * g->n, ws->rows.p, sizeof(int32_t) * (size_t)count * g->n,
+                         hipMemcpyDeviceToHost));
+    float ms = 0.f;
+    DAWN_HIP(hipEventElapsedTime(&ms, ws->ev0, ws->ev1));
+    if (stats) stats->device_ms += ms;
+    int64_t steps = 0;
+    for (int32_t i = 0; i < count; i++) {
+      if (sums) sums[b0 + i] = (int64_t)h[(size_t)i * 4];
+      if (!stats) continue;
+      stats->vertices_reached += (int64_t)h[(size_t)i * 4 + 1];
+      stats->edges_reached += (int64_t)h[(size_t)i * 4 + 2];
+      // Batches of 64 sources, as the engine of lanes counts them: the steps
+      // of one are those of its longest source.
+      steps = std::max<int64_t>(i % 64 ? steps : 0, (int64_t)h[(size_t)i * 4 + 3]);
+      if (i % 64 != 63 && i != count - 1) continue;
+      stats->steps += steps;
+      stats->mode_steps[DAWN_MODE_PUSH] += steps;
+      stats->batches += 1;
+    }
+  }
+  return DAWN_OK;
+}
+
+void sources_workspace_free(SourcesWorkspace* ws) {
+  if (!ws) return;
+  for (hipEvent_t e : {ws->ev0, ws->ev1})
+    if (e) (void)hipEventDestroy(e);
+  delete ws;
+}
+
 }  // namespace dawn
 
 using namespace dawn;

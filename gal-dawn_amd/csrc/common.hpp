@@ -94,6 +94,16 @@ struct SsWorkspace;   // single-source engines state (bfs.hip / sssp.hip)
 struct WmsWorkspace;  // batched weighted engine state (wmsbfs.hip)
 struct MsView;        // hub-first order of the batched engine (view.hip)
 
+// Weighted sources, a workgroup each (batch.hip): kept with the batched
+// weighted engine's state.
+struct SourcesWorkspace {
+  DevBuf<unsigned char> graph;
+  DevBuf<unsigned long long> wsum, acc;
+  DevBuf<unsigned> counter;
+  DevBuf<int32_t> sources, rows;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+};
+
 }  // namespace dawn
 
 // Device-resident graph.  For undirected graphs the in-edge arrays alias the
@@ -475,5 +485,10 @@ bool tuned_knobs_for(const dawn_graph* g, TuneKnobs* out);
 void ms_workspace_free(MsWorkspace* ws);
 void ss_workspace_free(SsWorkspace* ws);
 void wms_workspace_free(WmsWorkspace* ws);
+// At most this many vertices, fewer than this many edges.
+constexpr int64_t kSourcesN = 134000, kSourcesMaxM = 1 << 30;
+int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources, int32_t S, int32_t* dist,
+                    int64_t* sums, dawn_stats* stats);
+void sources_workspace_free(SourcesWorkspace* ws);
 
 }  // namespace dawn

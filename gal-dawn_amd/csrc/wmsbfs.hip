@@ -29,6 +29,8 @@
 // workgroup).  A K-step loop is captured once into a
 // hipGraph; every kernel reads the step and the done flag from device
 // state, so the graph is replayed until the frontier empties.
+//
+// Graphs small enough for a workgroup's LDS take another route (by_workgroup).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -485,6 +487,7 @@ struct WmsWorkspace {
   WBatch* h_batch = nullptr;
   std::map<int, hipGraphExec_t> graphs;  // by (L, policy, steps per graph)
   int32_t last_steps = 0;                // steps the last batch took
+  SourcesWorkspace* sources = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
@@ -496,6 +499,7 @@ void wms_invalidate_graphs(WmsWorkspace* ws) {
 
 void wms_workspace_free(WmsWorkspace* ws) {
   if (!ws) return;
+  sources_workspace_free(ws->sources);
   for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
   if (ws->h_state) (void)hipHostFree(ws->h_state);
   if (ws->h_batch) (void)hipHostFree(ws->h_batch);
@@ -647,13 +651,45 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
 
 }  // namespace
 
-// Weighted multi-source traversal, batches of up to 64 sources.
+// Graphs whose state fits a workgroup's LDS: every source in a workgroup of
+// its own (batch.hip), 256 at a time, instead of 64 lanes that share steps of
+// four launches.  Measured (ms, lanes / workgroups):
+//   ER 16,384, 131,000 edges: 1 source 1.04 / 0.24, 64 3.2 / 0.27, 1024 51 / 0.97
+//   ER 60,000, 480,000 edges: 1 source 1.4 / 1.0, 64 3.5 / 1.05, 1024 57 / 5.9
+//   grid 360 x 360: 1 source 2.3 / 1.7, 64 4.7 / 1.9, 1024 75 / 8.8
+// A workgroup relaxes 1 to 1.5 G edges/s alone, so that few sources of a graph
+// of many edges leave the chip idle:
+//   ER 130,000, 3.9 M edges: 8 sources 2.9 / 3.5, 16 3.7 / 3.4, 64 11 / 3.5
+//   RMAT-17, 3.7 M edges: 8 sources 2.7 / 4.5, 16 4.2 / 4.3, 64 23 / 6.6
+// hence the two lines below.  A forced mode is one of the lanes' steps.
+constexpr int64_t kSourcesM = 1500000;  // edges up to which any number of sources
+constexpr int32_t kSourcesS = 32;       // sources from which any number of edges
+
+static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
+  if (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED) return false;
+  return g->n <= kSourcesN && (g->m <= kSourcesM || (S >= kSourcesS && g->m < kSourcesMaxM));
+}
+
+// Weighted multi-source traversal: a workgroup per source, or batches of up to
+// 64 sources.
 int run_wmsbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64_t* sums,
                int32_t policy, dawn_stats* stats) {
   if (!g || !g->weighted || S < 0 || (S > 0 && !sources) || g->n <= 0) return DAWN_ERR_INVALID_ARG;
   if (S == 0) return DAWN_OK;
   std::lock_guard<std::mutex> guard(g->lock);
   DAWN_HIP(hipSetDevice(g->device));
+  if (by_workgroup(g, S, policy)) {
+    if (!g->wms) g->wms = new WmsWorkspace();
+    if (!g->wms->sources) g->wms->sources = new SourcesWorkspace();
+    std::vector<int32_t> src(S);
+    for (int32_t i = 0; i < S; i++) {
+      int64_t v = sources[i] % (int64_t)g->n;
+      if (v < 0) v += g->n;
+      src[i] = (int32_t)v;
+      if (stats && g->h_row_ptr[v] == g->h_row_ptr[v + 1]) stats->skipped_sources += 1;
+    }
+    return run_sources_lds(g, g->wms->sources, src.data(), S, dist, sums, stats);
+  }
   const int32_t per = std::min<int32_t>(S, 64);
   if (per <= 8) return run_w<8>(g, sources, S, dist, sums, policy, stats);
   if (per <= 16) return run_w<16>(g, sources, S, dist, sums, policy, stats);

@@ -213,7 +213,9 @@ int dawn_bfs_noalloc(const dawn_graph* g, int32_t source, int32_t* dist,
 /* Multi-source shortest paths.  Unweighted graphs run 64*W sources per
  * bit-packed batch (W = the lane-words knob, up to 16: 1024 sources);
  * weighted graphs run the batched min-plus engine, up to 64 sources per
- * batch.
+ * batch, or, where a graph's state fits a workgroup's LDS (up to 134,000
+ * vertices, a few edges or many sources; fixed and learned policies), a
+ * workgroup per source.
  * sources are taken modulo n (reference: msource[i] % rows, mssp.cpp:15);
  * isolated sources are skipped (dist row left INF except dist[src]=0, sum 0).
  * dist: S*n int32 row-major (host or device), or NULL to keep only sums
