@@ -412,22 +412,22 @@ __device__ __forceinline__ Cols4 cols_at(GlobalInts p, int r) {
   return Cols4{{p[0], p[min(1, r)], p[r], p[r]}};
 }
 
-template <int BS>
-__device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask& T, LdsTask& s,
-                        int32_t* qv, int2* ent, int* s_off, int* s_beg, uint32_t* s_f, int* s_scan,
-                        unsigned* s_cnt, uint32_t* s_red) {
+// sources, lanes, bits: of the task.  gstage: levels that do not fit the LDS.
+// levels(v, b) afterwards: kInf, or the level, by any thread.
+template <int BS, typename Out>
+__device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lanes, int bits, int32_t* drow,
+                       uint8_t* gstage, LdsTask& s, int32_t* qv, int2* ent, int* s_off, int* s_beg,
+                       uint32_t* s_f, int* s_scan, unsigned* s_cnt, uint32_t* s_red, Out out) {
   const int32_t n = G.n;
   const int t = threadIdx.x;
-  const bool one = T.bits == 0;
-  const int L = 1 << T.bits, fw = one ? 0 : T.bits + 1, fpw = 5 - fw;  // log2 field width, fields per word
+  const bool one = bits == 0;
+  const int L = 1 << bits, fw = one ? 0 : bits + 1, fpw = 5 - fw;  // log2 field width, fields per word
   const uint32_t fmask = (1u << L) - 1u;
   uint32_t bmask = 0;  // the B halves of a word
   if (!one)
     for (int k = 0; k < 32; k += 2 * L) bmask |= fmask << (k + L);
   const int words = (int)((((int64_t)n << fw) + 31) >> 5);
-  int32_t* drow = a.dist + G.dist_off + (int64_t)T.lane0 * n;
   uint8_t* lstage = reinterpret_cast<uint8_t*>(s.W + words);
-  uint8_t* gstage = a.stage + (int64_t)blockIdx.x * a.stage_cap;
   const bool in_lds = (int64_t)words * 4 + (int64_t)n * L <= (int64_t)kLdsWords * 4;
   auto word_of = [&](int32_t v) { return v >> fpw; };
   auto shift_of = [&](int32_t v) { return (v & ((1 << fpw) - 1)) << fw; };
@@ -445,8 +445,8 @@ __device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask
   for (int i = t; i < words; i += BS) s.W[i] = 0u;
   if (t == 0) s_cnt[0] = 0u;
   __syncthreads();
-  if (t < T.lanes) {
-    const int32_t v = a.sources[(int64_t)T.graph * a.spg + T.lane0 + t];
+  if (t < lanes) {
+    const int32_t v = sources[t];
     const uint32_t bit = 1u << t;
     const uint32_t old = atomicOr(&s.W[word_of(v)], mark(bit) << shift_of(v)) >> shift_of(v);
     put_level(v, bit, 0);
@@ -493,7 +493,7 @@ __device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask
       } else {
         if (t < 1 << kMaxBits) s.lane_edges[t] = 0u;
         __syncthreads();
-        for (int b0 = 0; b0 < T.lanes; b0 += 4) {
+        for (int b0 = 0; b0 < lanes; b0 += 4) {
           unsigned c[4] = {0, 0, 0, 0};
           for (unsigned i = t; i < qn; i += BS) {
             const unsigned df = (unsigned)ent[i].y;
@@ -503,11 +503,11 @@ __device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask
 #pragma unroll
           for (int b = 0; b < 4; b++) {
             for (int o = 32; o >= 1; o >>= 1) c[b] += (unsigned)__shfl_xor((int)c[b], o);
-            if (lane_id() == 0 && c[b] && b0 + b < T.lanes) atomicAdd(&s.lane_edges[b0 + b], c[b]);
+            if (lane_id() == 0 && c[b] && b0 + b < lanes) atomicAdd(&s.lane_edges[b0 + b], c[b]);
           }
         }
         __syncthreads();
-        for (int b = 0; b < T.lanes; b++)
+        for (int b = 0; b < lanes; b++)
           if ((unsigned long long)s.lane_edges[b] * kPullShare > (unsigned long long)G.m) pull |= 1u << b;
       }
     }
@@ -654,20 +654,30 @@ __device__ void run_lds(const BatchArgs& a, const BatchGraph& G, const BatchTask
       __syncthreads();
     }
   }
+  out([&](int32_t v, int b) -> int32_t {
+    if (!((s.W[word_of(v)] >> (shift_of(v) + b)) & 1u)) return kInf;
+    const int64_t at = (int64_t)v * L + b;
+    const uint32_t l = in_lds ? lstage[at] : gstage[at];
+    return l == kStaged8 ? drow[(int64_t)b * n + v] : (int32_t)l;
+  });
+  return level;
+}
+
+template <int BS>
+__device__ void lds_task(const BatchArgs& a, const BatchGraph& G, const BatchTask& T, LdsTask& s,
+                         int32_t* qv, int2* ent, int* s_off, int* s_beg, uint32_t* s_f, int* s_scan,
+                         unsigned* s_cnt, uint32_t* s_red) {
+  const int32_t n = G.n;
+  int32_t* drow = a.dist + G.dist_off + (int64_t)T.lane0 * n;
   // Rows: a row store of a wave covers 64 consecutive vertices.
-  for (int32_t v = t; v < n; v += BS) {
-    const uint32_t got = s.W[word_of(v)] >> shift_of(v);
-    for (int b = 0; b < T.lanes; b++) {
-      const int64_t at = (int64_t)v * L + b;
-      if (!((got >> b) & 1u)) {
-        drow[(int64_t)b * n + v] = kInf;
-      } else {
-        const uint32_t l = in_lds ? lstage[at] : gstage[at];
-        if (l != kStaged8) drow[(int64_t)b * n + v] = (int32_t)l;
-      }
-    }
-  }
-  if (t == 0) atomicAdd(a.levels_total, (unsigned long long)level);
+  const int levels = run_lds<BS>(
+      G, a.sources + (int64_t)T.graph * a.spg + T.lane0, T.lanes, T.bits, drow,
+      a.stage + (int64_t)blockIdx.x * a.stage_cap, s, qv, ent, s_off, s_beg, s_f, s_scan, s_cnt, s_red,
+      [&](auto level_of) {
+        for (int32_t v = threadIdx.x; v < n; v += BS)
+          for (int b = 0; b < T.lanes; b++) drow[(int64_t)b * n + v] = level_of(v, b);
+      });
+  if (threadIdx.x == 0) atomicAdd(a.levels_total, (unsigned long long)levels);
 }
 
 // One weighted source.  The reference's initialisation
@@ -1236,7 +1246,7 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
                          (int*)s_f, s_scan, s_cnt, s_red);
     } else {
       if (T.bits >= 0)
-        run_lds<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
+        lds_task<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
                     a.entries + (int64_t)blockIdx.x * a.max_lds_n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or);
       else if (T.lanes <= 8)
         run_unweighted<BS, uint8_t>(a, G, T, (uint8_t*)seen, (uint8_t*)next, qv, (uint8_t*)qw,
@@ -1315,80 +1325,136 @@ __global__ void __launch_bounds__(BS) sources_kernel(SourcesArgs a) {
   }
 }
 
+// The same unweighted: levels in LDS (n <= kSourcesN), one lane.
+struct BfsSourcesArgs {
+  BatchGraph G;
+  const int32_t* sources;
+  int32_t count;
+  int32_t* rows;            // [count][n], or null
+  int32_t* scratch;         // without rows: [grid][n], for levels beyond a byte
+  int32_t* qv;              // [grid][n]
+  int2* ent;                // [grid][n]
+  unsigned* counter;
+  unsigned long long* acc;  // as above, levels for steps
+};
+
+template <int BS>
+__global__ void __launch_bounds__(BS) bfs_sources_kernel(BfsSourcesArgs a) {
+  __shared__ int s_off[BS];
+  __shared__ int s_beg[BS];
+  __shared__ uint32_t s_lf[BS];
+  __shared__ int s_scan[BS / kWave];
+  __shared__ unsigned s_cnt[5];
+  __shared__ uint32_t s_or[1];
+  __shared__ int s_next;
+  __shared__ unsigned long long s_acc[3];
+  __shared__ LdsTask s_lds;
+  const int t = threadIdx.x;
+  const int32_t n = a.G.n;
+  for (;;) {
+    if (t == 0) s_next = (int)atomicAdd(a.counter, 1u);
+    if (t < 3) s_acc[t] = 0ull;
+    __syncthreads();
+    const int i = __builtin_amdgcn_readfirstlane(s_next);
+    __syncthreads();
+    if (i >= a.count) break;  // every workgroup leaves once the sources are taken
+    int32_t* row = a.rows ? a.rows + (int64_t)i * n : a.scratch + (int64_t)blockIdx.x * n;
+    const int levels = run_lds<BS>(
+        a.G, a.sources + i, 1, 0, row, nullptr, s_lds, a.qv + (int64_t)blockIdx.x * n,
+        a.ent + (int64_t)blockIdx.x * n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or, [&](auto level_of) {
+          unsigned long long sum = 0;
+          unsigned reached = 0, edges = 0;  // m < 2^31
+          for (int32_t v = t; v < n; v += BS) {
+            const int32_t d = level_of(v, 0);
+            if (a.rows) row[v] = d;
+            if (d != kInf) {
+              sum += (unsigned)d;
+              reached++;
+              edges += (unsigned)(a.G.row_ptr[v + 1] - a.G.row_ptr[v]);
+            }
+          }
+          sum = wave_sum_u64(sum);
+          const unsigned long long many = wave_sum_u64((unsigned long long)reached);
+          const unsigned long long es = wave_sum_u64((unsigned long long)edges);
+          if (lane_id() == 0) {
+            atomicAdd(&s_acc[0], sum);
+            atomicAdd(&s_acc[1], many);
+            atomicAdd(&s_acc[2], es);
+          }
+        });
+    __syncthreads();
+    if (t < 4) a.acc[(int64_t)i * 4 + t] = t < 3 ? s_acc[t] : (unsigned long long)levels;
+    __syncthreads();
+  }
+}
+
 }  // namespace
 
-// The batched min-plus engine's route for graphs whose state fits a
-// workgroup's LDS (wmsbfs.hip says when): sources already reduced mod n.
+// Sources (reduced mod n) a workgroup each, for graphs whose state fits its
+// LDS; the engines of lanes say when.  acc: per source the distance sum, the
+// vertices reached, their out-degrees, the steps (levels); device time in *ms.
 int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources, int32_t S, int32_t* dist,
-                    int64_t* sums, dawn_stats* stats) {
-  if (g->n > kBoundN || g->m >= kLdsM) return DAWN_ERR_UNSUPPORTED;
+                    std::vector<unsigned long long>& acc, double* ms) {
+  if (g->n > kSourcesN || g->m >= kSourcesMaxM) return DAWN_ERR_UNSUPPORTED;
   const bool dl = g->n <= kDistN;
   const bool dev_out = dist && is_device_pointer(dist);
   int cus = 0;
   DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
   hipStream_t s = g->stream;
   // Rows go to the caller's device memory; host rows in blocks of a full launch.
-  const int32_t per = dist && !dev_out ? std::min<int32_t>(S, std::max(cus / 64, 1) * 64) : S;
+  const int32_t per = dist && !dev_out ? std::min<int32_t>(S, cus) : S;
   const int grid = std::max(1, std::min<int>(per, cus));
-  SourcesArgs a{};
-  a.G = BatchGraph{g->n, 1, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col, (GlobalInts)g->weight,
-                   (GlobalInts)g->in_row_ptr, (GlobalInts)g->in_col, 0, g->max_out_degree, 0};
-  if (!ws->graph.p) {
-    DAWN_TRY(ws->graph.alloc(sizeof(BatchGraph)));
-    DAWN_TRY(ws->wsum.alloc(1));
-    DAWN_HIP(hipMemcpyAsync(ws->graph.p, &a.G, sizeof(BatchGraph), hipMemcpyHostToDevice, s));
-    DAWN_HIP(hipMemsetAsync(ws->wsum.p, 0, sizeof(unsigned long long), s));
-    wsum_kernel<<<kWsumParts, kBlock, 0, s>>>((const BatchGraph*)ws->graph.p, ws->wsum.p);
-    DAWN_HIP(hipGetLastError());
-  }
-  for (hipEvent_t* e : {&ws->ev0, &ws->ev1})
-    if (!*e) DAWN_HIP(hipEventCreate(e));
+  const size_t gn = (size_t)grid * g->n;
+  const BatchGraph G{g->n, g->weighted, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col,
+                     (GlobalInts)g->weight, (GlobalInts)g->in_row_ptr, (GlobalInts)g->in_col, 0,
+                     g->max_out_degree, 0};
   DAWN_TRY(ws->counter.alloc(1));
   DAWN_TRY(ws->sources.alloc((size_t)per));
   DAWN_TRY(ws->acc.alloc((size_t)per * 4));
   if (dist && !dev_out) DAWN_TRY(ws->rows.alloc((size_t)per * g->n));
-  else if (!dist && !dl) DAWN_TRY(ws->rows.alloc((size_t)grid * g->n));
-  a.sources = ws->sources.p;
-  a.scratch = ws->rows.p;
-  a.counter = ws->counter.p;
-  a.acc = ws->acc.p;
-  a.wsum = ws->wsum.p;
-  std::vector<unsigned long long> h((size_t)per * 4);
+  else if (!dist && !(g->weighted && dl)) DAWN_TRY(ws->rows.alloc(gn));
+  for (hipEvent_t* e : {&ws->ev0, &ws->ev1})
+    if (!*e) DAWN_HIP(hipEventCreate(e));
+  if (!g->weighted) {
+    DAWN_TRY(ws->queue.alloc(gn));
+    DAWN_TRY(ws->entries.alloc(gn));
+  } else if (!ws->wsum.p) {
+    DAWN_TRY(ws->graph.alloc(sizeof(BatchGraph)));
+    DAWN_TRY(ws->wsum.alloc(1));
+    DAWN_HIP(hipMemcpyAsync(ws->graph.p, &G, sizeof(BatchGraph), hipMemcpyHostToDevice, s));
+    DAWN_HIP(hipMemsetAsync(ws->wsum.p, 0, sizeof(unsigned long long), s));
+    wsum_kernel<<<kWsumParts, kBlock, 0, s>>>((const BatchGraph*)ws->graph.p, ws->wsum.p);
+    DAWN_HIP(hipGetLastError());
+  }
+  acc.resize((size_t)S * 4);
+  *ms = 0;
   for (int32_t b0 = 0; b0 < S; b0 += per) {
     const int32_t count = std::min(per, S - b0);
-    a.count = count;
-    a.rows = !dist ? nullptr : dev_out ? dist + (int64_t)b0 * g->n : ws->rows.p;
+    int32_t* rows = !dist ? nullptr : dev_out ? dist + (int64_t)b0 * g->n : ws->rows.p;
     DAWN_HIP(hipMemcpyAsync(ws->sources.p, sources + b0, sizeof(int32_t) * (size_t)count,
                             hipMemcpyHostToDevice, s));
     DAWN_HIP(hipEventRecord(ws->ev0, s));
     DAWN_HIP(hipMemsetAsync(ws->counter.p, 0, sizeof(unsigned), s));
-    if (dl) sources_kernel<kBatchBlock, true><<<grid, kBatchBlock, 0, s>>>(a);
-    else sources_kernel<kBatchBlock, false><<<grid, kBatchBlock, 0, s>>>(a);
+    if (g->weighted) {
+      const SourcesArgs a{G, ws->sources.p, count, rows, ws->rows.p, ws->counter.p, ws->acc.p, ws->wsum.p};
+      if (dl) sources_kernel<kBatchBlock, true><<<grid, kBatchBlock, 0, s>>>(a);
+      else sources_kernel<kBatchBlock, false><<<grid, kBatchBlock, 0, s>>>(a);
+    } else {
+      const BfsSourcesArgs a{G, ws->sources.p, count, rows, ws->rows.p, ws->queue.p, ws->entries.p,
+                             ws->counter.p, ws->acc.p};
+      bfs_sources_kernel<kBatchBlock><<<grid, kBatchBlock, 0, s>>>(a);
+    }
     DAWN_HIP(hipGetLastError());
     DAWN_HIP(hipEventRecord(ws->ev1, s));
-    DAWN_HIP(hipMemcpyAsync(h.data(), ws->acc.p, sizeof(unsigned long long) * 4 * (size_t)count,
-                            hipMemcpyDeviceToHost, s));
+    DAWN_HIP(hipMemcpyAsync(acc.data() + (size_t)b0 * 4, ws->acc.p,
+                            sizeof(unsigned long long) * 4 * (size_t)count, hipMemcpyDeviceToHost, s));
     DAWN_HIP(hipStreamSynchronize(s));
     if (dist && !dev_out)
       DAWN_HIP(hipMemcpy(dist + (int64_t)b0 * g->n, ws->rows.p, sizeof(int32_t) * (size_t)count * g->n,
                          hipMemcpyDeviceToHost));
-    float ms = 0.f;
-    DAWN_HIP(hipEventElapsedTime(&ms, ws->ev0, ws->ev1));
-    if (stats) stats->device_ms += ms;
-    int64_t steps = 0;
-    for (int32_t i = 0; i < count; i++) {
-      if (sums) sums[b0 + i] = (int64_t)h[(size_t)i * 4];
-      if (!stats) continue;
-      stats->vertices_reached += (int64_t)h[(size_t)i * 4 + 1];
-      stats->edges_reached += (int64_t)h[(size_t)i * 4 + 2];
-      // Batches of 64 sources, as the engine of lanes counts them: the steps
-      // of one are those of its longest source.
-      steps = std::max<int64_t>(i % 64 ? steps : 0, (int64_t)h[(size_t)i * 4 + 3]);
-      if (i % 64 != 63 && i != count - 1) continue;
-      stats->steps += steps;
-      stats->mode_steps[DAWN_MODE_PUSH] += steps;
-      stats->batches += 1;
-    }
+    float x = 0.f;
+    DAWN_HIP(hipEventElapsedTime(&x, ws->ev0, ws->ev1));
+    *ms += x;
   }
   return DAWN_OK;
 }

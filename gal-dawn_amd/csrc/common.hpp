@@ -94,13 +94,13 @@ struct SsWorkspace;   // single-source engines state (bfs.hip / sssp.hip)
 struct WmsWorkspace;  // batched weighted engine state (wmsbfs.hip)
 struct MsView;        // hub-first order of the batched engine (view.hip)
 
-// Weighted sources, a workgroup each (batch.hip): kept with the batched
-// weighted engine's state.
+// Sources a workgroup each (batch.hip).
 struct SourcesWorkspace {
   DevBuf<unsigned char> graph;
   DevBuf<unsigned long long> wsum, acc;
   DevBuf<unsigned> counter;
-  DevBuf<int32_t> sources, rows;
+  DevBuf<int32_t> sources, rows, queue;
+  DevBuf<int2> entries;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
@@ -147,6 +147,10 @@ struct dawn_graph {
   hipStream_t stream2 = nullptr;
   dawn::SsWorkspace* ss = nullptr;
   dawn::WmsWorkspace* wms = nullptr;
+  dawn::SourcesWorkspace* sources = nullptr;
+  // Multi-source calls keep to the engine of lanes: its knobs were set, or
+  // are being tuned.
+  bool lanes_only = false;
   dawn::MsView* view = nullptr;
 };
 
@@ -488,7 +492,7 @@ void wms_workspace_free(WmsWorkspace* ws);
 // At most this many vertices, fewer than this many edges.
 constexpr int64_t kSourcesN = 134000, kSourcesMaxM = 1 << 30;
 int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources, int32_t S, int32_t* dist,
-                    int64_t* sums, dawn_stats* stats);
+                    std::vector<unsigned long long>& acc, double* ms);
 void sources_workspace_free(SourcesWorkspace* ws);
 
 }  // namespace dawn

@@ -227,6 +227,7 @@ int dawn_graph_destroy(dawn_graph* g) {
   ms_workspace_free(g->ms_tail);
   ss_workspace_free(g->ss);
   wms_workspace_free(g->wms);
+  sources_workspace_free(g->sources);
   ms_view_free(g);
   if (g->directed) {
     if (g->in_row_ptr) (void)hipFree(g->in_row_ptr);

@@ -2316,6 +2316,68 @@ void split_live(const dawn_graph* g, const int32_t* sources, int32_t S, std::vec
   }
 }
 
+// Graphs whose state fits a workgroup's LDS: every source in a workgroup of its
+// own (batch.hip), 256 at a time, while that is faster than the shared steps of
+// a batch of lanes, seven launches each.  Measured (ms, lanes / workgroups):
+//   ER 4,096, 65,000 edges: 16 sources 0.47 / 0.07, 1024 0.57 / 0.18
+//   ER 16,384, 131,000 edges: 256 sources 0.57 / 0.16, 1024 0.61 / 0.46
+//   ER 60,000, 240,000 edges: 256 sources 0.74 / 0.44, 512 0.89 / 0.79, 1024 1.1 / 1.4
+//   ER 65,536, 1 M edges: 65 sources 0.53 / 0.37, 256 0.62 / 0.35, 1024 0.72 / 1.1
+//   RMAT-15, 0.9 M edges: 256 sources 0.71 / 0.22, 512 0.78 / 0.36
+//   grid 250 x 250: 64 sources 1.3 / 0.34, 1024 2.6 / 1.3
+//   RMAT-17, 3.7 M edges: 64 sources 0.67 / 0.70, 256 0.80 / 0.72
+// A source costs its edges and about 16 edges' time per vertex (levels of few
+// vertices, the row); a graph of more than kSourcesWork of those or kSourcesM
+// edges, or a call of more than kSourcesCall, goes to the lanes, and so do
+// forced modes and graphs whose knobs were set.
+constexpr int64_t kSourcesWork = 1 << 22, kSourcesCall = 1 << 30, kSourcesM = 1 << 21;
+constexpr int32_t kSourcesS = 1024;
+
+static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
+  if (g->lanes_only || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
+  const int64_t work = g->m + 16 * (int64_t)g->n;
+  return g->n <= kSourcesN && g->m <= kSourcesM && work <= kSourcesWork && S <= kSourcesS &&
+         S * work <= kSourcesCall;
+}
+
+// live: the sources that take lanes in batches of 64 words, as the lanes count.
+static int run_msbfs_sources(dawn_graph* g, const int32_t* sources, int32_t S, const std::vector<int32_t>& live_row,
+                             int words, int32_t* dist, int64_t* sums, int64_t* reached, int64_t* edges,
+                             dawn_stats* stats) {
+  if (!g->sources) g->sources = new SourcesWorkspace();
+  std::vector<int32_t> src(S);
+  for (int32_t i = 0; i < S; i++) {
+    int64_t v = sources[i] % (int64_t)g->n;
+    if (v < 0) v += g->n;
+    src[i] = (int32_t)v;
+  }
+  std::vector<unsigned long long> acc;
+  double ms = 0;
+  DAWN_TRY(run_sources_lds(g, g->sources, src.data(), S, dist, acc, &ms));
+  for (int32_t i = 0; i < S; i++) {
+    const unsigned long long* x = acc.data() + (size_t)i * 4;
+    if (sums) sums[i] = (int64_t)x[0];
+    if (reached) reached[i] = (int64_t)x[1];
+    if (edges) edges[i] = (int64_t)x[2];
+  }
+  if (!stats) return DAWN_OK;
+  stats->device_ms += ms;
+  const int32_t L = (int32_t)live_row.size();
+  int64_t steps = 0;
+  for (int32_t k = 0; k < L; k++) {
+    const unsigned long long* x = acc.data() + (size_t)live_row[k] * 4;
+    stats->vertices_reached += (int64_t)x[1];
+    stats->edges_reached += (int64_t)x[2];
+    stats->frontier_edges += (int64_t)x[2];  // each reached vertex is expanded once
+    steps = std::max<int64_t>(k % (64 * words) ? steps : 0, (int64_t)x[3]);
+    if ((k + 1) % (64 * words) && k != L - 1) continue;
+    stats->steps += steps;
+    stats->mode_steps[DAWN_MODE_PUSH] += steps;
+    stats->batches += 1;
+  }
+  return DAWN_OK;
+}
+
 int run_msbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64_t* sums,
               int64_t* reached, int64_t* edges, int32_t policy, dawn_stats* stats, bool rows) {
   if (!g || S < 0 || (S > 0 && !sources) || g->n <= 0) return DAWN_ERR_INVALID_ARG;
@@ -2329,9 +2391,20 @@ int run_msbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, i
   const int32_t L = (int32_t)live.size();
   const IsoRows isr{iso.data(), (int32_t)(iso.size() / 2)};
   const bool dist_dev = dist && is_device_pointer(dist);
+  int rc0 = DAWN_ERR_UNSUPPORTED;
+  if (by_workgroup(g, S, policy)) {
+    rc0 = run_msbfs_sources(g, sources, S, live_row, words_for(g, L), dist, sums, reached, edges, stats);
+    if (rc0 == DAWN_ERR_OUT_OF_MEMORY) {  // nothing has run yet: the lanes try
+      sources_workspace_free(g->sources);
+      g->sources = nullptr;
+      (void)hipGetLastError();
+    } else if (rc0 != DAWN_OK) {
+      return rc0;
+    }
+  }
   // Workspaces are sized by the batch width; if the device cannot hold them
   // (they are allocated before any batch runs), narrower batches are tried.
-  for (int w = words_for(g, L);; w >>= 1) {
+  for (int w = words_for(g, L); rc0 != DAWN_OK; w >>= 1) {
     int rc;
     const int32_t* ls = live.data();
     const int32_t* lr = live_row.data();

@@ -487,7 +487,6 @@ struct WmsWorkspace {
   WBatch* h_batch = nullptr;
   std::map<int, hipGraphExec_t> graphs;  // by (L, policy, steps per graph)
   int32_t last_steps = 0;                // steps the last batch took
-  SourcesWorkspace* sources = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
@@ -499,7 +498,6 @@ void wms_invalidate_graphs(WmsWorkspace* ws) {
 
 void wms_workspace_free(WmsWorkspace* ws) {
   if (!ws) return;
-  sources_workspace_free(ws->sources);
   for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
   if (ws->h_state) (void)hipHostFree(ws->h_state);
   if (ws->h_batch) (void)hipHostFree(ws->h_batch);
@@ -666,8 +664,17 @@ constexpr int64_t kSourcesM = 1500000;  // edges up to which any number of sourc
 constexpr int32_t kSourcesS = 32;       // sources from which any number of edges
 
 static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
-  if (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED) return false;
+  if (g->lanes_only || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
   return g->n <= kSourcesN && (g->m <= kSourcesM || (S >= kSourcesS && g->m < kSourcesMaxM));
+}
+
+static int run_lanes(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64_t* sums,
+                     int32_t policy, dawn_stats* stats) {
+  const int32_t per = std::min<int32_t>(S, 64);
+  if (per <= 8) return run_w<8>(g, sources, S, dist, sums, policy, stats);
+  if (per <= 16) return run_w<16>(g, sources, S, dist, sums, policy, stats);
+  if (per <= 32) return run_w<32>(g, sources, S, dist, sums, policy, stats);
+  return run_w<64>(g, sources, S, dist, sums, policy, stats);
 }
 
 // Weighted multi-source traversal: a workgroup per source, or batches of up to
@@ -679,22 +686,43 @@ int run_wmsbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, 
   std::lock_guard<std::mutex> guard(g->lock);
   DAWN_HIP(hipSetDevice(g->device));
   if (by_workgroup(g, S, policy)) {
-    if (!g->wms) g->wms = new WmsWorkspace();
-    if (!g->wms->sources) g->wms->sources = new SourcesWorkspace();
+    if (!g->sources) g->sources = new SourcesWorkspace();
     std::vector<int32_t> src(S);
     for (int32_t i = 0; i < S; i++) {
       int64_t v = sources[i] % (int64_t)g->n;
       if (v < 0) v += g->n;
       src[i] = (int32_t)v;
-      if (stats && g->h_row_ptr[v] == g->h_row_ptr[v + 1]) stats->skipped_sources += 1;
     }
-    return run_sources_lds(g, g->wms->sources, src.data(), S, dist, sums, stats);
+    std::vector<unsigned long long> acc;
+    double ms = 0;
+    const int rc = run_sources_lds(g, g->sources, src.data(), S, dist, acc, &ms);
+    if (rc == DAWN_ERR_OUT_OF_MEMORY) {  // nothing has run yet: the lanes try
+      sources_workspace_free(g->sources);
+      g->sources = nullptr;
+      (void)hipGetLastError();
+      return run_lanes(g, sources, S, dist, sums, policy, stats);
+    }
+    if (rc != DAWN_OK) return rc;
+    int64_t steps = 0;
+    for (int32_t i = 0; i < S; i++) {
+      const unsigned long long* x = acc.data() + (size_t)i * 4;
+      if (sums) sums[i] = (int64_t)x[0];
+      if (!stats) continue;
+      if (g->h_row_ptr[src[i]] == g->h_row_ptr[src[i] + 1]) stats->skipped_sources += 1;
+      stats->vertices_reached += (int64_t)x[1];
+      stats->edges_reached += (int64_t)x[2];
+      // Batches of 64 sources, as the lanes count them: the steps of one are
+      // those of its longest source.
+      steps = std::max<int64_t>(i % 64 ? steps : 0, (int64_t)x[3]);
+      if (i % 64 != 63 && i != S - 1) continue;
+      stats->steps += steps;
+      stats->mode_steps[DAWN_MODE_PUSH] += steps;
+      stats->batches += 1;
+    }
+    if (stats) stats->device_ms += ms;
+    return DAWN_OK;
   }
-  const int32_t per = std::min<int32_t>(S, 64);
-  if (per <= 8) return run_w<8>(g, sources, S, dist, sums, policy, stats);
-  if (per <= 16) return run_w<16>(g, sources, S, dist, sums, policy, stats);
-  if (per <= 32) return run_w<32>(g, sources, S, dist, sums, policy, stats);
-  return run_w<64>(g, sources, S, dist, sums, policy, stats);
+  return run_lanes(g, sources, S, dist, sums, policy, stats);
 }
 
 }  // namespace dawn

@@ -47,3 +47,45 @@ def test_host_rows_and_sums_only(orc, n):
     _, s2, _ = g.closeness(src)
     assert np.array_equal(s2, sums)
     g.close()
+
+
+@pytest.mark.parametrize("n,degree", [(2, 1), (300, 4), (20_000, 10), (60_000, 12), (100_000, 3)])
+@pytest.mark.parametrize("count", [1, 64, 257])
+def test_unweighted_against_lanes(orc, n, degree, count):
+    """Rows, sums and counts equal those of the engine of lanes (knobs set),
+    with isolated, negative and repeated sources."""
+    print(f"case: {n} vertices, degree {degree}, {count} sources", flush=True)
+    rng = np.random.default_rng(n + count)
+    u, v = (rng.integers(0, n, n * degree).astype(np.int32) for _ in range(2))
+    h = dawn.HostGraph.from_edges(n, u, v, symmetrize=n % 3 != 0)
+    g = dawn.Graph(h)
+    src = rng.integers(-n, 2 * n, count).astype(np.int32)
+    src[-1] = src[0]
+    rows, sums, st = device_rows(g, src, "learned")
+    hrows, hsums = g.mssp(src)
+    _, csums, _ = g.closeness(src)
+    g.set_knobs()
+    want, wsums, wst = device_rows(g, src, "learned")
+    assert np.array_equal(rows, want) and np.array_equal(hrows, want)
+    assert all(np.array_equal(x, wsums) for x in (sums, hsums, csums))
+    for f in ("vertices_reached", "edges_reached", "skipped_sources", "batches", "steps"):
+        assert st[f] == wst[f], f
+    g.close()
+
+
+def test_unweighted_long_levels(orc):
+    """Levels beyond a byte (rows, and sums without rows) on a path with a
+    random graph at its end."""
+    print("case: path of 5,000 vertices into a random graph, 40 sources", flush=True)
+    rng = np.random.default_rng(3)
+    p = np.arange(5_000, dtype=np.int32)
+    u = np.concatenate([p, 5_000 + rng.integers(0, 4_000, 12_000)]).astype(np.int32)
+    v = np.concatenate([p + 1, 5_000 + rng.integers(0, 4_000, 12_000)]).astype(np.int32)
+    h = dawn.HostGraph.from_edges(9_000, u, v)
+    g = dawn.Graph(h)
+    src = np.concatenate([[0, 4_999, 5_000], rng.integers(0, 9_000, 37)]).astype(np.int32)
+    odist, osums, _, _ = orc.mssp(h.row_ptr, h.col, None, src)
+    dist, sums = g.mssp(src)
+    assert np.array_equal(dist, odist) and np.array_equal(sums, osums)
+    assert np.array_equal(g.closeness(src)[1], osums)
+    g.close()
