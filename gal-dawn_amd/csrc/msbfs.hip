@@ -174,7 +174,6 @@ struct MsWorkspace {
   hipEvent_t ev0 = nullptr, ev1 = nullptr, e_a = nullptr, e_b = nullptr;
 };
 
-void wms_invalidate_graphs(WmsWorkspace* ws);
 
 // Captured step graphs bake grid sizes, knobs and buffer addresses (the
 // heavy-chunk lists among them); the autotuner and workspace re-layouts
@@ -185,7 +184,6 @@ void invalidate_graphs(dawn_graph* g) {
     for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
     ws->graphs.clear();
   }
-  wms_invalidate_graphs(g->wms);
 }
 
 void ms_workspace_free(MsWorkspace* ws) {

@@ -16,26 +16,28 @@
 //   dist   int32[n][L]   L = 8, 16, 32 or 64 lanes (the smallest power of
 //                        two >= the batch's sources, at least 8), so one
 //                        vertex's distances of all lanes share cache lines
-//   act    u64[2][n]     lanes of v improved in the step (step parity)
-//   q      int32[2][n]   vertices with any improved lane (step parity)
-// Step (push, chaotic like GOVMP): a frontier vertex u of out-degree < 16
-// gets one lane, which relaxes dist[v][b] = min(dist[v][b], dist[u][b] + w)
-// for each lane b active at u and each edge (edge by edge, 16 lanes at a
-// time from 16-byte record loads); a heavier u gets one
-// wave, split into 64/L groups of L lanes, group g taking edges g, g+64/L,
-// ... and lane b of a group relaxing source lane b.  Improved lanes are
-// OR-ed into act_next[v]; the first improvement appends v to the next
-// queue (staged per workgroup in LDS, one global reservation per
-// workgroup).  A K-step loop is captured once into a
-// hipGraph; every kernel reads the step and the done flag from device
-// state, so the graph is replayed until the frontier empties.
+//   act    u64[3][n]     lanes of v improved in a step (step k reads k % 3,
+//                        writes k + 1 and clears what step k - 1 read)
+//   q      int32[3][n]   vertices with any improved lane, in the same order
+// One kernel a step, launched with its number k: every workgroup derives the
+// mode from the frontier's size, the queue lengths rotate over four slots, so
+// nothing is decided, swapped or cleared between steps (four kernels a step,
+// two of them idle, cost 30 us of each).  The host launches a chunk of steps
+// and reads whether the frontier emptied.
+//
+// A group of L / 4 threads holds a vertex's record, four lanes a thread, so
+// that a wave's 16-byte loads cover whole lines (a thread per record took 64
+// lines an instruction: 285 us per pull step of a 2048 x 2048 grid, 16 lanes,
+// the L1's rate).  Push: a group per queued vertex relaxes its edges four at a
+// time; improved lanes are OR-ed into act[k + 1], the first improvement appends
+// the vertex (staged per workgroup in LDS).  Edge lists of heavy vertices go by
+// chunks, a wave each.
 //
 // Graphs small enough for a workgroup's LDS take another route (by_workgroup).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstring>
-#include <map>
 #include <vector>
 
 #include "common.hpp"
@@ -44,21 +46,27 @@ namespace dawn {
 
 namespace {
 
-constexpr int kWChunk = 32;  // steps per captured graph before a traversal's depth is known
-constexpr int kWLight = 16;  // out-degree below which a queued vertex gets one lane, not a wave
+constexpr int kWChunk = 32;       // steps per wait before a traversal's depth is known
 constexpr int kWStageCap = 4096;  // next-queue entries a workgroup stages in LDS
+// Vertices per workgroup of a step: what a pull may append stays within half of
+// kWStageCap (past it every wave's append is an atomic on one address: with
+// 4096 vertices to 2048 entries a step of a 2048 x 2048 grid took 0.8 ms).
+constexpr int kWSpan = 2048;
+constexpr int kWSlots = 4, kWSlotPad = 32;  // queue lengths, a line each
 
 struct WState {
-  int32_t step;      // parity of the current queue = step & 1
+  int32_t steps;       // steps taken
+  int32_t pull_steps;  // of those, pulled
   int32_t done;
-  unsigned qlen[2];
-  int32_t mode;        // DAWN_MODE_PUSH or DAWN_MODE_PULL for the current step
-  int32_t pull_steps;  // steps taken in pull mode so far
+  int32_t pad[29];
+  unsigned qlen[kWSlots * kWSlotPad];
 };
 
 // Pull when the frontier holds at least n / kWPullDiv vertices (policy
-// FIXED / LEARNED); PUSH and PULL policies force one mode.
-constexpr int64_t kWPullDiv = 16;
+// FIXED / LEARNED); PUSH and PULL policies force one mode.  Measured, 16 lanes,
+// n/16, n/8, n/5: 2048 x 2048 10.6, 10.1, 9.9 ms; ER 1,000,000 3.2, 3.0, 2.9;
+// RMAT-18 2.3, 2.4, 3.0; RMAT-20 6.4, 6.3, 6.9.
+constexpr int64_t kWPullDiv = 8;
 
 struct WBatch {
   int32_t nlanes;
@@ -79,10 +87,14 @@ struct WArgs {
   const int32_t* hc_beg;
   const int32_t* hc_end;
   int64_t num_hc;
+  const int32_t* oc_v;        // the same of out-edges
+  const int32_t* oc_beg;
+  const int32_t* oc_end;
+  int64_t num_oc;
   int32_t heavy;
   int32_t* dist;        // [n][L]
-  uint64_t* act;        // [2][n]
-  int32_t* q;           // [2][n]
+  uint64_t* act;        // [3][n]
+  int32_t* q;           // [3][n]
   WState* st;
   const WBatch* batch;
 };
@@ -90,31 +102,38 @@ struct WArgs {
 template <int L>
 __global__ void w_fill_kernel(WArgs a) {
   const int64_t gs = (int64_t)gridDim.x * blockDim.x;
-  const int64_t total = (int64_t)a.n * L;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gs) a.dist[i] = kInf;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < 2 * (int64_t)a.n; i += gs)
-    a.act[i] = 0ull;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    WState st{};
-    st.mode = a.policy == DAWN_POLICY_PULL ? DAWN_MODE_PULL : DAWN_MODE_PUSH;
-    *a.st = st;
-  }
+  const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t quads = (int64_t)a.n * L / 4;
+  for (int64_t i = t0; i < quads; i += gs)
+    reinterpret_cast<int4*>(a.dist)[i] = make_int4(kInf, kInf, kInf, kInf);
+  for (int64_t i = t0; i < 3 * (int64_t)a.n; i += gs) a.act[i] = 0ull;
+  uint32_t* st = reinterpret_cast<uint32_t*>(a.st);
+  if (t0 < (int64_t)(sizeof(WState) / 4)) st[t0] = 0u;
 }
 
-// Reference initialisation, one thread per source lane (each owns its
-// column of dist): the listed out-edges write their weight in row order,
-// then dist[source] = 0; the out-neighbours other than the source form the
-// first frontier.  Isolated sources keep an empty frontier (row INF except
-// the source), as MSSP skips them.
+// Reference initialisation, one workgroup per source lane (each owns its
+// column of dist): of the listed out-edges to a neighbour the last gives its
+// weight (first a tag, -1 - edge, whose minimum is that edge's), then
+// dist[source] = 0; the out-neighbours other than the source form the first
+// frontier.  Isolated sources keep an empty frontier (row INF except the
+// source), as MSSP skips them.
 template <int L>
-__global__ void w_seed_kernel(WArgs a) {
-  const int b = threadIdx.x;
-  if (blockIdx.x != 0 || b >= a.batch->nlanes) return;
+__global__ void __launch_bounds__(kBlock) w_seed_kernel(WArgs a) {
+  const int b = blockIdx.x;
+  if (b >= a.batch->nlanes) return;
   const int32_t s = a.batch->src[b];
   const int32_t beg = a.row_ptr[s], end = a.row_ptr[s + 1];
-  for (int32_t k = beg; k < end; k++) a.dist[(int64_t)a.col[k] * L + b] = a.w[k];
-  a.dist[(int64_t)s * L + b] = 0;
-  for (int32_t k = beg; k < end; k++) {
+  auto at = [&](int32_t v) { return a.dist + (int64_t)v * L + b; };
+  for (int32_t k = beg + threadIdx.x; k < end; k += kBlock) atomicMin(at(a.col[k]), -1 - k);
+  __syncthreads();
+  for (int32_t k = beg + threadIdx.x; k < end; k += kBlock) {
+    int32_t* p = at(a.col[k]);
+    if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == -1 - k)
+      __hip_atomic_store(p, a.w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(at(s), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int32_t k = beg + threadIdx.x; k < end; k += kBlock) {
     const int32_t v = a.col[k];
     if (v == s) continue;
     const unsigned long long old = atomicOr((unsigned long long*)&a.act[v], 1ull << b);
@@ -122,351 +141,403 @@ __global__ void w_seed_kernel(WArgs a) {
   }
 }
 
-template <int L>
-__global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a) {
-  constexpr int G = kWave / L;  // edge groups per wave
-  const WState st = *a.st;
-  if (st.done || st.mode != DAWN_MODE_PUSH) return;
-  const int p = st.step & 1;
-  const unsigned qn = st.qlen[p];
-  const int32_t* q_in = a.q + (int64_t)p * a.n;
-  int32_t* q_out = a.q + (int64_t)(p ^ 1) * a.n;
-  uint64_t* act_in = a.act + (int64_t)p * a.n;
-  uint64_t* act_out = a.act + (int64_t)(p ^ 1) * a.n;
-  unsigned* qlen_out = &a.st->qlen[p ^ 1];
+// Of two distances, kInf for none (both are >= 0).
+__device__ __forceinline__ int32_t w_plus(int32_t x, int32_t y) {
+  return (int32_t)min((uint32_t)x + (uint32_t)y, (uint32_t)kInf);
+}
+
+__device__ __forceinline__ bool w_pulls(unsigned qn, int32_t n, int32_t policy) {
+  if (policy == DAWN_POLICY_PULL) return true;
+  return policy != DAWN_POLICY_PUSH && (int64_t)qn * kWPullDiv >= (int64_t)n;
+}
+
+// OR over the groups of VL threads; every thread of a group receives it.
+template <int VL>
+__device__ __forceinline__ uint64_t group_or(uint64_t x) {
+#pragma unroll
+  for (int o = 1; o < VL; o <<= 1) {
+    uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)x, o), hi = 0;
+    if (VL == 16) hi = (uint32_t)__shfl_xor((int)(uint32_t)(x >> 32), o);
+    x |= (uint64_t)hi << 32 | lo;
+  }
+  return x;
+}
+
+constexpr int kRound = 4;  // edges in flight per group
+
+// Step k.  A pull, for large frontiers: every vertex v takes, per source lane
+// b, the minimum of dist[u][b] + w over its in-edges (u, w) whose tail improved
+// lane b in the last step, and stores the lanes that improve with plain stores
+// (v's record is written by v's group only; a concurrent reader of it sees the
+// old or the new value of each lane, both path lengths, so the fixed point is
+// unchanged).  Vertices of in-degree >= heavy are done by in-edge chunks, a
+// wave each, merged with atomicMin.
+template <int L, bool Wide>
+__global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a, int k) {
+  constexpr int VL = L / 4;          // threads per record
+  constexpr int VW = kWave / VL;     // records per wave
+  if (a.st->done) return;  // set by an earlier step, or by this one where qn == 0
+  const unsigned qn = a.st->qlen[(k % kWSlots) * kWSlotPad];
+  if (qn == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.st->done = 1;
+    return;
+  }
+  const bool pull = w_pulls(qn, a.n, a.policy);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    a.st->qlen[((k + 2) % kWSlots) * kWSlotPad] = 0u;
+    a.st->steps = k + 1;
+    a.st->pull_steps += pull;
+  }
+  const int32_t* q_in = a.q + (int64_t)(k % 3) * a.n;
+  int32_t* q_out = a.q + (int64_t)((k + 1) % 3) * a.n;
+  const uint64_t* act_in = a.act + (int64_t)(k % 3) * a.n;
+  uint64_t* act_out = a.act + (int64_t)((k + 1) % 3) * a.n;
+  unsigned* qlen_out = &a.st->qlen[((k + 1) % kWSlots) * kWSlotPad];
+  const int64_t t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t threads = (int64_t)gridDim.x * kBlock;
+  // The masks step k - 1 read: by its queue, or all where that held many.
+  if (k > 0) {
+    uint64_t* clr = a.act + (int64_t)((k + 2) % 3) * a.n;
+    const int32_t* q_prev = a.q + (int64_t)((k + 2) % 3) * a.n;
+    const unsigned pn = a.st->qlen[((k + kWSlots - 1) % kWSlots) * kWSlotPad];
+    if ((int64_t)pn * 16 >= a.n) {
+      for (int64_t i = t0; i < a.n; i += threads) clr[i] = 0ull;
+    } else {
+      for (int64_t i = t0; i < pn; i += threads) clr[q_prev[i]] = 0ull;
+    }
+  }
   __shared__ LdsQueue<kWStageCap> s_q;
   if (threadIdx.x == 0) s_q.init();
   __syncthreads();
   const int lane = lane_id();
-  const int b = lane % L;
-  const int grp = lane / L;
-  const uint64_t gmask = L == 64 ? ~0ull : ((1ull << L) - 1);
-  // Light vertices (out-degree < kWLight): one lane per queued vertex -- on
-  // sparse graphs a vertex is usually active in few lanes, so a wave per
-  // vertex would leave most lanes idle.  The lane takes u's edges in turn;
-  // per edge it works through the record in chunks of CH = min(L, 16)
-  // source lanes that hold an active lane of u: 16-byte loads of u's and
-  // the neighbour's distances (u's held in registers when L <= 16), atomics
-  // only for the lanes that improve, and one act_next OR per edge.  The
-  // wave loops until its busiest lane is done, so every lane of the wave
-  // takes part in each (LDS-staged) append.
-  {
-    constexpr int CH = L < 16 ? L : 16;
-    constexpr int NC = L / CH;
-    constexpr uint64_t kChunk = CH == 64 ? ~0ull : ((1ull << CH) - 1);
-    auto load_chunk = [](const int32_t* p, int32_t (&x)[CH]) {
+  const int sub = lane % VL, grp = lane / VL;
+  const int64_t wave = t0 / kWave, nwaves = threads / kWave;
+  auto quad = [&](int32_t v) { return reinterpret_cast<int4*>(a.dist + (int64_t)v * L) + sub; };
+  // This thread's lanes of a mask; inactive lanes' distances count as kInf.
+  auto bits4 = [&](uint64_t m) { return (unsigned)(m >> (4 * sub)) & 15u; };
+  auto masked = [&](int4 d, unsigned m) {
+    return make_int4(m & 1 ? d.x : kInf, m & 2 ? d.y : kInf, m & 4 ? d.z : kInf, m & 8 ? d.w : kInf);
+  };
+  if (!pull) {
+    // kRound edges of this group's vertex (v < 0: none), whose distances are du.
+    auto relax = [&](const int32_t (&v)[kRound], const int32_t (&wt)[kRound], int4 du) {
+      int4 dv[kRound];
+      int32_t old[kRound][4], nd[kRound][4];
 #pragma unroll
-      for (int t = 0; t < CH / 4; t++) {
-        const int4 y = reinterpret_cast<const int4*>(p)[t];
-        x[4 * t] = y.x;
-        x[4 * t + 1] = y.y;
-        x[4 * t + 2] = y.z;
-        x[4 * t + 3] = y.w;
+      for (int r = 0; r < kRound; r++) dv[r] = v[r] >= 0 ? *quad(v[r]) : make_int4(0, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < kRound; r++) {
+        nd[r][0] = w_plus(du.x, wt[r]), nd[r][1] = w_plus(du.y, wt[r]);
+        nd[r][2] = w_plus(du.z, wt[r]), nd[r][3] = w_plus(du.w, wt[r]);
+        int32_t* p = reinterpret_cast<int32_t*>(quad(v[r]));
+        old[r][0] = nd[r][0] < dv[r].x ? atomicMin(p, nd[r][0]) : -1;
+        old[r][1] = nd[r][1] < dv[r].y ? atomicMin(p + 1, nd[r][1]) : -1;
+        old[r][2] = nd[r][2] < dv[r].z ? atomicMin(p + 2, nd[r][2]) : -1;
+        old[r][3] = nd[r][3] < dv[r].w ? atomicMin(p + 3, nd[r][3]) : -1;
       }
+      // Opaque to the compiler, which else moves each comparison, and with it
+      // the wait for its atomic, up before the next atomic.
+#pragma unroll
+      for (int r = 0; r < kRound; r++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) asm volatile("" : "+v"(old[r][c]));
+      unsigned long long was[kRound];
+      uint64_t imp[kRound];
+#pragma unroll
+      for (int r = 0; r < kRound; r++) {
+        unsigned x = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) x |= (nd[r][c] < old[r][c] ? 1u : 0u) << c;
+        imp[r] = group_or<VL>((uint64_t)x << (4 * sub));
+        was[r] = 1ull;
+        if (sub == 0 && imp[r]) was[r] = atomicOr((unsigned long long*)&act_out[v[r]], imp[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < kRound; r++) asm volatile("" : "+v"(was[r]));
+#pragma unroll
+      for (int r = 0; r < kRound; r++)
+        s_q.append(sub == 0 && imp[r] != 0 && was[r] == 0ull, v[r], qlen_out, q_out);
     };
-    for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); base < qn;
-         base += (int64_t)gridDim.x * kBlock) {  // wave-uniform
-      const int64_t i = base + lane;
+    for (int64_t i0 = wave * VW; i0 < qn; i0 += nwaves * VW) {  // wave-uniform
+      const int64_t i = i0 + grp;
       int32_t u = 0;
-      uint64_t m = 0;
       int beg = 0, deg = 0;
+      int4 du = make_int4(kInf, kInf, kInf, kInf);
       if (i < qn) {
         u = q_in[i];
         beg = a.row_ptr[u];
         deg = a.row_ptr[u + 1] - beg;
-        if (deg < kWLight) m = act_in[u];
+        const unsigned m = bits4(act_in[u]);
+        du = masked(*quad(u), m);
+        if (deg >= a.heavy) deg = 0;
       }
-      const bool light = i < qn && deg < kWLight;
-      const int most = wave_max_i32(m ? deg : 0);
-      const int32_t* up = a.dist + (int64_t)u * L;
-      int32_t du[CH];
-      if (NC == 1 && m) load_chunk(up, du);
-      for (int e = 0; e < most; e++) {
-        bool append = false;
-        int32_t v = -1;
-        if (m && e < deg) {
-          v = a.col[beg + e];
-          const int32_t wt = a.w[beg + e];
-          int32_t* vp = a.dist + (int64_t)v * L;
-          uint64_t imp = 0;
-#pragma unroll 1
-          for (int c = 0; c < NC; c++) {
-            const uint64_t mc = (m >> (c * CH)) & kChunk;
-            if (!mc) continue;
-            if (NC > 1) load_chunk(up + c * CH, du);
-            int32_t dv[CH];
-            load_chunk(vp + c * CH, dv);
+      const int most = wave_max_i32(deg);
+      for (int j = 0; j < most; j += kRound) {
+        int32_t v[kRound], wt[kRound];
 #pragma unroll
-            for (int bl = 0; bl < CH; bl++) {
-              if (((mc >> bl) & 1ull) && du[bl] != kInf) {
-                const int32_t nd = minplus(du[bl], wt);
-                if (nd < dv[bl] && nd < atomicMin(vp + c * CH + bl, nd)) imp |= 1ull << (c * CH + bl);
+        for (int r = 0; r < kRound; r++) v[r] = j + r < deg ? a.col[beg + j + r] : -1;
+#pragma unroll
+        for (int r = 0; r < kRound; r++) wt[r] = j + r < deg ? a.w[beg + j + r] : 0;
+        relax(v, wt, du);
+      }
+    }
+    // Heavy vertices by out-edge chunks: a wave looks at 64 chunks, then takes
+    // the active ones, kRound edges per group at a time.
+    for (int64_t c0 = wave * kWave; c0 < a.num_oc; c0 += nwaves * kWave) {  // wave-uniform
+      const int64_t c = c0 + lane;
+      uint64_t hot = __ballot(c < a.num_oc && act_in[a.oc_v[c < a.num_oc ? c : 0]] != 0ull);
+      for (; hot; hot &= hot - 1) {
+        const int64_t hc = c0 + __ffsll((unsigned long long)hot) - 1;
+        const int32_t u = a.oc_v[hc];
+        const int kb = a.oc_beg[hc], ke = a.oc_end[hc];
+        const int4 du = masked(*quad(u), bits4(act_in[u]));
+        for (int j = kb; j < ke; j += kRound * VW) {
+          int32_t v[kRound], wt[kRound];
+#pragma unroll
+          for (int r = 0; r < kRound; r++) v[r] = j + r * VW + grp < ke ? a.col[j + r * VW + grp] : -1;
+#pragma unroll
+          for (int r = 0; r < kRound; r++) wt[r] = j + r * VW + grp < ke ? a.w[j + r * VW + grp] : 0;
+          relax(v, wt, du);
+        }
+      }
+    }
+  } else {
+    // Minima over kRound in-edges (u < 0: none) of this thread's lanes.
+    auto gather = [&](const int32_t (&u)[kRound], const int32_t (&wt)[kRound], int4& best) {
+      unsigned m[kRound];
+      int4 du[kRound];
+#pragma unroll
+      for (int r = 0; r < kRound; r++) m[r] = u[r] >= 0 ? bits4(act_in[u[r]]) : 0u;
+#pragma unroll
+      for (int r = 0; r < kRound; r++)
+        du[r] = m[r] ? *quad(u[r]) : make_int4(kInf, kInf, kInf, kInf);
+#pragma unroll
+      for (int r = 0; r < kRound; r++) {
+        const int4 d = masked(du[r], m[r]);
+        best.x = min(best.x, w_plus(d.x, wt[r])), best.y = min(best.y, w_plus(d.y, wt[r]));
+        best.z = min(best.z, w_plus(d.z, wt[r])), best.w = min(best.w, w_plus(d.w, wt[r]));
+      }
+    };
+    // Lanes of best below dv, moved there.
+    auto take = [](const int4& best, int4& dv) {
+      unsigned x = 0;
+      if (best.x < dv.x) dv.x = best.x, x |= 1;
+      if (best.y < dv.y) dv.y = best.y, x |= 2;
+      if (best.z < dv.z) dv.z = best.z, x |= 4;
+      if (best.w < dv.w) dv.w = best.w, x |= 8;
+      return x;
+    };
+    if constexpr (Wide) {
+      // Records of 64 lanes, or of 32 where heavy vertices hold the edges: a
+      // group takes a vertex, list and all (the minima of 64 vertices would
+      // take 32 or 64 registers and leave two or three waves per SIMD to the
+      // heavy vertices: RMAT-20, 64 sources, 23 -> 32 ms, 32 sources 13 -> 18;
+      // without heavy vertices, 2048 x 2048, 32 sources, 28 -> 22).
+      for (int64_t v0 = wave * VW; v0 < a.n; v0 += nwaves * VW) {  // wave-uniform
+        const int64_t vv = v0 + grp;
+        const int32_t v = vv < a.n ? (int32_t)vv : 0;
+        int beg = 0, deg = 0;
+        if (vv < a.n) {
+          beg = a.in_row_ptr[v];
+          deg = a.in_row_ptr[v + 1] - beg;
+          if (deg >= a.heavy) deg = 0;
+        }
+        int4 best = make_int4(kInf, kInf, kInf, kInf);
+        for (int j = 0; j < deg; j += kRound) {
+          int32_t u[kRound], wt[kRound];
+#pragma unroll
+          for (int r = 0; r < kRound; r++) u[r] = j + r < deg ? a.in_col[beg + j + r] : -1;
+#pragma unroll
+          for (int r = 0; r < kRound; r++) wt[r] = j + r < deg ? a.in_w[beg + j + r] : 0;
+          gather(u, wt, best);
+        }
+        unsigned x = 0;
+        if (min(min(best.x, best.y), min(best.z, best.w)) != kInf) {
+          int4 dv = *quad(v);
+          x = take(best, dv);
+          if (x) *quad(v) = dv;
+        }
+        const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
+        if (sub == 0 && imp) act_out[v] = imp;  // v's own slot (heavy vertices are not here)
+        s_q.append(sub == 0 && imp != 0, v, qlen_out, q_out);
+      }
+    } else {
+      // Light vertices, 64 a wave: a thread per vertex reads its list, kRound
+      // edges at a time, and their tails' masks; then the groups, VW vertices at
+      // a time, read the records.  Without branches (a tail that did not improve
+      // gives way to the vertex's own record, read below in any case), so that a
+      // stage's loads are all in flight (16 vertices a wave, list and records by
+      // the group: 390 us for 2048 x 2048, a chain of six latencies each).
+      for (int64_t v0 = wave * kWave; v0 < a.n; v0 += nwaves * kWave) {  // wave-uniform
+        int beg = 0, deg = 0;
+        if (v0 + lane < a.n) {
+          beg = a.in_row_ptr[v0 + lane];
+          deg = a.in_row_ptr[v0 + lane + 1] - beg;
+          if (deg >= a.heavy) deg = 0;
+        }
+        int4 best[VL];
+#pragma unroll
+        for (int q = 0; q < VL; q++) best[q] = make_int4(kInf, kInf, kInf, kInf);
+        auto vertex = [&](int q) { return (int32_t)min(v0 + q * VW + grp, (int64_t)a.n - 1); };
+        const int most = wave_max_i32(deg);
+        bool any = false;
+        for (int j = 0; j < most; j += kRound) {
+          int32_t u[kRound], wt[kRound];
+          uint64_t m[kRound];
+#pragma unroll
+          for (int r = 0; r < kRound; r++) {
+            const int k = j + r < deg ? beg + j + r : 0;
+            u[r] = a.in_col[k];
+            wt[r] = a.in_w[k];
+          }
+#pragma unroll
+          for (int r = 0; r < kRound; r++) m[r] = act_in[u[r]];
+          uint64_t seen = 0;
+#pragma unroll
+          for (int r = 0; r < kRound; r++) {
+            m[r] = j + r < deg ? m[r] : 0ull;
+            seen |= m[r];
+          }
+          if (!__ballot(seen != 0)) continue;
+          any = true;
+#pragma unroll
+          for (int q = 0; q < VL; q += 2) {
+            int4 du[2][kRound];
+            int32_t w2[2][kRound];
+            unsigned m2[2][kRound];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+              const int from = (q + h) * VW + grp;
+#pragma unroll
+              for (int r = 0; r < kRound; r++) {
+                m2[h][r] = bits4((uint32_t)__shfl((int)(uint32_t)m[r], from));
+                w2[h][r] = __shfl(wt[r], from);
+                const int32_t t = __shfl(u[r], from);
+                du[h][r] = *quad(m2[h][r] ? t : vertex(q + h));
               }
             }
-          }
-          if (imp) append = atomicOr((unsigned long long*)&act_out[v], (unsigned long long)imp) == 0ull;
-        }
-        s_q.append(append, v, qlen_out, q_out);
-      }
-      if (light) act_in[u] = 0ull;  // consumed
-    }
-  }
-  // Heavy vertices: one wave each, split into groups of L lanes.
-  const int64_t wave = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
-  const int64_t nwaves = (int64_t)gridDim.x * (kBlock / kWave);
-  for (int64_t i = wave; i < qn; i += nwaves) {
-    const int32_t u = q_in[i];
-    if (a.row_ptr[u + 1] - a.row_ptr[u] < kWLight) continue;
-    const uint64_t mask = act_in[u];
-    const bool active = (mask >> b) & 1ull;
-    const int32_t du = active ? a.dist[(int64_t)u * L + b] : kInf;
-    const int beg = a.row_ptr[u], end = a.row_ptr[u + 1];
-    for (int e0 = beg; e0 < end; e0 += G) {
-      const int e = e0 + grp;
-      bool improved = false;
-      int32_t v = -1;
-      if (e < end) {
-        v = a.col[e];
-        if (active && du != kInf) {
-          const int32_t nd = minplus(du, a.w[e]);
-          int32_t* dv = a.dist + (int64_t)v * L + b;
-          if (nd < *dv) improved = nd < atomicMin(dv, nd);
-        }
-      }
-      const uint64_t bal = __ballot(improved);
-      const uint64_t mine = (bal >> (grp * L)) & gmask;
-      // One atomic per group and edge; the first improvement of v in this
-      // step appends it to the next queue.
-      bool append = false;
-      if (b == 0 && mine) append = atomicOr((unsigned long long*)&act_out[v], mine) == 0ull;
-      s_q.append(append, v, qlen_out, q_out);
-    }
-    if (lane == 0) act_in[u] = 0ull;  // consumed (each u is in the queue once)
-  }
-  s_q.flush(qlen_out, q_out);
-}
-
-// Pull step, for large frontiers: every vertex v takes, per source lane b,
-// the minimum of dist[u][b] + w over its in-edges (u, w) whose tail
-// improved lane b in the last step, and stores the lanes that improve with
-// plain stores (v's record is written by v's thread only; a concurrent
-// reader of it sees the old or the new value of each lane, both path
-// lengths, so the fixed point is unchanged).  Vertices of in-degree >=
-// heavy are done by in-edge chunks, a wave each: per lane minima reduced
-// over the wave, merged with atomicMin (a vertex's chunks may run in
-// different waves).  Light vertices take 16 source lanes at a time from
-// 16-byte record loads.
-// In-edges per round of a light vertex in the batched pull step.
-constexpr int kPullRound = 4;
-
-template <int L>
-__global__ void __launch_bounds__(kBlock) w_pull_kernel(WArgs a) {
-  constexpr int CH = L < 16 ? L : 16;
-  constexpr int NC = L / CH;
-  constexpr uint64_t kChunk = CH == 64 ? ~0ull : ((1ull << CH) - 1);
-  const WState st = *a.st;
-  if (st.done || st.mode != DAWN_MODE_PULL) return;
-  const int p = st.step & 1;
-  const uint64_t* act_in = a.act + (int64_t)p * a.n;
-  uint64_t* act_out = a.act + (int64_t)(p ^ 1) * a.n;
-  int32_t* q_out = a.q + (int64_t)(p ^ 1) * a.n;
-  unsigned* qlen_out = &a.st->qlen[p ^ 1];
-  __shared__ LdsQueue<kWStageCap> s_q;
-  if (threadIdx.x == 0) s_q.init();
-  __syncthreads();
-  const int lane = lane_id();
-  auto load_chunk = [](const int32_t* q, int32_t (&x)[CH]) {
 #pragma unroll
-    for (int t = 0; t < CH / 4; t++) {
-      const int4 y = reinterpret_cast<const int4*>(q)[t];
-      x[4 * t] = y.x;
-      x[4 * t + 1] = y.y;
-      x[4 * t + 2] = y.z;
-      x[4 * t + 3] = y.w;
-    }
-  };
-  for (int64_t base = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~(kWave - 1)); base < a.n;
-       base += (int64_t)gridDim.x * kBlock) {  // wave-uniform
-    const int64_t vv = base + lane;
-    const int32_t v = vv < a.n ? (int32_t)vv : 0;
-    int beg = 0, deg = 0;
-    if (vv < a.n) {
-      beg = a.in_row_ptr[v];
-      deg = a.in_row_ptr[v + 1] - beg;
-    }
-    uint64_t imp = 0;
-    if (vv < a.n && deg > 0 && deg < a.heavy) {
-      int32_t* vp = a.dist + (int64_t)v * L;
-#pragma unroll 1
-      for (int c = 0; c < NC; c++) {
-        int32_t best[CH];
+            for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int bl = 0; bl < CH; bl++) best[bl] = kInf;
-        bool any = false;
-        // Rounds of kPullRound in-edges: their columns and weights, then
-        // their tails' masks, then the improved tails' records, so that a
-        // lane waits on memory once per stage and round, not per edge.
-        for (int j0 = 0; j0 < deg; j0 += kPullRound) {
-          int32_t u[kPullRound], wt[kPullRound];
-#pragma unroll
-          for (int t = 0; t < kPullRound; t++) {
-            const bool ok = j0 + t < deg;
-            u[t] = ok ? a.in_col[beg + j0 + t] : -1;
-            wt[t] = ok ? a.in_w[beg + j0 + t] : 0;
-          }
-          uint64_t m[kPullRound];
-#pragma unroll
-          for (int t = 0; t < kPullRound; t++) m[t] = u[t] >= 0 ? (act_in[u[t]] >> (c * CH)) & kChunk : 0ull;
-#pragma unroll
-          for (int t = 0; t < kPullRound; t++) {
-            if (!m[t]) continue;
-            any = true;
-            int32_t du[CH];
-            load_chunk(a.dist + (int64_t)u[t] * L + c * CH, du);
-#pragma unroll
-            for (int bl = 0; bl < CH; bl++)
-              if (((m[t] >> bl) & 1ull) && du[bl] != kInf) best[bl] = min(best[bl], minplus(du[bl], wt[t]));
+              for (int r = 0; r < kRound; r++) {
+                const int4 d = masked(du[h][r], m2[h][r]);
+                int4& b = best[q + h];
+                b.x = min(b.x, w_plus(d.x, w2[h][r])), b.y = min(b.y, w_plus(d.y, w2[h][r]));
+                b.z = min(b.z, w_plus(d.z, w2[h][r])), b.w = min(b.w, w_plus(d.w, w2[h][r]));
+              }
           }
         }
         if (!any) continue;
-        int32_t dv[CH];
-        load_chunk(vp + c * CH, dv);
-        uint64_t ci = 0;
 #pragma unroll
-        for (int bl = 0; bl < CH; bl++)
-          if (best[bl] < dv[bl]) {
-            dv[bl] = best[bl];
-            ci |= 1ull << bl;
+        for (int q = 0; q < VL; q += 2) {
+          int4 dv[2];
+#pragma unroll
+          for (int h = 0; h < 2; h++) dv[h] = *quad(vertex(q + h));
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            const int4 b = best[q + h];
+            const int32_t v = vertex(q + h);
+            const bool in = v0 + (q + h) * VW + grp < a.n;
+            const unsigned x = in ? take(b, dv[h]) : 0u;
+            if (x) *quad(v) = dv[h];
+            const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
+            if (sub == 0 && imp) act_out[v] = imp;  // v's own slot (heavy vertices are not here)
+            s_q.append(sub == 0 && imp != 0, v, qlen_out, q_out);
           }
-        if (ci) {
-#pragma unroll
-          for (int t = 0; t < CH / 4; t++)
-            reinterpret_cast<int4*>(vp + c * CH)[t] =
-                make_int4(dv[4 * t], dv[4 * t + 1], dv[4 * t + 2], dv[4 * t + 3]);
-          imp |= ci << (c * CH);
         }
       }
-      if (imp) act_out[v] = imp;  // v's own slot (heavy vertices are not here)
     }
-    s_q.append(imp != 0, v, qlen_out, q_out);
-  }
-  // Heavy vertices by in-edge chunks, one wave each.
-  const int64_t wave = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kWave;
-  const int64_t nwaves = (int64_t)gridDim.x * (kBlock / kWave);
-  for (int64_t hc = wave; hc < a.num_hc; hc += nwaves) {  // wave-uniform
-    const int32_t v = a.hc_v[hc];
-    const int kb = a.hc_beg[hc], ke = a.hc_end[hc];
-    uint64_t vimp = 0;
-#pragma unroll 1
-    for (int c = 0; c < NC; c++) {
-      int32_t best[CH];
+    for (int64_t hc = wave; hc < a.num_hc; hc += nwaves) {  // wave-uniform
+      const int32_t v = a.hc_v[hc];
+      const int kb = a.hc_beg[hc], ke = a.hc_end[hc];
+      int4 best = make_int4(kInf, kInf, kInf, kInf);
+      for (int j = kb; j < ke; j += kRound * VW) {
+        int32_t u[kRound], wt[kRound];
 #pragma unroll
-      for (int bl = 0; bl < CH; bl++) best[bl] = kInf;
-      for (int k = kb + lane; k < ke; k += kWave) {
-        const int32_t u = a.in_col[k];
-        const uint64_t m = (act_in[u] >> (c * CH)) & kChunk;
-        if (!m) continue;
-        const int32_t wt = a.in_w[k];
-        int32_t du[CH];
-        load_chunk(a.dist + (int64_t)u * L + c * CH, du);
+        for (int r = 0; r < kRound; r++) u[r] = j + r * VW + grp < ke ? a.in_col[j + r * VW + grp] : -1;
 #pragma unroll
-        for (int bl = 0; bl < CH; bl++)
-          if (((m >> bl) & 1ull) && du[bl] != kInf) best[bl] = min(best[bl], minplus(du[bl], wt));
+        for (int r = 0; r < kRound; r++) wt[r] = j + r * VW + grp < ke ? a.in_w[j + r * VW + grp] : 0;
+        gather(u, wt, best);
       }
-      int32_t mine = kInf;
-#pragma unroll
-      for (int bl = 0; bl < CH; bl++) {
-        const int32_t x = wave_min_i32(best[bl]);
-        if (lane == bl) mine = x;
+      for (int o = VL; o < kWave; o <<= 1) {
+        best.x = min(best.x, __shfl_xor(best.x, o)), best.y = min(best.y, __shfl_xor(best.y, o));
+        best.z = min(best.z, __shfl_xor(best.z, o)), best.w = min(best.w, __shfl_xor(best.w, o));
       }
-      bool improved = false;
-      if (lane < CH && mine != kInf) {
-        int32_t* dp = a.dist + (int64_t)v * L + c * CH + lane;
-        if (mine < *dp) improved = mine < atomicMin(dp, mine);
+      unsigned x = 0;
+      if (grp == 0 && min(min(best.x, best.y), min(best.z, best.w)) != kInf) {
+        int32_t* p = reinterpret_cast<int32_t*>(quad(v));
+        const int4 dv = *quad(v);
+        if (best.x < dv.x && best.x < atomicMin(p, best.x)) x |= 1;
+        if (best.y < dv.y && best.y < atomicMin(p + 1, best.y)) x |= 2;
+        if (best.z < dv.z && best.z < atomicMin(p + 2, best.z)) x |= 4;
+        if (best.w < dv.w && best.w < atomicMin(p + 3, best.w)) x |= 8;
       }
-      vimp |= (__ballot(improved) & kChunk) << (c * CH);
+      const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
+      bool append = false;
+      if (lane == 0 && imp) append = atomicOr((unsigned long long*)&act_out[v], (unsigned long long)imp) == 0ull;
+      s_q.append(append, v, qlen_out, q_out);
     }
-    bool append = false;
-    if (lane == 0 && vimp) append = atomicOr((unsigned long long*)&act_out[v], (unsigned long long)vimp) == 0ull;
-    s_q.append(append, v, qlen_out, q_out);
   }
   s_q.flush(qlen_out, q_out);
 }
 
-// After a pull step: clears the consumed frontier masks (a push step clears
-// each as it consumes it; a pull step reads them from many threads).
-__global__ void w_clear_kernel(WArgs a) {
-  const WState st = *a.st;
-  if (st.done || st.mode != DAWN_MODE_PULL) return;
-  const int p = st.step & 1;
-  const unsigned qn = st.qlen[p];
-  const int32_t* q_in = a.q + (int64_t)p * a.n;
-  uint64_t* act_in = a.act + (int64_t)p * a.n;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < qn;
-       i += (int64_t)gridDim.x * blockDim.x)
-    act_in[q_in[i]] = 0ull;
-}
-
-// Ends a step: the next queue becomes current, and the next step's mode is
-// chosen from its size.
-__global__ void w_advance_kernel(WState* st, int32_t n, int32_t policy) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (st->done) return;
-  const int p = st->step & 1;
-  if (st->mode == DAWN_MODE_PULL) st->pull_steps += 1;
-  st->qlen[p] = 0;
-  st->step += 1;
-  const unsigned nq = st->qlen[p ^ 1];
-  if (nq == 0) {
-    st->done = 1;
-    return;
-  }
-  int mode = DAWN_MODE_PUSH;
-  if (policy == DAWN_POLICY_PULL) mode = DAWN_MODE_PULL;
-  else if (policy != DAWN_POLICY_PUSH && (int64_t)nq * kWPullDiv >= (int64_t)n) mode = DAWN_MODE_PULL;
-  st->mode = mode;
-}
-
 // Distance rows (lane b at out + b * stride) and per-lane sums: a workgroup
-// stages 256 vertices x L lanes in LDS (one contiguous read), then each
-// wave writes its 64 vertices of every lane as one coalesced row segment.
-template <int L>
+// stages 256 / 128 vertices x L lanes in LDS (one contiguous read, records at
+// an odd stride), then wave w writes the rows of lanes w, w + 4, ... segment by
+// segment.  Sums stay in registers, per thread and lane, until the end
+// (reduced per 64 vertices they took 395 us of a 2048 x 2048 grid's 16 lanes).
 // acc: [0..63] distance sums, [64..127] reached vertices, [128..191] sum of
 // out-degrees of reached vertices, per lane.
+template <int L>
 __global__ void __launch_bounds__(kBlock) w_final_kernel(WArgs a, int32_t* out, int64_t stride,
                                                          unsigned long long* acc) {
-  __shared__ int32_t s_tile[kBlock * L];
-  __shared__ unsigned long long s_acc[3 * 64];
+  constexpr int T = L <= 32 ? 256 : 128;  // vertices per tile
+  constexpr int W = kBlock / kWave, B = L / W;
+  __shared__ int32_t s_tile[T * (L + 1)];
+  __shared__ int32_t s_deg[T];
   const int nl = a.batch->nlanes;
-  if (threadIdx.x < 3 * 64) s_acc[threadIdx.x] = 0;
   const int lane = lane_id();
   const int wv = threadIdx.x / kWave;
-  for (int64_t b0 = (int64_t)blockIdx.x * kBlock; b0 < a.n; b0 += (int64_t)gridDim.x * kBlock) {
-    const int64_t cnt = std::min<int64_t>(kBlock, a.n - b0);  // block-uniform
-    const int32_t* src = a.dist + b0 * L;
+  unsigned long long sum[B], edges[B];
+  unsigned reached[B];
+#pragma unroll
+  for (int r = 0; r < B; r++) sum[r] = edges[r] = 0, reached[r] = 0;
+  for (int64_t b0 = (int64_t)blockIdx.x * T; b0 < a.n; b0 += (int64_t)gridDim.x * T) {
+    const int cnt = (int)std::min<int64_t>(T, a.n - b0);  // block-uniform
+    const int4* src = reinterpret_cast<const int4*>(a.dist + b0 * L);
     __syncthreads();
-    for (int64_t i = threadIdx.x; i < cnt * L; i += kBlock) s_tile[i] = src[i];
+    for (int i = threadIdx.x; i < cnt * (L / 4); i += kBlock) {
+      const int4 x = src[i];
+      int32_t* p = s_tile + (i / (L / 4)) * (L + 1) + i % (L / 4) * 4;
+      p[0] = x.x, p[1] = x.y, p[2] = x.z, p[3] = x.w;
+    }
+    for (int i = threadIdx.x; i < cnt; i += kBlock) s_deg[i] = a.row_ptr[b0 + i + 1] - a.row_ptr[b0 + i];
     __syncthreads();
-    const int64_t v = b0 + wv * kWave + lane;
-    const bool ok = v < a.n;
-    const unsigned deg = ok ? (unsigned)(a.row_ptr[v + 1] - a.row_ptr[v]) : 0u;
-    for (int bl = 0; bl < nl; bl++) {
-      const int32_t d = ok ? s_tile[(wv * kWave + lane) * L + bl] : kInf;
-      if (out && ok) out[(int64_t)bl * stride + v] = d;
-      const bool r = d != kInf;
-      const unsigned long long sm = wave_sum_u64(r ? (unsigned long long)d : 0ull);
-      const unsigned long long em = wave_sum_u64(r ? (unsigned long long)deg : 0ull);
-      const unsigned long long rc = (unsigned long long)__popcll(__ballot(r));
-      if (lane == 0) {
-        if (sm) atomicAdd(&s_acc[bl], sm);
-        if (rc) atomicAdd(&s_acc[64 + bl], rc);
-        if (em) atomicAdd(&s_acc[128 + bl], em);
+#pragma unroll
+    for (int r = 0; r < B; r++) {
+      const int bl = r * W + wv;
+      if (bl >= nl) continue;
+      for (int i = lane; i < cnt; i += kWave) {
+        const int32_t d = s_tile[i * (L + 1) + bl];
+        if (out) out[(int64_t)bl * stride + b0 + i] = d;
+        if (d != kInf) {
+          sum[r] += (unsigned)d;
+          reached[r]++;
+          edges[r] += (unsigned)s_deg[i];
+        }
       }
     }
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 3 * 64; i += kBlock)
-    if ((i & 63) < nl && s_acc[i]) atomicAdd(&acc[i], s_acc[i]);
+#pragma unroll
+  for (int r = 0; r < B; r++) {
+    const int bl = r * W + wv;
+    const unsigned long long s1 = wave_sum_u64(sum[r]), s2 = wave_sum_u64(reached[r]), s3 = wave_sum_u64(edges[r]);
+    if (lane == 0 && bl < nl) {
+      if (s1) atomicAdd(&acc[bl], s1);
+      if (s2) atomicAdd(&acc[64 + bl], s2);
+      if (s3) atomicAdd(&acc[128 + bl], s3);
+    }
+  }
 }
 
 __global__ void w_zero_kernel(unsigned long long* p, int n) {
@@ -485,20 +556,12 @@ struct WmsWorkspace {
   DevBuf<unsigned long long> sums;
   WState* h_state = nullptr;
   WBatch* h_batch = nullptr;
-  std::map<int, hipGraphExec_t> graphs;  // by (L, policy, steps per graph)
-  int32_t last_steps = 0;                // steps the last batch took
+  int32_t last_steps = 0;  // steps the last batch took
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
 
-void wms_invalidate_graphs(WmsWorkspace* ws) {
-  if (!ws) return;
-  for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
-  ws->graphs.clear();
-}
-
 void wms_workspace_free(WmsWorkspace* ws) {
   if (!ws) return;
-  for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
   if (ws->h_state) (void)hipHostFree(ws->h_state);
   if (ws->h_batch) (void)hipHostFree(ws->h_batch);
   for (hipEvent_t e : {ws->ev0, ws->ev1})
@@ -512,15 +575,13 @@ int ensure_wms(dawn_graph* g, int L) {
   if (!g->wms) g->wms = new WmsWorkspace();
   WmsWorkspace* ws = g->wms;
   if (ws->n == g->n && ws->lanes == L && ws->dist.p) return DAWN_OK;
-  for (auto& kv : ws->graphs) (void)hipGraphExecDestroy(kv.second);
-  ws->graphs.clear();
   ws->dist.release();
   ws->rows.release();
   ws->n = g->n;
   ws->lanes = L;
   DAWN_TRY(ws->dist.alloc((size_t)g->n * L));
-  DAWN_TRY(ws->act.alloc((size_t)2 * g->n));
-  DAWN_TRY(ws->q.alloc((size_t)2 * g->n));
+  DAWN_TRY(ws->act.alloc((size_t)3 * g->n));
+  DAWN_TRY(ws->q.alloc((size_t)3 * g->n));
   DAWN_TRY(ws->st.alloc(1));
   DAWN_TRY(ws->batch.alloc(1));
   DAWN_TRY(ws->sums.alloc(3 * 64));
@@ -552,6 +613,10 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
   a.hc_beg = g->hc_beg;
   a.hc_end = g->hc_end;
   a.num_hc = g->num_hc;
+  a.oc_v = g->oc_v;
+  a.oc_beg = g->oc_beg;
+  a.oc_end = g->oc_end;
+  a.num_oc = g->num_oc;
   a.heavy = g->knobs.heavy_degree;
   a.dist = ws->dist.p;
   a.act = ws->act.p;
@@ -559,35 +624,13 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
   a.st = ws->st.p;
   a.batch = ws->batch.p;
   const unsigned fill_grid = grid_for((int64_t)g->n * L);
-  const unsigned step_grid = 2048;  // 8 workgroups per CU, waves stride the queue
-  // (1024-8192 workgroups measured within noise of each other.)
-  const unsigned pull_grid = grid_for(std::max<int32_t>(g->n, 1), kBlock, 4096);
-  const unsigned fin_grid = grid_for(std::max<int32_t>(g->n, 1), kBlock, 2048);
+  const unsigned step_grid = (unsigned)std::max<int64_t>(1024, (g->n + kWSpan - 1) / kWSpan);
+  const unsigned fin_grid = 1024;
+  const bool wide = g->num_hc * 64 > g->n;  // heavy vertices hold many of the edges
 
-  // Steps per captured graph: what the last batch took (+ the one that
-  // finds the frontier empty), rounded up to a multiple of 8, so that one
-  // graph launch and one read of the done flag usually suffice.
-  const int chunk = ws->last_steps > 0 ? std::min(256, (ws->last_steps + 1 + 7) & ~7) : kWChunk;
-  const int key = (chunk * 128 + L) * 8 + (policy & 7);
-  hipGraphExec_t exec = nullptr;
-  auto it = ws->graphs.find(key);
-  if (it != ws->graphs.end()) {
-    exec = it->second;
-  } else {
-    hipGraph_t graph;
-    DAWN_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < chunk; i++) {
-      w_step_kernel<L><<<step_grid, kBlock, 0, s>>>(a);
-      w_pull_kernel<L><<<pull_grid, kBlock, 0, s>>>(a);
-      w_clear_kernel<<<step_grid, kBlock, 0, s>>>(a);
-      w_advance_kernel<<<1, 1, 0, s>>>(a.st, a.n, policy);
-    }
-    DAWN_HIP(hipStreamEndCapture(s, &graph));
-    hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    DAWN_HIP(e);
-    ws->graphs[key] = exec;
-  }
+  // Steps per wait: what the last batch took and the one that finds the
+  // frontier empty, so that one read of the done flag usually suffices.
+  const int chunk = ws->last_steps > 0 ? std::min(256, ws->last_steps + 1) : kWChunk;
 
   float total_ms = 0.f;
   std::vector<unsigned long long> h_sums(3 * 64);
@@ -605,10 +648,14 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
     DAWN_HIP(hipMemcpyAsync(ws->batch.p, ws->h_batch, sizeof(WBatch), hipMemcpyHostToDevice, s));
     DAWN_HIP(hipEventRecord(ws->ev0, s));
     w_fill_kernel<L><<<fill_grid, kBlock, 0, s>>>(a);
-    w_seed_kernel<L><<<1, 64, 0, s>>>(a);
+    w_seed_kernel<L><<<(unsigned)lanes, kBlock, 0, s>>>(a);
     int64_t launched = 0;
     for (;;) {
-      DAWN_HIP(hipGraphLaunch(exec, s));
+      for (int i = 0; i < chunk; i++) {
+        const int k = (int)(launched + i);
+        if (wide) w_step_kernel<L, L >= 32><<<step_grid, kBlock, 0, s>>>(a, k);
+        else w_step_kernel<L, L >= 64><<<step_grid, kBlock, 0, s>>>(a, k);
+      }
       launched += chunk;
       DAWN_HIP(hipMemcpyAsync(ws->h_state, ws->st.p, sizeof(WState), hipMemcpyDeviceToHost, s));
       DAWN_HIP(hipStreamSynchronize(s));
@@ -631,15 +678,15 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
                          hipMemcpyDeviceToHost));
     for (int i = 0; i < lanes; i++)
       if (sums) sums[b0 + i] = (int64_t)h_sums[i];
-    ws->last_steps = ws->h_state->step;
+    ws->last_steps = ws->h_state->steps;
     if (stats) {
       for (int i = 0; i < lanes; i++) {
         stats->vertices_reached += (int64_t)h_sums[64 + i];
         stats->edges_reached += (int64_t)h_sums[128 + i];
       }
       stats->batches += 1;
-      stats->steps += ws->h_state->step;
-      stats->mode_steps[DAWN_MODE_PUSH] += ws->h_state->step - ws->h_state->pull_steps;
+      stats->steps += ws->h_state->steps;
+      stats->mode_steps[DAWN_MODE_PUSH] += ws->h_state->steps - ws->h_state->pull_steps;
       stats->mode_steps[DAWN_MODE_PULL] += ws->h_state->pull_steps;
     }
   }

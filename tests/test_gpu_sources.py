@@ -89,3 +89,31 @@ def test_unweighted_long_levels(orc):
     assert np.array_equal(dist, odist) and np.array_equal(sums, osums)
     assert np.array_equal(g.closeness(src)[1], osums)
     g.close()
+
+
+@pytest.mark.parametrize("count", [1, 8, 16, 20, 32, 40, 64, 70])
+@pytest.mark.parametrize("kind", ["grid", "rmat", "directed"])
+def test_weighted_lanes(orc, kind, count):
+    """The engine of lanes (knobs set, and forced modes): every record width,
+    light lists, heavy vertices by chunks, in-edges of a directed graph,
+    zero weights, hub sources."""
+    print(f"case: {kind}, {count} sources", flush=True)
+    rng = np.random.default_rng(count)
+    if kind == "grid":
+        h = dawn.HostGraph.grid(70, 0.02, 3, weighted=True)
+    elif kind == "rmat":
+        h = dawn.HostGraph.rmat(12, 16, 4, weighted=True)
+    else:
+        u, v = rng.integers(0, 3001, 40_000) % rng.integers(1, 3001, 40_000), rng.integers(0, 3001, 40_000)
+        h = dawn.HostGraph.from_edges(3001, u.astype(np.int32), v.astype(np.int32),
+                                      rng.integers(0, 90, 40_000).astype(np.int32), symmetrize=False)
+    g = dawn.Graph(h)
+    g.set_knobs()
+    src = rng.integers(0, h.n, count).astype(np.int32)
+    src[0] = int(np.argmax(h.degrees()))
+    odist, osums, _, _ = orc.mssp(h.row_ptr, h.col, h.weight, src)
+    for p in ("fixed", "push", "pull"):
+        dist, sums = g.mssp(src, policy=p)
+        assert np.array_equal(dist, odist), p
+        assert np.array_equal(sums, osums), p
+    g.close()
