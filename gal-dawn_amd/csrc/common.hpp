@@ -130,12 +130,13 @@ struct dawn_graph {
   int32_t* hc_beg = nullptr;
   int32_t* hc_end = nullptr;
   int64_t num_hc = 0;
+  int64_t num_hv = 0;             // heavy vertices: their first chunks come first
   // Same for out-edge lists (dense top-down step).  Alias the hc_* arrays
   // for undirected graphs.
   int32_t* oc_v = nullptr;
   int32_t* oc_beg = nullptr;
   int32_t* oc_end = nullptr;
-  int64_t num_oc = 0;
+  int64_t num_oc = 0, num_ov = 0;
   std::vector<int32_t> h_row_ptr; // host copy of offsets (degrees for drivers)
   std::vector<int32_t> h_in_row_ptr;  // host CSC offsets (directed graphs)
   dawn::TuneKnobs knobs;
@@ -167,7 +168,7 @@ struct MsView {
   int32_t* in_col = nullptr;
   int32_t* perm = nullptr;
   int32_t *hc_v = nullptr, *hc_beg = nullptr, *hc_end = nullptr;
-  int64_t num_hc = 0;
+  int64_t num_hc = 0, num_hv = 0;
   int32_t *oc_v = nullptr, *oc_beg = nullptr, *oc_end = nullptr;
   int64_t num_oc = 0;
 };

@@ -75,19 +75,28 @@ void free_chunks(dawn_graph* g) {
 }  // namespace
 
 // Chunk list of the rows of `rp` with at least `heavy` entries, cut into
-// pieces of at most `chunk`: (row, first, end) triples on the device.
+// pieces of at most `chunk`: (row, first, end) triples on the device.  The
+// first chunks of all rows come first, then the second ones, and so on: a
+// pull's first chunk of a row (its hubs) often finds all that is missing, and
+// the later ones, reached after it, find the row complete.  *rows: the number
+// of first chunks.
 int build_chunk_list(const std::vector<int32_t>& rp, int heavy, int chunk, int32_t** dv,
-                     int32_t** db, int32_t** de, int64_t* count) {
-  std::vector<int32_t> hv, hb, he;
+                     int32_t** db, int32_t** de, int64_t* count, int64_t* rows) {
+  std::vector<int32_t> hv, hb, he, left;
   const int32_t n = (int32_t)rp.size() - 1;
-  for (int32_t v = 0; v < n; v++) {
-    const int32_t b = rp[v], e = rp[v + 1];
-    if (e - b < heavy) continue;
-    for (int32_t k = b; k < e; k += chunk) {
+  for (int32_t v = 0; v < n; v++)
+    if (rp[v + 1] - rp[v] >= heavy) left.push_back(v);
+  *rows = (int64_t)left.size();
+  for (int64_t at = 0; !left.empty(); at += chunk) {
+    size_t keep = 0;
+    for (const int32_t v : left) {
+      const int64_t b = rp[v] + at, e = rp[v + 1];
       hv.push_back(v);
-      hb.push_back(k);
-      he.push_back(std::min(e, k + chunk));
+      hb.push_back((int32_t)b);
+      he.push_back((int32_t)std::min(e, b + chunk));
+      if (b + chunk < e) left[keep++] = v;
     }
+    left.resize(keep);
   }
   *count = (int64_t)hv.size();
   DAWN_TRY(upload_i32(dv, hv));
@@ -101,15 +110,16 @@ int build_chunks(dawn_graph* g) {
   free_chunks(g);
   const int heavy = g->knobs.heavy_degree, chunk = g->knobs.pull_chunk;
   DAWN_TRY(build_chunk_list(g->directed ? g->h_in_row_ptr : g->h_row_ptr, heavy, chunk, &g->hc_v,
-                            &g->hc_beg, &g->hc_end, &g->num_hc));
+                            &g->hc_beg, &g->hc_end, &g->num_hc, &g->num_hv));
   if (g->directed) {
     DAWN_TRY(build_chunk_list(g->h_row_ptr, heavy, chunk, &g->oc_v, &g->oc_beg, &g->oc_end,
-                              &g->num_oc));
+                              &g->num_oc, &g->num_ov));
   } else {
     g->oc_v = g->hc_v;
     g->oc_beg = g->hc_beg;
     g->oc_end = g->hc_end;
     g->num_oc = g->num_hc;
+    g->num_ov = g->num_hv;
   }
   return DAWN_OK;
 }

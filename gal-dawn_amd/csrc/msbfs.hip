@@ -115,6 +115,7 @@ struct MsArgs {
   const int32_t* hc_beg;
   const int32_t* hc_end;
   int64_t num_hc;
+  int64_t num_hv;         // heavy vertices: the first chunks, one each
   const int32_t* oc_v;    // heavy out-edge chunks (dense top-down)
   const int32_t* oc_beg;
   const int32_t* oc_end;
@@ -915,7 +916,18 @@ __global__ void __launch_bounds__(kBlock) ms_pull_kernel(MsArgs a) {
   }
   // Heavy vertices: their in-edge lists are cut into chunks of at most
   // knobs.pull_chunk edges, one wave per chunk (lane pairs per edge at
-  // W = 16), merged with atomicOr.
+  // W = 16), merged with atomicOr.  The lists hold the hubs first: where the
+  // first 64 edges of a chunk hold kFullHits frontier vertices the wave looks
+  // whether they found all that is missing (about a hundred lane exchanges, the
+  // time of 64 records) and leaves the rest of the chunk.
+  constexpr int R = 4;  // rounds of 64 edges whose columns are in flight
+  constexpr int kFullHits = 24;
+  auto all_found = [](const uint64_t (&p)[HW], const uint64_t (&want)[HW]) {
+    uint64_t lack = 0;
+#pragma unroll
+    for (int t = 0; t < HW; t++) lack |= want[t] & ~wave_or_mod<TPV>(p[t]);
+    return __ballot(lack != 0) == 0ull;
+  };
   const int64_t wave = (int64_t)(blockIdx.x * kBlock + threadIdx.x) / kWave;
   const int64_t nwaves = (int64_t)gridDim.x * (kBlock / kWave);
   for (int64_t c = wave; c < a.num_hc; c += nwaves) {  // wave-uniform
@@ -939,14 +951,29 @@ __global__ void __launch_bounds__(kBlock) ms_pull_kernel(MsArgs a) {
     const int he = a.hc_end[c];
     uint64_t part[HW] = {};
     if constexpr (TPV == 1) {
-      for (int k = a.hc_beg[c] + lane; k < he; k += kWave) {
-        const int32_t u = a.in_col[k];
-        if ((fb[u >> 5] >> (u & 31)) & 1u) {
-          uint64_t f[HW];
-          load_words<HW>(prev + (int64_t)u * W, f);
+      for (int k0 = a.hc_beg[c]; k0 < he; k0 += R * kWave) {  // wave-uniform
+        int32_t u[R];
 #pragma unroll
-          for (int t = 0; t < HW; t++) part[t] |= f[t];
+        for (int r = 0; r < R; r++) {
+          const int k = k0 + r * kWave + lane;
+          u[r] = k < he ? a.in_col[k] : -1;
         }
+        uint32_t fw[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) fw[r] = u[r] >= 0 ? fb[u[r] >> 5] : 0u;
+        bool full = false;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          const bool hit = u[r] >= 0 && ((fw[r] >> (u[r] & 31)) & 1u);
+          if (hit && !full) {
+            uint64_t f[HW];
+            load_words<HW>(prev + (int64_t)u[r] * W + h * HW, f);
+#pragma unroll
+            for (int t = 0; t < HW; t++) part[t] |= f[t];
+          }
+          if (r == 0 && k0 + kWave < he && __popcll(__ballot(hit)) >= kFullHits) full = all_found(part, miss);
+        }
+        if (full) break;
       }
     } else {
       // Split records: every lane probes one in-edge (64 per round), the
@@ -955,7 +982,6 @@ __global__ void __launch_bounds__(kBlock) ms_pull_kernel(MsArgs a) {
       // Sparse frontiers cost one probe per edge, not one per lane pair.
       // The column reads and bitmap probes of R rounds are issued before
       // any is examined, so a wave waits once per R*64 edges, not per round.
-      constexpr int R = 8;
       int* hits = s_hits + (threadIdx.x / kWave) * kWave;
       for (int k0 = a.hc_beg[c]; k0 < he; k0 += R * kWave) {  // wave-uniform
         int32_t u[R];
@@ -967,6 +993,7 @@ __global__ void __launch_bounds__(kBlock) ms_pull_kernel(MsArgs a) {
         uint32_t fw[R];
 #pragma unroll
         for (int r = 0; r < R; r++) fw[r] = u[r] >= 0 ? fb[u[r] >> 5] : 0u;
+        bool full = false;
 #pragma unroll
         for (int r = 0; r < R; r++) {
           const bool hit = u[r] >= 0 && ((fw[r] >> (u[r] & 31)) & 1u);
@@ -985,7 +1012,9 @@ __global__ void __launch_bounds__(kBlock) ms_pull_kernel(MsArgs a) {
             }
           }
           wave_lds_sync();  // the list is rewritten by the next round
+          if (r == 0 && k0 + kWave < he && nh >= kFullHits && (full = all_found(part, miss))) break;
         }
+        if (full) break;
       }
     }
 #pragma unroll
@@ -1135,8 +1164,7 @@ __global__ void __launch_bounds__(kBlock) ms_finalize_kernel(MsArgs a) {
 
 // Fold of a pull step's heavy vertices (in-degree >= knobs.heavy_degree),
 // whose chunks merged their arrivals in next[] (the pull kernel folded the
-// light ones): one group of TPV threads per chunk entry, acting on the
-// first chunk of each vertex not yet done.  Same arithmetic as the
+// light ones): one group of TPV threads per heavy vertex not yet done.  Same arithmetic as the
 // finalize pass; bitmap bits are OR-ed into the words the pull wrote.
 template <int W>
 __global__ void __launch_bounds__(kBlock) ms_fold_heavy_kernel(MsArgs a) {
@@ -1156,18 +1184,15 @@ __global__ void __launch_bounds__(kBlock) ms_fold_heavy_kernel(MsArgs a) {
 #pragma unroll
   for (int i = 0; i < WPV; i++) alive_prev[i] = al[sub * WPT + i];
   MsAcc<W, WPV> acc;
-  // Pull step: the pull kernel folded the light vertices.  Fold the heavy
-  // ones (merged by their chunks in next[]): one group of TPV threads per
-  // chunk entry, acting on the first chunk of each vertex not yet done.
   const int64_t gstride = (int64_t)gridDim.x * (kBlock / TPV);
   for (int64_t cb = (int64_t)blockIdx.x * (kBlock / TPV) + (threadIdx.x / kWave) * (kWave / TPV);
-       cb < a.num_hc; cb += gstride) {  // wave-uniform
+       cb < a.num_hv; cb += gstride) {  // wave-uniform
     const int64_t c = cb + lane / TPV;
     int32_t v = 0;
     bool work = false;
-    if (c < a.num_hc) {
+    if (c < a.num_hv) {
       v = a.hc_v[c];
-      work = (c == 0 || a.hc_v[c - 1] != v) && !((a.done[v >> 5] >> (v & 31)) & 1u);
+      work = !((a.done[v >> 5] >> (v & 31)) & 1u);
     }
     uint64_t nx[WPV], sv[WPV], nw[WPV];
 #pragma unroll
@@ -1711,6 +1736,7 @@ MsArgs make_args(dawn_graph* g, MsWorkspace* ws) {
   a.hc_beg = vw ? vw->hc_beg : g->hc_beg;
   a.hc_end = vw ? vw->hc_end : g->hc_end;
   a.num_hc = vw ? vw->num_hc : g->num_hc;
+  a.num_hv = vw ? vw->num_hv : g->num_hv;
   a.oc_v = vw ? vw->oc_v : g->oc_v;
   a.oc_beg = vw ? vw->oc_beg : g->oc_beg;
   a.oc_end = vw ? vw->oc_end : g->oc_end;

@@ -23,7 +23,7 @@ namespace dawn {
 
 int upload_i32(int32_t** dst, const std::vector<int32_t>& src);
 int build_chunk_list(const std::vector<int32_t>& rp, int heavy, int chunk, int32_t** dv,
-                     int32_t** db, int32_t** de, int64_t* count);
+                     int32_t** db, int32_t** de, int64_t* count, int64_t* rows);
 
 namespace {
 
@@ -141,11 +141,12 @@ int ms_view_ensure(dawn_graph* g) {
   }
   const int heavy = g->knobs.heavy_degree, chunk = g->knobs.pull_chunk;
   if ((rc = build_chunk_list(g->directed ? view->h_in_row_ptr : view->h_row_ptr, heavy, chunk,
-                             &view->hc_v, &view->hc_beg, &view->hc_end, &view->num_hc)))
+                             &view->hc_v, &view->hc_beg, &view->hc_end, &view->num_hc, &view->num_hv)))
     return fail(rc);
   if (g->directed) {
+    int64_t num_ov = 0;
     if ((rc = build_chunk_list(view->h_row_ptr, heavy, chunk, &view->oc_v, &view->oc_beg,
-                               &view->oc_end, &view->num_oc)))
+                               &view->oc_end, &view->num_oc, &num_ov)))
       return fail(rc);
   } else {
     view->oc_v = view->hc_v;
