@@ -480,7 +480,14 @@ inline unsigned grid_for(int64_t items, int per_block = kBlock, unsigned cap = 8
 bool is_device_pointer(const void* p);
 
 // (Re)builds the heavy chunk lists of g from g->knobs (graph_dev.hip).
-int build_chunks(dawn_graph* g);
+struct RowStats {
+  int32_t max_deg = 0;  // largest row
+  int64_t empty = 0;    // rows without entries
+};
+int build_chunks(dawn_graph* g, RowStats* out_rows = nullptr, RowStats* in_rows = nullptr);
+// A list of row chunks (graph_dev.hip) from offsets on the device.
+int chunk_list_device(const int32_t* rp, int32_t n, int heavy, int chunk, hipStream_t s, int32_t** dv,
+                      int32_t** db, int32_t** de, int64_t* count, int64_t* rows, RowStats* stats);
 // Drops captured step graphs (their launch shapes depend on the knobs).
 void invalidate_graphs(dawn_graph* g);
 // Knobs cached for the graph's class, if any (tune.hip).

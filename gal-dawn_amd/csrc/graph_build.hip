@@ -37,7 +37,6 @@
 
 namespace dawn {
 
-int build_chunks(dawn_graph* g);
 int validate_csr(const dawn_csr* csr);
 
 namespace {
@@ -579,6 +578,100 @@ int compact(const uint64_t* keys, const int32_t* w, int64_t E, int dedup, int vb
   return DAWN_OK;
 }
 
+// ---- degrees and chunk lists -------------------------------------------------
+
+// Per tile of kScanTile rows: rows of at least `heavy` entries (hv), their
+// chunks beyond the first (ex); over all rows the largest degree and the
+// number of empty rows.
+__global__ void __launch_bounds__(kBlock) row_count_kernel(const int32_t* rp, int32_t n, int heavy,
+                                                           int chunk, uint32_t* hv, uint32_t* ex,
+                                                           unsigned* max_deg, unsigned* empty) {
+  const int64_t t0 = (int64_t)blockIdx.x * kScanTile;
+  uint32_t h = 0, x = 0, z = 0;
+  int32_t big = 0;
+#pragma unroll
+  for (int r = 0; r < kScanPer; r++) {
+    const int64_t v = t0 + r * kBlock + threadIdx.x;
+    if (v >= n) continue;
+    const int32_t d = rp[v + 1] - rp[v];
+    big = max(big, d);
+    z += d == 0;
+    if (d < heavy) continue;
+    h++;
+    x += (uint32_t)((d - 1) / chunk);
+  }
+  uint32_t th, tx, tz;
+  (void)block_excl_scan(h, &th);
+  (void)block_excl_scan(x, &tx);
+  (void)block_excl_scan(z, &tz);
+  for (int o = 32; o >= 1; o >>= 1) big = max(big, __shfl_xor(big, o));
+  if (lane_id() == 0 && big) atomicMax(max_deg, (unsigned)big);
+  if (threadIdx.x == 0) {
+    hv[blockIdx.x] = th;
+    ex[blockIdx.x] = tx;
+    if (tz) atomicAdd(empty, tz);
+  }
+}
+
+// The lists: first chunks of the heavy rows in row order, then the others,
+// row by row.  hv / ex: the tiles' first positions.
+__global__ void __launch_bounds__(kBlock) row_chunks_kernel(const int32_t* rp, int32_t n, int heavy,
+                                                            int chunk, const uint32_t* hv,
+                                                            const uint32_t* ex, int32_t* cv,
+                                                            int32_t* cb, int32_t* ce) {
+  constexpr int kWaves = kBlock / kWave, kGroups = kScanPer * kWaves;
+  static_assert(kGroups <= kWave, "one wave scans the groups");
+  __shared__ uint32_t s_h[kGroups], s_x[kGroups];
+  const int tid = threadIdx.x, lane = lane_id(), wv = tid / kWave;
+  const int64_t t0 = (int64_t)blockIdx.x * kScanTile;
+  int32_t beg[kScanPer], deg[kScanPer];
+#pragma unroll
+  for (int r = 0; r < kScanPer; r++) {
+    const int64_t v = t0 + r * kBlock + tid;
+    beg[r] = v < n ? rp[v] : 0;
+    deg[r] = v < n ? rp[v + 1] - beg[r] : -1;
+  }
+  uint32_t at_h[kScanPer], at_x[kScanPer];  // within the group of 64 rows
+#pragma unroll
+  for (int r = 0; r < kScanPer; r++) {
+    const bool in = deg[r] >= heavy;
+    const uint64_t m = __ballot(in);
+    const uint32_t x = in ? (uint32_t)((deg[r] - 1) / chunk) : 0u;
+    const uint32_t inc = wave_incl_scan_u32(x);
+    at_h[r] = (uint32_t)__popcll(m & lanes_below_mask());
+    at_x[r] = inc - x;
+    if (lane == kWave - 1) {
+      s_h[r * kWaves + wv] = (uint32_t)__popcll(m);
+      s_x[r * kWaves + wv] = inc;
+    }
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const uint32_t h = lane < kGroups ? s_h[lane] : 0u, x = lane < kGroups ? s_x[lane] : 0u;
+    const uint32_t ih = wave_incl_scan_u32(h), ix = wave_incl_scan_u32(x);
+    if (lane < kGroups) {
+      s_h[lane] = hv[blockIdx.x] + ih - h;
+      s_x[lane] = ex[blockIdx.x] + ix - x;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kScanPer; r++) {
+    if (deg[r] < heavy) continue;
+    const int32_t v = (int32_t)(t0 + r * kBlock + tid), end = beg[r] + deg[r];
+    const uint32_t h = s_h[r * kWaves + wv] + at_h[r];
+    cv[h] = v;
+    cb[h] = beg[r];
+    ce[h] = deg[r] > chunk ? beg[r] + chunk : end;
+    uint32_t x = s_x[r * kWaves + wv] + at_x[r];
+    for (int64_t k = (int64_t)beg[r] + chunk; k < end; k += chunk, x++) {
+      cv[x] = v;
+      cb[x] = (int32_t)k;
+      ce[x] = (int32_t)min(k + chunk, (int64_t)end);
+    }
+  }
+}
+
 int key_bits(int32_t n) {
   int b = 1;
   while (b < 31 && (1ll << b) < (int64_t)n) b++;
@@ -715,19 +808,13 @@ int build_device(EmitArgs ea, int dedup, int32_t wmax_bound, dawn_graph** out) {
                   hipMemcpyDeviceToHost) != hipSuccess)
       return fail(DAWN_ERR_HIP);
   }
-  int32_t maxo = 0, maxi = 0;
-  int64_t z = 0;
-  const std::vector<int32_t>& ip = g->directed ? g->h_in_row_ptr : g->h_row_ptr;
-  for (int32_t v = 0; v < n; v++) {
-    maxo = std::max(maxo, g->h_row_ptr[v + 1] - g->h_row_ptr[v]);
-    maxi = std::max(maxi, ip[v + 1] - ip[v]);
-    z += ip[v + 1] == ip[v];
-  }
-  g->max_out_degree = maxo;
-  g->max_in_degree = maxi;
-  g->zero_in = z;
+  // Degree statistics come with the chunk lists: largest degrees and empty rows.
   (void)tuned_knobs_for(g, &g->knobs);
-  if ((rc = build_chunks(g))) return fail(rc);
+  RowStats out_rows, in_rows;
+  if ((rc = build_chunks(g, &out_rows, &in_rows))) return fail(rc);
+  g->max_out_degree = out_rows.max_deg;
+  g->max_in_degree = in_rows.max_deg;
+  g->zero_in = in_rows.empty;
   *out = g;
   return DAWN_OK;
 }
@@ -751,6 +838,48 @@ bool weights_ok(int32_t weighted, int32_t wmin, int32_t wmax) {
 }
 
 }  // namespace
+
+int chunk_list_device(const int32_t* rp, int32_t n, int heavy, int chunk, hipStream_t s, int32_t** dv,
+                      int32_t** db, int32_t** de, int64_t* count, int64_t* rows, RowStats* stats) {
+  const int64_t tiles = (n + (int64_t)kScanTile - 1) / kScanTile;
+  // Per tile: heavy rows, further chunks; then the largest degree, the empty rows.
+  DevBuf<uint32_t> cnt;
+  std::vector<uint32_t> h((size_t)tiles * 2 + 2);
+  const size_t bytes = sizeof(uint32_t) * h.size();
+  DAWN_TRY(cnt.alloc(h.size()));
+  DAWN_HIP(hipMemsetAsync(cnt.p, 0, bytes, s));
+  row_count_kernel<<<(unsigned)tiles, kBlock, 0, s>>>(rp, n, heavy, chunk, cnt.p, cnt.p + tiles,
+                                                      cnt.p + 2 * tiles, cnt.p + 2 * tiles + 1);
+  DAWN_HIP(hipGetLastError());
+  DAWN_HIP(hipMemcpyAsync(h.data(), cnt.p, bytes, hipMemcpyDeviceToHost, s));
+  DAWN_HIP(hipStreamSynchronize(s));
+  uint64_t at = 0;
+  for (int64_t i = 0; i < 2 * tiles; i++) {
+    if (i == tiles) *rows = (int64_t)at;
+    const uint32_t x = h[i];
+    h[i] = (uint32_t)at;
+    at += x;  // at most m
+  }
+  *count = (int64_t)at;
+  if (stats) *stats = RowStats{(int32_t)h[2 * tiles], (int64_t)h[2 * tiles + 1]};
+  for (int32_t** p : {dv, db, de}) {
+    const hipError_t e = hipMalloc((void**)p, sizeof(int32_t) * std::max<uint64_t>(at, 1));
+    if (e != hipSuccess) {
+      *p = nullptr;
+      set_hip_error(e, "hipMalloc", __FILE__, __LINE__);
+      return e == hipErrorOutOfMemory ? DAWN_ERR_OUT_OF_MEMORY : DAWN_ERR_HIP;
+    }
+  }
+  if (at) {
+    DAWN_HIP(hipMemcpyAsync(cnt.p, h.data(), sizeof(uint32_t) * 2 * (size_t)tiles, hipMemcpyHostToDevice, s));
+    row_chunks_kernel<<<(unsigned)tiles, kBlock, 0, s>>>(rp, n, heavy, chunk, cnt.p, cnt.p + tiles, *dv,
+                                                         *db, *de);
+    DAWN_HIP(hipGetLastError());
+  }
+  DAWN_HIP(hipStreamSynchronize(s));
+  return DAWN_OK;
+}
+
 }  // namespace dawn
 
 using namespace dawn;

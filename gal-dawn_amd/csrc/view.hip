@@ -22,8 +22,9 @@
 namespace dawn {
 
 int upload_i32(int32_t** dst, const std::vector<int32_t>& src);
-int build_chunk_list(const std::vector<int32_t>& rp, int heavy, int chunk, int32_t** dv,
-                     int32_t** db, int32_t** de, int64_t* count, int64_t* rows);
+int build_chunk_list(const std::vector<int32_t>& rp, const int32_t* d_rp, hipStream_t s, int heavy,
+                     int chunk, int32_t** dv, int32_t** db, int32_t** de, int64_t* count, int64_t* rows,
+                     RowStats* stats);
 
 namespace {
 
@@ -140,13 +141,14 @@ int ms_view_ensure(dawn_graph* g) {
     view->in_col = view->col;
   }
   const int heavy = g->knobs.heavy_degree, chunk = g->knobs.pull_chunk;
-  if ((rc = build_chunk_list(g->directed ? view->h_in_row_ptr : view->h_row_ptr, heavy, chunk,
-                             &view->hc_v, &view->hc_beg, &view->hc_end, &view->num_hc, &view->num_hv)))
+  if ((rc = build_chunk_list(g->directed ? view->h_in_row_ptr : view->h_row_ptr, view->in_row_ptr,
+                             g->stream, heavy, chunk, &view->hc_v, &view->hc_beg, &view->hc_end,
+                             &view->num_hc, &view->num_hv, nullptr)))
     return fail(rc);
   if (g->directed) {
     int64_t num_ov = 0;
-    if ((rc = build_chunk_list(view->h_row_ptr, heavy, chunk, &view->oc_v, &view->oc_beg,
-                               &view->oc_end, &view->num_oc, &num_ov)))
+    if ((rc = build_chunk_list(view->h_row_ptr, view->row_ptr, g->stream, heavy, chunk, &view->oc_v,
+                               &view->oc_beg, &view->oc_end, &view->num_oc, &num_ov, nullptr)))
       return fail(rc);
   } else {
     view->oc_v = view->hc_v;
