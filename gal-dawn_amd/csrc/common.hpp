@@ -161,7 +161,7 @@ namespace dawn {
 // Device arrays are in the new numbering; perm maps old ids to new ones.
 struct MsView {
   int32_t k = 0;
-  std::vector<int32_t> h_perm, h_row_ptr, h_in_row_ptr;
+  std::vector<int32_t> h_perm;
   int32_t* row_ptr = nullptr;
   int32_t* col = nullptr;
   int32_t* in_row_ptr = nullptr;  // == row_ptr / col for undirected graphs
@@ -485,6 +485,11 @@ struct RowStats {
   int64_t empty = 0;    // rows without entries
 };
 int build_chunks(dawn_graph* g, RowStats* out_rows = nullptr, RowStats* in_rows = nullptr);
+// The k vertices of largest out-degree first (descending, ties by id), the
+// others in their order: perm[old] = new, inv[new] = old, on the device.
+int hub_order_device(const dawn_graph* g, int32_t k, int32_t* perm, int32_t* inv);
+// Offsets (n + 1) of the rows in that order.
+int permuted_offsets_device(const int32_t* rp, const int32_t* inv, int32_t n, hipStream_t s, int32_t* out);
 // A list of row chunks (graph_dev.hip) from offsets on the device.
 int chunk_list_device(const int32_t* rp, int32_t n, int heavy, int chunk, hipStream_t s, int32_t** dv,
                       int32_t** db, int32_t** de, int64_t* count, int64_t* rows, RowStats* stats);

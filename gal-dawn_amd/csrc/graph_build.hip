@@ -672,6 +672,45 @@ __global__ void __launch_bounds__(kBlock) row_chunks_kernel(const int32_t* rp, i
   }
 }
 
+// ---- hub-first order ---------------------------------------------------------
+
+// Sort keys: the degree counted down from the largest, the vertex above it.
+__global__ void order_keys_kernel(const int32_t* rp, int32_t n, int32_t max_deg, uint64_t* keys,
+                                  uint32_t* rest) {
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
+       v += (int64_t)gridDim.x * blockDim.x) {
+    keys[v] = (uint64_t)v << 32 | (uint32_t)(max_deg - (rp[v + 1] - rp[v]));
+    rest[v] = 1u;
+  }
+}
+
+__global__ void order_hubs_kernel(const uint64_t* keys, int32_t k, int32_t* perm, int32_t* inv,
+                                  uint32_t* rest) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < k;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t v = (int32_t)(keys[i] >> 32);
+    perm[v] = (int32_t)i;
+    inv[i] = v;
+    rest[v] = 0u;
+  }
+}
+
+// after: the scanned `rest`, the rank of a vertex among those that are no hubs.
+__global__ void order_rest_kernel(const uint32_t* after, int32_t n, int32_t k, int32_t* perm, int32_t* inv) {
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
+       v += (int64_t)gridDim.x * blockDim.x) {
+    if ((v + 1 < n ? after[v + 1] : (uint32_t)(n - k)) == after[v]) continue;  // a hub
+    perm[v] = k + (int32_t)after[v];
+    inv[k + after[v]] = (int32_t)v;
+  }
+}
+
+__global__ void order_degrees_kernel(const int32_t* rp, const int32_t* inv, int32_t n, uint32_t* out) {
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r <= n;
+       r += (int64_t)gridDim.x * blockDim.x)
+    out[r] = r < n ? (uint32_t)(rp[inv[r] + 1] - rp[inv[r]]) : 0u;
+}
+
 int key_bits(int32_t n) {
   int b = 1;
   while (b < 31 && (1ll << b) < (int64_t)n) b++;
@@ -838,6 +877,38 @@ bool weights_ok(int32_t weighted, int32_t wmin, int32_t wmax) {
 }
 
 }  // namespace
+
+int hub_order_device(const dawn_graph* g, int32_t k, int32_t* perm, int32_t* inv) {
+  const int32_t n = g->n;
+  hipStream_t s = g->stream;
+  SortTemp t;
+  DevBuf<uint64_t> ka, kb;
+  DevBuf<uint32_t> rest;
+  DAWN_TRY(ka.alloc((size_t)n));
+  DAWN_TRY(kb.alloc((size_t)n));
+  DAWN_TRY(rest.alloc((size_t)n));
+  const unsigned grid = grid_for(n);
+  order_keys_kernel<<<grid, kBlock, 0, s>>>(g->row_ptr, n, g->max_out_degree, ka.p, rest.p);
+  DAWN_HIP(hipGetLastError());
+  bool in1 = false;
+  DAWN_TRY(radix_sort(ka.p, kb.p, nullptr, nullptr, n, weight_bits(g->max_out_degree), s, t, &in1));
+  order_hubs_kernel<<<grid_for(k), kBlock, 0, s>>>(in1 ? kb.p : ka.p, k, perm, inv, rest.p);
+  DAWN_HIP(hipGetLastError());
+  DAWN_TRY(excl_scan(rest.p, n, s, t.scan));
+  order_rest_kernel<<<grid, kBlock, 0, s>>>(rest.p, n, k, perm, inv);
+  DAWN_HIP(hipGetLastError());
+  DAWN_HIP(hipStreamSynchronize(s));
+  return DAWN_OK;
+}
+
+int permuted_offsets_device(const int32_t* rp, const int32_t* inv, int32_t n, hipStream_t s, int32_t* out) {
+  ScanTemp t;
+  order_degrees_kernel<<<grid_for((int64_t)n + 1), kBlock, 0, s>>>(rp, inv, n, (uint32_t*)out);
+  DAWN_HIP(hipGetLastError());
+  DAWN_TRY(excl_scan((uint32_t*)out, (int64_t)n + 1, s, t));
+  DAWN_HIP(hipStreamSynchronize(s));
+  return DAWN_OK;
+}
 
 int chunk_list_device(const int32_t* rp, int32_t n, int heavy, int chunk, hipStream_t s, int32_t** dv,
                       int32_t** db, int32_t** de, int64_t* count, int64_t* rows, RowStats* stats) {

@@ -14,23 +14,19 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <numeric>
 #include <vector>
 
 #include "common.hpp"
 
 namespace dawn {
 
-int upload_i32(int32_t** dst, const std::vector<int32_t>& src);
-int build_chunk_list(const std::vector<int32_t>& rp, const int32_t* d_rp, hipStream_t s, int heavy,
-                     int chunk, int32_t** dv, int32_t** db, int32_t** de, int64_t* count, int64_t* rows,
-                     RowStats* stats);
-
 namespace {
 
 // Row r of the new adjacency = row inv[r] of the old one, columns mapped
-// through perm: one wave per row, lanes stride the edges.
-__global__ void view_copy_kernel(int32_t n, const int32_t* old_rp, const int32_t* old_col,
+// through perm, the hubs (new ids below k) first: a pull finds most lanes at
+// them and leaves the row.  One wave per row, 64 edges at a time, placed by
+// ballots: hubs from the front, then the others.
+__global__ void view_copy_kernel(int32_t n, int32_t k, const int32_t* old_rp, const int32_t* old_col,
                                  const int32_t* new_rp, int32_t* new_col, const int32_t* inv,
                                  const int32_t* perm) {
   const int lane = lane_id();
@@ -38,8 +34,27 @@ __global__ void view_copy_kernel(int32_t n, const int32_t* old_rp, const int32_t
   const int64_t nwaves = (int64_t)gridDim.x * blockDim.x / kWave;
   for (int64_t r = wave; r < n; r += nwaves) {
     const int32_t o = inv[r];
-    const int32_t b = old_rp[o], e = old_rp[o + 1], nb = new_rp[r];
-    for (int32_t k = b + lane; k < e; k += kWave) new_col[nb + (k - b)] = perm[old_col[k]];
+    const int32_t b = old_rp[o], deg = old_rp[o + 1] - b, nb = new_rp[r];
+    if (deg <= kWave) {
+      const int32_t c = lane < deg ? perm[old_col[b + lane]] : 0;
+      const uint64_t in = __ballot(lane < deg), hub = __ballot(lane < deg && c < k);
+      const uint64_t mine = c < k ? hub : in & ~hub;
+      const int at = (c < k ? 0 : __popcll(hub)) + __popcll(mine & lanes_below_mask());
+      if (lane < deg) new_col[nb + at] = c;
+      continue;
+    }
+    int hubs = 0;
+    for (int j = lane; j - lane < deg; j += kWave)  // wave-uniform
+      hubs += __popcll(__ballot(j < deg && perm[old_col[b + (j < deg ? j : 0)]] < k));
+    int front = 0, back = hubs;
+    for (int j = lane; j - lane < deg; j += kWave) {
+      const int32_t c = j < deg ? perm[old_col[b + j]] : 0;
+      const uint64_t in = __ballot(j < deg), hub = __ballot(j < deg && c < k), rest = in & ~hub;
+      const int at = c < k ? front + __popcll(hub & lanes_below_mask()) : back + __popcll(rest & lanes_below_mask());
+      if (j < deg) new_col[nb + at] = c;
+      front += __popcll(hub);
+      back += __popcll(rest);
+    }
   }
 }
 
@@ -75,80 +90,55 @@ int ms_view_ensure(dawn_graph* g) {
   if (g->view) return DAWN_OK;
   const int32_t n = g->n;
   const int32_t k = std::max<int32_t>(1, n / 16);
-  std::vector<int32_t> deg(n), order(n);
-  for (int32_t v = 0; v < n; v++) deg[v] = g->h_row_ptr[v + 1] - g->h_row_ptr[v];
-  std::iota(order.begin(), order.end(), 0);
-  auto hotter = [&](int32_t x, int32_t y) { return deg[x] != deg[y] ? deg[x] > deg[y] : x < y; };
-  std::nth_element(order.begin(), order.begin() + (k - 1), order.end(), hotter);
-  std::sort(order.begin(), order.begin() + k, hotter);
-  std::vector<char> hub(n, 0);
-  for (int32_t i = 0; i < k; i++) hub[order[i]] = 1;
   MsView* view = new MsView();
   view->k = k;
-  view->h_perm.resize(n);
-  std::vector<int32_t> inv(n);
-  for (int32_t i = 0; i < k; i++) {
-    view->h_perm[order[i]] = i;
-    inv[i] = order[i];
-  }
-  int32_t next = k;
-  for (int32_t v = 0; v < n; v++)
-    if (!hub[v]) {
-      view->h_perm[v] = next;
-      inv[next++] = v;
-    }
-  auto offsets = [&](const std::vector<int32_t>& rp) {
-    std::vector<int32_t> out((size_t)n + 1);
-    out[0] = 0;
-    for (int32_t r = 0; r < n; r++) out[r + 1] = out[r] + (rp[inv[r] + 1] - rp[inv[r]]);
-    return out;
-  };
-  view->h_row_ptr = offsets(g->h_row_ptr);
-  if (g->directed) view->h_in_row_ptr = offsets(g->h_in_row_ptr);
   g->view = view;
   auto fail = [&](int rc) {
     ms_view_free(g);
     return rc;
   };
+  auto dalloc = [&](int32_t** p, int64_t count) -> int {
+    const hipError_t e = hipMalloc((void**)p, sizeof(int32_t) * std::max<int64_t>(count, 1));
+    if (e == hipSuccess) return DAWN_OK;
+    *p = nullptr;
+    set_hip_error(e, "hipMalloc", __FILE__, __LINE__);
+    return e == hipErrorOutOfMemory ? DAWN_ERR_OUT_OF_MEMORY : DAWN_ERR_HIP;
+  };
+  DevBuf<int32_t> inv;
   int rc;
-  int32_t* d_inv = nullptr;
-  if ((rc = upload_i32(&view->perm, view->h_perm)) || (rc = upload_i32(&d_inv, inv))) {
-    free_ptr(d_inv);
+  if ((rc = dalloc(&view->perm, n)) || (rc = inv.alloc((size_t)n)) ||
+      (rc = hub_order_device(g, k, view->perm, inv.p)))
     return fail(rc);
-  }
-  auto relabel = [&](const std::vector<int32_t>& new_rp, const int32_t* old_rp,
-                     const int32_t* old_col, int32_t** rp_out, int32_t** col_out) -> int {
-    DAWN_TRY(upload_i32(rp_out, new_rp));
-    const hipError_t e = hipMalloc((void**)col_out, sizeof(int32_t) * std::max<int64_t>(g->m, 1));
-    if (e != hipSuccess) {
-      *col_out = nullptr;
-      set_hip_error(e, "hipMalloc", __FILE__, __LINE__);
-      return e == hipErrorOutOfMemory ? DAWN_ERR_OUT_OF_MEMORY : DAWN_ERR_HIP;
-    }
-    view_copy_kernel<<<2048, kBlock, 0, g->stream>>>(n, old_rp, old_col, *rp_out, *col_out, d_inv,
+  view->h_perm.resize(n);
+  auto relabel = [&](const int32_t* old_rp, const int32_t* old_col, int32_t** rp_out,
+                     int32_t** col_out) -> int {
+    DAWN_TRY(dalloc(rp_out, (int64_t)n + 1));
+    DAWN_TRY(dalloc(col_out, g->m));
+    DAWN_TRY(permuted_offsets_device(old_rp, inv.p, n, g->stream, *rp_out));
+    view_copy_kernel<<<2048, kBlock, 0, g->stream>>>(n, k, old_rp, old_col, *rp_out, *col_out, inv.p,
                                                      view->perm);
     DAWN_HIP(hipGetLastError());
     return DAWN_OK;
   };
-  rc = relabel(view->h_row_ptr, g->row_ptr, g->col, &view->row_ptr, &view->col);
-  if (!rc && g->directed)
-    rc = relabel(view->h_in_row_ptr, g->in_row_ptr, g->in_col, &view->in_row_ptr, &view->in_col);
-  if (!rc && hipStreamSynchronize(g->stream) != hipSuccess) rc = DAWN_ERR_HIP;
-  free_ptr(d_inv);
+  rc = relabel(g->row_ptr, g->col, &view->row_ptr, &view->col);
+  if (!rc && g->directed) rc = relabel(g->in_row_ptr, g->in_col, &view->in_row_ptr, &view->in_col);
+  if (!rc && (hipMemcpyAsync(view->h_perm.data(), view->perm, sizeof(int32_t) * (size_t)n,
+                             hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
+              hipStreamSynchronize(g->stream) != hipSuccess))
+    rc = DAWN_ERR_HIP;
   if (rc) return fail(rc);
   if (!g->directed) {
     view->in_row_ptr = view->row_ptr;
     view->in_col = view->col;
   }
   const int heavy = g->knobs.heavy_degree, chunk = g->knobs.pull_chunk;
-  if ((rc = build_chunk_list(g->directed ? view->h_in_row_ptr : view->h_row_ptr, view->in_row_ptr,
-                             g->stream, heavy, chunk, &view->hc_v, &view->hc_beg, &view->hc_end,
-                             &view->num_hc, &view->num_hv, nullptr)))
+  if ((rc = chunk_list_device(view->in_row_ptr, n, heavy, chunk, g->stream, &view->hc_v, &view->hc_beg,
+                              &view->hc_end, &view->num_hc, &view->num_hv, nullptr)))
     return fail(rc);
   if (g->directed) {
     int64_t num_ov = 0;
-    if ((rc = build_chunk_list(view->h_row_ptr, view->row_ptr, g->stream, heavy, chunk, &view->oc_v,
-                               &view->oc_beg, &view->oc_end, &view->num_oc, &num_ov, nullptr)))
+    if ((rc = chunk_list_device(view->row_ptr, n, heavy, chunk, g->stream, &view->oc_v, &view->oc_beg,
+                                &view->oc_end, &view->num_oc, &num_ov, nullptr)))
       return fail(rc);
   } else {
     view->oc_v = view->hc_v;
