@@ -934,7 +934,8 @@ __device__ void run_weighted(const BatchArgs& a, const BatchGraph& G, const Batc
 // one edge per thread in flight.  What bounds it now is the instructions of a
 // relaxation (RMAT-17, one CU: 2 G relaxations/s of 60 VALU and 15 LDS
 // operations per wave and edge) and, for small graphs, the step's scan (3 us).
-constexpr int64_t kDistN = kLdsWords - 3;  // words, rounded up to four
+constexpr int64_t kDistN = kSourcesDistN;  // words, rounded up to four
+static_assert(kDistN + 3 <= kLdsWords, "distances");
 constexpr int64_t kBoundN = kSourcesN;     // a byte and a bit per vertex
 constexpr int64_t kSerialM = 4;            // edges of one load
 constexpr int64_t kLdsM = kSourcesMaxM;    // edges reached by 32-bit byte offsets

@@ -2350,26 +2350,26 @@ void split_live(const dawn_graph* g, const int32_t* sources, int32_t S, std::vec
 
 // Graphs whose state fits a workgroup's LDS: every source in a workgroup of its
 // own (batch.hip), 256 at a time, while that is faster than the shared steps of
-// a batch of lanes, seven launches each.  Measured (ms, lanes / workgroups):
-//   ER 4,096, 65,000 edges: 16 sources 0.47 / 0.07, 1024 0.57 / 0.18
-//   ER 16,384, 131,000 edges: 256 sources 0.57 / 0.16, 1024 0.61 / 0.46
-//   ER 60,000, 240,000 edges: 256 sources 0.74 / 0.44, 512 0.89 / 0.79, 1024 1.1 / 1.4
-//   ER 65,536, 1 M edges: 65 sources 0.53 / 0.37, 256 0.62 / 0.35, 1024 0.72 / 1.1
-//   RMAT-15, 0.9 M edges: 256 sources 0.71 / 0.22, 512 0.78 / 0.36
-//   grid 250 x 250: 64 sources 1.3 / 0.34, 1024 2.6 / 1.3
-//   RMAT-17, 3.7 M edges: 64 sources 0.67 / 0.70, 256 0.80 / 0.72
-// A source costs its edges and about 16 edges' time per vertex (levels of few
-// vertices, the row); a graph of more than kSourcesWork of those or kSourcesM
-// edges, or a call of more than kSourcesCall, goes to the lanes, and so do
-// forced modes and graphs whose knobs were set.
-constexpr int64_t kSourcesWork = 1 << 22, kSourcesCall = 1 << 30, kSourcesM = 1 << 21;
-constexpr int32_t kSourcesS = 1024;
+// a batch of lanes, seven launches each.  Measured (ms, workgroups / lanes):
+//   ER 1,000, degree 8: 1 source 0.08 / 0.28, 1024 0.20 / 0.48
+//   ER 16,384, degree 8: 256 sources 0.16 / 0.43, 1024 0.47 / 0.59
+//   ER 32,768, degree 16: 256 sources 0.26 / 0.42, 512 0.47 / 0.51, 1024 0.82 / 0.61
+//   ER 65,536, degree 8: 64 sources 0.37 / 0.39, 256 0.40 / 0.50, 512 0.72 / 0.62
+//   ER 100,000, degree 8: 64 sources 0.54 / 0.43, 256 0.58 / 0.56
+//   RMAT-15: 256 sources 0.22 / 0.51, 512 0.34 / 0.63; RMAT-16: 64 0.35 / 0.44
+//   grid 250 x 250: 64 sources 0.34 / 1.3, 512 0.70 / 1.9; 360 x 360: 64 0.61 / 1.4
+// One round of 256 sources: up to kSourcesVerts vertices (short lists, many
+// levels: the LDS's limit) and kSourcesM edges.  More rounds: while their
+// work, edges and 16 per vertex (levels of few vertices, the row), stays below
+// kSourcesWork.  Forced modes and graphs whose knobs were set keep the lanes.
+constexpr int64_t kSourcesVerts = 80000, kSourcesM = 1 << 21, kSourcesWork = 2600000;
+constexpr int32_t kSourcesRound = 256, kSourcesShortDeg = 12;
 
 static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
   if (g->lanes_only || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
-  const int64_t work = g->m + 16 * (int64_t)g->n;
-  return g->n <= kSourcesN && g->m <= kSourcesM && work <= kSourcesWork && S <= kSourcesS &&
-         S * work <= kSourcesCall;
+  if (g->n > (g->max_out_degree <= kSourcesShortDeg ? kSourcesN : kSourcesVerts) || g->m > kSourcesM) return false;
+  const int64_t rounds = ((int64_t)S + kSourcesRound - 1) / kSourcesRound;
+  return rounds <= 1 || rounds * (g->m + 16 * (int64_t)g->n) <= kSourcesWork;
 }
 
 // live: the sources that take lanes in batches of 64 words, as the lanes count.

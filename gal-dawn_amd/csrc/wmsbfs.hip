@@ -697,22 +697,26 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
 }  // namespace
 
 // Graphs whose state fits a workgroup's LDS: every source in a workgroup of
-// its own (batch.hip), 256 at a time, instead of 64 lanes that share steps of
-// four launches.  Measured (ms, lanes / workgroups):
-//   ER 16,384, 131,000 edges: 1 source 1.04 / 0.24, 64 3.2 / 0.27, 1024 51 / 0.97
-//   ER 60,000, 480,000 edges: 1 source 1.4 / 1.0, 64 3.5 / 1.05, 1024 57 / 5.9
-//   grid 360 x 360: 1 source 2.3 / 1.7, 64 4.7 / 1.9, 1024 75 / 8.8
-// A workgroup relaxes 1 to 1.5 G edges/s alone, so that few sources of a graph
-// of many edges leave the chip idle:
-//   ER 130,000, 3.9 M edges: 8 sources 2.9 / 3.5, 16 3.7 / 3.4, 64 11 / 3.5
-//   RMAT-17, 3.7 M edges: 8 sources 2.7 / 4.5, 16 4.2 / 4.3, 64 23 / 6.6
-// hence the two lines below.  A forced mode is one of the lanes' steps.
-constexpr int64_t kSourcesM = 1500000;  // edges up to which any number of sources
-constexpr int32_t kSourcesS = 32;       // sources from which any number of edges
+// its own (batch.hip), 256 at a time, instead of 64 lanes that share steps.
+// Measured (ms, workgroups / lanes):
+//   ER 16,384, degree 8: 1 source 0.25 / 0.42, 64 0.27 / 0.65, 256 0.29 / 2.9
+//   ER 32,768, degree 16: 1 source 0.50 / 0.54, 64 0.56 / 1.05, 256 0.59 / 4.1
+//   RMAT-14, 0.43 M edges: 1 source 0.54 / 0.61, 64 0.61 / 3.2
+//   RMAT-15, 0.88 M edges: 8 sources 0.97 / 0.72, 16 1.01 / 1.15, 64 1.03 / 4.0
+//   ER 65,536, degree 8: 32 sources 1.12 / 0.91, 64 1.13 / 1.21, 256 1.65 / 4.9
+//   ER 130,000, degree 3: 32 sources 1.51 / 1.02, 64 1.54 / 1.38, 256 2.0 / 5.4
+//   grid 360 x 360: 32 sources 1.84 / 1.37, 64 1.85 / 2.6, 256 2.3 / 9.6
+// With the distances in LDS (up to kSourcesDistN vertices) the lines are
+// kSourcesM edges and kSourcesS sources; with bounds there and distances in
+// memory, more sources than one batch of lanes.  A forced mode is one of the
+// lanes' steps, and knobs set by hand are theirs.
+constexpr int64_t kSourcesM = 600000;
+constexpr int32_t kSourcesS = 16;
 
 static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
   if (g->lanes_only || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
-  return g->n <= kSourcesN && (g->m <= kSourcesM || (S >= kSourcesS && g->m < kSourcesMaxM));
+  if (g->n > kSourcesN || g->m >= kSourcesMaxM) return false;
+  return g->n <= kSourcesDistN ? g->m <= kSourcesM || S >= kSourcesS : S > 64;
 }
 
 static int run_lanes(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64_t* sums,

@@ -211,14 +211,13 @@ int dawn_bfs_noalloc(const dawn_graph* g, int32_t source, int32_t* dist,
                      int32_t policy, dawn_stats* stats);
 
 /* Multi-source shortest paths.  Unweighted graphs run 64*W sources per
- * bit-packed batch (W = the lane-words knob, up to 16: 1024 sources), or, on
- * small graphs (up to 134,000 vertices and 2 million edges, up to 1024
- * sources, fixed and learned policies, knobs not set by hand), a workgroup
- * per source; its counts are those of the batches (steps all push);
+ * bit-packed batch (W = the lane-words knob, up to 16: 1024 sources);
  * weighted graphs run the batched min-plus engine, up to 64 sources per
- * batch, or, where a graph's state fits a workgroup's LDS (up to 134,000
- * vertices; up to 1.5 million edges, or 32 sources), a
- * workgroup per source.
+ * batch.  On graphs whose state fits a workgroup's LDS (up to 80,000 vertices
+ * and 2 million edges unweighted, 134,000 vertices weighted) a call that is
+ * faster so runs a workgroup per source instead (fixed and learned policies,
+ * knobs not set by hand); its counts are those of the batches, its steps
+ * count as push, its frontier edges per source.
  * sources are taken modulo n (reference: msource[i] % rows, mssp.cpp:15);
  * isolated sources are skipped (dist row left INF except dist[src]=0, sum 0).
  * dist: S*n int32 row-major (host or device), or NULL to keep only sums
