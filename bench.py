@@ -160,10 +160,8 @@ def summarize_rocprof(out_dir, profiles_dir):
 def summarize_rocprof_c2(out_dir):
     """Kernel table and per-step times of the rocprofv3 kernel trace of
     `--quick-profile-c2` (one SSSP and one 16-source MSSP on the weighted
-    2048^2 grid, each run twice: the first run captures the step graphs).
-    A captured weighted step launches the push, pull, clear and advance
-    kernels; the mode not chosen returns at once.  Captured chunks end with
-    steps that return at once after the traversal is done."""
+    2048^2 grid, each run twice: the first run does not know the depth).  A
+    step is one kernel; launches past the end of a traversal return at once."""
     import csv
     import glob
 
@@ -187,25 +185,17 @@ def summarize_rocprof_c2(out_dir):
                      f"{float(r['AverageNs']) / 1e3:.1f} | {float(r['MaxNs']) / 1e3:.1f} | {len(w)} | "
                      f"{(sum(w) / len(w)) if w else 0:.1f} |")
     # Per-step times of the second (timed) run of each traversal.
-    ss = [dur(r) for r in trace if "sssp_expand_kernel" in r["Kernel_Name"]]
-    half = len(ss) // 2
-    steps_ss = ss[half:]
-    runs, cur = [], None
-    for r in trace:
-        k = r["Kernel_Name"]
-        if "w_fill_kernel" in k:
-            cur = []
-            runs.append(cur)
-        elif cur is not None and ("w_step_kernel" in k or "w_pull_kernel" in k):
-            cur.append(("push" if "w_step_kernel" in k else "pull", dur(r)))
-        elif "w_final_kernel" in k:
-            cur = None
-    steps_ms = []
-    for i in range(0, len(runs[-1]), 2):
-        (m1, t1), (m2, t2) = runs[-1][i], runs[-1][i + 1]
-        steps_ms.append(("P" if t2 > t1 else "S") + f"{max(t1, t2):.0f}")
-    return "\n".join(lines), {"sssp_step_us": [round(x) for x in steps_ss],
-                              "mssp16_step_us": steps_ms}
+    def last_run(fill, step):
+        runs = []
+        for r in trace:
+            if fill in r["Kernel_Name"]:
+                runs.append([])
+            elif runs and step in r["Kernel_Name"]:
+                runs[-1].append(round(dur(r)))
+        return runs[-1]
+
+    return "\n".join(lines), {"sssp_step_us": last_run("ss_fill_kernel", "ss_step_kernel"),
+                              "mssp16_step_us": last_run("w_fill_kernel", "w_step_kernel")}
 
 
 def host_cpu():

@@ -1,7 +1,8 @@
 // Step scheduler shared by the frontier engines: per-level counters, the
 // per-step feature vector, the GAPBS alpha/beta rule and MLP inference.
-// The decision runs on the device (one wave) so that step loops can be
-// captured in a hipGraph without host round trips.
+// The decision runs on the device so that steps follow each other without
+// host round trips: one wave between the batched engine's captured steps,
+// every workgroup for itself in the single-source ones.
 #pragma once
 #include <hip/hip_runtime.h>
 
