@@ -1364,6 +1364,7 @@ __global__ void __launch_bounds__(BS) sources_kernel(SourcesArgs a) {
 }
 
 // The same unweighted: levels in LDS (n <= kSourcesN), one lane.
+static_assert((kSourcesN + 31) / 32 * 4 + kSourcesN <= (int64_t)kLdsWords * 4, "a bit and a level each");
 struct BfsSourcesArgs {
   BatchGraph G;
   const int32_t* sources;

@@ -76,3 +76,19 @@ def test_hubs(orc, leaves):
     u, v = np.concatenate([ru, np.full(leaves, 7, np.int32)]), np.concatenate([r.col, leaf])
     w = np.concatenate([r.weight, (leaf % 977).astype(np.int32)])
     check(orc, dawn.HostGraph.from_edges(r.n + leaves, u, v, w), [7, r.n + 3])
+
+
+def test_mixed_batch(orc):
+    """Weighted and unweighted graphs of every state in one batch."""
+    print("case: 6 graphs, weighted and not, in LDS and in memory, 3 sources each", flush=True)
+    hosts = [dawn.HostGraph.grid(60, 0.01, 1, weighted=True), dawn.HostGraph.er(2_000, 9.0, 2),
+             dawn.HostGraph.er(45_000, 6.0, 3, weighted=True), dawn.HostGraph.rmat(12, 16, 4),
+             dawn.HostGraph.er(140_000, 3.0, 5, weighted=True), dawn.HostGraph.er(1_220_000, 2.0, 6)]
+    graphs = [dawn.Graph(h) for h in hosts]
+    src = np.concatenate([np.flatnonzero(h.degrees() > 0)[[0, 7, -1]] for h in hosts]).astype(np.int32)
+    rows, _ = dawn.batch_mssp(graphs, src, 3)
+    for i, h in enumerate(hosts):
+        want = orc.mssp(h.row_ptr, h.col, h.weight if h.weighted else None, src[3 * i:3 * i + 3])[0]
+        for j in range(3):
+            assert np.array_equal(rows[i][j], want[j]), (i, j)
+        graphs[i].close()
