@@ -1429,6 +1429,8 @@ __global__ void __launch_bounds__(BS) bfs_sources_kernel(BfsSourcesArgs a) {
 
 }  // namespace
 
+constexpr int32_t kSourcesLaunch = 1 << 16;  // sources of one launch
+
 // Sources (reduced mod n) a workgroup each, for graphs whose state fits its
 // LDS; the engines of lanes say when.  acc: per source the distance sum, the
 // vertices reached, their out-degrees, the steps (levels); device time in *ms.
@@ -1440,8 +1442,8 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
   int cus = 0;
   DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
   hipStream_t s = g->stream;
-  // Rows go to the caller's device memory; host rows in blocks of a full launch.
-  const int32_t per = dist && !dev_out ? std::min<int32_t>(S, cus) : S;
+  // Rows go to the caller's device memory; host rows in blocks of a workgroup per CU.
+  const int32_t per = std::min<int32_t>(S, dist && !dev_out ? cus : kSourcesLaunch);
   const int grid = std::max(1, std::min<int>(per, cus));
   const size_t gn = (size_t)grid * g->n;
   const BatchGraph G{g->n, g->weighted, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col,

@@ -117,3 +117,17 @@ def test_weighted_lanes(orc, kind, count):
         assert np.array_equal(dist, odist), p
         assert np.array_equal(sums, osums), p
     g.close()
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_more_sources_than_a_launch(orc, weighted):
+    print(f"case: path of 5 vertices, 70,000 sources, weighted={weighted}", flush=True)
+    u = np.arange(4, dtype=np.int32)
+    h = dawn.HostGraph.from_edges(5, u, u + 1, np.array([3, 1, 4, 1], np.int32) if weighted else None)
+    g = dawn.Graph(h)
+    src = (np.arange(70_000) * 7 % 5).astype(np.int32)
+    rows, sums, st = device_rows(g, src, "fixed")
+    odist, osums, _, _ = orc.mssp(h.row_ptr, h.col, h.weight if weighted else None, np.arange(5, dtype=np.int32))
+    assert np.array_equal(rows, odist[src]) and np.array_equal(sums, osums[src])
+    assert st["vertices_reached"] == 5 * len(src)
+    g.close()
