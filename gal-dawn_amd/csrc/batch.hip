@@ -185,6 +185,7 @@ __device__ __forceinline__ int lds_append(unsigned* s_count, bool pred) {
 
 // Stage entry of a level that does not fit 16 bits (written to its row).
 constexpr uint16_t kStaged = 0xFFFF;
+constexpr int32_t kStageLanes = 8;  // tasks with their state in memory: lanes that stage their levels
 
 // atomicOr on a lane word of type LT; sub-word types go through the
 // aligned 32-bit word that holds them.  Returns the old value of *p.
@@ -218,11 +219,12 @@ __device__ void run_unweighted(const BatchArgs& a, const BatchGraph& G, const Ba
   // Lane b of the task is source lane0 + b of the graph: row drow + b * n.
   int32_t* drow = a.dist + G.dist_off + (int64_t)T.lane0 * n;
   const LT lanemask = (LT)(T.lanes >= 64 ? ~0ull : ((1ull << T.lanes) - 1));
-  // Tasks of at most 8 lanes stage each arrival level in stage[v][b]
+  // Tasks of at most kStageLanes lanes stage each arrival level in stage[v][b]
   // (16 bits; kStaged marks a level that did not fit, written to its row at
   // once) and write the rows in one coalesced pass at the end, instead of
   // 4-byte stores scattered over the rows as vertices are reached.
   constexpr bool kStage = sizeof(LT) == 1;
+  static_assert(!kStage || kStageLanes == 8, "a byte of lanes");
   uint16_t* stage = reinterpret_cast<uint16_t*>(a.stage + (int64_t)blockIdx.x * a.stage_cap);
   for (int32_t v = threadIdx.x; v < n; v += blockDim.x) {
     seen[v] = (LT)~lanemask;
@@ -395,6 +397,14 @@ inline int lds_bits(int64_t n, int lanes, int32_t max_deg) {
   int b = 0;
   while ((1 << b) < lanes) b++;
   return b <= kMaxBits && (b == 0 || max_deg < 65536) && lds_field_words(n, b) <= kLdsWords ? b : -1;
+}
+
+// Bytes of arrival levels that a task of `lanes` sources keeps in memory
+// (BatchArgs::stage); bits as in BatchTask.
+inline int64_t stage_bytes(int64_t n, int lanes, int bits) {
+  if (bits < 0) return lanes <= kStageLanes ? n * kStageLanes * (int64_t)sizeof(uint16_t) : 0;
+  const bool in_lds = lds_field_words(n, bits) * 4 + (n << bits) <= (int64_t)kLdsWords * 4;
+  return in_lds ? 0 : n << bits;
 }
 
 struct LdsTask {
@@ -1286,7 +1296,7 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
       if (T.bits >= 0)
         lds_task<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
                     a.entries + (int64_t)blockIdx.x * a.max_lds_n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or);
-      else if (T.lanes <= 8)
+      else if (T.lanes <= kStageLanes)
         run_unweighted<BS, uint8_t>(a, G, T, (uint8_t*)seen, (uint8_t*)next, qv, (uint8_t*)qw,
                                     touched, s_off, s_beg, s_f, s_scan, s_cnt);
       else if (T.lanes <= 16)
@@ -1560,7 +1570,6 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
         // Graphs beyond the LDS: state in memory, lanes as wide as 64.
         per = g->m >= 2000000 ? 1 : g->m >= 500000 ? std::max(1, spg / 2) : spg;
         max_n = std::max<int64_t>(max_n, g->n);
-        if (per <= 8) stage_cap = std::max<int64_t>(stage_cap, (int64_t)g->n * 16);
       } else {
         max_lds_n = std::max<int64_t>(max_lds_n, g->n);
       }
@@ -1568,8 +1577,7 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
         const int32_t lanes = std::min(per, spg - j);
         const int bits =
             lds_bits(g->n, per, g->max_out_degree) < 0 ? -1 : lds_bits(g->n, lanes, g->max_out_degree);
-        if (bits >= 0 && lds_field_words(g->n, bits) * 4 + ((int64_t)g->n << bits) > (int64_t)kLdsWords * 4)
-          stage_cap = std::max<int64_t>(stage_cap, (int64_t)g->n << bits);
+        stage_cap = std::max(stage_cap, stage_bytes(g->n, lanes, bits));  // a last task may have fewer lanes
         ht.push_back(BatchTask{i, j, lanes, bits});
       }
     }
