@@ -27,6 +27,9 @@ void set_hip_error(hipError_t e, const char* what, const char* file, int line) {
   char buf[512];
   std::snprintf(buf, sizeof buf, "%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
   g_last_error = buf;
+  // The runtime keeps a failed call's error for the next hipGetLastError: the
+  // launch check of a later call would report it again.
+  (void)hipGetLastError();
   if (std::getenv("DAWN_VERBOSE")) std::fprintf(stderr, "dawn: %s\n", buf);
 }
 
