@@ -585,11 +585,10 @@ namespace {
 int ensure_wms(dawn_graph* g, int L) {
   if (!g->wms) g->wms = new WmsWorkspace();
   WmsWorkspace* ws = g->wms;
-  if (ws->n == g->n && ws->lanes == L && ws->dist.p) return DAWN_OK;
+  if (ws->n == g->n && ws->lanes == L) return DAWN_OK;
+  ws->n = ws->lanes = 0;  // set once every buffer is in place
   ws->dist.release();
   ws->rows.release();
-  ws->n = g->n;
-  ws->lanes = L;
   DAWN_TRY(ws->dist.alloc((size_t)g->n * L));
   DAWN_TRY(ws->act.alloc((size_t)3 * g->n));
   DAWN_TRY(ws->q.alloc((size_t)3 * g->n));
@@ -600,6 +599,8 @@ int ensure_wms(dawn_graph* g, int L) {
   if (!ws->h_batch) DAWN_HIP(hipHostMalloc((void**)&ws->h_batch, sizeof(WBatch)));
   for (hipEvent_t* e : {&ws->ev0, &ws->ev1})
     if (!*e) DAWN_HIP(hipEventCreate(e));
+  ws->n = g->n;
+  ws->lanes = L;
   return DAWN_OK;
 }
 

@@ -161,6 +161,8 @@ std::map<std::string, Op> ops() {
   return {
       {"bfs", {300, false, one(false)}},
       {"sssp", {300, true, one(true)}},
+      {"weighted_lanes_8", {300, true, many(300, 5, DAWN_POLICY_PUSH, true)}},
+      {"weighted_lanes_64", {300, true, many(300, 70, DAWN_POLICY_PUSH, true)}},
       {"weighted_workgroups", {300, true, many(300, 70, DAWN_POLICY_FIXED, true)}},
       {"lanes", {300, false, many(300, 130, DAWN_POLICY_PUSH, true)}},
       {"lanes_hub_order", {66000, false, many(66000, 3, DAWN_POLICY_PUSH, false)}},

@@ -11,7 +11,7 @@ import pytest
 from conftest import ROOT
 
 PKG = os.path.join(ROOT, "gal-dawn_amd")
-OPERATIONS = ("bfs", "sssp", "weighted_workgroups", "lanes",
+OPERATIONS = ("bfs", "sssp", "weighted_lanes_8", "weighted_lanes_64", "weighted_workgroups", "lanes",
               "lanes_hub_order", "workgroups", "workgroups_no_rows", "batch", "batch_weighted")
 
 
