@@ -1328,10 +1328,13 @@ __global__ void __launch_bounds__(kSsBlock, 8) ss_step_kernel(SsRun run, int k) 
   SsStage& sg = lds.wide.sg;
   sg.init();
   Acc acc;
-  // A frontier vertex at or beyond the threshold stays in the frontier.
+  // A frontier vertex at or beyond the threshold stays in the frontier, but for
+  // one without a distance (its edge from the source weighs INT32_MAX): no path
+  // goes on from it, and it would never get below.
   const int32_t thr = MP && ctl.st.delta > 0 ? (int32_t)min(ctl.st.thr, (long long)kInf) : kInf;
   auto defer = [&](bool yes, int32_t u, int du, int deg) {
     const uint32_t bit = 1u << (u & 31);
+    yes = yes && du != kInf;
     const bool first = yes && (atomicOr(&bm_out[u >> 5], bit) & bit) == 0;
     if (yes) acc.dist(du);
     if (first) acc.de += (unsigned)deg;
