@@ -1448,12 +1448,14 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
                     std::vector<unsigned long long>& acc, double* ms) {
   if (g->n > kSourcesN || g->m >= kSourcesMaxM) return DAWN_ERR_UNSUPPORTED;
   const bool dl = g->n <= kDistN;
-  const bool dev_out = dist && is_device_pointer(dist);
+  // Rows go to the caller's device memory itself; with bounds in LDS the
+  // distances are lowered there, in plain memory of the device only.
+  const bool direct = g->weighted && !dl ? in_place(g->device, dist) : is_device_pointer(dist);
   int cus = 0;
   DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
   hipStream_t s = g->stream;
-  // Rows go to the caller's device memory; host rows in blocks of a workgroup per CU.
-  const int32_t per = std::min<int32_t>(S, dist && !dev_out ? cus : kSourcesLaunch);
+  // Other rows are copied, in blocks of a workgroup per CU.
+  const int32_t per = std::min<int32_t>(S, dist && !direct ? cus : kSourcesLaunch);
   const int grid = std::max(1, std::min<int>(per, cus));
   const size_t gn = (size_t)grid * g->n;
   const BatchGraph G{g->n, g->weighted, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col,
@@ -1462,7 +1464,7 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
   DAWN_TRY(ws->counter.alloc(1));
   DAWN_TRY(ws->sources.alloc((size_t)per));
   DAWN_TRY(ws->acc.alloc((size_t)per * 4));
-  if (dist && !dev_out) DAWN_TRY(ws->rows.alloc((size_t)per * g->n));
+  if (dist && !direct) DAWN_TRY(ws->rows.alloc((size_t)per * g->n));
   else if (!dist && !(g->weighted && dl)) DAWN_TRY(ws->rows.alloc(gn));
   for (hipEvent_t* e : {&ws->ev0, &ws->ev1})
     if (!*e) DAWN_HIP(hipEventCreate(e));
@@ -1481,7 +1483,7 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
   *ms = 0;
   for (int32_t b0 = 0; b0 < S; b0 += per) {
     const int32_t count = std::min(per, S - b0);
-    int32_t* rows = !dist ? nullptr : dev_out ? dist + (int64_t)b0 * g->n : ws->rows.p;
+    int32_t* rows = !dist ? nullptr : direct ? dist + (int64_t)b0 * g->n : ws->rows.p;
     DAWN_HIP(hipMemcpyAsync(ws->sources.p, sources + b0, sizeof(int32_t) * (size_t)count,
                             hipMemcpyHostToDevice, s));
     DAWN_HIP(hipEventRecord(ws->ev0, s));
@@ -1500,9 +1502,11 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
     DAWN_HIP(hipMemcpyAsync(acc.data() + (size_t)b0 * 4, ws->acc.p,
                             sizeof(unsigned long long) * 4 * (size_t)count, hipMemcpyDeviceToHost, s));
     DAWN_HIP(hipStreamSynchronize(s));
-    if (dist && !dev_out)
+    if (dist && !direct) {
       DAWN_HIP(hipMemcpy(dist + (int64_t)b0 * g->n, ws->rows.p, sizeof(int32_t) * (size_t)count * g->n,
-                         hipMemcpyDeviceToHost));
+                         hipMemcpyDefault));
+      DAWN_HIP(hipStreamSynchronize(nullptr));  // rows that are no host memory
+    }
     float x = 0.f;
     DAWN_HIP(hipEventElapsedTime(&x, ws->ev0, ws->ev1));
     *ms += x;
@@ -1616,9 +1620,17 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   const size_t o_touch = cut(g1 * mx, sizeof(int32_t)), o_stage = cut(g1 * (size_t)stage_cap, 1);
   const size_t o_ldsq = cut(g1 * lx, sizeof(int32_t)), o_ent = cut(g1 * lx, sizeof(int2));
   DAWN_TRY(mem.alloc(bytes));
-  const bool dev_out = is_device_pointer(dist);
+  bool any_weighted = false;
+  bool all_weighted = true;
+  for (const BatchGraph& x : hg) {
+    any_weighted = any_weighted || x.weighted;
+    all_weighted = all_weighted && x.weighted;
+  }
+  // Weighted tasks lower the distances in the rows: in plain memory of the
+  // device only.
+  const bool direct = any_weighted ? in_place(device, dist) : is_device_pointer(dist);
   int32_t* out = dist;
-  if (!dev_out) {
+  if (!direct) {
     DAWN_TRY(dout.alloc((size_t)total));
     out = dout.p;
   }
@@ -1652,12 +1664,6 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   hipEvent_t e0, e1;
   DAWN_HIP(hipEventCreate(&e0));
   DAWN_HIP(hipEventCreate(&e1));
-  bool any_weighted = false;
-  bool all_weighted = true;
-  for (const BatchGraph& x : hg) {
-    any_weighted = any_weighted || x.weighted;
-    all_weighted = all_weighted && x.weighted;
-  }
   DAWN_HIP(hipEventRecord(e0, s));
   if (any_weighted) wsum_kernel<<<num_graphs * kWsumParts, kBlock, 0, s>>>(a.graphs, (unsigned long long*)(M + o_wsum));
   if (!any_weighted) batch_kernel<kBatchBlock, 0><<<grid, kBatchBlock, 0, s>>>(a);
@@ -1672,8 +1678,14 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   (void)hipEventDestroy(e1);
   unsigned long long levels = 0;
   DAWN_HIP(hipMemcpy(&levels, a.levels_total, sizeof levels, hipMemcpyDeviceToHost));
-  if (dist && !dev_out)
+  if (dist && !direct && !is_device_pointer(dist)) {
     DAWN_HIP(hipMemcpy(dist, out, sizeof(int32_t) * (size_t)total, hipMemcpyDeviceToHost));
+  } else if (dist && !direct) {  // what lies between the graphs' rows stays
+    for (int32_t i = 0; i < num_graphs; i++)
+      DAWN_HIP(hipMemcpyAsync(dist + dist_offsets[i], out + dist_offsets[i],
+                              sizeof(int32_t) * (size_t)spg * hg[i].n, hipMemcpyDefault, s));
+    DAWN_HIP(hipStreamSynchronize(s));
+  }
   if (stats) {
     stats->device_ms += ms;
     stats->steps += (int64_t)levels;

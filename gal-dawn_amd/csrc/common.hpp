@@ -478,6 +478,9 @@ inline unsigned grid_for(int64_t items, int per_block = kBlock, unsigned cap = 8
 
 // Pointer kind of a caller buffer.
 bool is_device_pointer(const void* p);
+// Whether a traversal may run in the caller's buffer itself, with atomics:
+// plain memory of the graph's own device, at int32 alignment.
+bool in_place(int device, const void* p);
 
 // (Re)builds the heavy chunk lists of g from g->knobs (graph_dev.hip).
 struct RowStats {

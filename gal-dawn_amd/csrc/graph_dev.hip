@@ -51,6 +51,16 @@ bool is_device_pointer(const void* p) {
   return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
 }
 
+bool in_place(int device, const void* p) {
+  if (!p || ((uintptr_t)p & 3)) return false;
+  hipPointerAttribute_t attr;
+  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return attr.type == hipMemoryTypeDevice && attr.device == device;
+}
+
 int upload_i32(int32_t** dst, const std::vector<int32_t>& src) {
   hipError_t e = hipMalloc((void**)dst, sizeof(int32_t) * std::max<size_t>(src.size(), 1));
   if (e != hipSuccess) {

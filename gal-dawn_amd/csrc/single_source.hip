@@ -1481,18 +1481,6 @@ int ss_stats(const dawn_graph* g, const SsState& h, dawn_stats* stats) {
   return DAWN_OK;
 }
 
-// Whether the traversal may run in the caller's buffer itself: plain memory
-// of the graph's own device, at int32 alignment.
-bool in_place(const dawn_graph* g, const void* p) {
-  if (!p || ((uintptr_t)p & 3)) return false;
-  hipPointerAttribute_t attr;
-  if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return attr.type == hipMemoryTypeDevice && attr.device == g->device;
-}
-
 }  // namespace
 
 // Runs one single-source traversal.  kind 0: BOVM, 1: min-plus.
@@ -1505,7 +1493,7 @@ int run_single_source(dawn_graph* g, int kind, int32_t source, int32_t* dist_out
   DAWN_HIP(hipSetDevice(g->device));
   DAWN_TRY(ensure_ss(g));
   SsWorkspace* ws = g->ss;
-  const bool direct = in_place(g, dist_out);
+  const bool direct = in_place(g->device, dist_out);
   if (!direct) DAWN_TRY(ws->dist.alloc(g->n));
   SsRun r = make_run(g, source, policy);
   use_workspace(r, ws);

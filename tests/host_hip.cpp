@@ -1,12 +1,14 @@
 // The library's host code on stand-ins for the HIP runtime: device memory is
-// host memory, kernels are not run, and allocations can be made to fail from a
-// chosen one on.  The definitions here come before the runtime's own, as the
-// program is searched first.
+// host memory, kernels are not run (their arguments can be looked at), and
+// allocations can be made to fail from a chosen one on.  The definitions here
+// come before the runtime's own, as the program is searched first.
 //
 //   host_hip list                 the operations
 //   host_hip memory <operation>   from every allocation of the operation on,
 //                                 memory is short: the call and the one after
 //                                 it say so, the next one works, nothing leaks
+//   host_hip managed              a traversal that lowers distances in its rows
+//                                 is not given rows in managed memory
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -23,6 +25,8 @@ namespace {
 long g_allocs = 0, g_fail_from = -1, g_failed = 0, g_live = 0;
 hipError_t g_last = hipSuccess;  // kept until hipGetLastError, as the runtime does
 std::map<const void*, size_t> g_blocks;
+const void* g_managed = nullptr;  // a buffer of managed memory
+long g_seen_managed = 0;          // launches of 1024 threads whose first argument holds its address
 
 hipError_t give(void** p, size_t bytes) {
   if (g_fail_from >= 0 && g_allocs++ >= g_fail_from) {
@@ -79,8 +83,9 @@ hipError_t hipMemset(void* p, int v, size_t n) { return std::memset(p, v, n), hi
 hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) { return std::memset(p, v, n), hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
   std::memset(a, 0, sizeof *a);
-  if (!on_device(p)) return g_last = hipErrorInvalidValue;
-  a->type = hipMemoryTypeDevice;
+  if (p && p == g_managed) a->type = hipMemoryTypeManaged;
+  else if (on_device(p)) a->type = hipMemoryTypeDevice;
+  else return g_last = hipErrorInvalidValue;
   return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t)8, hipSuccess; }
@@ -105,7 +110,11 @@ hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t sh, hipStream_t s) 
 hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, hipStream_t* s) {
   return *g = g_grid, *b = g_block, *sh = g_shared, *s = g_stream, hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void*, dim3, dim3 block, void** args, size_t, hipStream_t) {
+  if (g_managed && block.x == 1024)  // their argument structs hold more than 128 bytes
+    for (int i = 0; i < 128; i += 8) g_seen_managed += !std::memcmp((const char*)args[0] + i, &g_managed, 8);
+  return hipSuccess;
+}
 }
 
 namespace {
@@ -212,6 +221,32 @@ int memory(const Op& op) {
     if (g_live != before) return fail("memory is lost", k, (int)(g_live - before));
   }
 }
+
+// Weighted sources a workgroup each on more vertices than their distances fit
+// the LDS for, as a call of their own and in a batch: the kernel lowers them in
+// the rows by atomics.
+int managed() {
+  constexpr int32_t n = 40000, most = 65;
+  const Ring r(n, true);
+  dawn_graph* g = nullptr;
+  if (dawn_graph_create(&r.csr, &g)) return 1;
+  int bad = 0;
+  for (const bool batch : {false, true}) {
+    const int32_t count = batch ? 3 : most;
+    const int64_t first = batch ? 5 : 0;  // a batch's rows may lie anywhere in the buffer
+    std::vector<int32_t> src((size_t)count, 1), rows((size_t)(first + (int64_t)count * n), 7);
+    g_managed = rows.data();
+    g_seen_managed = 0;
+    const int rc = batch ? dawn_batch_mssp(&g, 1, src.data(), count, rows.data(), &first, nullptr)
+                         : dawn_mssp(g, src.data(), count, rows.data(), nullptr, DAWN_POLICY_FIXED, nullptr);
+    g_managed = nullptr;
+    std::printf("status %d, %ld launches hold the rows, entries %d %d\n", rc, g_seen_managed, rows[first], rows.back());
+    // The kernels did not run: the entries are those of fresh memory.
+    bad |= rc || g_seen_managed || rows[first] != 0 || rows.back() != 0 || (first && rows[first - 1] != 7);
+  }
+  dawn_graph_destroy(g);
+  return bad;
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -221,5 +256,6 @@ int main(int argc, char** argv) {
     return 0;
   }
   if (what == "memory" && argc > 2) return memory(ops().at(argv[2]));
+  if (what == "managed") return managed();
   return 2;
 }

@@ -1,6 +1,7 @@
 """Shortage of device memory: at every allocation of an operation the call
 reports it, a second call on the same graph does too (it does not go on with
 what the first one left), a call with memory again works, and nothing is lost.
+Rows in managed memory: not for a kernel that lowers distances in them.
 The library's host code runs on stand-ins for the HIP runtime
 (tests/host_hip.cpp); no GPU."""
 import os
@@ -32,4 +33,9 @@ def test_operations_listed(host_hip):
 @pytest.mark.parametrize("operation", OPERATIONS)
 def test_memory_shortage(host_hip, operation):
     r = subprocess.run([host_hip, "memory", operation], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_managed_rows(host_hip):
+    r = subprocess.run([host_hip, "managed"], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
