@@ -1381,6 +1381,7 @@ struct BfsSourcesArgs {
   int32_t count;
   int32_t* rows;            // [count][n], or null
   int32_t* scratch;         // without rows: [grid][n], for levels beyond a byte
+  int32_t write;            // rows are written: to `rows`, else each over the last in `scratch`
   int32_t* qv;              // [grid][n]
   int2* ent;                // [grid][n]
   unsigned* counter;
@@ -1415,7 +1416,7 @@ __global__ void __launch_bounds__(BS) bfs_sources_kernel(BfsSourcesArgs a) {
           unsigned reached = 0, edges = 0;  // m < 2^31
           for (int32_t v = t; v < n; v += BS) {
             const int32_t d = level_of(v, 0);
-            if (a.rows) row[v] = d;
+            if (a.write) row[v] = d;
             if (d != kInf) {
               sum += (unsigned)d;
               reached++;
@@ -1442,10 +1443,11 @@ __global__ void __launch_bounds__(BS) bfs_sources_kernel(BfsSourcesArgs a) {
 constexpr int32_t kSourcesLaunch = 1 << 16;  // sources of one launch
 
 // Sources (reduced mod n) a workgroup each, for graphs whose state fits its
-// LDS; the engines of lanes say when.  acc: per source the distance sum, the
+// LDS; the engines of lanes say when.  compute_rows: unweighted rows are
+// computed without an output too (dawn_mssp).  acc: per source the distance sum, the
 // vertices reached, their out-degrees, the steps (levels); device time in *ms.
 int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources, int32_t S, int32_t* dist,
-                    std::vector<unsigned long long>& acc, double* ms) {
+                    bool compute_rows, std::vector<unsigned long long>& acc, double* ms) {
   if (g->n > kSourcesN || g->m >= kSourcesMaxM) return DAWN_ERR_UNSUPPORTED;
   const bool dl = g->n <= kDistN;
   // Rows go to the caller's device memory itself; with bounds in LDS the
@@ -1493,8 +1495,8 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
       if (dl) sources_kernel<kBatchBlock, true><<<grid, kBatchBlock, 0, s>>>(a);
       else sources_kernel<kBatchBlock, false><<<grid, kBatchBlock, 0, s>>>(a);
     } else {
-      const BfsSourcesArgs a{G, ws->sources.p, count, rows, ws->rows.p, ws->queue.p, ws->entries.p,
-                             ws->counter.p, ws->acc.p};
+      const BfsSourcesArgs a{G, ws->sources.p, count, rows, ws->rows.p, dist || compute_rows,
+                             ws->queue.p, ws->entries.p, ws->counter.p, ws->acc.p};
       bfs_sources_kernel<kBatchBlock><<<grid, kBatchBlock, 0, s>>>(a);
     }
     DAWN_HIP(hipGetLastError());

@@ -509,7 +509,7 @@ void wms_workspace_free(WmsWorkspace* ws);
 constexpr int64_t kSourcesN = 134000, kSourcesMaxM = 1 << 30;
 constexpr int64_t kSourcesDistN = 37797;  // weighted: distances in LDS up to here
 int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources, int32_t S, int32_t* dist,
-                    std::vector<unsigned long long>& acc, double* ms);
+                    bool compute_rows, std::vector<unsigned long long>& acc, double* ms);
 void sources_workspace_free(SourcesWorkspace* ws);
 
 }  // namespace dawn

@@ -2375,7 +2375,7 @@ static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
 // live: the sources that take lanes in batches of 64 words, as the lanes count.
 static int run_msbfs_sources(dawn_graph* g, const int32_t* sources, int32_t S, const std::vector<int32_t>& live_row,
                              int words, int32_t* dist, int64_t* sums, int64_t* reached, int64_t* edges,
-                             dawn_stats* stats) {
+                             dawn_stats* stats, bool rows) {
   if (!g->sources) g->sources = new SourcesWorkspace();
   std::vector<int32_t> src(S);
   for (int32_t i = 0; i < S; i++) {
@@ -2385,7 +2385,7 @@ static int run_msbfs_sources(dawn_graph* g, const int32_t* sources, int32_t S, c
   }
   std::vector<unsigned long long> acc;
   double ms = 0;
-  DAWN_TRY(run_sources_lds(g, g->sources, src.data(), S, dist, acc, &ms));
+  DAWN_TRY(run_sources_lds(g, g->sources, src.data(), S, dist, rows, acc, &ms));
   for (int32_t i = 0; i < S; i++) {
     const unsigned long long* x = acc.data() + (size_t)i * 4;
     if (sums) sums[i] = (int64_t)x[0];
@@ -2425,7 +2425,8 @@ int run_msbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, i
   const bool dist_dev = dist && is_device_pointer(dist);
   int rc0 = DAWN_ERR_UNSUPPORTED;
   if (by_workgroup(g, S, policy)) {
-    rc0 = run_msbfs_sources(g, sources, S, live_row, words_for(g, L), dist, sums, reached, edges, stats);
+    rc0 = run_msbfs_sources(g, sources, S, live_row, words_for(g, L), dist, sums, reached, edges, stats,
+                            rows);
     if (rc0 == DAWN_ERR_OUT_OF_MEMORY) {  // nothing has run yet: the lanes try
       sources_workspace_free(g->sources);
       g->sources = nullptr;

@@ -758,7 +758,7 @@ int run_wmsbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, 
     }
     std::vector<unsigned long long> acc;
     double ms = 0;
-    const int rc = run_sources_lds(g, g->sources, src.data(), S, dist, acc, &ms);
+    const int rc = run_sources_lds(g, g->sources, src.data(), S, dist, false, acc, &ms);
     if (rc == DAWN_ERR_OUT_OF_MEMORY) {  // nothing has run yet: the lanes try
       sources_workspace_free(g->sources);
       g->sources = nullptr;
