@@ -84,6 +84,12 @@ struct TuneKnobs {
                                 // 2 per lane 8 in flight, 3 as 2 with streaming column loads
   int32_t lane_words = 16;      // batched engine: 64-lane words per vertex (1, 2, 4, 8, 16)
   int32_t hub_order = 1;        // batched engine: hub-first vertex order (MsView)
+
+  // Equal but for the single-source engine's.
+  bool same_batched(const TuneKnobs& o) const {
+    return dense_blocks == o.dense_blocks && heavy_degree == o.heavy_degree && pull_chunk == o.pull_chunk &&
+           pull_variant == o.pull_variant && lane_words == o.lane_words && hub_order == o.hub_order;
+  }
 };
 
 // Graphs below this size keep their own order in the batched engine.
@@ -140,6 +146,8 @@ struct dawn_graph {
   std::vector<int32_t> h_row_ptr; // host copy of offsets (degrees for drivers)
   std::vector<int32_t> h_in_row_ptr;  // host CSC offsets (directed graphs)
   dawn::TuneKnobs knobs;
+  dawn::TuneKnobs own_knobs;      // the library's choice: defaults, the tune cache's or the tuner's
+  bool tuning = false;
   hipStream_t stream = nullptr;
   std::mutex lock;                // one traversal per graph at a time
   dawn::MsWorkspace* ms = nullptr;
@@ -149,9 +157,9 @@ struct dawn_graph {
   dawn::SsWorkspace* ss = nullptr;
   dawn::WmsWorkspace* wms = nullptr;
   dawn::SourcesWorkspace* sources = nullptr;
-  // Multi-source calls keep to the engine of lanes: its knobs were set, or
-  // are being tuned.
-  bool lanes_only = false;
+  // Multi-source calls keep to the engine of lanes: its knobs are not the
+  // library's choice, or are being tuned.
+  bool lanes_only() const { return tuning || !knobs.same_batched(own_knobs); }
   dawn::MsView* view = nullptr;
 };
 

@@ -849,6 +849,7 @@ int build_device(EmitArgs ea, int dedup, int32_t wmax_bound, dawn_graph** out) {
   }
   // Degree statistics come with the chunk lists: largest degrees and empty rows.
   (void)tuned_knobs_for(g, &g->knobs);
+  g->own_knobs = g->knobs;
   RowStats out_rows, in_rows;
   if ((rc = build_chunks(g, &out_rows, &in_rows))) return fail(rc);
   g->max_out_degree = out_rows.max_deg;

@@ -249,6 +249,7 @@ int dawn_graph_create(const dawn_csr* csr, dawn_graph** out) {
     g->zero_in = z;
   }
   (void)tuned_knobs_for(g, &g->knobs);
+  g->own_knobs = g->knobs;
   if ((rc = build_chunks(g))) return fail(rc);
   *out = g;
   return DAWN_OK;

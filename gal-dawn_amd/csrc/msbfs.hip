@@ -2366,7 +2366,7 @@ constexpr int64_t kSourcesVerts = 80000, kSourcesM = 1 << 21, kSourcesWork = 260
 constexpr int32_t kSourcesRound = 256, kSourcesShortDeg = 12;
 
 static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
-  if (g->lanes_only || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
+  if (g->lanes_only() || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
   if (g->n > (g->max_out_degree <= kSourcesShortDeg ? kSourcesN : kSourcesVerts) || g->m > kSourcesM) return false;
   const int64_t rounds = ((int64_t)S + kSourcesRound - 1) / kSourcesRound;
   return rounds <= 1 || rounds * (g->m + 16 * (int64_t)g->n) <= kSourcesWork;

@@ -55,9 +55,12 @@ std::string class_key(const dawn_graph* g) {
 int sample_ms(dawn_graph* g, const std::vector<int32_t>& src, double* ms) {
   struct Lanes {  // the knobs are those of the engine of lanes
     dawn_graph* g;
-    bool was;
-    explicit Lanes(dawn_graph* x) : g(x), was(x->lanes_only) { g->lanes_only = true; }
-    ~Lanes() { g->lanes_only = was; }
+    explicit Lanes(dawn_graph* x) : g(x) { set(true); }
+    ~Lanes() { set(false); }
+    void set(bool on) {
+      std::lock_guard<std::mutex> guard(g->lock);
+      g->tuning = on;
+    }
   } lanes(g);
   double best = 1e300;
   for (int rep = 0; rep < 3; rep++) {  // the first run also warms up
@@ -86,12 +89,14 @@ bool knobs_valid(const TuneKnobs& k) {
          (k.hub_order == 0 || k.hub_order == 1);
 }
 
-int apply(dawn_graph* g, const TuneKnobs& k) {
+// own: the library's choice (else set by hand, or a candidate of the tuner).
+int apply(dawn_graph* g, const TuneKnobs& k, bool own = false) {
   std::lock_guard<std::mutex> guard(g->lock);  // traversals hold it while they run
   if (g->stream) DAWN_HIP(hipStreamSynchronize(g->stream));
   const bool rechunk = k.heavy_degree != g->knobs.heavy_degree || k.pull_chunk != g->knobs.pull_chunk;
   const bool reorder = rechunk || k.hub_order != g->knobs.hub_order;
   g->knobs = k;
+  if (own) g->own_knobs = k;
   invalidate_graphs(g);
   if (reorder) ms_view_free(g);  // rebuilt by the next batched traversal
   if (rechunk) {
@@ -222,7 +227,7 @@ int dawn_tune(const dawn_graph* gc, int32_t verbose) {
       }
     }
   }
-  DAWN_TRY(apply(g, best));
+  DAWN_TRY(apply(g, best, true));
   {
     std::lock_guard<std::mutex> l(g_tune_lock);
     g_tune_cache[class_key(g)] = best;
@@ -294,9 +299,7 @@ int dawn_graph_set_knobs(dawn_graph* g, const int32_t* knobs) {
   k.lane_words = knobs[DAWN_KNOB_LANE_WORDS];
   k.hub_order = knobs[DAWN_KNOB_HUB_ORDER];
   if (!knobs_valid(k)) return DAWN_ERR_INVALID_ARG;
-  DAWN_TRY(apply(g, k));
-  g->lanes_only = true;
-  return DAWN_OK;
+  return apply(g, k);
 }
 
 }  // extern "C"

@@ -726,7 +726,7 @@ constexpr int64_t kSourcesM = 600000;
 constexpr int32_t kSourcesS = 16;
 
 static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
-  if (g->lanes_only || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
+  if (g->lanes_only() || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
   if (g->n > kSourcesN || g->m >= kSourcesMaxM) return false;
   return g->n <= kSourcesDistN ? g->m <= kSourcesM || S >= kSourcesS : S > 64;
 }

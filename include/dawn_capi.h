@@ -216,7 +216,7 @@ int dawn_bfs_noalloc(const dawn_graph* g, int32_t source, int32_t* dist,
  * batch.  On graphs whose state fits a workgroup's LDS (up to 80,000 vertices
  * and 2 million edges unweighted, 134,000 vertices weighted) a call that is
  * faster so runs a workgroup per source instead (fixed and learned policies,
- * knobs not set by hand); its counts are those of the batches, its steps
+ * the batched engine's knobs as the library chose them); its counts are those of the batches, its steps
  * count as push, its frontier edges per source.
  * sources are taken modulo n (reference: msource[i] % rows, mssp.cpp:15);
  * isolated sources are skipped (dist row left INF except dist[src]=0, sum 0).
