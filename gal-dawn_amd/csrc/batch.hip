@@ -372,10 +372,14 @@ __device__ void run_unweighted(const BatchArgs& a, const BatchGraph& G, const Ba
 //   gather  the queue's vertices give their B bits, offsets and degrees to
 //           the entry list; B is cleared
 //   pull    of the lanes whose frontier holds more than 1 / kPullShare of the
-//           graph's edges: every vertex that misses one of them ORs its in-
-//           neighbours' A bits until it has found them all (a lane that an
-//           in-neighbour has and the vertex lacks arrived there one level
-//           ago, or the vertex would have it); they enter A afterwards
+//           graph's edges, if there are more edges than a push takes in one
+//           round (counting them per lane costs more than that round): every
+//           vertex that misses one of them ORs its in-neighbours' A bits until
+//           it has found them all (a lane that an in-neighbour has and the
+//           vertex lacks arrived there one level ago, or the vertex would have
+//           it); they enter A afterwards.  Without that bound 1500 grids of 150
+//           vertices, 16 sources each, took 2.2 times as long, 1500 random graphs
+//           of 150 vertices and degree 16 1.4 times
 //   push    of the other lanes: short lists by a thread per entry, else the
 //           entries' edges spread over the threads (LDS degree scan), four
 //           edges in flight per thread: bits new in A arrive; the first
@@ -481,11 +485,23 @@ __device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lane
     __syncthreads();
     unsigned fe = 0;  // at most m < 2^31
     uint32_t live = 0;
+    // B is cleared at the queue's vertices, or in all words if those are fewer:
+    // levels of a few vertices leave the words alone.  A thread's first entry
+    // stays in a register.
+    const bool few = qn <= (unsigned)words;
+    int2 mine = make_int2(0, 0);
     for (unsigned i = t; i < qn; i += BS) {
       const int32_t v = qv[i];
-      const uint32_t f = one ? 1u : (s.W[word_of(v)] >> (shift_of(v) + L)) & fmask;
+      uint32_t f = 1u;
+      if (!one) {
+        uint32_t* w = &s.W[word_of(v)];
+        const int at = shift_of(v) + L;
+        f = ((few ? atomicAnd(w, ~(fmask << at)) : *w) >> at) & fmask;
+      }
       const int rb = G.row_ptr[v], d = G.row_ptr[v + 1] - rb;
-      ent[i] = make_int2(rb, one ? d : d | (int)(f << 16));
+      const int2 e2 = make_int2(rb, one ? d : d | (int)(f << 16));
+      if (i < (unsigned)BS) mine = e2;
+      else ent[i] = e2;
       fe += (unsigned)d;
       live |= f;
     }
@@ -499,8 +515,9 @@ __device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lane
     }
     __syncthreads();
     live = s_red[0];
+    auto entry = [&](unsigned i) { return i < (unsigned)BS ? mine : ent[i]; };  // of this thread
     uint32_t pull = 0;  // lanes to pull
-    if ((unsigned long long)s_cnt[1] * kPullShare > (unsigned long long)G.m) {
+    if (s_cnt[1] > 4u * BS && (unsigned long long)s_cnt[1] * kPullShare > (unsigned long long)G.m) {
       // The frontier's edges lane by lane: the lanes with many are pulled
       // (a lane with few would make every vertex scan its whole list).
       if (one) {
@@ -511,7 +528,7 @@ __device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lane
         for (int b0 = 0; b0 < lanes; b0 += 4) {
           unsigned c[4] = {0, 0, 0, 0};
           for (unsigned i = t; i < qn; i += BS) {
-            const unsigned df = (unsigned)ent[i].y;
+            const unsigned df = (unsigned)entry(i).y;
 #pragma unroll
             for (int b = 0; b < 4; b++) c[b] += (df >> (16 + b0 + b)) & 1u ? df & 0xFFFFu : 0u;
           }
@@ -526,7 +543,7 @@ __device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lane
           if ((unsigned long long)s.lane_edges[b] * kPullShare > (unsigned long long)G.m) pull |= 1u << b;
       }
     }
-    if (!one)
+    if (!one && !few)
       for (int i = t; i < words; i += BS) s.W[i] &= ~bmask;
     if (t == 0) s_cnt[0] = 0u;
     __syncthreads();
@@ -663,7 +680,7 @@ __device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lane
       for (unsigned c0 = t & ~(kWave - 1); c0 < qn; c0 += BS) {  // wave-uniform
         const unsigned i = c0 + lane_id();
         int2 e2 = make_int2(0, 0);
-        if (i < qn) e2 = ent[i];
+        if (i < qn) e2 = entry(i);
         const uint32_t f = (one ? 1u : (uint32_t)e2.y >> 16) & ~pull;
         const int d = !f ? 0 : one ? e2.y : e2.y & 0xFFFF;
         const int most = wave_max_i32(d);
@@ -681,7 +698,7 @@ __device__ int run_lds(const BatchGraph& G, const int32_t* sources, int32_t lane
     for (unsigned c0 = 0; c0 < qn; c0 += BS) {
       const unsigned i = c0 + t;
       int2 e2 = make_int2(0, 0);
-      if (i < qn) e2 = ent[i];
+      if (i < qn) e2 = entry(i);
       const uint32_t f0 = (one ? 1u : (uint32_t)e2.y >> 16) & ~pull;
       int total;
       const int off = scan_bs<BS>(!f0 ? 0 : one ? e2.y : e2.y & 0xFFFF, s_scan, &total);
@@ -1261,7 +1278,7 @@ __global__ void __launch_bounds__(kBlock) wsum_kernel(const BatchGraph* graphs,
 
 // KIND: the tasks of the batch are all unweighted (0), all weighted (1) or
 // mixed (2); with one kind alone the compiler keeps the registers the other
-// would take (mixed: 145 scalar and 12 vector spills).
+// would take (mixed: 134 scalar and 14 vector spills).
 template <int BS, int KIND>
 __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
   __shared__ int s_off[BS];
