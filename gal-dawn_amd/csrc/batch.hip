@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "common.hpp"
@@ -70,6 +71,7 @@ struct BatchArgs {
   int32_t* dist;
   unsigned* task_counter;
   unsigned long long* levels_total;
+  int32_t* graph_levels;     // per unweighted graph: levels of its longest task
   const unsigned long long* wsum;  // per graph: sum of edge weights (weighted)
   // Per-workgroup scratch, sized for the largest graph (max_n).
   int64_t max_n;
@@ -97,9 +99,6 @@ namespace {
 // spilled) made the batches slower (18.7 -> 24-27 ms unweighted, 46 -> 51 ms
 // weighted): twice the concurrent tasks' state no longer fits the caches.
 constexpr int kBatchBlock = 1024;
-constexpr int64_t kSpanFlat = 116000, kSpan = 262144;
-constexpr int32_t kHubDeg = 1024;
-constexpr int64_t kSplit2 = 500000, kSplit1 = 2000000;
 
 template <int BS>
 __device__ __forceinline__ int owner(const int* off, int e) {
@@ -357,7 +356,10 @@ __device__ void run_unweighted(const BatchArgs& a, const BatchGraph& G, const Ba
       }
     }
   }
-  if (threadIdx.x == 0) atomicAdd(a.levels_total, (unsigned long long)level);
+  if (threadIdx.x == 0) {
+    atomicAdd(a.levels_total, (unsigned long long)level);
+    atomicMax(&a.graph_levels[T.graph], level);
+  }
 }
 
 // ---- unweighted tasks with their state in LDS -----------------------------
@@ -745,7 +747,10 @@ __device__ void lds_task(const BatchArgs& a, const BatchGraph& G, const BatchTas
         for (int32_t v = threadIdx.x; v < n; v += BS)
           for (int b = 0; b < T.lanes; b++) drow[(int64_t)b * n + v] = level_of(v, b);
       });
-  if (threadIdx.x == 0) atomicAdd(a.levels_total, (unsigned long long)levels);
+  if (threadIdx.x == 0) {
+    atomicAdd(a.levels_total, (unsigned long long)levels);
+    atomicMax(&a.graph_levels[T.graph], levels);
+  }
 }
 
 // One weighted source.  The reference's initialisation
@@ -1276,9 +1281,10 @@ __global__ void __launch_bounds__(kBlock) wsum_kernel(const BatchGraph* graphs,
   if (threadIdx.x == 0 && s_t) atomicAdd(&out[blockIdx.x / kWsumParts], s_t);
 }
 
-// KIND: the tasks of the batch are all unweighted (0), all weighted (1) or
-// mixed (2); with one kind alone the compiler keeps the registers the other
-// would take (mixed: 134 scalar and 14 vector spills).
+// KIND: the tasks of the batch are all unweighted (0), all weighted (1), mixed
+// (2) or all unweighted with their state in memory (3); with one kind alone the
+// compiler keeps the registers the others would take (mixed: 105 scalar and 14
+// vector spills).
 template <int BS, int KIND>
 __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
   __shared__ int s_off[BS];
@@ -1315,7 +1321,7 @@ __global__ void __launch_bounds__(BS) batch_kernel(BatchArgs a) {
         run_weighted<BS>(a, G, T, (uint8_t*)next, qv, (int32_t*)qw, s_off, s_beg,
                          (int*)s_f, s_scan, s_cnt, s_red);
     } else {
-      if (T.bits >= 0)
+      if (KIND != 3 && T.bits >= 0)
         lds_task<BS>(a, G, T, s_lds, a.lds_q + (int64_t)blockIdx.x * a.max_lds_n,
                     a.entries + (int64_t)blockIdx.x * a.max_lds_n, s_off, s_beg, s_lf, s_scan, s_cnt, s_or);
       else if (T.lanes <= kStageLanes)
@@ -1538,6 +1544,54 @@ int run_sources_lds(dawn_graph* g, SourcesWorkspace* ws, const int32_t* sources,
   return DAWN_OK;
 }
 
+namespace {
+
+// Unweighted tasks of the uneven batch.  The sources of a graph share one task
+// as lanes of a field, except on the largest graphs, whose tasks would be the
+// batch's critical path, and where fewer lanes keep the fields and staged
+// levels in LDS (kSpan*: lanes x vertices; graphs with hubs pull most of their
+// edges once for all lanes and take more, deep ones pay for their levels in
+// every task).  512 graphs of 1k-130k vertices, 8 sources: one task per graph
+// 4.6 ms, at most 65,536 lanes x vertices 3.6, at most 116,000 with the levels
+// in LDS 2.6.
+constexpr int64_t kSpanFlat = 116000, kSpan = 262144;
+constexpr int32_t kHubDeg = 1024;
+constexpr int64_t kSplit2 = 500000, kSplit1 = 2000000;
+
+// Graphs of many levels of few edges each: as batches have found it, before
+// that those of hardly more edges than vertices (paths, trees, road maps).  A
+// level takes a task 3-4 us whatever its lanes, so their tasks take as many
+// lanes as fit: 300 trees of 20,000 vertices and some 1000 levels, 16 sources,
+// take 22 ms as four tasks of 4 lanes, 10 as one of 16.  Grids of 20,000
+// vertices have 285 edges a level and are not among them (four tasks 4.9 ms,
+// one in memory 13.1).
+bool deep(const dawn_graph* g) {
+  const int64_t levels = g->batch_levels.load(std::memory_order_relaxed);
+  return levels ? g->m < 128 * levels : g->m * 5 <= 13 * (int64_t)g->n;
+}
+
+// Lanes per task with its state in LDS, 0: it does not fit.
+int32_t lds_lanes(const dawn_graph* g, int32_t spg) {
+  int32_t per = std::min(spg, 1 << kMaxBits);
+  if (g->m >= kSplit1) per = 1;
+  else if (g->m >= kSplit2) per = std::max(1, spg / 2);
+  const int64_t span = deep(g) || g->max_out_degree > kHubDeg ? kSpan : kSpanFlat;
+  while (per > 1 && (lds_bits(g->n, per, g->max_out_degree) < 0 || g->n * (int64_t)per > span))
+    per = (per + 1) / 2;
+  return lds_bits(g->n, per, g->max_out_degree) < 0 ? 0 : per;
+}
+
+// Whether `k` tasks of a graph in LDS take longer than one of up to 64 lanes in
+// memory, where tasks wait for a CU anyway.  Measured on 1500 graphs, LDS over
+// memory: four tasks, random graphs of degree 4 with 2000, 6000 and 8000 edges
+// 1.5, 1.09 and 0.93, paths of 150 and 1000 vertices 2.4 and 2.6; two tasks,
+// random graphs with 600, 2000 and 3000 edges 1.3, 1.06 and 0.98.
+bool memory_faster(const dawn_graph* g, int32_t k) {
+  return k > 1 && (deep(g) || g->m <= (k > 2 ? 8000 : 2500));
+}
+
+}  // namespace
+
 void sources_workspace_free(SourcesWorkspace* ws) {
   if (!ws) return;
   for (hipEvent_t e : {ws->ev0, ws->ev1})
@@ -1561,9 +1615,18 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   std::vector<BatchGraph> hg(num_graphs);
   std::vector<BatchTask> ht;
   std::vector<int32_t> hs((size_t)num_graphs * spg);
+  int cus = 0;
+  DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  int64_t tasks = 0;  // with their state in LDS where it fits
   for (int32_t i = 0; i < num_graphs; i++) {
-    dawn_graph* g = graphs[i];
+    const dawn_graph* g = graphs[i];
     if (!g || g->device != device || g->n <= 0) return DAWN_ERR_INVALID_ARG;
+    const int32_t per = g->weighted ? 1 : lds_lanes(g, spg);
+    tasks += per ? (spg + per - 1) / per : 1;
+  }
+  const bool queued = tasks > cus;
+  for (int32_t i = 0; i < num_graphs; i++) {
+    const dawn_graph* g = graphs[i];
     hg[i] = BatchGraph{g->n, g->weighted, g->m, (GlobalInts)g->row_ptr, (GlobalInts)g->col,
                        (GlobalInts)g->weight, (GlobalInts)g->in_row_ptr, (GlobalInts)g->in_col,
                        dist_offsets[i], g->max_out_degree, 0};
@@ -1581,30 +1644,17 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
       for (int32_t j = 0; j < spg; j++) ht.push_back(BatchTask{i, j, 1, state});
       if (state == kWeightedMemory) max_n = std::max<int64_t>(max_n, g->n);
     } else {
-      // The sources of a graph share one task as lanes of a field, except
-      // on the largest graphs, whose tasks would be the batch's critical
-      // path, and where fewer lanes keep the fields and staged levels in LDS
-      // (kSpan*: lanes x vertices; graphs with hubs pull most of their edges
-      // once for all lanes and take more).  512 graphs of 1k-130k vertices, 8
-      // sources: one task per graph 4.6 ms, at most 65,536 lanes x vertices
-      // 3.6, at most 116,000 with the levels in LDS 2.6.
-      int32_t per = std::min(spg, 1 << kMaxBits);
-      if (g->m >= kSplit1) per = 1;
-      else if (g->m >= kSplit2) per = std::max(1, spg / 2);
-      const int64_t span = g->max_out_degree <= kHubDeg ? kSpanFlat : kSpan;
-      while (per > 1 && (lds_bits(g->n, per, g->max_out_degree) < 0 || g->n * (int64_t)per > span))
-        per = (per + 1) / 2;
-      if (lds_bits(g->n, per, g->max_out_degree) < 0) {
-        // Graphs beyond the LDS: state in memory, lanes as wide as 64.
-        per = g->m >= 2000000 ? 1 : g->m >= 500000 ? std::max(1, spg / 2) : spg;
+      int32_t per = lds_lanes(g, spg);
+      const bool memory = per == 0 || (queued && memory_faster(g, (spg + per - 1) / per));
+      if (memory) {  // lanes as wide as 64
+        per = g->m >= kSplit1 ? 1 : g->m >= kSplit2 ? std::max(1, spg / 2) : spg;
         max_n = std::max<int64_t>(max_n, g->n);
       } else {
         max_lds_n = std::max<int64_t>(max_lds_n, g->n);
       }
       for (int32_t j = 0; j < spg; j += per) {
         const int32_t lanes = std::min(per, spg - j);
-        const int bits =
-            lds_bits(g->n, per, g->max_out_degree) < 0 ? -1 : lds_bits(g->n, lanes, g->max_out_degree);
+        const int bits = memory ? -1 : lds_bits(g->n, lanes, g->max_out_degree);
         stage_cap = std::max(stage_cap, stage_bytes(g->n, lanes, bits));  // a last task may have fewer lanes
         ht.push_back(BatchTask{i, j, lanes, bits});
       }
@@ -1619,8 +1669,6 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   std::stable_sort(ht.begin(), ht.end(),
                    [&](const BatchTask& x, const BatchTask& y) { return cost(x) > cost(y); });
   DAWN_HIP(hipSetDevice(device));
-  int cus = 0;
-  DAWN_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   // One workgroup per CU: as many as are resident at once.
   const int grid = std::max(1, std::min<int>((int)ht.size(), cus));
 
@@ -1638,6 +1686,7 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   const size_t o_graphs = cut(hg.size(), sizeof(BatchGraph)), o_tasks = cut(ht.size(), sizeof(BatchTask));
   const size_t o_src = cut(hs.size(), sizeof(int32_t));
   const size_t o_cnt = cut(1, sizeof(unsigned)), o_lev = cut(1, sizeof(unsigned long long));
+  const size_t o_glev = cut(hg.size(), sizeof(int32_t)), o_levels_end = bytes;
   const size_t o_wsum = cut(hg.size(), sizeof(unsigned long long)), o_zero_end = bytes;
   const size_t o_seen = cut(g1 * mx, sizeof(uint64_t)), o_next = cut(g1 * mx, sizeof(uint64_t));
   const size_t o_q = cut(g1 * 2 * mx, sizeof(int32_t)), o_qw = cut(g1 * 2 * mx, sizeof(uint64_t));
@@ -1674,6 +1723,7 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   a.task_counter = (unsigned*)(M + o_cnt);
   a.levels_total = (unsigned long long*)(M + o_lev);
   a.wsum = (const unsigned long long*)(M + o_wsum);
+  a.graph_levels = (int32_t*)(M + o_glev);
   a.max_n = max_n;
   a.seen = (uint64_t*)(M + o_seen);
   a.next = (uint64_t*)(M + o_next);
@@ -1690,7 +1740,8 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   DAWN_HIP(hipEventCreate(&e1));
   DAWN_HIP(hipEventRecord(e0, s));
   if (any_weighted) wsum_kernel<<<num_graphs * kWsumParts, kBlock, 0, s>>>(a.graphs, (unsigned long long*)(M + o_wsum));
-  if (!any_weighted) batch_kernel<kBatchBlock, 0><<<grid, kBatchBlock, 0, s>>>(a);
+  if (!any_weighted && max_lds_n == 0) batch_kernel<kBatchBlock, 3><<<grid, kBatchBlock, 0, s>>>(a);
+  else if (!any_weighted) batch_kernel<kBatchBlock, 0><<<grid, kBatchBlock, 0, s>>>(a);
   else if (all_weighted) batch_kernel<kBatchBlock, 1><<<grid, kBatchBlock, 0, s>>>(a);
   else batch_kernel<kBatchBlock, 2><<<grid, kBatchBlock, 0, s>>>(a);
   DAWN_HIP(hipGetLastError());
@@ -1700,8 +1751,16 @@ extern "C" int dawn_batch_mssp(dawn_graph* const* graphs, int32_t num_graphs,
   DAWN_HIP(hipEventElapsedTime(&ms, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
+  std::vector<unsigned char> lev(o_levels_end - o_lev);
+  DAWN_HIP(hipMemcpy(lev.data(), M + o_lev, lev.size(), hipMemcpyDeviceToHost));
   unsigned long long levels = 0;
-  DAWN_HIP(hipMemcpy(&levels, a.levels_total, sizeof levels, hipMemcpyDeviceToHost));
+  std::memcpy(&levels, lev.data(), sizeof levels);
+  for (int32_t i = 0; i < num_graphs; i++) {
+    int32_t most = 0;
+    std::memcpy(&most, lev.data() + (o_glev - o_lev) + sizeof(int32_t) * (size_t)i, sizeof most);
+    if (most > graphs[i]->batch_levels.load(std::memory_order_relaxed))
+      graphs[i]->batch_levels.store(most, std::memory_order_relaxed);
+  }
   if (dist && !direct && !is_device_pointer(dist)) {
     DAWN_HIP(hipMemcpy(dist, out, sizeof(int32_t) * (size_t)total, hipMemcpyDeviceToHost));
   } else if (dist && !direct) {  // what lies between the graphs' rows stays

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <vector>
@@ -161,6 +162,8 @@ struct dawn_graph {
   // library's choice, or are being tuned.
   bool lanes_only() const { return tuning || !knobs.same_batched(own_knobs); }
   dawn::MsView* view = nullptr;
+  // Unweighted: most levels a task of an uneven batch has taken (0: none has run).
+  std::atomic<int32_t> batch_levels{0};
 };
 
 namespace dawn {
