@@ -2424,7 +2424,7 @@ int run_msbfs(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, i
   const IsoRows isr{iso.data(), (int32_t)(iso.size() / 2)};
   const bool dist_dev = dist && is_device_pointer(dist);
   int rc0 = DAWN_ERR_UNSUPPORTED;
-  if (by_workgroup(g, S, policy)) {
+  if (L > 0 && by_workgroup(g, S, policy)) {  // nothing to traverse: the rows are filled below
     rc0 = run_msbfs_sources(g, sources, S, live_row, words_for(g, L), dist, sums, reached, edges, stats,
                             rows);
     if (rc0 == DAWN_ERR_OUT_OF_MEMORY) {  // nothing has run yet: the lanes try
