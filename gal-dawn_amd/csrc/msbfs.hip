@@ -2356,20 +2356,38 @@ void split_live(const dawn_graph* g, const int32_t* sources, int32_t S, std::vec
 //   ER 32,768, degree 16: 256 sources 0.26 / 0.42, 512 0.47 / 0.51, 1024 0.82 / 0.61
 //   ER 65,536, degree 8: 64 sources 0.37 / 0.39, 256 0.40 / 0.50, 512 0.72 / 0.62
 //   ER 100,000, degree 8: 64 sources 0.54 / 0.43, 256 0.58 / 0.56
-//   RMAT-15: 256 sources 0.22 / 0.51, 512 0.34 / 0.63; RMAT-16: 64 0.35 / 0.44
+//   RMAT-15: 256 sources 0.22 / 0.51, 512 0.34 / 0.63
+//   RMAT-16, degree 2 to 28: 1 source 0.26-0.29 / 0.30, 64 0.29-0.35 / 0.42-0.47
 //   grid 250 x 250: 64 sources 0.34 / 1.3, 512 0.70 / 1.9; 360 x 360: 64 0.61 / 1.4
 // One round of 256 sources: up to kSourcesVerts vertices (short lists, many
 // levels: the LDS's limit) and kSourcesM edges.  More rounds: while their
 // work, edges and 16 per vertex (levels of few vertices, the row), stays below
 // kSourcesWork.  Forced modes and graphs whose knobs were set keep the lanes.
+//
+// Few sources of larger graphs without hubs: where the level before the last
+// large one holds a fifth of the vertices, a workgroup's pull looks at several
+// edges of most of the others.  ER, 1 and 64 sources:
+//   60,000: degree 16 0.23 / 0.30 and 0.27 / 0.37; 20 0.41 / 0.32 and 0.41 / 0.36
+//           (256: 0.43 / 0.44); 25 0.32 / 0.32 and 0.39 / 0.38; 32 0.25 / 0.37 and
+//           0.28 / 0.51
+//   72,000: degree 8 0.32 / 0.37 and 0.40 / 0.43; 16 0.26 / 0.33 and 0.33 / 0.38;
+//           20 0.52 / 0.31 and 0.50 / 0.36; 25 0.43 / 0.33 and 0.46 / 0.41
+//   80,000: degree 5 0.43 / 0.45 and 0.47 / 0.54; 8 0.40 / 0.38 and 0.45 / 0.44; 12
+//           0.47 / 0.34 and 0.48 / 0.38; 25 0.52 / 0.34 and 0.51 / 0.41 (256: 0.55 / 0.54)
 constexpr int64_t kSourcesVerts = 80000, kSourcesM = 1 << 21, kSourcesWork = 2600000;
+constexpr int64_t kFewSources = 128, kFewVerts = 54000, kFewVertsSparse = 74000;
 constexpr int32_t kSourcesRound = 256, kSourcesShortDeg = 12;
 
 static bool by_workgroup(const dawn_graph* g, int32_t S, int32_t policy) {
   if (g->lanes_only() || (policy != DAWN_POLICY_FIXED && policy != DAWN_POLICY_LEARNED)) return false;
   if (g->n > (g->max_out_degree <= kSourcesShortDeg ? kSourcesN : kSourcesVerts) || g->m > kSourcesM) return false;
+  const int64_t n = g->n, m = g->m;
+  const bool hubs = (int64_t)g->max_out_degree * n > 16 * m;
+  if (S <= kFewSources && !hubs && g->max_out_degree > kSourcesShortDeg &&
+      ((n > kFewVerts && m > 17 * n && m < 28 * n) || (n > kFewVertsSparse && m > 7 * n)))
+    return false;
   const int64_t rounds = ((int64_t)S + kSourcesRound - 1) / kSourcesRound;
-  return rounds <= 1 || rounds * (g->m + 16 * (int64_t)g->n) <= kSourcesWork;
+  return rounds <= 1 || rounds * (m + 16 * n) <= kSourcesWork;
 }
 
 // live: the sources that take lanes in batches of 64 words, as the lanes count.
