@@ -19,7 +19,7 @@ namespace dawn {
 
 int validate_csr(const dawn_csr* csr);
 int build_csc(const dawn_csr* csr, std::vector<int32_t>& ip, std::vector<int32_t>& ic,
-              std::vector<int32_t>& iw, int32_t* max_in_degree);
+              std::vector<int32_t>& iw);
 
 static thread_local std::string g_last_error;
 
@@ -193,9 +193,6 @@ int dawn_graph_create(const dawn_csr* csr, dawn_graph** out) {
   g->weighted = csr->weight ? 1 : 0;
   DAWN_HIP(hipGetDevice(&g->device));
   g->h_row_ptr.assign(csr->row_ptr, csr->row_ptr + n + 1);
-  int32_t maxd = 0;
-  for (int32_t i = 0; i < n; i++) maxd = std::max(maxd, csr->row_ptr[i + 1] - csr->row_ptr[i]);
-  g->max_out_degree = maxd;
 
   auto fail = [&](int rc) {
     dawn_graph_destroy(g);
@@ -229,28 +226,24 @@ int dawn_graph_create(const dawn_csr* csr, dawn_graph** out) {
     g->in_row_ptr = g->row_ptr;
     g->in_col = g->col;
     g->in_weight = g->weight;
-    g->max_in_degree = maxd;
   } else {
     // In-edge CSC on the host (rows ascending within each column).
     std::vector<int32_t> ip, ic, iw;
-    int32_t maxi = 0;
-    if ((rc = build_csc(csr, ip, ic, iw, &maxi))) return fail(rc);
-    g->max_in_degree = maxi;
+    if ((rc = build_csc(csr, ip, ic, iw))) return fail(rc);
     in_rp_host = ip;
     if ((rc = up(&g->in_row_ptr, ip.data(), (size_t)n + 1))) return fail(rc);
     if ((rc = up(&g->in_col, ic.data(), (size_t)m))) return fail(rc);
     if (csr->weight && (rc = up(&g->in_weight, iw.data(), (size_t)m))) return fail(rc);
   }
   if (g->directed) g->h_in_row_ptr = in_rp_host;
-  {
-    const std::vector<int32_t>& ip = g->directed ? g->h_in_row_ptr : g->h_row_ptr;
-    int64_t z = 0;
-    for (int32_t v = 0; v < n; v++) z += ip[v + 1] == ip[v];
-    g->zero_in = z;
-  }
+  // Degree statistics come with the chunk lists: largest degrees and empty rows.
   (void)tuned_knobs_for(g, &g->knobs);
   g->own_knobs = g->knobs;
-  if ((rc = build_chunks(g))) return fail(rc);
+  RowStats out_rows, in_rows;
+  if ((rc = build_chunks(g, &out_rows, &in_rows))) return fail(rc);
+  g->max_out_degree = out_rows.max_deg;
+  g->max_in_degree = in_rows.max_deg;
+  g->zero_in = in_rows.empty;
   *out = g;
   return DAWN_OK;
 }

@@ -201,18 +201,14 @@ int validate_csr(const dawn_csr* csr) {
 // In-edge CSC (column-major copy of the adjacency): ip[n+1], ic[m] = source
 // rows ascending within each column, iw[m] their weights.
 int build_csc(const dawn_csr* csr, std::vector<int32_t>& ip, std::vector<int32_t>& ic,
-              std::vector<int32_t>& iw, int32_t* max_in_degree) {
+              std::vector<int32_t>& iw) {
   const int32_t n = csr->n;
   const int64_t m = csr->m;
   ip.assign((size_t)n + 1, 0);
   ic.resize((size_t)m);
   iw.resize(csr->weight ? (size_t)m : 0);
   for (int64_t k = 0; k < m; k++) ip[csr->col[k] + 1]++;
-  int32_t maxi = 0;
-  for (int32_t i = 0; i < n; i++) {
-    maxi = std::max(maxi, ip[i + 1]);
-    ip[i + 1] += ip[i];
-  }
+  for (int32_t i = 0; i < n; i++) ip[i + 1] += ip[i];
   std::vector<int32_t> cur(ip.begin(), ip.end() - 1);
   for (int32_t r = 0; r < n; r++)
     for (int32_t k = csr->row_ptr[r]; k < csr->row_ptr[r + 1]; k++) {
@@ -220,7 +216,6 @@ int build_csc(const dawn_csr* csr, std::vector<int32_t>& ip, std::vector<int32_t
       ic[p] = r;
       if (csr->weight) iw[p] = csr->weight[k];
     }
-  *max_in_degree = maxi;
   return DAWN_OK;
 }
 
