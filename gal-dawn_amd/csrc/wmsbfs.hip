@@ -293,12 +293,15 @@ __global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a, int k) {
       }
     }
     // Heavy vertices by out-edge chunks: a wave looks at 64 chunks, then takes
-    // the active ones, kRound edges per group at a time.
-    for (int64_t c0 = wave * kWave; c0 < a.num_oc; c0 += nwaves * kWave) {  // wave-uniform
-      const int64_t c = c0 + lane;
+    // the active ones, kRound edges per group at a time.  The 64 lie a grid
+    // apart: few neighbouring ones would leave most waves without any and the
+    // others with 64 in turn (3000 vertices of degree 50, 64 sources, pushed: 6.8
+    // ms, so 0.72; RMAT-17, 64 sources, by the rule 6.1 and 3.4).
+    for (int64_t c0 = wave; c0 < a.num_oc; c0 += nwaves * kWave) {  // wave-uniform
+      const int64_t c = c0 + lane * nwaves;
       uint64_t hot = __ballot(c < a.num_oc && act_in[a.oc_v[c < a.num_oc ? c : 0]] != 0);
       for (; hot; hot &= hot - 1) {
-        const int64_t hc = c0 + __ffsll((unsigned long long)hot) - 1;
+        const int64_t hc = c0 + (__ffsll((unsigned long long)hot) - 1) * nwaves;
         const int32_t u = a.oc_v[hc];
         const int kb = a.oc_beg[hc], ke = a.oc_end[hc];
         const int4 du = masked(*quad(u), bits4(act_in[u]));
