@@ -346,34 +346,62 @@ __global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a, int k) {
       // group takes a vertex, list and all (the minima of 64 vertices would
       // take 32 or 64 registers and leave two or three waves per SIMD to the
       // heavy vertices: RMAT-20, 64 sources, 23 -> 32 ms, 32 sources 13 -> 18;
-      // without heavy vertices, 2048 x 2048, 32 sources, 28 -> 22).
-      for (int64_t v0 = wave * VW; v0 < a.n; v0 += nwaves * VW) {  // wave-uniform
-        const int64_t vv = v0 + grp;
-        const int32_t v = vv < a.n ? (int32_t)vv : 0;
-        int beg = 0, deg = 0;
-        if (vv < a.n) {
-          beg = a.in_row_ptr[v];
-          deg = a.in_row_ptr[v + 1] - beg;
-          if (deg >= a.heavy) deg = 0;
+      // without heavy vertices, 2048 x 2048, 32 sources, 28 -> 22).  Which
+      // vertices have a tail that improved is found first, a thread each, unless
+      // most will have one: most of a step's vertices often have none, and a
+      // group waits on three accesses for each (1000 x 1000 with shortcuts, 33
+      // sources, all steps pulled: 16.3 -> 10.6 ms, by the rule 10.4 -> 9.8; RMAT-20
+      // of degree 8, 64 sources, pulled 16.3 -> 11.7; random graph of 1,000,000,
+      // degree 12, by the rule 16.4 -> 16.7).
+      const bool dense = (int64_t)qn * 4 >= a.n;
+      for (int64_t v0 = wave * kWave; v0 < a.n; v0 += nwaves * kWave) {  // wave-uniform
+        int vbeg = 0, vdeg = 0;
+        if (v0 + lane < a.n) {
+          vbeg = a.in_row_ptr[v0 + lane];
+          vdeg = a.in_row_ptr[v0 + lane + 1] - vbeg;
+          if (vdeg >= a.heavy) vdeg = 0;
         }
-        int4 best = make_int4(kInf, kInf, kInf, kInf);
-        for (int j = 0; j < deg; j += kRound) {
-          int32_t u[kRound], wt[kRound];
+        bool hot = dense && vdeg > 0;
+        for (int j = 0; __ballot(!hot && j < vdeg); j += kRound) {
+          int32_t u[kRound];
+          Mask m[kRound];
 #pragma unroll
-          for (int r = 0; r < kRound; r++) u[r] = j + r < deg ? a.in_col[beg + j + r] : -1;
+          for (int r = 0; r < kRound; r++) u[r] = !hot && j + r < vdeg ? a.in_col[vbeg + j + r] : -1;
 #pragma unroll
-          for (int r = 0; r < kRound; r++) wt[r] = j + r < deg ? a.in_w[beg + j + r] : 0;
-          gather(u, wt, best);
+          for (int r = 0; r < kRound; r++) m[r] = u[r] >= 0 ? act_in[u[r]] : (Mask)0;
+#pragma unroll
+          for (int r = 0; r < kRound; r++) hot |= m[r] != 0;
         }
-        unsigned x = 0;
-        if (min(min(best.x, best.y), min(best.z, best.w)) != kInf) {
-          int4 dv = *quad(v);
-          x = take(best, dv);
-          if (x) *quad(v) = dv;
+        uint64_t todo = __ballot(hot);
+        while (todo) {  // VW of them at a time
+          int at = -1;
+#pragma unroll
+          for (int q = 0; q < VW; q++) {
+            if (grp == q && todo) at = __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1;
+          }
+          const int from = at < 0 ? 0 : at, beg = __shfl(vbeg, from), len = __shfl(vdeg, from);
+          const int deg = at < 0 ? 0 : len;
+          const int32_t v = (int32_t)v0 + from;
+          int4 best = make_int4(kInf, kInf, kInf, kInf);
+          for (int j = 0; j < deg; j += kRound) {
+            int32_t u[kRound], wt[kRound];
+#pragma unroll
+            for (int r = 0; r < kRound; r++) u[r] = j + r < deg ? a.in_col[beg + j + r] : -1;
+#pragma unroll
+            for (int r = 0; r < kRound; r++) wt[r] = j + r < deg ? a.in_w[beg + j + r] : 0;
+            gather(u, wt, best);
+          }
+          unsigned x = 0;
+          if (min(min(best.x, best.y), min(best.z, best.w)) != kInf) {
+            int4 dv = *quad(v);
+            x = take(best, dv);
+            if (x) *quad(v) = dv;
+          }
+          const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
+          if (sub == 0 && imp) act_out[v] = (Mask)imp;  // v's own slot (heavy vertices are not here)
+          s_q.append(sub == 0 && imp != 0, v, qlen_out, q_out);
         }
-        const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
-        if (sub == 0 && imp) act_out[v] = (Mask)imp;  // v's own slot (heavy vertices are not here)
-        s_q.append(sub == 0 && imp != 0, v, qlen_out, q_out);
       }
     } else {
       // Light vertices, 64 a wave: a thread per vertex reads its list, kRound
