@@ -352,7 +352,12 @@ __global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a, int k) {
       // group waits on three accesses for each (1000 x 1000 with shortcuts, 33
       // sources, all steps pulled: 16.3 -> 10.6 ms, by the rule 10.4 -> 9.8; RMAT-20
       // of degree 8, 64 sources, pulled 16.3 -> 11.7; random graph of 1,000,000,
-      // degree 12, by the rule 16.4 -> 16.7).
+      // degree 12, by the rule 16.4 -> 16.7).  A group takes two vertices at a
+      // time, without branches, so that both chains are in flight (2048 x 2048, 64
+      // sources, pulled 3.24 -> 2.86 s, by the rule 3.13 -> 2.76; the random graph
+      // 16.7 -> 15.8 ms, RMAT-20 18.2 -> 18.0).  An edge past a list's end reads the
+      // list's first one; a group that has a first vertex and no second reads the
+      // edge at the lists' start of the wave's first vertex, not past the first's.
       const bool dense = (int64_t)qn * 4 >= a.n;
       for (int64_t v0 = wave * kWave; v0 < a.n; v0 += nwaves * kWave) {  // wave-uniform
         int vbeg = 0, vdeg = 0;
@@ -373,34 +378,69 @@ __global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a, int k) {
           for (int r = 0; r < kRound; r++) hot |= m[r] != 0;
         }
         uint64_t todo = __ballot(hot);
-        while (todo) {  // VW of them at a time
-          int at = -1;
+        while (todo) {  // 2 VW of them at a time
+          int at[2] = {-1, -1}, beg[2], deg[2];
+          int32_t v[2];
+          int4 best[2];
 #pragma unroll
-          for (int q = 0; q < VW; q++) {
-            if (grp == q && todo) at = __ffsll((unsigned long long)todo) - 1;
-            todo &= todo - 1;
-          }
-          const int from = at < 0 ? 0 : at, beg = __shfl(vbeg, from), len = __shfl(vdeg, from);
-          const int deg = at < 0 ? 0 : len;
-          const int32_t v = (int32_t)v0 + from;
-          int4 best = make_int4(kInf, kInf, kInf, kInf);
-          for (int j = 0; j < deg; j += kRound) {
-            int32_t u[kRound], wt[kRound];
+          for (int h = 0; h < 2; h++) {
 #pragma unroll
-            for (int r = 0; r < kRound; r++) u[r] = j + r < deg ? a.in_col[beg + j + r] : -1;
+            for (int q = 0; q < VW; q++) {
+              if (grp == q && todo) at[h] = __ffsll((unsigned long long)todo) - 1;
+              todo &= todo - 1;
+            }
+            const int from = at[h] < 0 ? 0 : at[h];
+            beg[h] = __shfl(vbeg, from);
+            const int len = __shfl(vdeg, from);
+            deg[h] = at[h] < 0 ? 0 : len;
+            v[h] = (int32_t)v0 + from;
+            best[h] = make_int4(kInf, kInf, kInf, kInf);
+          }
+          for (int j = 0; j < max(deg[0], deg[1]); j += kRound) {
+            int32_t u[2][kRound], wt[2][kRound];
+            unsigned m[2][kRound];
+            int4 du[2][kRound];
 #pragma unroll
-            for (int r = 0; r < kRound; r++) wt[r] = j + r < deg ? a.in_w[beg + j + r] : 0;
-            gather(u, wt, best);
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+              for (int r = 0; r < kRound; r++) {
+                const int k = beg[h] + (j + r < deg[h] ? j + r : 0);
+                u[h][r] = a.in_col[k];
+                wt[h][r] = a.in_w[k];
+              }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+              for (int r = 0; r < kRound; r++) {
+                const Mask x = act_in[u[h][r]];
+                m[h][r] = j + r < deg[h] ? bits4(x) : 0u;
+              }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+              for (int r = 0; r < kRound; r++) du[h][r] = *quad(m[h][r] ? u[h][r] : v[h]);
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+              for (int r = 0; r < kRound; r++) {
+                const int4 d = masked(du[h][r], m[h][r]);
+                int4& b = best[h];
+                b.x = min(b.x, w_plus(d.x, wt[h][r])), b.y = min(b.y, w_plus(d.y, wt[h][r]));
+                b.z = min(b.z, w_plus(d.z, wt[h][r])), b.w = min(b.w, w_plus(d.w, wt[h][r]));
+              }
           }
-          unsigned x = 0;
-          if (min(min(best.x, best.y), min(best.z, best.w)) != kInf) {
-            int4 dv = *quad(v);
-            x = take(best, dv);
-            if (x) *quad(v) = dv;
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            unsigned x = 0;
+            if (min(min(best[h].x, best[h].y), min(best[h].z, best[h].w)) != kInf) {
+              int4 dv = *quad(v[h]);
+              x = take(best[h], dv);
+              if (x) *quad(v[h]) = dv;
+            }
+            const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
+            if (sub == 0 && imp) act_out[v[h]] = (Mask)imp;  // v's own slot (heavy vertices are not here)
+            s_q.append(sub == 0 && imp != 0, v[h], qlen_out, q_out);
           }
-          const uint64_t imp = group_or<VL>((uint64_t)x << (4 * sub));
-          if (sub == 0 && imp) act_out[v] = (Mask)imp;  // v's own slot (heavy vertices are not here)
-          s_q.append(sub == 0 && imp != 0, v, qlen_out, q_out);
         }
       }
     } else {
