@@ -350,18 +350,22 @@ __global__ void __launch_bounds__(kBlock) w_step_kernel(WArgs a, int k) {
       // vertices have a tail that improved is found first, a thread each, unless
       // most will have one: most of a step's vertices often have none, and a
       // group waits on three accesses for each (1000 x 1000 with shortcuts, 33
-      // sources, all steps pulled: 16.3 -> 10.6 ms, by the rule 10.4 -> 9.8; RMAT-20
-      // of degree 8, 64 sources, pulled 16.3 -> 11.7; random graph of 1,000,000,
-      // degree 12, by the rule 16.4 -> 16.7).  A group takes two vertices at a
-      // time, without branches, so that both chains are in flight (2048 x 2048, 64
-      // sources, pulled 3.24 -> 2.86 s, by the rule 3.13 -> 2.76; the random graph
-      // 16.7 -> 15.8 ms, RMAT-20 18.2 -> 18.0).  An edge past a list's end reads the
-      // list's first one; a group that has a first vertex and no second reads the
-      // edge at the lists' start of the wave's first vertex, not past the first's.
+      // sources, all steps pulled: 16.3 -> 10.8 ms, by the rule 10.4 -> 10.1;
+      // RMAT-20 of degree 8, 64 sources, pulled 16.3 -> 11.4).  A wave looks at 64
+      // vertices, or as many as give every wave some (random graph of 65,536,
+      // degree 8, 64 sources: 2.3 ms by 64 vertices, 1.3 so).
+      // A group takes two vertices at a time, without branches, so that both
+      // chains are in flight (2048 x 2048, 64 sources, pulled 3.24 -> 2.82 s, by the
+      // rule 3.13 -> 2.72; random graph of 1,000,000, degree 12, 16.7 -> 15.8 ms;
+      // RMAT-20 18.2 -> 18.0).  An edge past a list's end reads the list's first
+      // one; a group that has a first vertex and no second reads the edge at the
+      // lists' start of the wave's first vertex, which is not past the first's.
       const bool dense = (int64_t)qn * 4 >= a.n;
-      for (int64_t v0 = wave * kWave; v0 < a.n; v0 += nwaves * kWave) {  // wave-uniform
+      const int64_t each = (a.n + nwaves - 1) / nwaves;
+      const int span = (int)min((int64_t)kWave, (each + 2 * VW - 1) / (2 * VW) * (2 * VW));
+      for (int64_t v0 = wave * span; v0 < a.n; v0 += nwaves * span) {  // wave-uniform
         int vbeg = 0, vdeg = 0;
-        if (v0 + lane < a.n) {
+        if (lane < span && v0 + lane < a.n) {
           vbeg = a.in_row_ptr[v0 + lane];
           vdeg = a.in_row_ptr[v0 + lane + 1] - vbeg;
           if (vdeg >= a.heavy) vdeg = 0;
