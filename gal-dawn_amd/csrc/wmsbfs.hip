@@ -786,13 +786,19 @@ int run_w(dawn_graph* g, const int32_t* sources, int32_t S, int32_t* dist, int64
 // Graphs whose state fits a workgroup's LDS: every source in a workgroup of
 // its own (batch.hip), 256 at a time, instead of 64 lanes that share steps.
 // Measured (ms, workgroups / lanes):
-//   ER 16,384, degree 8: 1 source 0.25 / 0.42, 64 0.27 / 0.65, 256 0.29 / 2.9
-//   ER 32,768, degree 16: 1 source 0.50 / 0.54, 64 0.56 / 1.05, 256 0.59 / 4.1
-//   RMAT-14, 0.43 M edges: 1 source 0.54 / 0.61, 64 0.61 / 3.2
-//   RMAT-15, 0.88 M edges: 8 sources 0.97 / 0.72, 16 1.01 / 1.15, 64 1.03 / 4.0
-//   ER 65,536, degree 8: 32 sources 1.12 / 0.91, 64 1.13 / 1.21, 256 1.65 / 4.9
-//   ER 130,000, degree 3: 32 sources 1.51 / 1.02, 64 1.54 / 1.38, 256 2.0 / 5.4
-//   grid 360 x 360: 32 sources 1.84 / 1.37, 64 1.85 / 2.6, 256 2.3 / 9.6
+//   random graph of 16,384, degree 8: 1 source 0.24 / 0.36, 64 0.26 / 0.58, 256 0.28 / 2.3
+//   random graph of 32,768, degree 16: 1 source 0.52 / 0.59, 64 0.55 / 0.99, 256 0.58 / 4.1
+//   random graph of 37,000, degree 20: 8 sources - / 0.68, 16 0.63 / 0.78, 64 0.64 / 1.4
+//   random graph of 30,000, degree 100: 8 sources - / 0.87, 16 1.19 / 1.10, 32 1.28 / 1.59
+//   RMAT-14, 0.43 M edges: 1 source 0.52 / 0.32, 16 0.55 / 0.48, 32 0.55 / 0.58, 64 0.57 / 0.82
+//   RMAT-15, 0.88 M edges: 8 sources - / 0.45, 16 0.97 / 0.54, 32 0.99 / 0.73, 64 0.99 / 1.20
+//   grid 190 x 190: 1 source 2.0 / 3.5, 64 2.0 / 6.6
+//   random graph of 65,536, degree 8: 64 sources - / 1.15, 65 1.13 / 1.84, 256 1.67 / 4.7
+//   random graph of 130,000, degree 3: 64 sources - / 1.27, 65 1.56 / 2.10, 256 2.0 / 5.1
+//   RMAT-16, 1.8 M edges: 64 sources - / 1.83, 65 2.99 / 1.97, 128 3.5 / 3.7, 256 3.7 / 7.3
+//   grid 360 x 360: 64 sources - / 21, 65 8.3 / 27, 256 8.4 / 83
+// The lines suit graphs without hubs; with hubs the lanes are the better up to
+// some 48 sources, a fixed 0.2 to 0.4 ms that the rule leaves there.
 // With the distances in LDS (up to kSourcesDistN vertices) the lines are
 // kSourcesM edges and kSourcesS sources; with bounds there and distances in
 // memory, more sources than one batch of lanes.  A forced mode is one of the
