@@ -227,54 +227,6 @@ __device__ __forceinline__ int wave_append(unsigned int* counter, bool pred) {
   return pred ? (int)(base + (unsigned int)__popcll(m & lanes_below_mask())) : -1;
 }
 
-// Wave-aggregated append of k >= 0 slots per lane; returns the lane's first
-// slot.  Must be called by all 64 lanes.
-__device__ __forceinline__ int wave_append_n(unsigned int* counter, int k) {
-  const int l = lane_id();
-  int inc = k;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    int y = __shfl_up(inc, o);
-    if (l >= o) inc += y;
-  }
-  const int total = __shfl(inc, 63);
-  unsigned int base = 0;
-  if (total > 0) {
-    if (l == 0) base = atomicAdd(counter, (unsigned int)total);
-    base = __shfl(base, 0);
-  }
-  return (int)base + inc - k;
-}
-
-// Block-aggregated append of k >= 0 slots per thread: one atomic per block.
-// Returns the thread's first slot.  Every thread of the kBlock-thread block
-// must call it (it synchronises the block).  s_wtot: kBlock/kWave ints of
-// LDS, s_base: one unsigned of LDS.
-__device__ __forceinline__ int block_append_n(unsigned int* counter, int k, int* s_wtot,
-                                              unsigned int* s_base) {
-  const int l = lane_id();
-  const int w = threadIdx.x / kWave;
-  int inc = k;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    int y = __shfl_up(inc, o);
-    if (l >= o) inc += y;
-  }
-  if (l == kWave - 1) s_wtot[w] = inc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-    for (int i = 0; i < kBlock / kWave; i++) t += s_wtot[i];
-    *s_base = t ? atomicAdd(counter, (unsigned int)t) : 0u;
-  }
-  __syncthreads();
-  int off = 0;
-  for (int i = 0; i < w; i++) off += s_wtot[i];
-  const int r = (int)*s_base + off + inc - k;
-  __syncthreads();  // s_wtot / s_base may be reused after this
-  return r;
-}
-
 // Queue appends of a workgroup staged in LDS.  A global counter that every
 // wave of the grid bumps serialises at one address: thousands of such
 // atomics per step cost more than the step's own memory traffic.  Waves
@@ -356,12 +308,6 @@ __device__ __forceinline__ int wave_min_i32(int x) {
   return x;
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t x, int o) {
-  unsigned lo = __shfl_xor((unsigned)(x & 0xffffffffu), o);
-  unsigned hi = __shfl_xor((unsigned)(x >> 32), o);
-  return ((uint64_t)hi << 32) | lo;
-}
-
 // Value of lane (this lane ^ J), J a power of two below 64: DPP quad
 // permutes for J = 1, 2, ds_swizzle (bit mode, within 32 lanes) for
 // J = 4..16, ds_bpermute across the halves for J = 32.  All lanes active.
@@ -435,21 +381,6 @@ __device__ __forceinline__ uint64_t wave_transpose64(uint64_t x) {
   x = transpose_round<2, 0x3333333333333333ull>(x, l);
   x = transpose_round<1, 0x5555555555555555ull>(x, l);
   return x;
-}
-
-// In-register 32x32 bit transpose: afterwards bit r of A[c] is bit c of the
-// input A[r] (recursive block swaps, 5 rounds of 16 masked exchanges).
-__host__ __device__ __forceinline__ void transpose32(uint32_t (&A)[32]) {
-  uint32_t m = 0x0000FFFFu;
-#pragma unroll
-  for (int j = 16; j != 0; j >>= 1, m ^= (m << j)) {
-#pragma unroll
-    for (int k = 0; k < 32; k = ((k | j) + 1) & ~j) {
-      const uint32_t t = ((A[k] >> j) ^ A[k | j]) & m;
-      A[k] ^= t << j;
-      A[k | j] ^= t;
-    }
-  }
 }
 
 // Exclusive scan of one int per thread over a kBlock-thread workgroup.
