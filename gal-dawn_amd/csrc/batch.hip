@@ -11,7 +11,9 @@
 // Unweighted task: all sources of one graph (or a share of them) as lanes of
 // one field per vertex, level-synchronous BOVM with the fields in LDS, pushed
 // and pulled (run_lds).  Graphs too large for a workgroup's LDS (more than 1.2
-// million vertices) keep words of up to 64 lanes in memory, sparse BOVM:
+// million vertices), and those whose sources would be several tasks in LDS and
+// are done sooner as one where tasks wait for a CU (memory_faster: small graphs
+// and graphs of many levels), keep words of up to 64 lanes in memory, sparse BOVM:
 //   Q_l = [(v, lanes that reached v at level l)]
 //   expand: for (u, f) in Q_l, w in N(u): nv = f & ~seen[w]; if nv,
 //           atomicOr(next[w], nv); the first writer appends w to `touched`
@@ -89,15 +91,11 @@ struct BatchArgs {
 
 namespace {
 
-// Threads per workgroup of the persistent kernel: a task (one graph's
-// traversal) runs inside one workgroup, so the largest graphs' tasks are
-// the critical path of a batch, and wider workgroups shorten it (measured
-// on 512 graphs of 1k-130k vertices: 1024 threads 30 ms unweighted / 85 ms
-// weighted; 256 threads, two or eight per CU: 74 ms / 183-203 ms).  One
-// such workgroup is resident per CU (the kernel's scalar registers allow
-// seven waves per SIMD); forcing two per CU (eight waves, scalar registers
-// spilled) made the batches slower (18.7 -> 24-27 ms unweighted, 46 -> 51 ms
-// weighted): twice the concurrent tasks' state no longer fits the caches.
+// Threads per workgroup of the persistent kernels.  A task (one graph's
+// traversal) runs inside one workgroup, and the LDS that holds its state is a
+// CU's whole, so one workgroup is resident per CU and its own waves are all
+// that hides a step's latency: as many as a workgroup can have, 16, four per
+// SIMD, which leaves each thread 128 registers.
 constexpr int kBatchBlock = 1024;
 
 template <int BS>

@@ -1874,7 +1874,9 @@ int run_msbfs_slot(dawn_graph* g, MsWorkspace* ws, hipStream_t s, const int32_t*
   // The chunk: the last batch's levels, the step that finds the frontier empty
   // and one to spare, in steps of two (each length is captured once), kChunk
   // before a depth is known.  A step past the end is seven launches that
-  // return at once, 15 us (RMAT-17, 64 sources: 0.67 ms, 0.48 without).
+  // return at once, 15 us (RMAT-17, 64 sources: 0.67 ms, 0.48 without).  A new
+  // length costs the call that meets it 0.13-0.18 ms (RMAT-17, second call on a
+  // graph, 64 sources 0.68 ms, later ones 0.50; 0.71 by a chunk of kChunk).
   constexpr int kChunk = chunk_steps(W);
   auto get_graph = [&](int want_edges, int chunk, hipGraphExec_t* exec) -> int {
     const auto key = std::make_tuple(W, (int)policy, want_edges, (const void*)p.mlp, chunk);

@@ -103,8 +103,9 @@ __host__ __device__ inline void sched_features(const LevelCounters& c, int step,
   x[7] = log2p1((double)p.max_degree);
 }
 
-// One-wave MLP inference (8 -> 32 -> 32 -> 3, ReLU); returns argmin of the
-// predicted log step times over the allowed modes.  Called by all 64 lanes.
+// MLP inference (8 -> 32 -> 32 -> 3, ReLU) by a workgroup's first 32 threads;
+// returns argmin of the predicted log step times over the allowed modes.  Called
+// by all threads of the workgroup (it synchronises them).
 __device__ inline int sched_mlp_mode(const float* x, const SchedParams& p) {
   __shared__ float xin[8], h1[32], h2[32], out[3];
   const int t = threadIdx.x;
