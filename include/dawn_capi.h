@@ -216,13 +216,13 @@ int dawn_bfs_noalloc(const dawn_graph* g, int32_t source, int32_t* dist,
  * batch.  On graphs whose state fits a workgroup's LDS (up to 80,000 vertices
  * and 2 million edges unweighted, 134,000 vertices weighted) a call that is
  * faster so runs a workgroup per source instead (fixed and learned policies,
- * the batched engine's knobs as the library chose them); its counts are those of the batches, its steps
- * count as push, its frontier edges per source.
+ * the batched engine's knobs as the library chose them); its counts are those
+ * of the batches, its steps count as push, its frontier edges per source.
  * sources are taken modulo n (reference: msource[i] % rows, mssp.cpp:15);
  * isolated sources are skipped (dist row left INF except dist[src]=0, sum 0).
  * dist: S*n int32 row-major (host or device), or NULL to keep only sums
- * (the rows are still computed, each batch's into a device scratch buffer,
- * as the reference computes every source's distance array and discards it).
+ * (every distance is still computed, in device memory of the library's, as
+ * the reference computes every source's distance array and discards it).
  * sums: S int64 sums of distances over reached vertices, or NULL.
  * Reference: DAWN::MSSP_GPU::run / run_Weighted (src/algorithm/gpu/mssp.cu:9-102),
  * DAWN::MSSP_CPU::run (src/algorithm/cpu/mssp.cpp:9-32). */
